@@ -2289,6 +2289,7 @@ extern "C" int mcx_batch_create(mcx_batch** out, int nvol, const int* dims_xyz, 
   if (elem != MCX_ELEM_SHORT2 && elem != MCX_ELEM_F32) return MCX_ERR_ARG;
   std::vector<VolDesc> vols(nvol);
   std::vector<BatchVol> bvol(nvol);
+  std::vector<int64_t> blk_begin(nvol + 1);
   std::vector<Column> cols;
   int64_t tb = 0, cubes = 0, voxels = 0, blocks = 0, gblocks = 0;
   int maxX = 1;
@@ -2299,10 +2300,12 @@ extern "C" int mcx_batch_create(mcx_batch** out, int nvol, const int* dims_xyz, 
     if (!size_ok(X, Y, Z)) return MCX_ERR_UNSUPPORTED;
     vols[b] = make_vol(d_vols[b], X, Y, Z, h[b], nullptr, tb);
     const int64_t nv = (int64_t)X * Y * Z;
-    bvol[b] = BatchVol{X, Y, Z, h[b], voxels, blocks, gblocks, FastDiv((uint32_t)X),
-                       FastDiv((uint32_t)Y)};
+    const int rx = (X + 31) / 32, ry = (Y + 7) / 8, rz = (Z + 3) / 4;  // 32 x 8 x 4 voxels each
+    bvol[b] = BatchVol{X, Y, Z, h[b], voxels, blocks, gblocks, FastDiv((uint32_t)rx),
+                       FastDiv((uint32_t)ry)};
+    blk_begin[b] = blocks;
     voxels += nv;
-    blocks += (nv + 255) / 256;
+    blocks += (int64_t)rx * ry * rz;
     gblocks += ((int64_t)X * Y + kGatherSpan - 1) / kGatherSpan * Z;
     const int64_t nt = tiles_of(X, Y, Z);
     if (nt > 0) {
@@ -2331,7 +2334,8 @@ extern "C" int mcx_batch_create(mcx_batch** out, int nvol, const int* dims_xyz, 
   p->ncols = (int64_t)cols.size();
   p->cubes = cubes;
   p->voxels = voxels;
-  p->blocks = blocks;
+  p->blocks = blk_begin[nvol] = blocks;
+  p->blk_begin = std::move(blk_begin);
   p->gather_blocks = gblocks;
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&p->d_vols), sizeof(VolDesc) * nvol);
   if (e == hipSuccess)

@@ -7,11 +7,12 @@
 //   _cu_voxel_volumetric_integration       :534-549
 // The reference gives each thread one (y, z) row and walks x inside the
 // thread, so a wave strides the volume by 4*X bytes (uncoalesced), and it
-// sweeps the whole volume once per frame.  Here a thread owns one voxel, a
-// workgroup owns 256 consecutive voxels of a z-slab (x fastest, coalesced
-// 1 KiB per workgroup), and K frames are fused per sweep: the voxel is read
-// once, updated for every frame in order in registers, and written once, so a
-// sweep costs 8 B/voxel plus the depth reads instead of 8 B/voxel/frame.
+// sweeps the whole volume once per frame.  Here a wave owns a brick of
+// 8 x 8 x 4 voxels (a lane one x, y and four z) and a workgroup four bricks in
+// a row of x (32 consecutive voxels: whole 128-byte lines), and K frames are
+// fused per sweep: the voxel is read once, updated for every frame in order
+// in registers, and written once, so a sweep costs 8 B/voxel plus the depth
+// reads instead of 8 B/voxel/frame.
 //
 // Per voxel and frame (bit-for-bit the oracle's update_voxel):
 //   p = ((i + 0.5) h) per axis; q = R^T (p - t)          (camera-to-world pose)
@@ -23,9 +24,10 @@
 //   and max_t of the volume; one truncation gives clamp(sdf / trunc, -1, 1));
 //   running average with integer weights capped at max_w; tsdf stored as
 //   trunc(t * 32767) clamped to +-32767.
-// A workgroup first marks the frames that none of its voxels can observe
-// (frame_skip_flags) and passes over them; the per-voxel arithmetic and its
-// results are unchanged.
+// A wave first tests eight frames at a time against its brick (test_box) and
+// passes over those that none of its voxels can observe: out of the frame's
+// view, or behind everything the frame measured there.  The per-voxel
+// arithmetic and its results are those of every voxel taken by itself.
 #include <float.h>
 #include <hip/hip_runtime.h>
 
@@ -45,17 +47,6 @@ __global__ __launch_bounds__(256) void init_kernel(uint32_t* vol, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) vol[i] = v;
 }
 
-// Per-pixel ray-length factor sqrt(((u-cx)/fx)^2 + ((v-cy)/fy)^2 + 1)
-// (d_voxel_volumetric_depth_scaling, :416-425), shared by all frames.
-__global__ __launch_bounds__(256) void rayfac_kernel(float* out, int W, int H, float fx, float fy,
-                                                      float cx, float cy) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= W * H) return;
-  const int u = i % W, v = i / W;
-  const float ax = ((float)u - cx) / fx, ay = ((float)v - cy) / fy;
-  out[i] = sqrtf(__fmaf_rn(ay, ay, ax * ax) + 1.0f);
-}
-
 struct IntegrateParams {
   uint32_t* vol;
   int X, Y, Z;
@@ -66,18 +57,83 @@ struct IntegrateParams {
   const float* poses;      // [K][12] device
   const void* depth;       // [K][H][W] device, uint16 or float
   const float* rayfac;     // [H][W]
+  const float2* tiles;     // [tiled][TY][TX]: a tile's (largest, smallest) ray distance
   float depth_scale;
   int W, H, K;
-  FastDiv divX, divY;
-  int step_x, step_y, step_z;  // 256 voxels as x, y, z steps (step_x < X, step_y < Y)
-  int64_t first_block;   // workgroup index of this launch's blockIdx.x 0
+  int TX, TY;              // tiles of kTile x kTile pixels
+  int tiled;               // frames [0, tiled) have a tile table
+  FastDiv divX, divY;      // workgroups along x and y of the volume
+  int64_t first_block;     // workgroup index of this launch's blockIdx.x 0
 };
 
-// Depth value and ray factor of pixel pix (>= 0) of frame k, as buffer loads
-// from uniform per-frame bases with 32-bit offsets (no 64-bit address
-// arithmetic per voxel and frame).  Word 3 of a raw 32-bit-element buffer
-// resource on gfx950.
+// Ray-length factor sqrt(((u-cx)/fx)^2 + ((v-cy)/fy)^2 + 1) of a pixel
+// (d_voxel_volumetric_depth_scaling, :416-425), shared by all frames.
+__device__ __forceinline__ float ray_factor(int u, int v, float fx, float fy, float cx, float cy) {
+  const float ax = ((float)u - cx) / fx, ay = ((float)v - cy) / fy;
+  return sqrtf(__fmaf_rn(ay, ay, ax * ax) + 1.0f);
+}
+
+// Largest and smallest measured ray distance (depth * scale * factor, the
+// voxels' own operations; pixels without a measurement do not count) of every
+// kTile x kTile pixels of the window [0, W-2) x [0, H-2) that voxels can
+// observe: (0, inf) where a tile holds none.  A wave takes eight tiles of a
+// tile row, a lane eight pixels of one image row, for every gridDim.z-th
+// frame; the ray factors are computed once per lane and written for the
+// integration by the waves of blockIdx.z = 0.  Tiles of 8 pixels: an
+// 8 x 8 x 4 brick of a 512^3 scan covers about 14 pixels, so 3 x 3 tiles.
+constexpr int kTile = 8;
+template <typename DT>
+__global__ __launch_bounds__(64) void frame_tiles_kernel(const DT* __restrict__ depth, float scale,
+                                                         int W, int H, int frames, float fx,
+                                                         float fy, float cx, float cy,
+                                                         float* rayfac, int TX, int TY,
+                                                         int first_ty, int vec, float2* tiles) {
+  const int lane = threadIdx.x;
+  const int tx = blockIdx.x * 8 + (lane & 7), ty = first_ty + blockIdx.y;
+  const int u0 = tx * kTile, v = ty * kTile + (lane >> 3);
+  float rf[kTile];
+#pragma unroll
+  for (int i = 0; i < kTile; ++i) {
+    rf[i] = ray_factor(u0 + i, v, fx, fy, cx, cy);
+    if (blockIdx.z == 0 && v < H && u0 + i < W) rayfac[(int64_t)v * W + u0 + i] = rf[i];
+  }
+  for (int k = blockIdx.z; k < frames; k += gridDim.z) {
+    const DT* row = depth + (int64_t)k * W * H + (int64_t)v * W + u0;
+    DT d[kTile];
+    if (vec) {  // W a multiple of 8 and 16-byte aligned frames: whole 16-byte words
+      constexpr int NQ = kTile * (int)sizeof(DT) / 16;
+      uint4 q[NQ] = {};
+      if (v < H && u0 < W)
+        for (int i = 0; i < NQ; ++i) q[i] = reinterpret_cast<const uint4*>(row)[i];
+      __builtin_memcpy(d, q, sizeof(d));
+    } else {
+#pragma unroll
+      for (int i = 0; i < kTile; ++i) d[i] = v < H && u0 + i < W ? row[i] : (DT)0;
+    }
+    float hi = 0.0f, lo = INFINITY;
+#pragma unroll
+    for (int i = 0; i < kTile; ++i) {
+      const float z = v < H - 2 && u0 + i < W - 2 ? ((float)d[i] * scale) * rf[i] : 0.0f;
+      if (z > FLT_MIN) {
+        hi = fmaxf(hi, z);
+        lo = fminf(lo, z);
+      }
+    }
+#pragma unroll
+    for (int o = 8; o < 64; o <<= 1) {
+      hi = fmaxf(hi, __shfl_xor(hi, o));
+      lo = fminf(lo, __shfl_xor(lo, o));
+    }
+    if (lane < 8 && tx < TX) tiles[((int64_t)k * TY + ty) * TX + tx] = make_float2(hi, lo);
+  }
+}
+
+// Depth value and ray factor of pixel pix of frame k, as buffer loads from
+// uniform per-frame bases with 32-bit offsets (no 64-bit address arithmetic
+// per voxel and frame); a pixel of kNoPixel lies past the buffer and reads 0,
+// no measurement.  Word 3 of a raw 32-bit-element buffer resource on gfx950.
 constexpr int kRawBufferWord3 = 0x00020000;
+constexpr uint32_t kNoPixel = 0x20000000u;  // times 4 bytes: past every frame of < 2^31 bytes
 template <typename DT>
 __device__ __forceinline__ float frame_depth(const IntegrateParams& P, int k, uint32_t pix) {
   const int64_t wh = (int64_t)P.W * P.H;
@@ -95,119 +151,241 @@ __device__ __forceinline__ float frame_rayfac(const IntegrateParams& P, uint32_t
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, pix * 4u, 0, 0));
 }
 
-// Frames that no voxel of a workgroup can observe, as bits of s_skip (one per
-// frame).  The workgroup's voxels, linear indices [i0, i1] of one X x Y x Z
-// volume, lie in a box of voxel centres; frame k is skipped when the whole
-// box is behind its camera, or in front of it (every corner deeper than 1 cm)
-// and projecting past one edge of the pixel window: the image of a convex box
-// in front of the camera is the convex hull of its corners' images.  Eight
-// lanes take a frame, one corner each, with the voxels' own fp32 operations
-// (a corner is a voxel centre) up to the quotients, which come from the
-// hardware reciprocal (error within 2e-7 |u - cx| plus an ulp).  A voxel's
-// fp32 q differs from the exact one by at most d = 4e-7 * (|dx| + |dy| +
-// |dz|) per component (the subtraction and the fma chain, |R| <= 1), so its u
-// differs from the exact projection by at most (fx d / qz_min) (1 + |u -
-// cx|_max / fx), likewise v; the tests use four times that plus one pixel as
-// the margin ("behind": every corner below -max(1e-4 m, 4 d)); the pixel
-// covers the reciprocal's error wherever a test is close (|u|, |v| < 2^16:
-// under 0.02 pixel), so every voxel of a skipped frame would have taken its
-// q.z or window skip.  Called by every thread of the workgroup (barriers
-// inside).
-__device__ void frame_skip_flags(const float* s_pose, int K, const IntegrateParams& P,
-                                 int64_t i0, int64_t i1, uint32_t* s_skip) {
-  const int64_t XY = (int64_t)P.X * P.Y;
-  const int64_t z0 = i0 / XY, z1 = i1 / XY;
-  int64_t x0 = 0, x1 = P.X - 1, y0 = 0, y1 = P.Y - 1;
-  if (z0 == z1) {
-    const int64_t r0 = i0 - z0 * XY, r1 = i1 - z1 * XY;
-    y0 = r0 / P.X;
-    y1 = r1 / P.X;
-    if (y0 == y1) {
-      x0 = r0 - y0 * P.X;
-      x1 = r1 - y1 * P.X;
-    }
-  }
-  for (int w = threadIdx.x; w < (K + 31) / 32; w += blockDim.x) s_skip[w] = 0;
-  __syncthreads();
-  const int lane = threadIdx.x & 63, c = lane & 7;
-  const float px = ((float)((c & 1) ? x1 : x0) + 0.5f) * P.h;
-  const float py = ((float)((c & 2) ? y1 : y0) + 0.5f) * P.h;
-  const float pz = ((float)((c & 4) ? z1 : z0) + 0.5f) * P.h;
-  const int nf = (int)(blockDim.x >> 3);  // frames per round
-  for (int kb = (int)(threadIdx.x >> 6) * 8; kb < K; kb += nf) {
-    const int k = kb + (lane >> 3);
-    float qz = 0.0f, u = 0.0f, v = 0.0f, dist = 0.0f;
-    if (k < K) {
-      const float* R = s_pose + 12 * k;
-      const float dx = px - R[9], dy = py - R[10], dz = pz - R[11];
-      dist = fabsf(dx) + fabsf(dy) + fabsf(dz);
-      const float qx = __fmaf_rn(R[6], dz, __fmaf_rn(R[3], dy, R[0] * dx));
-      const float qy = __fmaf_rn(R[7], dz, __fmaf_rn(R[4], dy, R[1] * dx));
-      qz = __fmaf_rn(R[8], dz, __fmaf_rn(R[5], dy, R[2] * dx));
-      const float rz = __builtin_amdgcn_rcpf(qz);
-      u = __fmaf_rn(P.fx, qx * rz, P.cx);
-      v = __fmaf_rn(P.fy, qy * rz, P.cy);
-    }
-    float qzmin = qz, qzmax = qz, umin = u, umax = u, vmin = v, vmax = v, dmax = dist;
-#pragma unroll
-    for (int o = 1; o < 8; o <<= 1) {
-      dmax = fmaxf(dmax, __shfl_xor(dmax, o));
-      qzmin = fminf(qzmin, __shfl_xor(qzmin, o));
-      qzmax = fmaxf(qzmax, __shfl_xor(qzmax, o));
-      umin = fminf(umin, __shfl_xor(umin, o));
-      umax = fmaxf(umax, __shfl_xor(umax, o));
-      vmin = fminf(vmin, __shfl_xor(vmin, o));
-      vmax = fmaxf(vmax, __shfl_xor(vmax, o));
-    }
-    bool skip = false;
-    if (k < K) {
-      const float d = 4e-7f * dmax;  // bound on a voxel's fp32 error in q
-      if (qzmax < -fmaxf(1e-4f, 4.0f * d)) {
-        skip = true;
-      } else if (qzmin > 0.01f) {
-        // margins from reciprocals (relative error ~1e-7 in a bound taken
-        // four times over)
-        const float rq = __builtin_amdgcn_rcpf(qzmin);
-        const float au = fmaxf(fabsf(umin - P.cx), fabsf(umax - P.cx)) * __builtin_amdgcn_rcpf(P.fx);
-        const float av = fmaxf(fabsf(vmin - P.cy), fabsf(vmax - P.cy)) * __builtin_amdgcn_rcpf(P.fy);
-        const float tu = 1.0f + 4.0f * (P.fx * d * rq) * (1.0f + au);
-        const float tv = 1.0f + 4.0f * (P.fy * d * rq) * (1.0f + av);
-        // a voxel is observed only at rint(u) in [0, W - 2), rint(v) in [0, H - 2)
-        skip = umax < -0.5f - tu || umin > (float)P.W - 2.5f + tu || vmax < -0.5f - tv ||
-               vmin > (float)P.H - 2.5f + tv;
-      }
-    }
-    const uint64_t m = __ballot(skip && c == 0);  // bit 8 j: frame kb + j
-    if (lane == 0 && m) {
-      uint32_t bits = 0;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) bits |= (uint32_t)((m >> (8 * j)) & 1u) << j;
-      atomicOr(&s_skip[kb >> 5], bits << (kb & 31));
-    }
-  }
-  __syncthreads();
+// ---- bricks ---------------------------------------------------------------
+// A wave's 8 x 8 x NZ voxels (NZ = 4, or 1 in the backward of small volumes):
+// compact, so that its image is a few tiles (256 voxels in a row of x, the
+// former split, cover a line of some 300 pixels) and one test serves 256
+// voxels; a lane's NZ voxels share x, y and so two of the three products of
+// each row of R^T (p - t).  VALU-issue bound before and after: the observations
+// that are left out are the gain.  640x480 frames into 512^3: one frame a call
+// 405 -> 127 us, 300 frames 84.1 -> 19.4 ms; 64 volumes of 64-192 a side with
+// 16 frames each (a far wall: little is hidden) 5.2 -> 4.5 ms.
+constexpr int kBrick = 8, kBrickZ = 4;
+constexpr int kRegionX = 4 * kBrick;  // a workgroup's four bricks lie side by side in x
+
+// Reductions over the eight lanes of a frame (all 64 lanes active).
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141;
+__device__ __forceinline__ float min8(float v) {
+  v = fminf(v, dpp_f32<kDppXor1>(v));
+  v = fminf(v, dpp_f32<kDppXor2>(v));
+  return fminf(v, dpp_f32<kDppHalfMirror>(v));
+}
+__device__ __forceinline__ float max8(float v) {
+  v = fmaxf(v, dpp_f32<kDppXor1>(v));
+  v = fmaxf(v, dpp_f32<kDppXor2>(v));
+  return fmaxf(v, dpp_f32<kDppHalfMirror>(v));
 }
 
-// f(k) for every frame k < K not marked in s_skip, in order (a uniform
-// 32-frame mask at a time: one LDS read per 32 frames).
-template <typename F>
-__device__ __forceinline__ void for_active_frames(const uint32_t* s_skip, int K, F&& f) {
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    uint32_t act = ~s_skip[k0 >> 5];
-    if (K - k0 < 32) act &= (1u << (K - k0)) - 1u;
-    act = __builtin_amdgcn_readfirstlane(act);
+// Whether no voxel of a box of voxel centres can observe a frame.  Eight
+// lanes take a frame, lane c one corner (bit 0 of c: the far x, bit 1: y, bit
+// 2: z), with the voxels' own fp32 operations (a corner is a voxel centre) up
+// to the quotients, which come from the hardware reciprocal (error within
+// 2e-7 |u - cx| plus an ulp).
+//   Out of view: the whole box is behind the camera, or in front of it (every
+// corner deeper than 1 cm) and projecting past one edge of the pixel window:
+// the image of a convex box in front of the camera is the convex hull of its
+// corners' images.
+//   Behind what was measured: with the box in front of the camera, its pixels
+// lie in the rectangle of its corners' images; the largest ray distance z
+// measured there (the tiles that meet the rectangle) and a lower bound q of
+// the voxels' distances give sdf <= z - q (the subtraction rounds
+// monotonically), and nothing is updated where that is below -trunc_neg, or
+// where nothing was measured at all.  q is the least corner coordinate along
+// the direction n of the box's centre (|n| <= 1, so |q(p)| >= q(p) . n, which
+// is linear in p).
+// Margins: a voxel's fp32 q differs from the exact one by at most
+// d = 4e-7 * (|dx| + |dy| + |dz|) per component (the subtraction and the fma
+// chain, |R| <= 1), so its u differs from the exact projection by at most
+// (fx d / qz_min) (1 + |u - cx|_max / fx), likewise v; the tests use four
+// times that plus one pixel as the margin ("behind": every corner below
+// -max(1e-4 m, 4 d)); the pixel covers the reciprocal's error wherever a test
+// is close (|u|, |v| < 2^16: under 0.02 pixel) and the rounding to the
+// nearest pixel.  Distances differ by less than 1e-6 (|dx| + |dy| + |dz|),
+// taken four times over.  So every voxel of a skipped frame would have taken
+// its q.z, window, dropout or -trunc_neg skip.
+// Boxes over more than 8 x 8 tiles are not tested against them.
+__device__ bool test_box(const IntegrateParams& P, const float* R, int k, float px, float py,
+                         float pz) {
+  const float dx = px - R[9], dy = py - R[10], dz = pz - R[11];
+  const float dmax = max8(fabsf(dx) + fabsf(dy) + fabsf(dz));
+  const float qx = __fmaf_rn(R[6], dz, __fmaf_rn(R[3], dy, R[0] * dx));
+  const float qy = __fmaf_rn(R[7], dz, __fmaf_rn(R[4], dy, R[1] * dx));
+  const float qz = __fmaf_rn(R[8], dz, __fmaf_rn(R[5], dy, R[2] * dx));
+  const float qzmin = min8(qz), qzmax = max8(qz);
+  const float d = 4e-7f * dmax;  // bound on a voxel's fp32 error in q
+  if (qzmax < -fmaxf(1e-4f, 4.0f * d)) return true;
+  const float rz = __builtin_amdgcn_rcpf(qz);
+  const float u = __fmaf_rn(P.fx, qx * rz, P.cx), v = __fmaf_rn(P.fy, qy * rz, P.cy);
+  float umin = min8(u), umax = max8(u), vmin = min8(v), vmax = max8(v);
+  // the opposite corner sits in lane 7 - c: the sum is twice the centre
+  const float nx = qx + dpp_f32<kDppHalfMirror>(qx), ny = qy + dpp_f32<kDppHalfMirror>(qy),
+              nz = qz + dpp_f32<kDppHalfMirror>(qz);
+  const float rn = __builtin_amdgcn_rsqf(__fmaf_rn(nz, nz, __fmaf_rn(ny, ny, nx * nx)));
+  const float near = min8(__fmaf_rn(qz, nz, __fmaf_rn(qy, ny, qx * nx)) * rn);
+  if (!(qzmin > 0.01f)) return false;
+  // margins from reciprocals (relative error ~1e-7 in a bound taken four
+  // times over)
+  const float rq = __builtin_amdgcn_rcpf(qzmin);
+  const float fx = fabsf(P.fx), fy = fabsf(P.fy);
+  const float au = fmaxf(fabsf(umin - P.cx), fabsf(umax - P.cx)) * __builtin_amdgcn_rcpf(fx);
+  const float av = fmaxf(fabsf(vmin - P.cy), fabsf(vmax - P.cy)) * __builtin_amdgcn_rcpf(fy);
+  const float tu = 1.0f + 4.0f * (fx * d * rq) * (1.0f + au);
+  const float tv = 1.0f + 4.0f * (fy * d * rq) * (1.0f + av);
+  // a voxel is observed only at rint(u) in [0, W - 2), rint(v) in [0, H - 2)
+  if (umax < -0.5f - tu || umin > (float)P.W - 2.5f + tu || vmax < -0.5f - tv ||
+      vmin > (float)P.H - 2.5f + tv)
+    return true;
+  if (k >= P.tiled) return false;
+  umin = fmaxf(umin - tu, 0.0f);
+  vmin = fmaxf(vmin - tv, 0.0f);
+  umax = fminf(umax + tu, (float)(P.W - 3));
+  vmax = fminf(vmax + tv, (float)(P.H - 3));
+  if (!(umin <= umax && vmin <= vmax)) return false;  // (NaN) not decided here
+  const int tx0 = (int)umin / kTile, tx1 = (int)umax / kTile;
+  const int ty0 = (int)vmin / kTile, ty1 = (int)vmax / kTile;
+  if (tx1 - tx0 > 7 || ty1 - ty0 > 7) return false;
+  const int c = threadIdx.x & 7;
+  float far = 0.0f;
+  const float2* T = P.tiles + (int64_t)k * P.TY * P.TX;
+  for (int ty = ty0 + (c >> 2); ty <= ty1; ty += 2)
+    for (int tx = tx0 + (c & 3); tx <= tx1; tx += 4) far = fmaxf(far, T[ty * P.TX + tx].x);
+  far = max8(far);
+  return far == 0.0f || far - (near - 4e-6f * dmax) < -P.trunc_neg;
+}
+
+// A brick: its first voxel and this lane's column of NZ.
+template <int NZ>
+struct Brick {
+  int x0, y0, z0;
+  int nz;          // planes of the volume in it, 1 to NZ
+  bool inside;     // the lane's column lies in the volume
+  float px, py;    // the column's voxel centre
+  __device__ __forceinline__ Brick(const IntegrateParams& P, int bx, int by, int bz)
+      : x0(bx), y0(by), z0(bz) {
+    const int lane = threadIdx.x & 63, x = x0 + (lane & 7), y = y0 + (lane >> 3);
+    nz = min(NZ, P.Z - z0);
+    inside = x < P.X && y < P.Y;
+    px = ((float)x + 0.5f) * P.h;
+    py = ((float)y + 0.5f) * P.h;
+  }
+  __device__ __forceinline__ float pz(const IntegrateParams& P, int j) const {
+    return ((float)(z0 + j) + 0.5f) * P.h;
+  }
+  // index of the lane's first voxel (the next ones are a plane further each)
+  __device__ __forceinline__ int64_t first(const IntegrateParams& P) const {
+    const int lane = threadIdx.x & 63;
+    return ((int64_t)z0 * P.Y + (y0 + (lane >> 3))) * P.X + (x0 + (lane & 7));
+  }
+};
+
+// This wave's brick of workgroup `blk` of a volume; false past the volume's
+// edge (x0 is the same for all lanes).
+__device__ __forceinline__ bool brick_origin(const IntegrateParams& P, uint32_t blk, int zstep,
+                                             int* x0, int* y0, int* z0) {
+  const uint32_t row = P.divX.div(blk), plane = P.divY.div(row);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  *x0 = (int)(blk - row * P.divX.d) * kRegionX + wave * kBrick;
+  *y0 = (int)(row - plane * P.divY.d) * kBrick;
+  *z0 = (int)plane * zstep;
+  return *x0 < P.X;
+}
+
+// One corner of the box of a brick's voxel centres per lane (of eight).
+template <int NZ>
+__device__ __forceinline__ void brick_corner(const IntegrateParams& P, int x0, int y0, int z0,
+                                             float* px, float* py, float* pz) {
+  const int c = threadIdx.x & 7;
+  *px = ((float)((c & 1) ? min(x0 + kBrick - 1, P.X - 1) : x0) + 0.5f) * P.h;
+  *py = ((float)((c & 2) ? min(y0 + kBrick - 1, P.Y - 1) : y0) + 0.5f) * P.h;
+  *pz = ((float)((c & 4) ? min(z0 + NZ - 1, P.Z - 1) : z0) + 0.5f) * P.h;
+}
+
+// f(k) for every frame k that some voxel of the brick may observe, in order:
+// the wave tests eight frames at a time (every lane of the wave calls this).
+template <int NZ, typename F>
+__device__ __forceinline__ void for_active_frames(const IntegrateParams& P, const Brick<NZ>& B,
+                                                  F&& f) {
+  const int lane = threadIdx.x & 63;
+  float px, py, pz;
+  brick_corner<NZ>(P, B.x0, B.y0, B.z0, &px, &py, &pz);
+  for (int kb = 0; kb < P.K; kb += 8) {
+    const int k = min(kb + (lane >> 3), P.K - 1);
+    const bool skip = test_box(P, P.poses + 12 * k, k, px, py, pz);
+    uint64_t act = __ballot(!skip && (lane & 7) == 0 && kb + (lane >> 3) < P.K);
     while (act) {
-      const int k = k0 + __builtin_ctz(act);
-      act &= act - 1u;
-      f(k);
+      f(kb + (__builtin_ctzll(act) >> 3));
+      act &= act - 1;
     }
   }
 }
 
-// Packed short2 update of voxel i by frames [0, K) (the oracle's
-// update_voxel).  The voxel is read at its first update and written only if
-// some frame updated it: outside every frustum and behind every surface it
-// costs no memory traffic.
+// Poses are read with a uniform index through the constant address space
+// (scalar loads: the wave's registers hold no pose).
+typedef const float __attribute__((address_space(4))) cfloat;
+
+// Frame k's view of a brick: per voxel the pixel it is seen at (kNoPixel:
+// none) and its distance from the camera.
+template <int NZ>
+struct View {
+  uint32_t pix[NZ];
+  float qn[NZ];
+};
+
+template <int NZ>
+__device__ __forceinline__ View<NZ> view_brick(const IntegrateParams& P, const Brick<NZ>& B,
+                                               int k) {
+  cfloat* R = (cfloat*)(uintptr_t)(P.poses + 12 * k);
+  const float dx = B.px - R[9], dy = B.py - R[10];
+  const float ax = __fmaf_rn(R[3], dy, R[0] * dx), ay = __fmaf_rn(R[4], dy, R[1] * dx),
+              az = __fmaf_rn(R[5], dy, R[2] * dx);
+  View<NZ> V;
+#pragma unroll
+  for (int j = 0; j < NZ; ++j) {
+    const float dz = B.pz(P, j) - R[11];
+    const float qx = __fmaf_rn(R[6], dz, ax), qy = __fmaf_rn(R[7], dz, ay),
+                qz = __fmaf_rn(R[8], dz, az);
+    V.pix[j] = kNoPixel;
+    V.qn[j] = 0.0f;
+    if (!B.inside || j >= B.nz || qz < FLT_MIN) continue;
+    const float u = __fmaf_rn(P.fx, qx / qz, P.cx);
+    const float v = __fmaf_rn(P.fy, qy / qz, P.cy);
+    if (!(fabsf(u) < 1e9f) || !(fabsf(v) < 1e9f)) continue;
+    const int ui = (int)rintf(u), vi = (int)rintf(v);
+    if (ui < 0 || vi < 0 || ui >= P.W - 2 || vi >= P.H - 2) continue;
+    V.pix[j] = (uint32_t)(vi * P.W + ui);
+    V.qn[j] = sqrtf(__fmaf_rn(qz, qz, __fmaf_rn(qy, qy, qx * qx)));
+  }
+  return V;
+}
+
+// f(j, sdf, rayfac, pix) for the voxels j of the lane's column that frame k
+// updates (zval > FLT_MIN, sdf >= -trunc_neg); the loads of all its voxels are
+// in flight together.
+template <typename DT, int NZ, typename F>
+__device__ __forceinline__ void observe_brick(const IntegrateParams& P, const Brick<NZ>& B, int k,
+                                              F&& f) {
+  const View<NZ> V = view_brick(P, B, k);
+  float dm[NZ], rf[NZ];
+#pragma unroll
+  for (int j = 0; j < NZ; ++j) {
+    dm[j] = frame_depth<DT>(P, k, V.pix[j]);
+    rf[j] = frame_rayfac(P, V.pix[j]);
+  }
+#pragma unroll
+  for (int j = 0; j < NZ; ++j) {
+    const float zval = (dm[j] * P.depth_scale) * rf[j];
+    if (!(zval > FLT_MIN)) continue;
+    const float sdf = zval - V.qn[j];
+    if (!(sdf >= -P.trunc_neg)) continue;
+    f(j, sdf, rf[j], V.pix[j]);
+  }
+}
+
 // One packed update (the oracle's update_voxel after its lookups): the new
 // (tsdf, weight) word from the current one and the observation t.
 // A voxel at +1 observed at +1 (free space seen again) stays at +1 with no
@@ -235,176 +413,63 @@ __device__ __forceinline__ float truncated(float sdf, float trunc_pos, float tru
   return fminf(sdf / (sdf > 0.0f ? trunc_pos : trunc_neg), 1.0f);
 }
 
-// Coordinates of voxel i of an X x Y x Z volume (x fastest).  Below 2^32
-// voxels: two 32-bit magic-number divisions (i / X, then the row / Y), exact
-// for every 32-bit numerator; larger volumes divide in 64 bits.
-__device__ __forceinline__ void voxel_coords(const IntegrateParams& P, int64_t i, int* x, int* y,
-                                             int* z) {
-  if (i < ((int64_t)1 << 32)) {
-    const uint32_t row = P.divX.div((uint32_t)i);
-    const uint32_t zz = P.divY.div(row);
-    *x = (int)((uint32_t)i - row * (uint32_t)P.X);
-    *y = (int)(row - zz * (uint32_t)P.Y);
-    *z = (int)zz;
-  } else {
-    const uint32_t xy = (uint32_t)((int64_t)P.X * P.Y);
-    const int zz = (int)(i / xy);
-    const uint32_t rem = (uint32_t)(i - (int64_t)zz * xy);
-    const uint32_t yy = P.divX.div(rem);
-    *x = (int)(rem - yy * (uint32_t)P.X);
-    *y = (int)yy;
-    *z = zz;
-  }
-}
-
-// Packed short2 update of voxel i by frames [0, K) (the oracle's
-// update_voxel).  The voxel is read at its first update and written only if
-// some frame updated it: outside every frustum and behind every surface it
-// costs no memory traffic.
-template <typename DT>
-__device__ __forceinline__ void integrate_voxel(const IntegrateParams& P, const float* s_pose,
-                                                const uint32_t* s_skip, float px, float py,
-                                                float pz, int64_t i) {
-  uint32_t cur = 0;
-  bool have = false;
-  for_active_frames(s_skip, P.K, [&](int k) {
-    const float* R = s_pose + 12 * k;
-    const float dx = px - R[9], dy = py - R[10], dz = pz - R[11];
-    const float qx = __fmaf_rn(R[6], dz, __fmaf_rn(R[3], dy, R[0] * dx));
-    const float qy = __fmaf_rn(R[7], dz, __fmaf_rn(R[4], dy, R[1] * dx));
-    const float qz = __fmaf_rn(R[8], dz, __fmaf_rn(R[5], dy, R[2] * dx));
-    if (qz < FLT_MIN) return;
-    const float u = __fmaf_rn(P.fx, qx / qz, P.cx);
-    const float v = __fmaf_rn(P.fy, qy / qz, P.cy);
-    if (!(fabsf(u) < 1e9f) || !(fabsf(v) < 1e9f)) return;
-    const int ui = (int)rintf(u), vi = (int)rintf(v);
-    if (ui < 0 || vi < 0 || ui >= P.W - 2 || vi >= P.H - 2) return;
-    const uint32_t pix = (uint32_t)(vi * P.W + ui);
-    const float zval = (frame_depth<DT>(P, k, pix) * P.depth_scale) * frame_rayfac(P, pix);
-    if (!(zval > FLT_MIN)) return;
-    const float qn = sqrtf(__fmaf_rn(qz, qz, __fmaf_rn(qy, qy, qx * qx)));
-    const float sdf = zval - qn;
-    if (!(sdf >= -P.trunc_neg)) return;
-    const float tsdf = truncated(sdf, P.trunc, P.trunc_neg);
-    if (!have) {
-      cur = P.vol[i];
-      have = true;
-    }
-    cur = packed_update(cur, tsdf, P.max_w);
-  });
-  if (have) P.vol[i] = cur;
-}
-
-// Launches size the shared memory to K frames: poses (12 floats each), then
-// one skip bit per frame.
-__host__ __device__ constexpr size_t frames_lds_bytes(int K) {
-  return (size_t)K * 12 * sizeof(float) + (size_t)((K + 31) / 32) * sizeof(uint32_t);
-}
-
+// Packed short2 update of a brick by frames [0, K) (the oracle's
+// update_voxel).  The brick is read when its first frame comes up and a voxel
+// is written only if some frame updated it: outside every frustum and behind
+// every surface it costs no memory traffic.
 template <typename DT>
 __global__ __launch_bounds__(256) void integrate_kernel(IntegrateParams P) {
-  extern __shared__ float s_frames[];
-  float* const s_pose = s_frames;
-  uint32_t* const s_skip = reinterpret_cast<uint32_t*>(s_frames + 12 * P.K);
-  for (int i = threadIdx.x; i < P.K * 12; i += blockDim.x) s_pose[i] = P.poses[i];
-  __syncthreads();
-  const int64_t n = (int64_t)P.X * P.Y * P.Z;
-  const int64_t ib = (P.first_block + blockIdx.x) * (int64_t)blockDim.x;
-  frame_skip_flags(s_pose, P.K, P, ib, min(ib + (int64_t)blockDim.x, n) - 1, s_skip);
-  const int64_t i = ib + threadIdx.x;
-  if (i >= n) return;
-  int x, y, z;
-  voxel_coords(P, i, &x, &y, &z);
-  const float px = ((float)x + 0.5f) * P.h;
-  const float py = ((float)y + 0.5f) * P.h;
-  const float pz = ((float)z + 0.5f) * P.h;
-  integrate_voxel<DT>(P, s_pose, s_skip, px, py, pz, i);
+  int x0, y0, z0;
+  if (!brick_origin(P, (uint32_t)(P.first_block + blockIdx.x), kBrickZ, &x0, &y0, &z0)) return;
+  const Brick<kBrickZ> B(P, x0, y0, z0);
+  uint32_t* const v = P.vol + B.first(P);
+  const int64_t XY = (int64_t)P.X * P.Y;
+  uint32_t cur[kBrickZ] = {};
+  uint32_t changed = 0;
+  bool have = false;
+  for_active_frames(P, B, [&](int k) {
+    if (!have) {
+      have = true;
+#pragma unroll
+      for (int j = 0; j < kBrickZ; ++j)
+        if (B.inside && j < B.nz) cur[j] = v[j * XY];
+    }
+    observe_brick<DT>(P, B, k, [&](int j, float sdf, float, uint32_t) {
+      cur[j] = packed_update(cur[j], truncated(sdf, P.trunc, P.trunc_neg), P.max_w);
+      changed |= 1u << j;
+    });
+  });
+#pragma unroll
+  for (int j = 0; j < kBrickZ; ++j)
+    if (changed & (1u << j)) v[j * XY] = cur[j];
 }
 
-// One frame (the reference's per-frame call): eight voxels a thread (voxel
-// ib + t + 256 j of the workgroup's 2048, coalesced).  The thread's first
-// voxel has its coordinates from two divisions; each next one lies 256
-// voxels further, (step_x, step_y, step_z) with carries.  The projections
-// come first, then the depth, ray-factor and voxel loads of all eight are
-// issued together (at clamped, valid addresses), then the updates: the
-// operations and results of integrate_voxel, with the memory latency
-// overlapped.  The voxels are addressed from the workgroup's first one
-// (32-bit offsets).  Only voxels the frame updates are written.
-// 0.422 ms per 640x480 frame into 512^3 against 0.435 ms with four voxels a
-// thread, each by two divisions (four with steps: 0.445; eight by divisions:
-// 0.434; sixteen: 0.422 with steps, 0.444 by divisions).
-constexpr int kVoxelsPerThread1 = 8;
+// One frame (the reference's per-frame call): a wave takes `bricks` bricks
+// above one another (up to eight), tests all of them at once (eight lanes
+// each) and passes through those that can observe the frame.  Fewer bricks a
+// wave for small volumes, so that there are waves enough.
 template <typename DT>
-__global__ __launch_bounds__(256) void integrate1_kernel(IntegrateParams P) {
-  constexpr int NV = kVoxelsPerThread1;
-  __shared__ float s_pose[12];
-  __shared__ uint32_t s_skip[1];
-  if (threadIdx.x < 12) s_pose[threadIdx.x] = P.poses[threadIdx.x];
-  __syncthreads();
-  const int64_t n = (int64_t)P.X * P.Y * P.Z;
-  const int64_t ib = (P.first_block + blockIdx.x) * 256 * NV;
-  const int nloc = (int)min((int64_t)256 * NV, n - ib);  // voxels of the workgroup
-  frame_skip_flags(s_pose, 1, P, ib, ib + nloc - 1, s_skip);
-  if (s_skip[0] & 1u) return;  // no voxel of the workgroup can see the frame
-  const float* R = s_pose;
-  uint32_t* const vb = P.vol + ib;  // voxel ib + l is vb[l]
-  const int t = (int)threadIdx.x;
-  int x, y, z;
-  voxel_coords(P, ib + min(t, nloc - 1), &x, &y, &z);
-  int pix[NV];
-  float qn[NV];
+__global__ __launch_bounds__(256) void integrate1_kernel(IntegrateParams P, int bricks) {
+  int x0, y0, z0;
+  if (!brick_origin(P, (uint32_t)(P.first_block + blockIdx.x), kBrickZ * bricks, &x0, &y0, &z0))
+    return;
+  const int lane = threadIdx.x & 63;
+  const int zt = z0 + (lane >> 3) * kBrickZ;
+  float px, py, pz;
+  brick_corner<kBrickZ>(P, x0, y0, min(zt, P.Z - 1), &px, &py, &pz);
+  const bool skip = test_box(P, P.poses, 0, px, py, pz);
+  uint64_t act = __ballot(!skip && (lane & 7) == 0 && (lane >> 3) < bricks && zt < P.Z);
+  const int64_t XY = (int64_t)P.X * P.Y;
+  while (act) {
+    const Brick<kBrickZ> B(P, x0, y0, z0 + (__builtin_ctzll(act) >> 3) * kBrickZ);
+    act &= act - 1;
+    uint32_t* const v = P.vol + B.first(P);
+    uint32_t cur[kBrickZ];
 #pragma unroll
-  for (int j = 0; j < NV; ++j) {
-    if (j > 0) {  // x + step_x < 2X, y + step_y + 1 < 2Y
-      x += P.step_x;
-      y += P.step_y;
-      z += P.step_z;
-      if (x >= P.X) {
-        x -= P.X;
-        ++y;
-      }
-      if (y >= P.Y) {
-        y -= P.Y;
-        ++z;
-      }
-    }
-    pix[j] = -1;
-    qn[j] = 0.0f;
-    if (t + 256 * j >= nloc) continue;
-    const float px = ((float)x + 0.5f) * P.h;
-    const float py = ((float)y + 0.5f) * P.h;
-    const float pz = ((float)z + 0.5f) * P.h;
-    const float dx = px - R[9], dy = py - R[10], dz = pz - R[11];
-    const float qx = __fmaf_rn(R[6], dz, __fmaf_rn(R[3], dy, R[0] * dx));
-    const float qy = __fmaf_rn(R[7], dz, __fmaf_rn(R[4], dy, R[1] * dx));
-    const float qz = __fmaf_rn(R[8], dz, __fmaf_rn(R[5], dy, R[2] * dx));
-    if (qz < FLT_MIN) continue;
-    const float u = __fmaf_rn(P.fx, qx / qz, P.cx);
-    const float v = __fmaf_rn(P.fy, qy / qz, P.cy);
-    if (!(fabsf(u) < 1e9f) || !(fabsf(v) < 1e9f)) continue;
-    const int ui = (int)rintf(u), vv = (int)rintf(v);
-    if (ui < 0 || vv < 0 || ui >= P.W - 2 || vv >= P.H - 2) continue;
-    pix[j] = vv * P.W + ui;
-    qn[j] = sqrtf(__fmaf_rn(qz, qz, __fmaf_rn(qy, qy, qx * qx)));
-  }
-  DT dm[NV];
-  float rf[NV];
-  uint32_t cur[NV];
-#pragma unroll
-  for (int j = 0; j < NV; ++j) {
-    const int q = pix[j] >= 0 ? pix[j] : 0;
-    dm[j] = static_cast<const DT*>(P.depth)[(uint32_t)q];
-    rf[j] = P.rayfac[(uint32_t)q];
-    cur[j] = vb[min(t + 256 * j, nloc - 1)];
-  }
-#pragma unroll
-  for (int j = 0; j < NV; ++j) {
-    if (pix[j] < 0) continue;
-    const float zval = ((float)dm[j] * P.depth_scale) * rf[j];
-    if (!(zval > FLT_MIN)) continue;
-    const float sdf = zval - qn[j];
-    if (!(sdf >= -P.trunc_neg)) continue;
-    vb[t + 256 * j] = packed_update(cur[j], truncated(sdf, P.trunc, P.trunc_neg), P.max_w);
+    for (int j = 0; j < kBrickZ; ++j) cur[j] = B.inside && j < B.nz ? v[j * XY] : 0u;
+    observe_brick<DT>(P, B, 0, [&](int j, float sdf, float, uint32_t) {
+      v[j * XY] = packed_update(cur[j], truncated(sdf, P.trunc, P.trunc_neg), P.max_w);
+    });
   }
 }
 
@@ -413,102 +478,75 @@ __global__ __launch_bounds__(256) void integrate1_kernel(IntegrateParams P) {
 // tsdf (fp32) and weight (int32) in separate [z][y][x] arrays; the same
 // observation as above, stored unpacked:
 //   f <- fma(f, w, t) / (w + 1),  w <- min(w + 1, max_w),  t = clamp(sdf / trunc, -1, 1).
-// Observation k of voxel (px, py, pz): pixel, t and dt/d(depth value) (zero
-// where t is clamped).  Returns false where the voxel is not updated.
-template <typename DT>
-__device__ __forceinline__ bool observe(const IntegrateParams& P, const float* R, int k,
-                                        float px, float py, float pz, int* pix_out, float* t_out,
-                                        float* dtdd_out) {
-  const float dx = px - R[9], dy = py - R[10], dz = pz - R[11];
-  const float qx = __fmaf_rn(R[6], dz, __fmaf_rn(R[3], dy, R[0] * dx));
-  const float qy = __fmaf_rn(R[7], dz, __fmaf_rn(R[4], dy, R[1] * dx));
-  const float qz = __fmaf_rn(R[8], dz, __fmaf_rn(R[5], dy, R[2] * dx));
-  if (qz < FLT_MIN) return false;
-  const float u = __fmaf_rn(P.fx, qx / qz, P.cx);
-  const float v = __fmaf_rn(P.fy, qy / qz, P.cy);
-  if (!(fabsf(u) < 1e9f) || !(fabsf(v) < 1e9f)) return false;
-  const int ui = (int)rintf(u), vi = (int)rintf(v);
-  if (ui < 0 || vi < 0 || ui >= P.W - 2 || vi >= P.H - 2) return false;
-  const int pix = vi * P.W + ui;
-  const float rf = frame_rayfac(P, (uint32_t)pix);
-  const float d = frame_depth<DT>(P, k, (uint32_t)pix) * P.depth_scale;
-  const float zval = d * rf;
-  if (!(zval > FLT_MIN)) return false;
-  const float qn = sqrtf(__fmaf_rn(qz, qz, __fmaf_rn(qy, qy, qx * qx)));
-  const float sdf = zval - qn;
-  if (!(sdf >= -P.trunc)) return false;
-  *pix_out = pix;
-  if (sdf >= P.trunc) {
-    // sdf / trunc >= 1 before rounding, so after it: clamped to 1, no gradient
-    *t_out = 1.0f;
-    *dtdd_out = 0.0f;
-    return true;
-  }
+// The observation t of a signed distance (>= -trunc).
+__device__ __forceinline__ float truncated_f32(float sdf, float trunc) {
+  if (sdf >= trunc) return 1.0f;  // sdf / trunc >= 1 before rounding, so after it
+  return fminf(fmaxf(sdf / trunc, -1.0f), 1.0f);
+}
+
+// d(observation)/d(depth value): zero where t is clamped.
+__device__ __forceinline__ float observation_slope(const IntegrateParams& P, float sdf, float rf) {
+  if (sdf >= P.trunc) return 0.0f;
   const float ts = sdf / P.trunc;
-  *t_out = fminf(fmaxf(ts, -1.0f), 1.0f);
-  *dtdd_out = (ts > -1.0f && ts < 1.0f) ? P.depth_scale * rf / P.trunc : 0.0f;
-  return true;
+  return ts > -1.0f && ts < 1.0f ? P.depth_scale * rf / P.trunc : 0.0f;
 }
 
-// fp32 update of one voxel by frames [0, K).  With tsdf / wvol, (f, w) is
-// read from them at the first update (none: no memory traffic) and *changed
-// says whether any frame updated it; without, (f, w) holds the start value.
-__device__ __forceinline__ void integrate_tsdf_voxel(const IntegrateParams& P, const float* s_pose,
-                                                     const uint32_t* s_skip, float px, float py,
-                                                     float pz, float& f, int& w,
-                                                     const float* tsdf, const int32_t* wvol,
-                                                     bool* changed) {
-  bool have = tsdf == nullptr;
-  for_active_frames(s_skip, P.K, [&](int k) {
-    int pix;
-    float t, dtdd;
-    if (!observe<float>(P, s_pose + 12 * k, k, px, py, pz, &pix, &t, &dtdd)) return;
+// fp32 update of a brick by frames [0, K), from (f, w) as given.  Returns the
+// voxels (bits j) that some frame updated.
+template <typename LOAD>
+__device__ __forceinline__ uint32_t integrate_tsdf_brick(const IntegrateParams& P,
+                                                         const Brick<kBrickZ>& B,
+                                                         float (&f)[kBrickZ], int (&w)[kBrickZ],
+                                                         LOAD&& load) {
+  uint32_t changed = 0;
+  bool have = false;
+  for_active_frames(P, B, [&](int k) {
     if (!have) {
-      f = *tsdf;
-      w = *wvol;
       have = true;
+      load();
     }
-    *changed = true;
-    // f = 1 observed at 1 stays 1: fma(1, w, 1) = w + 1 = (float)(w + 1)
-    // exactly for 0 <= w < 2^24 (a weight read from the caller's volume may
-    // lie outside), and the quotient of equal values is 1
-    if (!(f == 1.0f && t == 1.0f && (uint32_t)w < (1u << 24)))
-      f = __fmaf_rn(f, (float)w, t) / (float)(w + 1);
-    w = w + 1 < P.max_w ? w + 1 : P.max_w;
+    observe_brick<float>(P, B, k, [&](int j, float sdf, float, uint32_t) {
+      const float t = truncated_f32(sdf, P.trunc);
+      changed |= 1u << j;
+      // f = 1 observed at 1 stays 1: fma(1, w, 1) = w + 1 = (float)(w + 1)
+      // exactly for 0 <= w < 2^24 (a weight read from the caller's volume may
+      // lie outside), and the quotient of equal values is 1
+      if (!(f[j] == 1.0f && t == 1.0f && (uint32_t)w[j] < (1u << 24)))
+        f[j] = __fmaf_rn(f[j], (float)w[j], t) / (float)(w[j] + 1);
+      w[j] = w[j] + 1 < P.max_w ? w[j] + 1 : P.max_w;
+    });
   });
+  return changed;
 }
 
-__device__ __forceinline__ void voxel_centre(const IntegrateParams& P, int64_t i, float* px,
-                                             float* py, float* pz) {
-  int x, y, z;
-  voxel_coords(P, i, &x, &y, &z);
-  *px = ((float)x + 0.5f) * P.h;
-  *py = ((float)y + 0.5f) * P.h;
-  *pz = ((float)z + 0.5f) * P.h;
+// The brick's voxels are read when the first frame that may observe it comes
+// up; only updated voxels are written.
+__device__ __forceinline__ void integrate_tsdf_stored(const IntegrateParams& P,
+                                                      const Brick<kBrickZ>& B, float* tsdf, int32_t* wvol) {
+  const int64_t i = B.first(P), XY = (int64_t)P.X * P.Y;
+  float f[kBrickZ] = {};
+  int w[kBrickZ] = {};
+  const uint32_t changed = integrate_tsdf_brick(P, B, f, w, [&]() {
+#pragma unroll
+    for (int j = 0; j < kBrickZ; ++j)
+      if (B.inside && j < B.nz) {
+        f[j] = tsdf[i + j * XY];
+        w[j] = wvol[i + j * XY];
+      }
+  });
+#pragma unroll
+  for (int j = 0; j < kBrickZ; ++j)
+    if (changed & (1u << j)) {
+      tsdf[i + j * XY] = f[j];
+      wvol[i + j * XY] = w[j];
+    }
 }
 
 __global__ __launch_bounds__(256) void integrate_tsdf_kernel(IntegrateParams P, float* tsdf,
                                                              int32_t* wvol) {
-  extern __shared__ float s_frames[];
-  float* const s_pose = s_frames;
-  uint32_t* const s_skip = reinterpret_cast<uint32_t*>(s_frames + 12 * P.K);
-  for (int i = threadIdx.x; i < P.K * 12; i += blockDim.x) s_pose[i] = P.poses[i];
-  __syncthreads();
-  const int64_t n = (int64_t)P.X * P.Y * P.Z;
-  const int64_t ib = (P.first_block + blockIdx.x) * (int64_t)blockDim.x;
-  frame_skip_flags(s_pose, P.K, P, ib, min(ib + (int64_t)blockDim.x, n) - 1, s_skip);
-  const int64_t i = ib + threadIdx.x;
-  if (i >= n) return;
-  float px, py, pz;
-  voxel_centre(P, i, &px, &py, &pz);
-  float f = 0.0f;
-  int w = 0;
-  bool changed = false;
-  integrate_tsdf_voxel(P, s_pose, s_skip, px, py, pz, f, w, tsdf + i, wvol + i, &changed);
-  if (changed) {
-    tsdf[i] = f;
-    wvol[i] = w;
-  }
+  int x0, y0, z0;
+  if (!brick_origin(P, (uint32_t)(P.first_block + blockIdx.x), kBrickZ, &x0, &y0, &z0)) return;
+  integrate_tsdf_stored(P, Brick<kBrickZ>(P, x0, y0, z0), tsdf, wvol);
 }
 
 // Deterministic max of |g| over n floats: per-block max, then an integer
@@ -534,101 +572,104 @@ __device__ __forceinline__ double grad_scale(uint32_t maxg_bits, float max_dtdd)
   return bound > 0.0 ? 4398046511104.0 / bound : 1.0;  // 2^42 / bound
 }
 
-// Backward of the fp32 update of one voxel for the K frames of one call:
-// recompute its observations; observation i (weight before it wb_i =
+// Backward of the fp32 update of a brick for the K frames of one call:
+// recompute its observations; a voxel's observation i (weight before it wb_i =
 // min(w0 + i, max_w)) has df/dt_i = 1/(wb_i + 1) * prod over later
 // observations j of wb_j / (wb_j + 1) (closed form: the uncapped part
 // telescopes, the capped part is a power of max_w / (max_w + 1)); the
 // contribution g * df/dt_i * dt_i/dd goes to the observed pixel of acc (K
 // frames of W x H) as an int64 fixed-point atomic add (integer sums do not
-// depend on the order).
-__device__ __forceinline__ void backward_voxel(const IntegrateParams& P, const float* s_pose,
-                                               const uint32_t* s_skip, float px, float py,
-                                               float pz, float gi, int w0, double scale,
+// depend on the order).  Bricks without a gradient (most: only the corners of
+// active cubes carry one) are left after reading it.
+template <int NZ>
+__device__ __forceinline__ void backward_brick(const IntegrateParams& P, const Brick<NZ>& B,
+                                               const float* __restrict__ g,
+                                               const int32_t* __restrict__ w0vol,
+                                               const uint32_t* maxg, float max_dtdd,
                                                unsigned long long* acc) {
+  const int64_t i = B.first(P), XY = (int64_t)P.X * P.Y;
+  float gi[NZ];
+#pragma unroll
+  for (int j = 0; j < NZ; ++j) gi[j] = B.inside && j < B.nz ? g[i + j * XY] : 0.0f;
+  bool any = false;
+#pragma unroll
+  for (int j = 0; j < NZ; ++j) any |= gi[j] != 0.0f;
+  if (!__any(any)) return;
+  const double scale = grad_scale(*maxg, max_dtdd);
   const int M = P.max_w;
-  int nobs = 0;
-  for_active_frames(s_skip, P.K, [&](int k) {
-    int pix;
-    float t, dtdd;
-    if (observe<float>(P, s_pose + 12 * k, k, px, py, pz, &pix, &t, &dtdd)) ++nobs;
+  int nobs[NZ] = {}, o[NZ] = {}, w0[NZ] = {};
+  if (w0vol) {
+#pragma unroll
+    for (int j = 0; j < NZ; ++j)
+      if (gi[j] != 0.0f) w0[j] = w0vol[i + j * XY];
+  }
+  for_active_frames(P, B, [&](int k) {
+    observe_brick<float>(P, B, k, [&](int j, float, float, uint32_t) { ++nobs[j]; });
   });
-  const int jc = M - w0 > 0 ? M - w0 : 0;  // first observation that sees the cap
   const double cap_a = (double)M / (double)(M + 1);
-  int o = 0;
-  for_active_frames(s_skip, P.K, [&](int k) {
-    int pix;
-    float t, dtdd;
-    if (!observe<float>(P, s_pose + 12 * k, k, px, py, pz, &pix, &t, &dtdd)) return;
-    const int wb = w0 + o < M ? w0 + o : M;
-    double c = 1.0 / (double)(wb + 1);
-    const int last_unc = (nobs - 1 < jc - 1) ? nobs - 1 : jc - 1;  // last uncapped index
-    if (o + 1 <= last_unc) c *= (double)(w0 + o + 1) / (double)(w0 + last_unc + 1);
-    const int first_cap = o + 1 > jc ? o + 1 : jc;
-    const int ncap = nobs - first_cap;
-    if (ncap > 0) {
-      // cap_a^ncap by squaring (a library pow inlined here costs the kernel
-      // registers on every path, capped or not)
-      double pw = 1.0, base = cap_a;
-      for (int e = ncap; e; e >>= 1) {
-        if (e & 1) pw *= base;
-        base *= base;
+  for_active_frames(P, B, [&](int k) {
+    observe_brick<float>(P, B, k, [&](int j, float sdf, float rf, uint32_t pix) {
+      const int oi = o[j]++;
+      if (gi[j] == 0.0f) return;
+      const float dtdd = observation_slope(P, sdf, rf);
+      if (dtdd == 0.0f) return;
+      const int w = w0[j], n = nobs[j];
+      const int jc = M - w > 0 ? M - w : 0;  // first observation that sees the cap
+      const int wb = w + oi < M ? w + oi : M;
+      double c = 1.0 / (double)(wb + 1);
+      const int last_unc = (n - 1 < jc - 1) ? n - 1 : jc - 1;  // last uncapped index
+      if (oi + 1 <= last_unc) c *= (double)(w + oi + 1) / (double)(w + last_unc + 1);
+      const int first_cap = oi + 1 > jc ? oi + 1 : jc;
+      const int ncap = n - first_cap;
+      if (ncap > 0) {
+        // cap_a^ncap by squaring (a library pow inlined here costs the kernel
+        // registers on every path, capped or not)
+        double pw = 1.0, base = cap_a;
+        for (int e = ncap; e; e >>= 1) {
+          if (e & 1) pw *= base;
+          base *= base;
+        }
+        c *= pw;
       }
-      c *= pw;
-    }
-    const double contrib = (double)gi * c * (double)dtdd;
-    if (contrib != 0.0) {
-      const long long q = llrint(contrib * scale);
-      atomicAdd(acc + (int64_t)k * P.W * P.H + pix, (unsigned long long)q);
-    }
-    ++o;
+      const double contrib = (double)gi[j] * c * (double)dtdd;
+      if (contrib != 0.0) {
+        const long long q = llrint(contrib * scale);
+        atomicAdd(acc + (int64_t)k * P.W * P.H + pix, (unsigned long long)q);
+      }
+    });
   });
 }
 
+template <int NZ>
 __global__ __launch_bounds__(256) void integrate_tsdf_backward_kernel(
     IntegrateParams P, const float* __restrict__ g, const int32_t* __restrict__ w0vol,
     const uint32_t* maxg, float max_dtdd, unsigned long long* acc) {
-  extern __shared__ float s_frames[];
-  float* const s_pose = s_frames;
-  uint32_t* const s_skip = reinterpret_cast<uint32_t*>(s_frames + 12 * P.K);
-  const int64_t n = (int64_t)P.X * P.Y * P.Z;
-  const int64_t ib = (P.first_block + blockIdx.x) * (int64_t)blockDim.x;
-  const int64_t i = ib + threadIdx.x;
-  // most blocks carry no gradient: they leave after reading it, before the
-  // poses and the frame tests
-  const float gi = i < n ? g[i] : 0.0f;
-  if (!__syncthreads_or(gi != 0.0f)) return;
-  for (int k = threadIdx.x; k < P.K * 12; k += blockDim.x) s_pose[k] = P.poses[k];
-  __syncthreads();
-  frame_skip_flags(s_pose, P.K, P, ib, min(ib + (int64_t)blockDim.x, n) - 1, s_skip);
-  if (i >= n || gi == 0.0f) return;
-  float px, py, pz;
-  voxel_centre(P, i, &px, &py, &pz);
-  backward_voxel(P, s_pose, s_skip, px, py, pz, gi, w0vol ? w0vol[i] : 0,
-                 grad_scale(*maxg, max_dtdd), acc);
+  int x0, y0, z0;
+  if (!brick_origin(P, (uint32_t)(P.first_block + blockIdx.x), NZ, &x0, &y0, &z0)) return;
+  backward_brick(P, Brick<NZ>(P, x0, y0, z0), g, w0vol, maxg, max_dtdd, acc);
 }
 
 // ---- batches of fp32 volumes (the per-volume layout of a batch plan:
 // concatenated per-voxel arrays, K frames of W x H and K poses per volume,
-// one set of intrinsics); one workgroup = 256 voxels of one volume.
+// one set of intrinsics); a workgroup takes four bricks of one volume.
 struct BatchIntegrateParams {
   IntegrateParams base;  // intrinsics, truncation, frames; depth / poses of volume 0
   const BatchVol* bvol;
   int nvol;
   int from_init;         // start every voxel from (init_value, 0) without reading it
   float init_value;
+  int tiled_vol;         // volumes [tiled_vol, tiled_vol + base.tiled / K) have tile tables
   int64_t first_block;   // workgroup index of this launch's blockIdx.x 0
 };
 
-// The volume of this workgroup's block (binary search over the block ranges).
-__device__ __forceinline__ int batch_block_volume(const BatchIntegrateParams& B) {
-  return batch_volume_of<&BatchVol::blk_begin>(B.bvol, B.nvol, B.first_block + blockIdx.x);
-}
-
-// This workgroup's volume vi: its launch parameters and its poses in LDS.
-__device__ __forceinline__ int batch_setup(const BatchIntegrateParams& B, int vi, IntegrateParams& P,
-                                           float* s_pose, int64_t* vox_begin, int64_t* i0) {
+// This workgroup's volume (binary search over the block ranges), its launch
+// parameters and this wave's brick; false past the volume's edge.
+__device__ __forceinline__ bool batch_setup(const BatchIntegrateParams& B, IntegrateParams& P,
+                                            int64_t* vox_begin, int* vol, int* x0, int* y0,
+                                            int* z0) {
   const int64_t blk = B.first_block + blockIdx.x;
+  const int vi = __builtin_amdgcn_readfirstlane(
+      batch_volume_of<&BatchVol::blk_begin>(B.bvol, B.nvol, blk));
   const BatchVol& V = B.bvol[vi];
   P = B.base;
   P.X = V.X;
@@ -637,75 +678,50 @@ __device__ __forceinline__ int batch_setup(const BatchIntegrateParams& B, int vi
   P.h = V.h;
   P.divX = V.divX;
   P.divY = V.divY;
-  const int64_t frames = (int64_t)P.K * P.W * P.H;
-  P.depth = static_cast<const float*>(B.base.depth) + (int64_t)vi * frames;
-  const float* poses = B.base.poses + (int64_t)vi * P.K * 12;
-  for (int i = threadIdx.x; i < P.K * 12; i += blockDim.x) s_pose[i] = poses[i];
+  P.depth = static_cast<const float*>(B.base.depth) + (int64_t)vi * P.K * P.W * P.H;
+  P.poses = B.base.poses + (int64_t)vi * P.K * 12;
+  P.tiled = vi >= B.tiled_vol ? max(0, min(P.K, P.tiled - (vi - B.tiled_vol) * P.K)) : 0;
+  P.tiles = B.base.tiles + (int64_t)(vi - B.tiled_vol) * P.K * P.TY * P.TX;
   *vox_begin = V.vox_begin;
-  *i0 = (blk - V.blk_begin) * 256;
-  __syncthreads();
-  return vi;
+  *vol = vi;
+  return brick_origin(P, (uint32_t)(blk - V.blk_begin), kBrickZ, x0, y0, z0);
 }
 
 __global__ __launch_bounds__(256) void integrate_tsdf_batched_kernel(BatchIntegrateParams B,
                                                                      float* tsdf, int32_t* wvol) {
-  extern __shared__ float s_frames[];
-  float* const s_pose = s_frames;
-  uint32_t* const s_skip = reinterpret_cast<uint32_t*>(s_frames + 12 * B.base.K);
   IntegrateParams P;
-  int64_t vb, ib;
-  batch_setup(B, batch_block_volume(B), P, s_pose, &vb, &ib);
-  const int64_t n = (int64_t)P.X * P.Y * P.Z;
-  frame_skip_flags(s_pose, P.K, P, ib, min(ib + 256, n) - 1, s_skip);
-  const int64_t i = ib + threadIdx.x;
-  if (i >= n) return;
-  float px, py, pz;
-  voxel_centre(P, i, &px, &py, &pz);
-  float f = B.init_value;
-  int w = 0;
-  bool changed = false;
-  if (B.from_init) {
-    // every voxel is written: the start value where no frame observes it
-    integrate_tsdf_voxel(P, s_pose, s_skip, px, py, pz, f, w, nullptr, nullptr, &changed);
-    tsdf[vb + i] = f;
-    wvol[vb + i] = w;
-  } else {
-    integrate_tsdf_voxel(P, s_pose, s_skip, px, py, pz, f, w, tsdf + vb + i, wvol + vb + i,
-                         &changed);
-    if (changed) {
-      tsdf[vb + i] = f;
-      wvol[vb + i] = w;
-    }
+  int64_t vb;
+  int vi, x0, y0, z0;
+  if (!batch_setup(B, P, &vb, &vi, &x0, &y0, &z0)) return;
+  const Brick<kBrickZ> K(P, x0, y0, z0);
+  if (!B.from_init) {
+    integrate_tsdf_stored(P, K, tsdf + vb, wvol + vb);
+    return;
   }
+  // every voxel is written: the start value where no frame observes it
+  float f[kBrickZ];
+  int w[kBrickZ] = {};
+#pragma unroll
+  for (int j = 0; j < kBrickZ; ++j) f[j] = B.init_value;
+  integrate_tsdf_brick(P, K, f, w, []() {});
+  const int64_t i = vb + K.first(P), XY = (int64_t)P.X * P.Y;
+#pragma unroll
+  for (int j = 0; j < kBrickZ; ++j)
+    if (K.inside && j < K.nz) {
+      tsdf[i + j * XY] = f[j];
+      wvol[i + j * XY] = w[j];
+    }
 }
 
 __global__ __launch_bounds__(256) void integrate_tsdf_backward_batched_kernel(
     BatchIntegrateParams B, const float* __restrict__ g, const int32_t* __restrict__ w0vol,
     const uint32_t* maxg, float max_dtdd, unsigned long long* acc) {
-  extern __shared__ float s_frames[];
-  float* const s_pose = s_frames;
-  uint32_t* const s_skip = reinterpret_cast<uint32_t*>(s_frames + 12 * B.base.K);
-  // most blocks carry no gradient: they leave after reading it, before the
-  // poses and the frame tests
-  const int vi = batch_block_volume(B);
-  float gi = 0.0f;
-  {
-    const BatchVol& V = B.bvol[vi];
-    const int64_t i = (B.first_block + blockIdx.x - V.blk_begin) * 256 + threadIdx.x;
-    if (i < (int64_t)V.X * V.Y * V.Z) gi = g[V.vox_begin + i];
-  }
-  if (!__syncthreads_or(gi != 0.0f)) return;
   IntegrateParams P;
-  int64_t vb, ib;
-  batch_setup(B, vi, P, s_pose, &vb, &ib);
-  const int64_t n = (int64_t)P.X * P.Y * P.Z;
-  frame_skip_flags(s_pose, P.K, P, ib, min(ib + 256, n) - 1, s_skip);
-  const int64_t i = ib + threadIdx.x;
-  if (i >= n || gi == 0.0f) return;
-  float px, py, pz;
-  voxel_centre(P, i, &px, &py, &pz);
-  backward_voxel(P, s_pose, s_skip, px, py, pz, gi, w0vol ? w0vol[vb + i] : 0,
-                 grad_scale(*maxg, max_dtdd), acc + (int64_t)vi * P.K * P.W * P.H);
+  int64_t vb;
+  int vi, x0, y0, z0;
+  if (!batch_setup(B, P, &vb, &vi, &x0, &y0, &z0)) return;
+  backward_brick(P, Brick<kBrickZ>(P, x0, y0, z0), g + vb, w0vol ? w0vol + vb : nullptr, maxg, max_dtdd,
+                 acc + (int64_t)vi * P.K * P.W * P.H);
 }
 
 __global__ __launch_bounds__(256) void fixed_to_float_kernel(const unsigned long long* acc,
@@ -827,23 +843,38 @@ extern "C" int mcx_volume_init(void* d_vol, int X, int Y, int Z, void* stream) {
   return MCX_OK;
 }
 
-extern "C" size_t mcx_integrate_workspace_size(int W, int H) {
+size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Tile tables: bytes per frame, and of as many frames as 32 MiB hold, at least
+// one (a 640x480 frame takes 38 KB, so a sweep's 512 frames fit; a 320x240
+// frame 9.6 KB: 3,495, the frames of 218 volumes of a batch with 16 each).
+size_t tile_bytes(int W, int H) {
+  return (size_t)((W + kTile - 1) / kTile) * ((H + kTile - 1) / kTile) * sizeof(float2);
+}
+size_t tile_tables_bytes(int W, int H) {
+  const size_t per = tile_bytes(W, H), most = (size_t)32 << 20;
+  return per * std::max((size_t)1, most / std::max(per, (size_t)1));
+}
+
+// The ray factors alone would do (they are what a call cannot run without);
+// the rest holds the frames' tile tables.
+size_t rayfac_bytes(int W, int H) {
   return (size_t)(W > 0 ? W : 0) * (size_t)(H > 0 ? H : 0) * sizeof(float);
+}
+extern "C" size_t mcx_integrate_workspace_size(int W, int H) {
+  const size_t rf = rayfac_bytes(W, H);
+  return rf ? al256(rf) + 256 + tile_tables_bytes(W, H) : 0;
 }
 
 // Checks shared by the integration entry points; fills the launch parameters
-// (all but vol, K, poses and depth) and computes the per-pixel ray factors.
+// (all but vol, K, poses, depth and the tile tables).
 int prepare_integrate(IntegrateParams& P, int X, int Y, int Z, float h, float trunc, int max_w,
-                      const float* intr, float depth_scale, int W, int H, int K, float* rayfac,
-                      hipStream_t s) {
+                      const float* intr, float depth_scale, int W, int H, int K, float* rayfac) {
   if (!intr || X < 1 || Y < 1 || Z < 1 || W < 3 || H < 3 || K < 0) return MCX_ERR_ARG;
   if (!(h > 0.f) || !(trunc > 0.f) || max_w < 1 || max_w > 65535) return MCX_ERR_ARG;
   if ((int64_t)X * Y > 0xffffffffll) return MCX_ERR_UNSUPPORTED;
   // frames are read through buffer resources of at most 2^31 - 1 bytes
   if ((int64_t)W * H * 4 >= ((int64_t)1 << 31)) return MCX_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(rayfac_kernel, dim3(blocks_for((int64_t)W * H)), dim3(256), 0, s, rayfac, W,
-                     H, intr[0], intr[1], intr[2], intr[3]);
-  MCX_HIP(hipGetLastError());
   P.vol = nullptr;
   P.X = X;
   P.Y = Y;
@@ -857,20 +888,52 @@ int prepare_integrate(IntegrateParams& P, int X, int Y, int Z, float h, float tr
   P.cx = intr[2];
   P.cy = intr[3];
   P.rayfac = rayfac;
+  P.tiles = nullptr;
+  P.tiled = 0;
+  P.TX = (W + kTile - 1) / kTile;
+  P.TY = (H + kTile - 1) / kTile;
   P.depth_scale = depth_scale;
   P.W = W;
   P.H = H;
-  P.divX = FastDiv((uint32_t)X);
-  P.divY = FastDiv((uint32_t)Y);
-  {
-    const int64_t XY = (int64_t)X * Y, r = 256 % XY;
-    P.step_z = (int)(256 / XY);
-    P.step_y = (int)(r / X);
-    P.step_x = (int)(r % X);
-  }
+  P.divX = FastDiv((uint32_t)((X + kRegionX - 1) / kRegionX));
+  P.divY = FastDiv((uint32_t)((Y + kBrick - 1) / kBrick));
   P.K = 0;
   P.poses = nullptr;
   P.depth = nullptr;
+  P.first_block = 0;
+  return MCX_OK;
+}
+
+// Workgroups of a volume, z planes taken zstep at a time.
+int64_t regions(int X, int Y, int Z, int zstep) {
+  return (int64_t)((X + kRegionX - 1) / kRegionX) * ((Y + kBrick - 1) / kBrick) *
+         ((Z + zstep - 1) / zstep);
+}
+
+// The ray factors, and the tile tables of as many of `frames` frames (from
+// `depth`) as [tables, end) holds; P.tiled says how many.
+template <typename DT>
+int frame_tiles(IntegrateParams& P, const DT* depth, int64_t frames, char* tables, char* end,
+                hipStream_t s) {
+  tables = reinterpret_cast<char*>(al256(reinterpret_cast<uintptr_t>(tables)));
+  const size_t per = tile_bytes(P.W, P.H);
+  const int64_t room = tables < end ? (int64_t)((size_t)(end - tables) / per) : 0;
+  P.tiles = reinterpret_cast<const float2*>(tables);
+  P.tiled = (int)std::min(frames, room);
+  const int gx = (P.TX + 7) / 8;
+  // about 16 waves per SIMD in all; each takes every gz-th frame
+  const int64_t gz = std::max<int64_t>(
+      1, std::min<int64_t>((16384 + (int64_t)gx * P.TY - 1) / ((int64_t)gx * P.TY), P.tiled));
+  const int vec = P.W % kTile == 0 && (reinterpret_cast<uintptr_t>(depth) & 15u) == 0 &&
+                  ((int64_t)P.W * P.H * (int64_t)sizeof(DT)) % 16 == 0;
+  for (int y0 = 0; y0 < P.TY; y0 += 65535) {
+    hipLaunchKernelGGL(frame_tiles_kernel<DT>,
+                       dim3((unsigned)gx, (unsigned)std::min(65535, P.TY - y0), (unsigned)gz),
+                       dim3(64), 0, s, depth, P.depth_scale, P.W, P.H, P.tiled, P.fx, P.fy, P.cx,
+                       P.cy, const_cast<float*>(P.rayfac), P.TX, P.TY, y0, vec,
+                       reinterpret_cast<float2*>(tables));
+    MCX_HIP(hipGetLastError());
+  }
   return MCX_OK;
 }
 
@@ -881,29 +944,35 @@ int integrate_impl(void* d_vol, int X, int Y, int Z, float h, float trunc_neg, f
                    void* stream) {
   if (!d_vol || !(trunc_neg > 0.f)) return MCX_ERR_ARG;
   if (K > 0 && (!d_poses || !d_depth)) return MCX_ERR_ARG;
-  if (!d_ws || ws_bytes < mcx_integrate_workspace_size(W, H)) return MCX_ERR_WORKSPACE;
+  if (!d_ws || ws_bytes < rayfac_bytes(W, H)) return MCX_ERR_WORKSPACE;
   if (K == 0) return MCX_OK;
   hipStream_t s = as_stream(stream);
   IntegrateParams P;
+  char* const ws = static_cast<char*>(d_ws);
   int rc = prepare_integrate(P, X, Y, Z, h, trunc, max_w, intr, depth_scale, W, H, K,
-                             static_cast<float*>(d_ws), s);
+                             reinterpret_cast<float*>(ws));
   if (rc) return rc;
   P.vol = static_cast<uint32_t*>(d_vol);
   P.trunc_neg = trunc_neg;
-  const int64_t n = (int64_t)X * Y * Z;
   for (int k0 = 0; k0 < K; k0 += kFramesPerPass) {
     P.K = K - k0 < kFramesPerPass ? K - k0 : kFramesPerPass;
     P.poses = d_poses + (int64_t)12 * k0;
     P.depth = d_depth + (int64_t)k0 * W * H;
-    const int64_t per = P.K == 1 ? 256 * kVoxelsPerThread1 : 256;
-    const int64_t nb = (n + per - 1) / per;
+    rc = frame_tiles(P, d_depth + (int64_t)k0 * W * H, P.K, ws + rayfac_bytes(W, H), ws + ws_bytes,
+                     s);
+    if (rc) return rc;
+    // one frame: up to eight bricks a wave, while that leaves 16384 waves
+    int bricks = 1;
+    if (P.K == 1)
+      while (bricks < 8 && (int64_t)X * Y * Z >= (int64_t)16384 * 256 * bricks * 2) bricks *= 2;
+    const int64_t nb = regions(X, Y, Z, kBrickZ * bricks);
     for (int64_t b0 = 0; b0 < nb; b0 += kMaxLaunchBlocks) {
       P.first_block = b0;
       const dim3 grid((unsigned)std::min(kMaxLaunchBlocks, nb - b0));
       if (P.K == 1)
-        hipLaunchKernelGGL(integrate1_kernel<DT>, grid, dim3(256), 0, s, P);
+        hipLaunchKernelGGL(integrate1_kernel<DT>, grid, dim3(256), 0, s, P, bricks);
       else
-        hipLaunchKernelGGL(integrate_kernel<DT>, grid, dim3(256), frames_lds_bytes(P.K), s, P);
+        hipLaunchKernelGGL(integrate_kernel<DT>, grid, dim3(256), 0, s, P);
       MCX_HIP(hipGetLastError());
     }
   }
@@ -922,8 +991,6 @@ float max_dtdd(const float* intr, float depth_scale, float trunc, int W, int H) 
     }
   return (float)(1.01 * m * (double)depth_scale / (double)trunc);
 }
-
-size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 extern "C" int mcx_integrate(void* d_vol, int X, int Y, int Z, float h, float trunc, int max_w,
                              const float* intr, const float* d_poses, const uint16_t* d_depth,
@@ -993,32 +1060,41 @@ extern "C" int mcx_integrate_tsdf(float* d_tsdf, int32_t* d_weight, int X, int Y
                                   void* stream) {
   if (!d_tsdf || !d_weight) return MCX_ERR_ARG;
   if (K > 0 && (!d_poses || !d_depth)) return MCX_ERR_ARG;
-  if (!d_ws || ws_bytes < mcx_integrate_workspace_size(W, H)) return MCX_ERR_WORKSPACE;
+  if (!d_ws || ws_bytes < rayfac_bytes(W, H)) return MCX_ERR_WORKSPACE;
   if (K == 0) return MCX_OK;
   hipStream_t s = as_stream(stream);
   IntegrateParams P;
+  char* const ws = static_cast<char*>(d_ws);
   int rc = prepare_integrate(P, X, Y, Z, h, trunc, max_w, intr, depth_scale, W, H, K,
-                             static_cast<float*>(d_ws), s);
+                             reinterpret_cast<float*>(ws));
   if (rc) return rc;
-  const int64_t n = (int64_t)X * Y * Z;
   for (int k0 = 0; k0 < K; k0 += kFramesPerPass) {
     P.K = K - k0 < kFramesPerPass ? K - k0 : kFramesPerPass;
     P.poses = d_poses + (int64_t)12 * k0;
     P.depth = d_depth + (int64_t)k0 * W * H;
-    const int64_t nb = (n + 255) / 256;
+    rc = frame_tiles(P, d_depth + (int64_t)k0 * W * H, P.K, ws + rayfac_bytes(W, H), ws + ws_bytes,
+                     s);
+    if (rc) return rc;
+    const int64_t nb = regions(X, Y, Z, kBrickZ);
     for (int64_t b0 = 0; b0 < nb; b0 += kMaxLaunchBlocks) {
       P.first_block = b0;
       hipLaunchKernelGGL(integrate_tsdf_kernel, dim3((unsigned)std::min(kMaxLaunchBlocks, nb - b0)),
-                         dim3(256), frames_lds_bytes(P.K), s, P, d_tsdf, d_weight);
+                         dim3(256), 0, s, P, d_tsdf, d_weight);
       MCX_HIP(hipGetLastError());
     }
   }
   return MCX_OK;
 }
 
+// Ray factors, max |g| and the accumulators of `frames` frames: what the
+// backward cannot run without (its workspace ends with the tile tables).
+size_t backward_bytes(int W, int H, int64_t frames) {
+  return al256((size_t)W * H * sizeof(float)) + 256 + (size_t)frames * W * H * 8;
+}
+
 extern "C" size_t mcx_integrate_tsdf_backward_workspace_size(int W, int H, int K) {
   if (W < 1 || H < 1 || K < 0) return 0;
-  return al256((size_t)W * H * sizeof(float)) + 256 + (size_t)K * W * H * 8;
+  return backward_bytes(W, H, K) + 256 + tile_bytes(W, H) * K;
 }
 
 extern "C" int mcx_integrate_tsdf_backward(const float* d_grad_tsdf, const int32_t* d_weight0,
@@ -1029,7 +1105,7 @@ extern "C" int mcx_integrate_tsdf_backward(const float* d_grad_tsdf, const int32
                                            size_t ws_bytes, void* stream) {
   if (!d_grad_tsdf) return MCX_ERR_ARG;
   if (K > 0 && (!d_poses || !d_depth || !d_grad_depth)) return MCX_ERR_ARG;
-  if (!d_ws || ws_bytes < mcx_integrate_tsdf_backward_workspace_size(W, H, K))
+  if (!d_ws || ws_bytes < (W < 1 || H < 1 || K < 0 ? 0 : backward_bytes(W, H, K)))
     return MCX_ERR_WORKSPACE;
   if (K == 0) return MCX_OK;
   if (K > kFramesPerPass) return MCX_ERR_UNSUPPORTED;  // one pass: weights known per voxel
@@ -1040,7 +1116,9 @@ extern "C" int mcx_integrate_tsdf_backward(const float* d_grad_tsdf, const int32
   unsigned long long* acc = reinterpret_cast<unsigned long long*>(
       b + al256((size_t)W * H * sizeof(float)) + 256);
   IntegrateParams P;
-  int rc = prepare_integrate(P, X, Y, Z, h, trunc, max_w, intr, depth_scale, W, H, K, rayfac, s);
+  int rc = prepare_integrate(P, X, Y, Z, h, trunc, max_w, intr, depth_scale, W, H, K, rayfac);
+  if (rc) return rc;
+  rc = frame_tiles(P, d_depth, K, b + backward_bytes(W, H, K), b + ws_bytes, s);
   if (rc) return rc;
   const int64_t n = (int64_t)X * Y * Z;
   const int64_t npix = (int64_t)K * W * H;
@@ -1054,12 +1132,19 @@ extern "C" int mcx_integrate_tsdf_backward(const float* d_grad_tsdf, const int32
   P.K = K;
   P.poses = d_poses;
   P.depth = d_depth;
-  const int64_t nb = (n + 255) / 256;
+  // One plane a wave below 2^23 voxels: few bricks hold a surface there, and
+  // each one's frames run in series.
+  const bool small = n < ((int64_t)1 << 23);
+  const int64_t nb = regions(X, Y, Z, small ? 1 : kBrickZ);
   for (int64_t b0 = 0; b0 < nb; b0 += kMaxLaunchBlocks) {
     P.first_block = b0;
-    hipLaunchKernelGGL(integrate_tsdf_backward_kernel,
-                       dim3((unsigned)std::min(kMaxLaunchBlocks, nb - b0)), dim3(256),
-                       frames_lds_bytes(K), s, P, d_grad_tsdf, d_weight0, maxg, mdt, acc);
+    const dim3 grid((unsigned)std::min(kMaxLaunchBlocks, nb - b0));
+    if (small)
+      hipLaunchKernelGGL(integrate_tsdf_backward_kernel<1>, grid, dim3(256), 0, s, P, d_grad_tsdf,
+                         d_weight0, maxg, mdt, acc);
+    else
+      hipLaunchKernelGGL(integrate_tsdf_backward_kernel<kBrickZ>, grid, dim3(256), 0, s, P,
+                         d_grad_tsdf, d_weight0, maxg, mdt, acc);
     MCX_HIP(hipGetLastError());
   }
   hipLaunchKernelGGL(fixed_to_float_kernel, dim3(blocks_for(npix)), dim3(256), 0, s, acc, npix,
@@ -1069,6 +1154,15 @@ extern "C" int mcx_integrate_tsdf_backward(const float* d_grad_tsdf, const int32
 }
 
 // ---- batched fp32 fusion (no counterpart in the reference) ----------------
+// Volumes of a batch whose K tile tables fit the workspace together (all of
+// them when not even one volume's do: they then run without).
+int volumes_per_turn(char* tables, char* end, int W, int H, int K, int nvol) {
+  tables = reinterpret_cast<char*>(al256(reinterpret_cast<uintptr_t>(tables)));
+  const int64_t fit =
+      tables < end ? (int64_t)((size_t)(end - tables) / tile_bytes(W, H)) / K : 0;
+  return fit < 1 ? nvol : (int)std::min<int64_t>(fit, nvol);
+}
+
 extern "C" int mcx_integrate_tsdf_batched(const mcx_batch* plan, float* d_tsdf, int32_t* d_weight,
                                           int from_init, float init_value, float trunc,
                                           int max_w, const float* intr, const float* d_poses,
@@ -1078,7 +1172,7 @@ extern "C" int mcx_integrate_tsdf_batched(const mcx_batch* plan, float* d_tsdf, 
   if (plan->elem != MCX_ELEM_F32) return MCX_ERR_ARG;
   if (K > 0 && (!d_poses || !d_depth)) return MCX_ERR_ARG;
   if (K > kFramesPerPass) return MCX_ERR_UNSUPPORTED;
-  if (!d_ws || ws_bytes < mcx_integrate_workspace_size(W, H)) return MCX_ERR_WORKSPACE;
+  if (!d_ws || ws_bytes < rayfac_bytes(W, H)) return MCX_ERR_WORKSPACE;
   hipStream_t s = as_stream(stream);
   if (K == 0) {
     if (!from_init) return MCX_OK;
@@ -1091,7 +1185,7 @@ extern "C" int mcx_integrate_tsdf_batched(const mcx_batch* plan, float* d_tsdf, 
   if (plan->blocks >= ((int64_t)1 << 31)) return MCX_ERR_UNSUPPORTED;
   BatchIntegrateParams B;
   int rc = prepare_integrate(B.base, 1, 1, 1, 1.0f, trunc, max_w, intr, depth_scale, W, H, K,
-                             static_cast<float*>(d_ws), s);
+                             static_cast<float*>(d_ws));
   if (rc) return rc;
   B.base.K = K;
   B.base.poses = d_poses;
@@ -1100,12 +1194,24 @@ extern "C" int mcx_integrate_tsdf_batched(const mcx_batch* plan, float* d_tsdf, 
   B.nvol = plan->nvol;
   B.from_init = from_init ? 1 : 0;
   B.init_value = init_value;
-  for (int64_t b0 = 0; b0 < plan->blocks; b0 += kMaxLaunchBlocks) {
-    B.first_block = b0;
-    hipLaunchKernelGGL(integrate_tsdf_batched_kernel,
-                       dim3((unsigned)std::min(kMaxLaunchBlocks, plan->blocks - b0)), dim3(256),
-                       frames_lds_bytes(K), s, B, d_tsdf, d_weight);
-    MCX_HIP(hipGetLastError());
+  // volumes in turn of as many as the workspace holds tile tables for
+  char* const ws = static_cast<char*>(d_ws);
+  const int64_t pixels = (int64_t)W * H * K;
+  const int turn = volumes_per_turn(ws + rayfac_bytes(W, H), ws + ws_bytes, W, H, K, plan->nvol);
+  for (int v0 = 0; v0 < plan->nvol; v0 += turn) {
+    const int v1 = std::min(plan->nvol, v0 + turn);
+    rc = frame_tiles(B.base, d_depth + v0 * pixels, (int64_t)(v1 - v0) * K,
+                     ws + rayfac_bytes(W, H), ws + ws_bytes, s);
+    if (rc) return rc;
+    B.tiled_vol = v0;
+    const int64_t end = plan->blk_begin[v1];
+    for (int64_t b0 = plan->blk_begin[v0]; b0 < end; b0 += kMaxLaunchBlocks) {
+      B.first_block = b0;
+      hipLaunchKernelGGL(integrate_tsdf_batched_kernel,
+                         dim3((unsigned)std::min(kMaxLaunchBlocks, end - b0)), dim3(256), 0, s, B,
+                         d_tsdf, d_weight);
+      MCX_HIP(hipGetLastError());
+    }
   }
   return MCX_OK;
 }
@@ -1113,7 +1219,8 @@ extern "C" int mcx_integrate_tsdf_batched(const mcx_batch* plan, float* d_tsdf, 
 extern "C" size_t mcx_integrate_tsdf_backward_batched_workspace_size(const mcx_batch* plan, int W,
                                                                      int H, int K) {
   if (!plan || W < 1 || H < 1 || K < 0) return 0;
-  return al256((size_t)W * H * sizeof(float)) + 256 + (size_t)plan->nvol * K * W * H * 8;
+  return backward_bytes(W, H, (int64_t)plan->nvol * K) + 256 +
+         tile_bytes(W, H) * plan->nvol * K;
 }
 
 extern "C" int mcx_integrate_tsdf_backward_batched(const mcx_batch* plan,
@@ -1128,7 +1235,8 @@ extern "C" int mcx_integrate_tsdf_backward_batched(const mcx_batch* plan,
   if (!plan || !d_grad_tsdf) return MCX_ERR_ARG;
   if (plan->elem != MCX_ELEM_F32) return MCX_ERR_ARG;
   if (K > 0 && (!d_poses || !d_depth || !d_grad_depth)) return MCX_ERR_ARG;
-  if (!d_ws || ws_bytes < mcx_integrate_tsdf_backward_batched_workspace_size(plan, W, H, K))
+  if (!d_ws ||
+      ws_bytes < (W < 1 || H < 1 || K < 0 ? 0 : backward_bytes(W, H, (int64_t)plan->nvol * K)))
     return MCX_ERR_WORKSPACE;
   if (K == 0) return MCX_OK;
   if (K > kFramesPerPass) return MCX_ERR_UNSUPPORTED;
@@ -1141,8 +1249,12 @@ extern "C" int mcx_integrate_tsdf_backward_batched(const mcx_batch* plan,
       b + al256((size_t)W * H * sizeof(float)) + 256);
   BatchIntegrateParams B;
   int rc = prepare_integrate(B.base, 1, 1, 1, 1.0f, trunc, max_w, intr, depth_scale, W, H, K,
-                             rayfac, s);
+                             rayfac);
   if (rc) return rc;
+  rc = frame_tiles(B.base, d_depth, (int64_t)plan->nvol * K,
+                   b + backward_bytes(W, H, (int64_t)plan->nvol * K), b + ws_bytes, s);
+  if (rc) return rc;
+  B.tiled_vol = 0;
   const int64_t npix = (int64_t)plan->nvol * K * W * H;
   if (d_maxabs) {
     rc = fill_bytes_zero(acc, (size_t)npix * 8, s);  // the accumulators
@@ -1169,7 +1281,7 @@ extern "C" int mcx_integrate_tsdf_backward_batched(const mcx_batch* plan,
     B.first_block = b0;
     hipLaunchKernelGGL(integrate_tsdf_backward_batched_kernel,
                        dim3((unsigned)std::min(kMaxLaunchBlocks, plan->blocks - b0)), dim3(256),
-                       frames_lds_bytes(K), s, B, d_grad_tsdf, d_weight0, mg, mdt, acc);
+                       0, s, B, d_grad_tsdf, d_weight0, mg, mdt, acc);
     MCX_HIP(hipGetLastError());
   }
   hipLaunchKernelGGL(fixed_to_float_kernel, dim3(blocks_for(npix)), dim3(256), 0, s, acc, npix,

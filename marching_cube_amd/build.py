@@ -112,6 +112,7 @@ def build_dropin():
 
 TEST_BIN = os.path.join(ROOT, "tests", "cpp", "test_dropin")
 EXACT_DIV_BIN = os.path.join(ROOT, "tests", "cpp", "exact_div_check")
+EXACT_FORMS_BIN = os.path.join(ROOT, "tests", "cpp", "exact_forms_check")
 
 
 def build_tests():
@@ -123,9 +124,9 @@ def build_tests():
           "-D__HIP_PLATFORM_AMD__", "-o", TEST_BIN, src, "-L", PKG, "-lmarching_cube_amd",
           "-lmcx", "-Wl,-rpath,$ORIGIN/../../marching_cube_amd", "-L/opt/rocm/lib",
           "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib"])
-    # device check of the exact fp32 forms (same flags as the library)
-    chk = os.path.join(ROOT, "tests", "cpp", "exact_div_check.hip")
-    _run([HIPCC, *HIP_FLAGS, "-I", INCLUDE, "-I", CSRC, "-o", EXACT_DIV_BIN, chk])
+    # device checks of the exact fp32 forms (same flags as the library)
+    for chk in (EXACT_DIV_BIN, EXACT_FORMS_BIN):
+        _run([HIPCC, *HIP_FLAGS, "-I", INCLUDE, "-I", CSRC, "-o", chk, chk + ".hip"])
     return TEST_BIN
 
 

@@ -49,6 +49,36 @@ __device__ __forceinline__ float div_weight_short2(float num, float den) {
   return __fmaf_rn(__fmaf_rn(-den, q, num), r, q);
 }
 
+// 1 / b correctly rounded for normal b with a normal reciprocal: the hardware
+// reciprocal refined by one Newton step (equal to IEEE division for all 2^23
+// significands; tests/cpp/exact_forms_check.hip checks them on the device).
+__device__ __forceinline__ float recip_rn(float b) {
+  const float r = __builtin_amdgcn_rcpf(b);
+  return __fmaf_rn(__fmaf_rn(-b, r, 1.0f), r, r);
+}
+
+// a / b correctly rounded from r = recip_rn(b), one multiply and one fused
+// correction, where no intermediate result leaves the normal range
+// (2^-60 <= |b| <= 2^60 and a = 0 or 2^-60 <= |a| <= 2^60 will do).
+// Before its last rounding the result is within 1.5 * 2^-47 (quotients below
+// 1; 2.5 * 2^-47 above) of a / b, times the quotient; a quotient that close to
+// the middle of two floats has |2^25 A - (2 M + 1) B| <= 6 for the 24-bit
+// significands A, B and M, and the same test solves that congruence for every
+// B and checks the 93 million pairs with |...| <= 16 against IEEE division.
+__device__ __forceinline__ float div_rn(float a, float b, float r) {
+  const float q = a * r;
+  return __fmaf_rn(__fmaf_rn(-b, q, a), r, q);
+}
+
+// sqrt(x) correctly rounded for normal x in [2^-100, 2^100]: one Newton step
+// from the hardware's reciprocal square root (equal to IEEE sqrt on all 2^24
+// floats of [1, 4); checked by the same device test).
+__device__ __forceinline__ float sqrt_rn(float x) {
+  const float y = __builtin_amdgcn_rsqf(x);
+  const float g = x * y;
+  return __fmaf_rn(__fmaf_rn(-g, g, x), 0.5f * y, g);
+}
+
 // ---------------------------------------------------------------- host side
 // Map a HIP error to a status code; keep the first HIP error for strerror.
 int hip_status(hipError_t e);

@@ -2294,13 +2294,19 @@ extern "C" int mcx_batch_create(mcx_batch** out, int nvol, const int* dims_xyz, 
   int64_t tb = 0, cubes = 0, voxels = 0, blocks = 0, gblocks = 0;
   int maxX = 1;
   bool wide = true;
+  // integration workgroups take one brick of 8 x 8 x 4 voxels a wave, or four
+  // above one another where that leaves 16 waves per SIMD (2^24 voxels)
+  double all = 0;
+  for (int b = 0; b < nvol; ++b)
+    all += (double)dims_xyz[3 * b] * dims_xyz[3 * b + 1] * dims_xyz[3 * b + 2];
+  const int bricks = all >= (double)(1 << 24) ? 4 : 1;
   for (int b = 0; b < nvol; ++b) {
     const int X = dims_xyz[3 * b], Y = dims_xyz[3 * b + 1], Z = dims_xyz[3 * b + 2];
     if (X < 1 || Y < 1 || Z < 1 || !d_vols[b]) return MCX_ERR_ARG;
     if (!size_ok(X, Y, Z)) return MCX_ERR_UNSUPPORTED;
     vols[b] = make_vol(d_vols[b], X, Y, Z, h[b], nullptr, tb);
     const int64_t nv = (int64_t)X * Y * Z;
-    const int rx = (X + 31) / 32, ry = (Y + 7) / 8, rz = (Z + 3) / 4;  // 32 x 8 x 4 voxels each
+    const int rx = (X + 31) / 32, ry = (Y + 7) / 8, rz = (Z + 4 * bricks - 1) / (4 * bricks);
     bvol[b] = BatchVol{X, Y, Z, h[b], voxels, blocks, gblocks, FastDiv((uint32_t)rx),
                        FastDiv((uint32_t)ry)};
     blk_begin[b] = blocks;
@@ -2336,6 +2342,7 @@ extern "C" int mcx_batch_create(mcx_batch** out, int nvol, const int* dims_xyz, 
   p->voxels = voxels;
   p->blocks = blk_begin[nvol] = blocks;
   p->blk_begin = std::move(blk_begin);
+  p->bricks = bricks;
   p->gather_blocks = gblocks;
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&p->d_vols), sizeof(VolDesc) * nvol);
   if (e == hipSuccess)

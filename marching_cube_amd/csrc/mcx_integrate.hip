@@ -59,14 +59,16 @@ struct IntegrateParams {
   const float* poses;      // [K][12] device
   const void* depth;       // [K][H][W] device, uint16 or float
   const float* rayfac;     // [H][W]
-  const float2* tiles;     // [tiled][TY][TX]: a tile's (largest, smallest) ray distance
+  const float2* tiles;     // per tiled frame: [TY][TX] tiles, then [TY1][TX1] large tiles,
+                           // each (largest, smallest) ray distance
   float depth_scale;
   int W, H, K;
-  int TX, TY;              // tiles of kTile x kTile pixels
+  int TX, TY, TX1, TY1;    // tiles of kTile x kTile pixels; of 4 x 4 tiles
   int tiled;               // frames [0, tiled) have a tile table
   int plain;               // camera, scale and truncation within the fast forms' ranges
   FastDiv divX, divY;      // workgroups along x and y of the volume
-  int64_t first_block;     // workgroup index of this launch's blockIdx.x 0
+  int64_t first_block;     // region of this launch's first workgroup
+  int log2_run;            // regions in a row of one XCD
 };
 
 // Ray-length factor sqrt(((u-cx)/fx)^2 + ((v-cy)/fy)^2 + 1) of a pixel
@@ -78,21 +80,25 @@ __device__ __forceinline__ float ray_factor(int u, int v, float fx, float fy, fl
 
 // Largest and smallest measured ray distance (depth * scale * factor, the
 // voxels' own operations; pixels without a measurement do not count) of every
-// kTile x kTile pixels of the window [0, W-2) x [0, H-2) that voxels can
-// observe: (0, inf) where a tile holds none.  A wave takes eight tiles of a
-// tile row, a lane eight pixels of one image row, for every gridDim.z-th
-// frame; the ray factors are computed once per lane and written for the
-// integration by the waves of blockIdx.z = 0.  Tiles of 8 pixels: an
+// 8 x 8 pixels, and of every 32 x 32, of the window [0, W-2) x [0, H-2) that
+// voxels can observe: (0, inf) where a tile holds none.  A wave takes eight
+// tiles of a tile row, a lane eight pixels of one image row, and the four
+// waves of a workgroup four tile rows (two large tiles), for every
+// gridDim.z-th frame; the ray factors are computed once per lane and written
+// for the integration by the waves of blockIdx.z = 0.  Tiles of 8 pixels: an
 // 8 x 8 x 4 brick of a 512^3 scan covers about 14 pixels, so 3 x 3 tiles.
-constexpr int kTile = 8;
+constexpr int kTile = 8, kTiles1 = 4;  // pixels a tile, tiles a large tile (each way)
 template <typename DT>
-__global__ __launch_bounds__(64) void frame_tiles_kernel(const DT* __restrict__ depth, float scale,
-                                                         int W, int H, int frames, float fx,
-                                                         float fy, float cx, float cy,
-                                                         float* rayfac, int TX, int TY,
-                                                         int first_ty, int vec, float2* tiles) {
-  const int lane = threadIdx.x;
-  const int tx = blockIdx.x * 8 + (lane & 7), ty = first_ty + blockIdx.y;
+__global__ __launch_bounds__(256) void frame_tiles_kernel(const DT* __restrict__ depth,
+                                                          float scale, int W, int H, int frames,
+                                                          float fx, float fy, float cx, float cy,
+                                                          float* rayfac, int TX, int TY, int TX1,
+                                                          int TY1, int first_row, int vec,
+                                                          float2* tiles) {
+  __shared__ float2 s_quad[2][4][2];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row1 = first_row + blockIdx.y;
+  const int tx = blockIdx.x * 8 + (lane & 7), ty = row1 * kTiles1 + wave;
   const int u0 = tx * kTile, v = ty * kTile + (lane >> 3);
   float rf[kTile];
 #pragma unroll
@@ -100,7 +106,8 @@ __global__ __launch_bounds__(64) void frame_tiles_kernel(const DT* __restrict__ 
     rf[i] = ray_factor(u0 + i, v, fx, fy, cx, cy);
     if (blockIdx.z == 0 && v < H && u0 + i < W) rayfac[(int64_t)v * W + u0 + i] = rf[i];
   }
-  for (int k = blockIdx.z; k < frames; k += gridDim.z) {
+  int buf = 0;
+  for (int k = blockIdx.z; k < frames; k += gridDim.z, buf ^= 1) {
     const DT* row = depth + (int64_t)k * W * H + (int64_t)v * W + u0;
     DT d[kTile];
     if (vec) {  // W a multiple of 8 and 16-byte aligned frames: whole 16-byte words
@@ -127,7 +134,24 @@ __global__ __launch_bounds__(64) void frame_tiles_kernel(const DT* __restrict__ 
       hi = fmaxf(hi, __shfl_xor(hi, o));
       lo = fminf(lo, __shfl_xor(lo, o));
     }
-    if (lane < 8 && tx < TX) tiles[((int64_t)k * TY + ty) * TX + tx] = make_float2(hi, lo);
+    float2* const T = tiles + (int64_t)k * (TX * TY + TX1 * TY1);
+    if (lane < 8 && tx < TX && ty < TY) T[ty * TX + tx] = make_float2(hi, lo);
+#pragma unroll
+    for (int o = 1; o < kTiles1; o <<= 1) {
+      hi = fmaxf(hi, __shfl_xor(hi, o));
+      lo = fminf(lo, __shfl_xor(lo, o));
+    }
+    // two buffers: a wave may be one frame ahead of the two lanes that read
+    if (lane == 0 || lane == 4) s_quad[buf][wave][lane >> 2] = make_float2(hi, lo);
+    __syncthreads();
+    if (threadIdx.x < 2) {
+      for (int w = 0; w < 4; ++w) {
+        hi = fmaxf(w ? hi : 0.0f, s_quad[buf][w][threadIdx.x].x);
+        lo = fminf(w ? lo : INFINITY, s_quad[buf][w][threadIdx.x].y);
+      }
+      const int tx1 = blockIdx.x * 2 + threadIdx.x;
+      if (tx1 < TX1) T[TX * TY + row1 * TX1 + tx1] = make_float2(hi, lo);
+    }
   }
 }
 
@@ -166,120 +190,116 @@ __device__ __forceinline__ float frame_rayfac(const IntegrateParams& P, uint32_t
 constexpr int kBrick = 8, kBrickZ = 4;
 constexpr int kRegionX = 4 * kBrick;  // a workgroup's four bricks lie side by side in x
 
-// Reductions over the eight lanes of a frame (all 64 lanes active).
-template <int CTRL>
-__device__ __forceinline__ float dpp_f32(float v) {
-  return __builtin_bit_cast(
-      float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
-constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141;
-__device__ __forceinline__ float min8(float v) {
-  v = fminf(v, dpp_f32<kDppXor1>(v));
-  v = fminf(v, dpp_f32<kDppXor2>(v));
-  return fminf(v, dpp_f32<kDppHalfMirror>(v));
-}
-__device__ __forceinline__ float max8(float v) {
-  v = fmaxf(v, dpp_f32<kDppXor1>(v));
-  v = fmaxf(v, dpp_f32<kDppXor2>(v));
-  return fmaxf(v, dpp_f32<kDppHalfMirror>(v));
-}
-
-// What a box of voxel centres has to do with a frame: kSkip, no voxel can
-// observe it; else kFast, the box is well in front of the camera (the quick
-// exact arithmetic applies); with it kInside, every voxel is seen at a pixel
-// of the window, and kFree, every measured pixel in sight lies at least
-// trunc in front of every voxel (observations are +1 or none).  Eight lanes
-// take a frame, lane c one corner (bit 0 of c: the far x, bit 1: y, bit
-// 2: z), with the voxels' own fp32 operations (a corner is a voxel centre) up
-// to the quotients, which come from the hardware reciprocal (error within
-// 2e-7 |u - cx| plus an ulp).
-//   Out of view: the whole box is behind the camera, or in front of it (every
-// corner deeper than 1 cm) and projecting past one edge of the pixel window:
-// the image of a convex box in front of the camera is the convex hull of its
-// corners' images.
-//   Behind what was measured: with the box in front of the camera, its pixels
-// lie in the rectangle of its corners' images; the largest ray distance z
-// measured there (the tiles that meet the rectangle) and a lower bound q of
-// the voxels' distances give sdf <= z - q (the subtraction rounds
-// monotonically), and nothing is updated where that is below -trunc_neg, or
-// where nothing was measured at all.  q is the least corner coordinate along
-// the direction n of the box's centre (|n| <= 1, so |q(p)| >= q(p) . n, which
-// is linear in p).
-// Margins: a voxel's fp32 q differs from the exact one by at most
-// d = 4e-7 * (|dx| + |dy| + |dz|) per component (the subtraction and the fma
-// chain, |R| <= 1), so its u differs from the exact projection by at most
-// (fx d / qz_min) (1 + |u - cx|_max / fx), likewise v; the tests use four
-// times that plus one pixel as the margin ("behind": every corner below
-// -max(1e-4 m, 4 d)); the pixel covers the reciprocal's error wherever a test
-// is close (|u|, |v| < 2^16: under 0.02 pixel) and the rounding to the
-// nearest pixel.  Distances differ by less than 1e-6 (|dx| + |dy| + |dz|),
-// taken four times over.  So every voxel of a skipped frame would have taken
-// its q.z, window, dropout or -trunc_neg skip.
-// Boxes over more than 8 x 8 tiles are not tested against them.  kFree is the
-// same argument from the other side: the least distance measured in the
-// rectangle against the largest of the corners' distances (|q| is convex).
+// What a brick has to do with a frame: kSkip, no voxel can observe it; else
+// kFast, the brick is well in front of the camera (the quick exact arithmetic
+// applies); with it kInside, every voxel is seen at a pixel of the window, and
+// kFree, every measured pixel in sight lies at least trunc in front of every
+// voxel (observations are +1 or none).  One lane decides for one brick and
+// frame, 64 of them at once (eight lanes per frame, one box corner each, took
+// eight times the instructions, half of a 300-frame sweep's: 15.8 -> 12.6 ms).
+//   The box of voxel centres maps to a parallelepiped around the centre's
+// q = R^T (p - t), with half extents e = |R^T| (half sides) per component.
+// Out of view: wholly behind the camera, or in front of it (every point deeper
+// than 1 cm) and past one edge of the pixel window; a point's image differs
+// from the centre's by |qx / qz - cx / cz| <= (ex + |cx / cz| ez) / (cz - ez)
+// times fx, likewise v.
+//   Behind what was measured: the largest ray distance z measured in that
+// rectangle of pixels (the tiles that meet it) and a lower bound q of the
+// voxels' distances give sdf <= z - q (the subtraction rounds monotonically),
+// and nothing is updated where that is below -trunc_neg, or where nothing was
+// measured at all.  q is the least value of q(p) . n over the box, n the
+// direction of its centre (|n| = 1, so |q(p)| >= q(p) . n, linear in p).
+//   kFree is the same argument from the other side: the least distance
+// measured against the centre's plus the half diagonal of e.
+// Margins: a voxel's fp32 q, and the box's, differ from the exact one by at
+// most d = 4e-7 * (|dx| + |dy| + |dz| + |p| + half sides) per component (the
+// coordinates, the subtraction and the fma chain, |R| <= 1), which widens e;
+// the rectangle is wider by one pixel, for the rounding to the nearest pixel
+// and the hardware reciprocals (|u|, |v| < 2^16: under 0.02 pixel).  Distances
+// differ by less than 1e-6 of the same sum, taken four times over.  So every
+// voxel of a skipped frame would have taken its q.z, window, dropout or
+// -trunc_neg skip.
+// Rectangles of up to 4 x 4 tiles are read from the table of 8-pixel tiles,
+// larger ones from the 32-pixel tiles; beyond that nothing is known of the
+// depth.
 constexpr int kSkip = 1, kFast = 2, kInside = 4, kFree = 8;
-__device__ int test_box(const IntegrateParams& P, const float* R, int k, float px, float py,
-                        float pz) {
+template <int NZ>
+__device__ int test_brick(const IntegrateParams& P, int x0, int y0, int z0, int k) {
+  const float* R = P.poses + 12 * k;
+  // box of voxel centres
+  const float wx = (float)(min(kBrick, P.X - x0) - 1), wy = (float)(min(kBrick, P.Y - y0) - 1),
+              wz = (float)(min(NZ, P.Z - z0) - 1);
+  const float hx = 0.5f * wx * P.h, hy = 0.5f * wy * P.h, hz = 0.5f * wz * P.h;
+  const float px = ((float)x0 + 0.5f + 0.5f * wx) * P.h, py = ((float)y0 + 0.5f + 0.5f * wy) * P.h,
+              pz = ((float)z0 + 0.5f + 0.5f * wz) * P.h;
+  const float r0 = R[0], r1 = R[1], r2 = R[2], r3 = R[3], r4 = R[4], r5 = R[5], r6 = R[6],
+              r7 = R[7], r8 = R[8];
   const float dx = px - R[9], dy = py - R[10], dz = pz - R[11];
-  const float dmax = max8(fabsf(dx) + fabsf(dy) + fabsf(dz));
-  const float qx = __fmaf_rn(R[6], dz, __fmaf_rn(R[3], dy, R[0] * dx));
-  const float qy = __fmaf_rn(R[7], dz, __fmaf_rn(R[4], dy, R[1] * dx));
-  const float qz = __fmaf_rn(R[8], dz, __fmaf_rn(R[5], dy, R[2] * dx));
-  const float qzmin = min8(qz), qzmax = max8(qz);
-  const float d = 4e-7f * dmax;  // bound on a voxel's fp32 error in q
-  if (qzmax < -fmaxf(1e-4f, 4.0f * d)) return kSkip;
-  const float rz = __builtin_amdgcn_rcpf(qz);
-  const float u = __fmaf_rn(P.fx, qx * rz, P.cx), v = __fmaf_rn(P.fy, qy * rz, P.cy);
-  float umin = min8(u), umax = max8(u), vmin = min8(v), vmax = max8(v);
-  // the opposite corner sits in lane 7 - c: the sum is twice the centre
-  const float nx = qx + dpp_f32<kDppHalfMirror>(qx), ny = qy + dpp_f32<kDppHalfMirror>(qy),
-              nz = qz + dpp_f32<kDppHalfMirror>(qz);
-  const float rn = __builtin_amdgcn_rsqf(__fmaf_rn(nz, nz, __fmaf_rn(ny, ny, nx * nx)));
-  const float near = min8(__fmaf_rn(qz, nz, __fmaf_rn(qy, ny, qx * nx)) * rn);
-  const float far = max8(__builtin_amdgcn_sqrtf(__fmaf_rn(qz, qz, __fmaf_rn(qy, qy, qx * qx))));
-  if (!(qzmin > 0.01f)) return 0;
-  // margins from reciprocals (relative error ~1e-7 in a bound taken four
-  // times over)
-  const float rq = __builtin_amdgcn_rcpf(qzmin);
-  const float fx = fabsf(P.fx), fy = fabsf(P.fy);
-  const float au = fmaxf(fabsf(umin - P.cx), fabsf(umax - P.cx)) * __builtin_amdgcn_rcpf(fx);
-  const float av = fmaxf(fabsf(vmin - P.cy), fabsf(vmax - P.cy)) * __builtin_amdgcn_rcpf(fy);
-  const float tu = 1.0f + 4.0f * (fx * d * rq) * (1.0f + au);
-  const float tv = 1.0f + 4.0f * (fy * d * rq) * (1.0f + av);
-  // a voxel is observed only at rint(u) in [0, W - 2), rint(v) in [0, H - 2)
-  if (umax < -0.5f - tu || umin > (float)P.W - 2.5f + tu || vmax < -0.5f - tv ||
-      vmin > (float)P.H - 2.5f + tv)
-    return kSkip;
+  const float sum = fabsf(dx) + fabsf(dy) + fabsf(dz) + (px + hx) + (py + hy) + (pz + hz);
+  const float d = 4e-7f * sum;
+  const float qx = __fmaf_rn(r6, dz, __fmaf_rn(r3, dy, r0 * dx));
+  const float qy = __fmaf_rn(r7, dz, __fmaf_rn(r4, dy, r1 * dx));
+  const float qz = __fmaf_rn(r8, dz, __fmaf_rn(r5, dy, r2 * dx));
+  const float ex = __fmaf_rn(fabsf(r6), hz, __fmaf_rn(fabsf(r3), hy, __fmaf_rn(fabsf(r0), hx, d)));
+  const float ey = __fmaf_rn(fabsf(r7), hz, __fmaf_rn(fabsf(r4), hy, __fmaf_rn(fabsf(r1), hx, d)));
+  const float ez = __fmaf_rn(fabsf(r8), hz, __fmaf_rn(fabsf(r5), hy, __fmaf_rn(fabsf(r2), hx, d)));
+  if (qz + ez < -fmaxf(1e-4f, 4.0f * d)) return kSkip;
+  const float zlo = qz - ez;
+  if (!(zlo > 0.01f)) return 0;
+  const float rz = __builtin_amdgcn_rcpf(qz), rl = __builtin_amdgcn_rcpf(zlo);
+  const float tx = qx * rz, ty = qy * rz;
+  const float u = __fmaf_rn(P.fx, tx, P.cx), v = __fmaf_rn(P.fy, ty, P.cy);
+  const float du = __fmaf_rn(fabsf(P.fx) * 1.00001f, __fmaf_rn(fabsf(tx), ez, ex) * rl, 1.0f);
+  const float dv = __fmaf_rn(fabsf(P.fy) * 1.00001f, __fmaf_rn(fabsf(ty), ez, ey) * rl, 1.0f);
+  const float wu = (float)(P.W - 3), wv = (float)(P.H - 3);  // the window's last pixel
+  float u0 = u - du, u1 = u + du, v0 = v - dv, v1 = v + dv;
+  if (u1 < 0.0f || u0 > wu || v1 < 0.0f || v0 > wv) return kSkip;
   int cls = 0;
-  if (P.plain && qzmin > 16.0f * d && dmax < 0x1p30f) {
+  if (P.plain && sum < 0x1p30f) {
     cls = kFast;
-    if (umin >= tu && umax <= (float)(P.W - 3) - tu && vmin >= tv && vmax <= (float)(P.H - 3) - tv)
+    if (u0 >= 0.0f && u1 <= wu && v0 >= 0.0f && v1 <= wv && wx == (float)(kBrick - 1) &&
+        wy == (float)(kBrick - 1) && wz == (float)(NZ - 1))
       cls |= kInside;
   }
   if (k >= P.tiled) return cls;
-  umin = fmaxf(umin - tu, 0.0f);
-  vmin = fmaxf(vmin - tv, 0.0f);
-  umax = fminf(umax + tu, (float)(P.W - 3));
-  vmax = fminf(vmax + tv, (float)(P.H - 3));
-  if (!(umin <= umax && vmin <= vmax)) return cls;  // (NaN) not decided here
-  const int tx0 = (int)umin / kTile, tx1 = (int)umax / kTile;
-  const int ty0 = (int)vmin / kTile, ty1 = (int)vmax / kTile;
-  if (tx1 - tx0 > 7 || ty1 - ty0 > 7) return cls;
-  const int c = threadIdx.x & 7;
+  u0 = fmaxf(u0, 0.0f);
+  v0 = fmaxf(v0, 0.0f);
+  u1 = fminf(u1, wu);
+  v1 = fminf(v1, wv);
+  if (!(u0 <= u1 && v0 <= v1)) return cls;  // (NaN) not decided here
+  const float2* T = P.tiles + (int64_t)k * (P.TX * P.TY + P.TX1 * P.TY1);
+  int a0 = (int)u0 / kTile, a1 = (int)u1 / kTile, b0 = (int)v0 / kTile, b1 = (int)v1 / kTile;
+  int stride = P.TX;
+  if (a1 - a0 > 3 || b1 - b0 > 3) {
+    a0 /= 4;
+    a1 /= 4;
+    b0 /= 4;
+    b1 /= 4;
+    T += P.TX * P.TY;
+    stride = P.TX1;
+    if (a1 - a0 > 3 || b1 - b0 > 3) return cls;
+  }
+  // two rows of four tiles (the last ones again where there are fewer) in
+  // flight together: a loop over single tiles waits for each
   float most = 0.0f, least = INFINITY;
-  const float2* T = P.tiles + (int64_t)k * P.TY * P.TX;
-  for (int ty = ty0 + (c >> 2); ty <= ty1; ty += 2)
-    for (int tx = tx0 + (c & 3); tx <= tx1; tx += 4) {
-      const float2 t = T[ty * P.TX + tx];
+  for (int b = b0; b <= b1; ++b)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float2 t = T[b * stride + min(a0 + i, a1)];
       most = fmaxf(most, t.x);
       least = fminf(least, t.y);
     }
-  most = max8(most);
-  least = min8(least);
-  const float margin = 4e-6f * dmax;
-  if (most == 0.0f || most - (near - margin) < -P.trunc_neg) return kSkip;
-  if ((cls & kFast) && least - (far + margin) >= P.trunc) cls |= kFree;
+  const float n2 = __fmaf_rn(qz, qz, __fmaf_rn(qy, qy, qx * qx));
+  const float rn = __builtin_amdgcn_rsqf(n2), dist = n2 * rn;
+  const float sx = fabsf(__fmaf_rn(qz, r2, __fmaf_rn(qy, r1, qx * r0)));
+  const float sy = fabsf(__fmaf_rn(qz, r5, __fmaf_rn(qy, r4, qx * r3)));
+  const float sz = fabsf(__fmaf_rn(qz, r8, __fmaf_rn(qy, r7, qx * r6)));
+  const float margin = 4e-6f * sum;
+  const float near = dist - __fmaf_rn(sz, hz, __fmaf_rn(sy, hy, sx * hx)) * rn - margin;
+  if (most == 0.0f || most - near < -P.trunc_neg) return kSkip;
+  const float far =
+      dist + __builtin_amdgcn_sqrtf(__fmaf_rn(ez, ez, __fmaf_rn(ey, ey, ex * ex))) + margin;
+  if ((cls & kFast) && least - far >= P.trunc) cls |= kFree;
   return cls;
 }
 
@@ -289,14 +309,12 @@ struct Brick {
   int x0, y0, z0;
   int nz;          // planes of the volume in it, 1 to NZ
   bool inside;     // the lane's column lies in the volume
-  int classes;     // all, or all but kInside where a lane's voxel leaves the volume
   float px, py;    // the column's voxel centre
   __device__ __forceinline__ Brick(const IntegrateParams& P, int bx, int by, int bz)
       : x0(bx), y0(by), z0(bz) {
     const int lane = threadIdx.x & 63, x = x0 + (lane & 7), y = y0 + (lane >> 3);
     nz = min(NZ, P.Z - z0);
     inside = x < P.X && y < P.Y;
-    classes = nz == NZ && __all(inside) ? ~0 : ~kInside;
     px = ((float)x + 0.5f) * P.h;
     py = ((float)y + 0.5f) * P.h;
   }
@@ -310,46 +328,116 @@ struct Brick {
   }
 };
 
-// This wave's brick of workgroup `blk` of a volume; false past the volume's
-// edge (x0 is the same for all lanes).
-__device__ __forceinline__ bool brick_origin(const IntegrateParams& P, uint32_t blk, int zstep,
-                                             int* x0, int* y0, int* z0) {
-  const uint32_t row = P.divX.div(blk), plane = P.divY.div(row);
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  *x0 = (int)(blk - row * P.divX.d) * kRegionX + wave * kBrick;
-  *y0 = (int)(row - plane * P.divY.d) * kBrick;
-  *z0 = (int)plane * zstep;
-  return *x0 < P.X;
+// A wave is a workgroup: the four waves of a region end at different times,
+// and a workgroup of four would hold the places of those that ended (3.1 waves
+// ran per SIMD where five fit; one frame into 512^3 111 -> 81 us, 300 frames
+// 12.6 -> 11.2 ms).  Workgroups go round the 8 XCDs, so a region's four waves
+// are those of every 8th workgroup: one L2 sees whole lines.  An XCD takes
+// 2^log2_run regions in a row.
+__device__ __forceinline__ int64_t region_of(int64_t first, int log2_run, int* wave) {
+  const uint32_t b = blockIdx.x, i = b >> 3, r = i >> 2;
+  *wave = (int)(i & 3);
+  return first + ((int64_t)(r >> log2_run) << (log2_run + 3)) + ((b & 7) << log2_run) +
+         (r & ((1u << log2_run) - 1));
 }
 
-// One corner of the box of a brick's voxel centres per lane (of eight).
+// A wave's first brick of region `blk` of a volume; false past the volume's
+// edge.  Regions are numbered x first, or (BLOCKS) in blocks of 2 x 8 x 4
+// regions, smaller at the far sides: waves that run together then see the same
+// part of each frame, and an XCD's L2 holds it (300 frames into 512^3: 10.9 ms
+// x first, where the waves of an XCD lie all over a slab, 8.8 ms in blocks).
+constexpr int kBlockX = 2, kBlockY = 8, kBlockZ = 4;
+template <bool BLOCKS>
+__device__ __forceinline__ bool brick_origin(const IntegrateParams& P, uint32_t blk, int wave,
+                                             int zstep, int* x0, int* y0, int* z0) {
+  uint32_t x, y, z;
+  if (BLOCKS) {
+    const uint32_t nx = P.divX.d, ny = P.divY.d, nz = (uint32_t)((P.Z + zstep - 1) / zstep);
+    const uint32_t bz = blk / (nx * ny * kBlockZ);
+    if (bz * kBlockZ >= nz) return false;
+    uint32_t r = blk - bz * (nx * ny * kBlockZ);
+    const uint32_t hz = min((uint32_t)kBlockZ, nz - bz * kBlockZ);
+    const uint32_t by = r / (nx * kBlockY * hz);
+    r -= by * (nx * kBlockY * hz);
+    const uint32_t hy = min((uint32_t)kBlockY, ny - by * kBlockY);
+    const uint32_t bx = r / (kBlockX * hy * hz);
+    r -= bx * (kBlockX * hy * hz);
+    const uint32_t hx = min((uint32_t)kBlockX, nx - bx * kBlockX);
+    const uint32_t iy = r / hx, iz = iy / hy;
+    x = bx * kBlockX + r - iy * hx;
+    y = by * kBlockY + iy - iz * hy;
+    z = bz * kBlockZ + iz;
+  } else {
+    const uint32_t row = P.divX.div(blk);
+    z = P.divY.div(row);
+    x = blk - row * P.divX.d;
+    y = row - z * P.divY.d;
+  }
+  *x0 = __builtin_amdgcn_readfirstlane((int)x) * kRegionX + wave * kBrick;
+  *y0 = __builtin_amdgcn_readfirstlane((int)y) * kBrick;
+  *z0 = __builtin_amdgcn_readfirstlane((int)z) * zstep;
+  return *x0 < P.X && *z0 < P.Z;
+}
+
+// The frames that bricks may observe.  A wave's 64 lanes test `lanes` frames
+// (a power of two, at least K up to 64) of 64 / lanes bricks above one another
+// at once; with more than 64 frames, 64 frames of one brick at a time.  Every
+// lane of the wave takes part.
 template <int NZ>
-__device__ __forceinline__ void brick_corner(const IntegrateParams& P, int x0, int y0, int z0,
-                                             float* px, float* py, float* pz) {
-  const int c = threadIdx.x & 7;
-  *px = ((float)((c & 1) ? min(x0 + kBrick - 1, P.X - 1) : x0) + 0.5f) * P.h;
-  *py = ((float)((c & 2) ? min(y0 + kBrick - 1, P.Y - 1) : y0) + 0.5f) * P.h;
-  *pz = ((float)((c & 4) ? min(z0 + NZ - 1, P.Z - 1) : z0) + 0.5f) * P.h;
-}
+struct Frames {
+  const IntegrateParams& P;
+  int x0, y0, z0;          // the first of the bricks tested together
+  int log2_lanes, shift;   // lanes per brick; this brick's first lane
+  bool tested;
+  int cls;                 // this lane's class (read from its lane at the frame's turn)
+  uint64_t act;
 
-// f(k, class) for every frame k that some voxel of the brick may observe, in
-// order: the wave tests eight frames at a time (every lane of the wave calls
-// this).  A brick that leaves the volume is never kInside.
-template <int NZ, typename F>
-__device__ __forceinline__ void for_active_frames(const IntegrateParams& P, const Brick<NZ>& B,
-                                                  F&& f) {
-  const int lane = threadIdx.x & 63;
-  float px, py, pz;
-  brick_corner<NZ>(P, B.x0, B.y0, B.z0, &px, &py, &pz);
-  for (int kb = 0; kb < P.K; kb += 8) {
-    const int k = min(kb + (lane >> 3), P.K - 1);
-    const int cls = test_box(P, P.poses + 12 * k, k, px, py, pz);
-    uint64_t act = __ballot(!(cls & kSkip) && (lane & 7) == 0 && kb + (lane >> 3) < P.K);
-    while (act) {
-      const int b = __builtin_ctzll(act);
-      f(kb + (b >> 3), __builtin_amdgcn_readlane(cls, b) & B.classes);
-      act &= act - 1;
+  __device__ __forceinline__ Frames(const IntegrateParams& p, int bx, int by, int bz)
+      : P(p), x0(bx), y0(by), z0(bz), shift(0), tested(false), cls(kSkip), act(0) {
+    log2_lanes = P.K > 32 ? 6 : P.K > 1 ? 32 - __builtin_clz((unsigned)(P.K - 1)) : 0;
+  }
+  __device__ __forceinline__ int bricks() const { return 64 >> log2_lanes; }
+  __device__ __forceinline__ void test(int kb) {
+    const int lane = threadIdx.x & 63, k = kb + (lane & ((1 << log2_lanes) - 1));
+    const int z = z0 + (lane >> log2_lanes) * NZ;
+    cls = k < P.K && z < P.Z ? test_brick<NZ>(P, x0, y0, z, k) : kSkip;
+    act = __ballot(!(cls & kSkip));
+    tested = true;
+  }
+  // f(k, class) for every frame k that some voxel of the brick may observe, in
+  // order.
+  template <typename F>
+  __device__ __forceinline__ void each(F&& f) {
+    for (int kb = 0; kb < P.K; kb += 64) {
+      if (!tested || P.K > 64) test(kb);
+      uint64_t m = act >> shift;
+      if (log2_lanes < 6) m &= (1ull << (1 << log2_lanes)) - 1;
+      while (m) {
+        const int b = __builtin_ctzll(m);
+        m &= m - 1;
+        f(kb + b, __builtin_amdgcn_readlane(cls, b + shift));
+      }
     }
+  }
+};
+
+// body(brick, frames) for the wave's `count` bricks above one another from
+// (x0, y0, z0) on.
+template <int NZ, typename F>
+__device__ __forceinline__ void for_bricks(const IntegrateParams& P, int x0, int y0, int z0,
+                                           int count, F&& body) {
+  Frames<NZ> fr(P, x0, y0, z0);
+  const int together = fr.bricks();
+  for (int b = 0; b < count; ++b) {
+    const int z = z0 + b * NZ;
+    if (z >= P.Z) break;
+    if (b % together == 0) {  // (a power of two)
+      fr.z0 = z;
+      fr.tested = false;
+    }
+    if (!fr.tested && P.K <= 64) fr.test(0);
+    fr.shift = (b % together) << fr.log2_lanes;
+    body(Brick<NZ>(P, x0, y0, z), fr);
   }
 }
 
@@ -519,69 +607,68 @@ __device__ __forceinline__ float truncated(const IntegrateParams& P, float sdf) 
   return fminf(FAST ? div_rn(sdf, t, front ? P.rtrunc : P.rtrunc_neg) : sdf / t, 1.0f);
 }
 
-// Packed short2 update of a brick by frames [0, K) (the oracle's
-// update_voxel).  The brick is read when its first frame comes up and a voxel
-// is written only if some frame updated it: outside every frustum and behind
+// Packed short2 update of a wave's bricks by frames [0, K) (the oracle's
+// update_voxel).  A brick is read when its first frame comes up and a voxel is
+// written only if some frame updated it: outside every frustum and behind
 // every surface it costs no memory traffic.
 template <typename DT>
-__global__ __launch_bounds__(256) void integrate_kernel(IntegrateParams P) {
-  int x0, y0, z0;
-  if (!brick_origin(P, (uint32_t)(P.first_block + blockIdx.x), kBrickZ, &x0, &y0, &z0)) return;
-  const Brick<kBrickZ> B(P, x0, y0, z0);
-  uint32_t* const v = P.vol + B.first(P);
+__global__ __launch_bounds__(64) void integrate_kernel(IntegrateParams P, int bricks) {
+  int wave, x0, y0, z0;
+  const uint32_t blk = (uint32_t)region_of(P.first_block, P.log2_run, &wave);
+  if (!brick_origin<true>(P, blk, wave, kBrickZ * bricks, &x0, &y0, &z0)) return;
   const int64_t XY = (int64_t)P.X * P.Y;
-  uint32_t cur[kBrickZ] = {};
-  uint32_t changed = 0;
-  bool have = false;
-  for_active_frames(P, B, [&](int k, int cls) {
-    if (!have) {
-      have = true;
+  for_bricks<kBrickZ>(P, x0, y0, z0, bricks, [&](const Brick<kBrickZ>& B, Frames<kBrickZ>& F) {
+    uint32_t* const v = P.vol + B.first(P);
+    uint32_t cur[kBrickZ] = {};
+    uint32_t changed = 0;
+    bool have = false;
+    F.each([&](int k, int cls) {
+      if (!have) {
+        have = true;
 #pragma unroll
-      for (int j = 0; j < kBrickZ; ++j)
-        if (B.inside && j < B.nz) cur[j] = v[j * XY];
-    }
-    observe_brick<DT>(
-        P, B, k, cls,
-        [&](auto fast, int j, float sdf, float, uint32_t) {
-          cur[j] = packed_update<fast.value>(cur[j], truncated<fast.value>(P, sdf), P.max_w);
-          changed |= 1u << j;
-        },
-        [&](int j) {
-          cur[j] = packed_update<true>(cur[j], 1.0f, P.max_w);
-          changed |= 1u << j;
-        });
+        for (int j = 0; j < kBrickZ; ++j)
+          if (B.inside && j < B.nz) cur[j] = v[j * XY];
+      }
+      observe_brick<DT>(
+          P, B, k, cls,
+          [&](auto fast, int j, float sdf, float, uint32_t) {
+            cur[j] = packed_update<fast.value>(cur[j], truncated<fast.value>(P, sdf), P.max_w);
+            changed |= 1u << j;
+          },
+          [&](int j) {
+            cur[j] = packed_update<true>(cur[j], 1.0f, P.max_w);
+            changed |= 1u << j;
+          });
+    });
+#pragma unroll
+    for (int j = 0; j < kBrickZ; ++j)
+      if (changed & (1u << j)) v[j * XY] = cur[j];
   });
-#pragma unroll
-  for (int j = 0; j < kBrickZ; ++j)
-    if (changed & (1u << j)) v[j * XY] = cur[j];
 }
 
-// One frame (the reference's per-frame call): a wave takes `bricks` bricks
-// above one another (up to eight), tests all of them at once (eight lanes
-// each) and passes through those that can observe the frame.  Fewer bricks a
-// wave for small volumes, so that there are waves enough.
+// One frame (the reference's per-frame call): a wave tests `bricks` bricks
+// above one another (up to eight, one lane each) and passes through those that
+// can observe the frame, the voxels loaded beside the depth.
 template <typename DT>
-__global__ __launch_bounds__(256) void integrate1_kernel(IntegrateParams P, int bricks) {
-  int x0, y0, z0;
-  if (!brick_origin(P, (uint32_t)(P.first_block + blockIdx.x), kBrickZ * bricks, &x0, &y0, &z0))
-    return;
-  const int lane = threadIdx.x & 63;
-  const int zt = z0 + (lane >> 3) * kBrickZ;
-  float px, py, pz;
-  brick_corner<kBrickZ>(P, x0, y0, min(zt, P.Z - 1), &px, &py, &pz);
-  const int cls = test_box(P, P.poses, 0, px, py, pz);
-  uint64_t act = __ballot(!(cls & kSkip) && (lane & 7) == 0 && (lane >> 3) < bricks && zt < P.Z);
+__global__ __launch_bounds__(64) void integrate1_kernel(IntegrateParams P, int bricks) {
+  int wave, x0, y0, z0;
+  const uint32_t blk = (uint32_t)region_of(P.first_block, P.log2_run, &wave);
+  if (!brick_origin<false>(P, blk, wave, kBrickZ * bricks, &x0, &y0, &z0)) return;
   const int64_t XY = (int64_t)P.X * P.Y;
+  const int lane = threadIdx.x & 63, zt = z0 + lane * kBrickZ;
+  const int cls =
+      lane < bricks && zt < P.Z ? test_brick<kBrickZ>(P, x0, y0, zt, 0) : kSkip;
+  uint64_t act = __ballot(!(cls & kSkip));
   while (act) {
     const int b = __builtin_ctzll(act);
-    const Brick<kBrickZ> B(P, x0, y0, z0 + (b >> 3) * kBrickZ);
+    const Brick<kBrickZ> B(P, x0, y0, z0 + b * kBrickZ);
     act &= act - 1;
     uint32_t* const v = P.vol + B.first(P);
     uint32_t cur[kBrickZ];
 #pragma unroll
     for (int j = 0; j < kBrickZ; ++j) cur[j] = B.inside && j < B.nz ? v[j * XY] : 0u;
     observe_brick<DT>(
-        P, B, 0, __builtin_amdgcn_readlane(cls, b) & B.classes,
+        P, B, 0, __builtin_amdgcn_readlane(cls, b),
         [&](auto fast, int j, float sdf, float, uint32_t) {
           v[j * XY] = packed_update<fast.value>(cur[j], truncated<fast.value>(P, sdf), P.max_w);
         },
@@ -631,11 +718,11 @@ __device__ __forceinline__ float observation_slope(const IntegrateParams& P, flo
 template <typename LOAD>
 __device__ __forceinline__ uint32_t integrate_tsdf_brick(const IntegrateParams& P,
                                                          const Brick<kBrickZ>& B,
-                                                         float (&f)[kBrickZ], int (&w)[kBrickZ],
-                                                         LOAD&& load) {
+                                                         Frames<kBrickZ>& F, float (&f)[kBrickZ],
+                                                         int (&w)[kBrickZ], LOAD&& load) {
   uint32_t changed = 0;
   bool have = false;
-  for_active_frames(P, B, [&](int k, int cls) {
+  F.each([&](int k, int cls) {
     if (!have) {
       have = true;
       load();
@@ -657,11 +744,13 @@ __device__ __forceinline__ uint32_t integrate_tsdf_brick(const IntegrateParams& 
 // The brick's voxels are read when the first frame that may observe it comes
 // up; only updated voxels are written.
 __device__ __forceinline__ void integrate_tsdf_stored(const IntegrateParams& P,
-                                                      const Brick<kBrickZ>& B, float* tsdf, int32_t* wvol) {
+                                                      const Brick<kBrickZ>& B,
+                                                      Frames<kBrickZ>& F, float* tsdf,
+                                                      int32_t* wvol) {
   const int64_t i = B.first(P), XY = (int64_t)P.X * P.Y;
   float f[kBrickZ] = {};
   int w[kBrickZ] = {};
-  const uint32_t changed = integrate_tsdf_brick(P, B, f, w, [&]() {
+  const uint32_t changed = integrate_tsdf_brick(P, B, F, f, w, [&]() {
 #pragma unroll
     for (int j = 0; j < kBrickZ; ++j)
       if (B.inside && j < B.nz) {
@@ -677,11 +766,14 @@ __device__ __forceinline__ void integrate_tsdf_stored(const IntegrateParams& P,
     }
 }
 
-__global__ __launch_bounds__(256) void integrate_tsdf_kernel(IntegrateParams P, float* tsdf,
-                                                             int32_t* wvol) {
-  int x0, y0, z0;
-  if (!brick_origin(P, (uint32_t)(P.first_block + blockIdx.x), kBrickZ, &x0, &y0, &z0)) return;
-  integrate_tsdf_stored(P, Brick<kBrickZ>(P, x0, y0, z0), tsdf, wvol);
+__global__ __launch_bounds__(64) void integrate_tsdf_kernel(IntegrateParams P, int bricks,
+                                                             float* tsdf, int32_t* wvol) {
+  int wave, x0, y0, z0;
+  const uint32_t blk = (uint32_t)region_of(P.first_block, P.log2_run, &wave);
+  if (!brick_origin<true>(P, blk, wave, kBrickZ * bricks, &x0, &y0, &z0)) return;
+  for_bricks<kBrickZ>(P, x0, y0, z0, bricks, [&](const Brick<kBrickZ>& B, Frames<kBrickZ>& F) {
+    integrate_tsdf_stored(P, B, F, tsdf, wvol);
+  });
 }
 
 // Deterministic max of |g| over n floats: per-block max, then an integer
@@ -738,13 +830,14 @@ __device__ __forceinline__ void backward_brick(const IntegrateParams& P, const B
     for (int j = 0; j < NZ; ++j)
       if (gi[j] != 0.0f) w0[j] = w0vol[i + j * XY];
   }
-  for_active_frames(P, B, [&](int k, int cls) {
+  Frames<NZ> F(P, B.x0, B.y0, B.z0);
+  F.each([&](int k, int cls) {
     observe_brick<float>(
         P, B, k, cls, [&](auto, int j, float, float, uint32_t) { ++nobs[j]; },
         [&](int j) { ++nobs[j]; });
   });
   const double cap_a = (double)M / (double)(M + 1);
-  for_active_frames(P, B, [&](int k, int cls) {
+  F.each([&](int k, int cls) {
     const auto add = [&](auto, int j, float sdf, float rf, uint32_t pix) {
       const int oi = o[j]++;
       if (gi[j] == 0.0f) return;
@@ -780,11 +873,12 @@ __device__ __forceinline__ void backward_brick(const IntegrateParams& P, const B
 }
 
 template <int NZ>
-__global__ __launch_bounds__(256) void integrate_tsdf_backward_kernel(
+__global__ __launch_bounds__(64) void integrate_tsdf_backward_kernel(
     IntegrateParams P, const float* __restrict__ g, const int32_t* __restrict__ w0vol,
     const uint32_t* maxg, float max_dtdd, unsigned long long* acc) {
-  int x0, y0, z0;
-  if (!brick_origin(P, (uint32_t)(P.first_block + blockIdx.x), NZ, &x0, &y0, &z0)) return;
+  int wave, x0, y0, z0;
+  const uint32_t blk = (uint32_t)region_of(P.first_block, P.log2_run, &wave);
+  if (!brick_origin<true>(P, blk, wave, NZ, &x0, &y0, &z0)) return;
   backward_brick(P, Brick<NZ>(P, x0, y0, z0), g, w0vol, maxg, max_dtdd, acc);
 }
 
@@ -797,6 +891,8 @@ struct BatchIntegrateParams {
   int nvol;
   int from_init;         // start every voxel from (init_value, 0) without reading it
   float init_value;
+  int bricks;            // bricks above one another in a workgroup
+  int64_t end_block;     // regions [first_block, end_block) are this launch's
   int tiled_vol;         // volumes [tiled_vol, tiled_vol + base.tiled / K) have tile tables
   int64_t first_block;   // workgroup index of this launch's blockIdx.x 0
 };
@@ -806,7 +902,9 @@ struct BatchIntegrateParams {
 __device__ __forceinline__ bool batch_setup(const BatchIntegrateParams& B, IntegrateParams& P,
                                             int64_t* vox_begin, int* vol, int* x0, int* y0,
                                             int* z0) {
-  const int64_t blk = B.first_block + blockIdx.x;
+  int wave;
+  const int64_t blk = region_of(B.first_block, B.base.log2_run, &wave);
+  if (blk >= B.end_block) return false;
   const int vi = __builtin_amdgcn_readfirstlane(
       batch_volume_of<&BatchVol::blk_begin>(B.bvol, B.nvol, blk));
   const BatchVol& V = B.bvol[vi];
@@ -820,47 +918,49 @@ __device__ __forceinline__ bool batch_setup(const BatchIntegrateParams& B, Integ
   P.depth = static_cast<const float*>(B.base.depth) + (int64_t)vi * P.K * P.W * P.H;
   P.poses = B.base.poses + (int64_t)vi * P.K * 12;
   P.tiled = vi >= B.tiled_vol ? max(0, min(P.K, P.tiled - (vi - B.tiled_vol) * P.K)) : 0;
-  P.tiles = B.base.tiles + (int64_t)(vi - B.tiled_vol) * P.K * P.TY * P.TX;
+  P.tiles = B.base.tiles + (int64_t)(vi - B.tiled_vol) * P.K * (P.TX * P.TY + P.TX1 * P.TY1);
   *vox_begin = V.vox_begin;
   *vol = vi;
-  return brick_origin(P, (uint32_t)(blk - V.blk_begin), kBrickZ, x0, y0, z0);
+  return brick_origin<true>(P, (uint32_t)(blk - V.blk_begin), wave, kBrickZ * B.bricks, x0, y0, z0);
 }
 
-__global__ __launch_bounds__(256) void integrate_tsdf_batched_kernel(BatchIntegrateParams B,
+__global__ __launch_bounds__(64) void integrate_tsdf_batched_kernel(BatchIntegrateParams B,
                                                                      float* tsdf, int32_t* wvol) {
   IntegrateParams P;
   int64_t vb;
   int vi, x0, y0, z0;
   if (!batch_setup(B, P, &vb, &vi, &x0, &y0, &z0)) return;
-  const Brick<kBrickZ> K(P, x0, y0, z0);
-  if (!B.from_init) {
-    integrate_tsdf_stored(P, K, tsdf + vb, wvol + vb);
-    return;
-  }
-  // every voxel is written: the start value where no frame observes it
-  float f[kBrickZ];
-  int w[kBrickZ] = {};
-#pragma unroll
-  for (int j = 0; j < kBrickZ; ++j) f[j] = B.init_value;
-  integrate_tsdf_brick(P, K, f, w, []() {});
-  const int64_t i = vb + K.first(P), XY = (int64_t)P.X * P.Y;
-#pragma unroll
-  for (int j = 0; j < kBrickZ; ++j)
-    if (K.inside && j < K.nz) {
-      tsdf[i + j * XY] = f[j];
-      wvol[i + j * XY] = w[j];
+  for_bricks<kBrickZ>(P, x0, y0, z0, B.bricks, [&](const Brick<kBrickZ>& K, Frames<kBrickZ>& F) {
+    if (!B.from_init) {
+      integrate_tsdf_stored(P, K, F, tsdf + vb, wvol + vb);
+      return;
     }
+    // every voxel is written: the start value where no frame observes it
+    float f[kBrickZ];
+    int w[kBrickZ] = {};
+#pragma unroll
+    for (int j = 0; j < kBrickZ; ++j) f[j] = B.init_value;
+    integrate_tsdf_brick(P, K, F, f, w, []() {});
+    const int64_t i = vb + K.first(P), XY = (int64_t)P.X * P.Y;
+#pragma unroll
+    for (int j = 0; j < kBrickZ; ++j)
+      if (K.inside && j < K.nz) {
+        tsdf[i + j * XY] = f[j];
+        wvol[i + j * XY] = w[j];
+      }
+  });
 }
 
-__global__ __launch_bounds__(256) void integrate_tsdf_backward_batched_kernel(
+__global__ __launch_bounds__(64) void integrate_tsdf_backward_batched_kernel(
     BatchIntegrateParams B, const float* __restrict__ g, const int32_t* __restrict__ w0vol,
     const uint32_t* maxg, float max_dtdd, unsigned long long* acc) {
   IntegrateParams P;
   int64_t vb;
   int vi, x0, y0, z0;
   if (!batch_setup(B, P, &vb, &vi, &x0, &y0, &z0)) return;
-  backward_brick(P, Brick<kBrickZ>(P, x0, y0, z0), g + vb, w0vol ? w0vol + vb : nullptr, maxg, max_dtdd,
-                 acc + (int64_t)vi * P.K * P.W * P.H);
+  for (int b = 0; b < B.bricks && z0 < P.Z; ++b, z0 += kBrickZ)
+    backward_brick(P, Brick<kBrickZ>(P, x0, y0, z0), g + vb, w0vol ? w0vol + vb : nullptr, maxg,
+                   max_dtdd, acc + (int64_t)vi * P.K * P.W * P.H);
 }
 
 __global__ __launch_bounds__(256) void fixed_to_float_kernel(const unsigned long long* acc,
@@ -988,7 +1088,10 @@ size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 // one (a 640x480 frame takes 38 KB, so a sweep's 512 frames fit; a 320x240
 // frame 9.6 KB: 3,495, the frames of 218 volumes of a batch with 16 each).
 size_t tile_bytes(int W, int H) {
-  return (size_t)((W + kTile - 1) / kTile) * ((H + kTile - 1) / kTile) * sizeof(float2);
+  const auto tiles = [&](int side) {
+    return (size_t)((W + side - 1) / side) * ((H + side - 1) / side);
+  };
+  return (tiles(kTile) + tiles(kTile * kTiles1)) * sizeof(float2);
 }
 size_t tile_tables_bytes(int W, int H) {
   const size_t per = tile_bytes(W, H), most = (size_t)32 << 20;
@@ -1046,6 +1149,8 @@ int prepare_integrate(IntegrateParams& P, int X, int Y, int Z, float h, float tr
   P.tiled = 0;
   P.TX = (W + kTile - 1) / kTile;
   P.TY = (H + kTile - 1) / kTile;
+  P.TX1 = (P.TX + kTiles1 - 1) / kTiles1;
+  P.TY1 = (P.TY + kTiles1 - 1) / kTiles1;
   P.depth_scale = depth_scale;
   P.W = W;
   P.H = H;
@@ -1056,6 +1161,7 @@ int prepare_integrate(IntegrateParams& P, int X, int Y, int Z, float h, float tr
   P.poses = nullptr;
   P.depth = nullptr;
   P.first_block = 0;
+  P.log2_run = 0;
   return MCX_OK;
 }
 
@@ -1077,19 +1183,40 @@ int frame_tiles(IntegrateParams& P, const DT* depth, int64_t frames, char* table
   P.tiled = (int)std::min(frames, room);
   const int gx = (P.TX + 7) / 8;
   // about 16 waves per SIMD in all; each takes every gz-th frame
-  const int64_t gz = std::max<int64_t>(
-      1, std::min<int64_t>((16384 + (int64_t)gx * P.TY - 1) / ((int64_t)gx * P.TY), P.tiled));
+  const int64_t plane = (int64_t)gx * P.TY1;
+  const int64_t gz = std::max<int64_t>(1, std::min<int64_t>((4096 + plane - 1) / plane, P.tiled));
   const int vec = P.W % kTile == 0 && (reinterpret_cast<uintptr_t>(depth) & 15u) == 0 &&
                   ((int64_t)P.W * P.H * (int64_t)sizeof(DT)) % 16 == 0;
-  for (int y0 = 0; y0 < P.TY; y0 += 65535) {
+  for (int y0 = 0; y0 < P.TY1; y0 += 65535) {
     hipLaunchKernelGGL(frame_tiles_kernel<DT>,
-                       dim3((unsigned)gx, (unsigned)std::min(65535, P.TY - y0), (unsigned)gz),
-                       dim3(64), 0, s, depth, P.depth_scale, P.W, P.H, P.tiled, P.fx, P.fy, P.cx,
-                       P.cy, const_cast<float*>(P.rayfac), P.TX, P.TY, y0, vec,
+                       dim3((unsigned)gx, (unsigned)std::min(65535, P.TY1 - y0), (unsigned)gz),
+                       dim3(256), 0, s, depth, P.depth_scale, P.W, P.H, P.tiled, P.fx, P.fy, P.cx,
+                       P.cy, const_cast<float*>(P.rayfac), P.TX, P.TY, P.TX1, P.TY1, y0, vec,
                        reinterpret_cast<float2*>(tables));
     MCX_HIP(hipGetLastError());
   }
   return MCX_OK;
+}
+
+// Workgroups of a launch over `n` regions (whole rounds of the 8 XCDs), and
+// the most regions of a launch.
+constexpr int64_t kMaxRegions = kMaxLaunchBlocks;
+unsigned region_groups(int64_t n, int log2_run) {
+  const int64_t round = (int64_t)8 << log2_run;
+  return (unsigned)((n + round - 1) / round * round * 4);
+}
+// Eight regions of a block in a row for one XCD, where several frames are
+// swept over regions enough for that (runs of 16 and 32 8.9 ms, of 64 10.7: the
+// XCDs' shares of the surfaces become uneven).
+int region_runs(int64_t n, int K) { return K > 1 && n >= 4096 ? 3 : 0; }
+
+// Bricks above one another that a wave takes (their frames are tested
+// together): as many as its 64 lanes can test at once, up to eight, while
+// that leaves 16 waves per SIMD.
+int bricks_per_wave(int64_t voxels, int K) {
+  int n = 1;
+  while (n < 8 && n * 2 * K <= 64 && voxels >= (int64_t)16384 * 256 * n * 2) n *= 2;
+  return n;
 }
 
 template <typename DT>
@@ -1116,18 +1243,16 @@ int integrate_impl(void* d_vol, int X, int Y, int Z, float h, float trunc_neg, f
     rc = frame_tiles(P, d_depth + (int64_t)k0 * W * H, P.K, ws + rayfac_bytes(W, H), ws + ws_bytes,
                      s);
     if (rc) return rc;
-    // one frame: up to eight bricks a wave, while that leaves 16384 waves
-    int bricks = 1;
-    if (P.K == 1)
-      while (bricks < 8 && (int64_t)X * Y * Z >= (int64_t)16384 * 256 * bricks * 2) bricks *= 2;
+    const int bricks = bricks_per_wave((int64_t)X * Y * Z, P.K);
     const int64_t nb = regions(X, Y, Z, kBrickZ * bricks);
-    for (int64_t b0 = 0; b0 < nb; b0 += kMaxLaunchBlocks) {
+    P.log2_run = region_runs(nb, P.K);
+    for (int64_t b0 = 0; b0 < nb; b0 += kMaxRegions) {
       P.first_block = b0;
-      const dim3 grid((unsigned)std::min(kMaxLaunchBlocks, nb - b0));
+      const dim3 grid(region_groups(std::min(kMaxRegions, nb - b0), P.log2_run));
       if (P.K == 1)
-        hipLaunchKernelGGL(integrate1_kernel<DT>, grid, dim3(256), 0, s, P, bricks);
+        hipLaunchKernelGGL(integrate1_kernel<DT>, grid, dim3(64), 0, s, P, bricks);
       else
-        hipLaunchKernelGGL(integrate_kernel<DT>, grid, dim3(256), 0, s, P);
+        hipLaunchKernelGGL(integrate_kernel<DT>, grid, dim3(64), 0, s, P, bricks);
       MCX_HIP(hipGetLastError());
     }
   }
@@ -1230,11 +1355,13 @@ extern "C" int mcx_integrate_tsdf(float* d_tsdf, int32_t* d_weight, int X, int Y
     rc = frame_tiles(P, d_depth + (int64_t)k0 * W * H, P.K, ws + rayfac_bytes(W, H), ws + ws_bytes,
                      s);
     if (rc) return rc;
-    const int64_t nb = regions(X, Y, Z, kBrickZ);
-    for (int64_t b0 = 0; b0 < nb; b0 += kMaxLaunchBlocks) {
+    const int bricks = bricks_per_wave((int64_t)X * Y * Z, P.K);
+    const int64_t nb = regions(X, Y, Z, kBrickZ * bricks);
+    P.log2_run = region_runs(nb, P.K);
+    for (int64_t b0 = 0; b0 < nb; b0 += kMaxRegions) {
       P.first_block = b0;
-      hipLaunchKernelGGL(integrate_tsdf_kernel, dim3((unsigned)std::min(kMaxLaunchBlocks, nb - b0)),
-                         dim3(256), 0, s, P, d_tsdf, d_weight);
+      const dim3 grid(region_groups(std::min(kMaxRegions, nb - b0), P.log2_run));
+      hipLaunchKernelGGL(integrate_tsdf_kernel, grid, dim3(64), 0, s, P, bricks, d_tsdf, d_weight);
       MCX_HIP(hipGetLastError());
     }
   }
@@ -1291,14 +1418,15 @@ extern "C" int mcx_integrate_tsdf_backward(const float* d_grad_tsdf, const int32
   // each one's frames run in series.
   const bool small = n < ((int64_t)1 << 23);
   const int64_t nb = regions(X, Y, Z, small ? 1 : kBrickZ);
-  for (int64_t b0 = 0; b0 < nb; b0 += kMaxLaunchBlocks) {
+  P.log2_run = region_runs(nb, K);
+  for (int64_t b0 = 0; b0 < nb; b0 += kMaxRegions) {
     P.first_block = b0;
-    const dim3 grid((unsigned)std::min(kMaxLaunchBlocks, nb - b0));
+    const dim3 grid(region_groups(std::min(kMaxRegions, nb - b0), P.log2_run));
     if (small)
-      hipLaunchKernelGGL(integrate_tsdf_backward_kernel<1>, grid, dim3(256), 0, s, P, d_grad_tsdf,
+      hipLaunchKernelGGL(integrate_tsdf_backward_kernel<1>, grid, dim3(64), 0, s, P, d_grad_tsdf,
                          d_weight0, maxg, mdt, acc);
     else
-      hipLaunchKernelGGL(integrate_tsdf_backward_kernel<kBrickZ>, grid, dim3(256), 0, s, P,
+      hipLaunchKernelGGL(integrate_tsdf_backward_kernel<kBrickZ>, grid, dim3(64), 0, s, P,
                          d_grad_tsdf, d_weight0, maxg, mdt, acc);
     MCX_HIP(hipGetLastError());
   }
@@ -1347,6 +1475,8 @@ extern "C" int mcx_integrate_tsdf_batched(const mcx_batch* plan, float* d_tsdf, 
   B.base.depth = d_depth;
   B.bvol = plan->d_bvol;
   B.nvol = plan->nvol;
+  B.bricks = plan->bricks;
+  B.base.log2_run = region_runs(plan->blocks, K);
   B.from_init = from_init ? 1 : 0;
   B.init_value = init_value;
   // volumes in turn of as many as the workspace holds tile tables for
@@ -1360,11 +1490,11 @@ extern "C" int mcx_integrate_tsdf_batched(const mcx_batch* plan, float* d_tsdf, 
     if (rc) return rc;
     B.tiled_vol = v0;
     const int64_t end = plan->blk_begin[v1];
-    for (int64_t b0 = plan->blk_begin[v0]; b0 < end; b0 += kMaxLaunchBlocks) {
+    for (int64_t b0 = plan->blk_begin[v0]; b0 < end; b0 += kMaxRegions) {
       B.first_block = b0;
-      hipLaunchKernelGGL(integrate_tsdf_batched_kernel,
-                         dim3((unsigned)std::min(kMaxLaunchBlocks, end - b0)), dim3(256), 0, s, B,
-                         d_tsdf, d_weight);
+      B.end_block = std::min(end, b0 + kMaxRegions);
+      const dim3 grid(region_groups(B.end_block - b0, B.base.log2_run));
+      hipLaunchKernelGGL(integrate_tsdf_batched_kernel, grid, dim3(64), 0, s, B, d_tsdf, d_weight);
       MCX_HIP(hipGetLastError());
     }
   }
@@ -1430,13 +1560,16 @@ extern "C" int mcx_integrate_tsdf_backward_batched(const mcx_batch* plan,
   B.base.depth = d_depth;
   B.bvol = plan->d_bvol;
   B.nvol = plan->nvol;
+  B.bricks = plan->bricks;
+  B.base.log2_run = region_runs(plan->blocks, K);
   B.from_init = 0;
   B.init_value = 0.0f;
-  for (int64_t b0 = 0; b0 < plan->blocks; b0 += kMaxLaunchBlocks) {
+  for (int64_t b0 = 0; b0 < plan->blocks; b0 += kMaxRegions) {
     B.first_block = b0;
-    hipLaunchKernelGGL(integrate_tsdf_backward_batched_kernel,
-                       dim3((unsigned)std::min(kMaxLaunchBlocks, plan->blocks - b0)), dim3(256),
-                       0, s, B, d_grad_tsdf, d_weight0, mg, mdt, acc);
+    B.end_block = std::min(plan->blocks, b0 + kMaxRegions);
+    const dim3 grid(region_groups(B.end_block - b0, B.base.log2_run));
+    hipLaunchKernelGGL(integrate_tsdf_backward_batched_kernel, grid, dim3(64), 0, s, B,
+                       d_grad_tsdf, d_weight0, mg, mdt, acc);
     MCX_HIP(hipGetLastError());
   }
   hipLaunchKernelGGL(fixed_to_float_kernel, dim3(blocks_for(npix)), dim3(256), 0, s, acc, npix,

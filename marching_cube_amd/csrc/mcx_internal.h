@@ -302,9 +302,9 @@ __device__ __forceinline__ int64_t lookback(const uint64_t* desc, int64_t t, uin
 // extraction, MC backward and integration kernels.  Per-voxel arrays of a
 // batch (fp32 TSDF, weights, gradients) are concatenated in volume order:
 // volume b's voxels start at vox_begin.  Workgroups of the integration kernels
-// take 32 x 8 x 4 voxels of one volume (blk_begin: the volume's first such
-// workgroup; divX, divY: workgroups along x and y); the batched gather takes
-// 1024 voxels of one plane (gblk_begin).
+// take 32 x 8 x (4 * the plan's bricks) voxels of one volume (blk_begin: the
+// volume's first such workgroup; divX, divY: workgroups along x and y); the
+// batched gather takes 1024 voxels of one plane (gblk_begin).
 struct BatchVol {
   int X, Y, Z;
   float h;
@@ -350,6 +350,7 @@ struct mcx_batch {
   int64_t voxels = 0;       // all volumes' voxels
   int64_t blocks = 0;       // workgroups of the integration kernels
   std::vector<int64_t> blk_begin;  // each volume's first one, then their number
+  int bricks = 1;           // bricks above one another that an integration wave takes
   int64_t gather_blocks = 0;
   mcx::VolDesc* d_vols = nullptr;
   mcx::Column* d_cols = nullptr;

@@ -57,7 +57,8 @@ def random_depth(rng, K, H, W, f32):
 @pytest.mark.parametrize("dims,K,W,H,f32", [
     ((33, 9, 5), 9, 96, 72, False), ((31, 8, 4), 1, 97, 71, True), ((64, 17, 37), 1, 40, 33, False),
     ((8, 40, 33), 17, 41, 24, True), ((1, 1, 9), 8, 96, 72, False), ((70, 7, 3), 2, 3, 3, True),
-    ((95, 41, 66), 24, 160, 120, False), ((40, 33, 12), 7, 16, 200, True)])
+    ((95, 41, 66), 24, 160, 120, False), ((40, 33, 12), 7, 16, 200, True),
+    ((20, 17, 9), 70, 64, 48, False), ((9, 20, 12), 64, 33, 40, True)])
 def test_integrate_brick_edges(dev, dims, K, W, H, f32):
     print(f"[case] bricks {dims} K={K} {W}x{H} f32={f32}", flush=True)
     rng = np.random.default_rng(sum(dims) + K)

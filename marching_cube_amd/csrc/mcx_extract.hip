@@ -438,11 +438,12 @@ __global__ __launch_bounds__(256) void count_kernel(ExtractParams P) {
 }
 
 // ============================================================ K1, wide form
-// SHORT2 volumes of any width.  128-bit loads: in chunk c (256 cubes) of a
-// tile, lane L holds the voxels 4L..4L+3 of each of the four corner rows
+// Volumes of any width, short2 or fp32.  128-bit loads: in chunk c (256 cubes)
+// of a tile, lane L holds the voxels 4L..4L+3 of each of the four corner rows
 // (rows y, y+1 of planes z, z+1); tiles start at multiples of 512 voxels,
 // rows and planes of a width X % 4 != 0 at 4-byte alignment, which the
 // vector memory path accepts.  The rows' tsdf signs become bytes (0xff:
+// negative; an fp32 voxel is first compared with 0, since -0 and NaN are not
 // negative); OR / AND over the four rows and over positions k and k + 1 (the
 // next lane's position 0 by one DPP lane shift) mark the cubes with both
 // signs, four per lane, masked by the cubes that exist (a row may end inside
@@ -451,8 +452,13 @@ __global__ __launch_bounds__(256) void count_kernel(ExtractParams P) {
 // is a sum of masked popcounts.  Records go to the column's quota, or, when
 // the tile does not fit there, to a shared overflow pool (one atomic per
 // overflowing tile); only when that is exhausted does the tile take the
-// staged path.  No active-cube masks are written (the backward runs on fp32
-// volumes, which take the 32-bit kernel).
+// staged path.  MASKS (the differentiable forms): the active-cube masks of
+// every tile, 16 words of 32 cubes, in one store of 16 lanes; a lane's four
+// cubes are four bits, OR-ed over eight lanes.  These forms have no overflow
+// pool: four columns share their quotas, so what fits with a quota a column
+// (the 32-bit kernel) fits here.
+// fp32 at 256^3 (bumps): 128-bit loads take the count from 54 to 46 us; a batch
+// of 64 fp32 volumes of 64-192 a side, with masks, from 425 to 193 us.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4a4 __attribute__((ext_vector_type(4), aligned(4)));  // 4-byte aligned
 
@@ -497,21 +503,37 @@ __device__ __forceinline__ uint32_t bfi(uint32_t m, uint32_t a, uint32_t b) {
 }
 
 // Byte k = 0xff when the tsdf of voxel position k is negative.
+template <int ELEM>
 __device__ __forceinline__ uint32_t sign_bytes(const u32x4& v) {
-  return __builtin_amdgcn_perm(v[1], v[0], kSignSel01) | __builtin_amdgcn_perm(v[3], v[2], kSignSel23);
+  if constexpr (ELEM == MCX_ELEM_SHORT2)
+    return __builtin_amdgcn_perm(v[1], v[0], kSignSel01) |
+           __builtin_amdgcn_perm(v[3], v[2], kSignSel23);
+  uint32_t n[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) n[k] = is_neg<ELEM>(v[k]) ? ~0u : 0u;
+  return bfi(0x000000ffu, n[0], bfi(0x0000ff00u, n[1], bfi(0x00ff0000u, n[2], n[3])));
 }
 
+template <int ELEM>
 __device__ __forceinline__ void plane_signs(Plane4& L) {
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    L.su[c] = sign_bytes(L.u[c]);
-    L.sw[c] = sign_bytes(L.w[c]);
+    L.su[c] = sign_bytes<ELEM>(L.u[c]);
+    L.sw[c] = sign_bytes<ELEM>(L.w[c]);
   }
+}
+
+// OR over the eight lanes of a group (all 64 lanes active).
+__device__ __forceinline__ uint32_t or8(uint32_t v) {
+  v |= __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true);   // lane ^ 1
+  v |= __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, true);   // lane ^ 2
+  v |= __builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, true);  // the other four
+  return v;
 }
 typedef const __attribute__((address_space(4))) uint32_t const_u32;  // scalar loads
 
-template <bool BATCH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+template <int ELEM, bool BATCH, bool MASKS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ELEM == MCX_ELEM_F32 ? 3 : 4)))
 void count4_kernel(ExtractParams P) {
   __shared__ uint8_t s_nv[256];
   __shared__ __attribute__((aligned(16))) uint32_t s_rec[4][256 * kRecWords];  // per wave: one chunk's records
@@ -599,6 +621,9 @@ void count4_kernel(ExtractParams P) {
     rsv[2] = __builtin_amdgcn_readfirstlane(rsv[2]);
     rsv[3] = __builtin_amdgcn_readfirstlane(rsv[3]);
   }
+  const __amdgpu_buffer_rsrc_t rsb = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint32_t*>(V.vol + (int64_t)z0 * XY), (short)0,
+      (int)((uint32_t)(z1 - z0 + 1) * plane_bytes), kBufferWord3);
   // the word after the tile in each row (the same for all lanes; an offset
   // past the resource, hence 0, when it lies outside the plane)
   const uint32_t xoffU = p0 + kTile < XY ? (uint32_t)(p0 + kTile) * 4u : 0x80000000u;
@@ -606,6 +631,15 @@ void count4_kernel(ExtractParams P) {
   auto load_plane = [&](int q, Plane4& L) {
     const uint32_t po = (uint32_t)(q - z0) * plane_bytes;
     const uint32_t a = voff + po, b = voffW + po;
+    if constexpr (ELEM == MCX_ELEM_F32) {
+      L.u[0] = __builtin_amdgcn_raw_buffer_load_b128(rsb, a, 0, 0);
+      L.u[1] = __builtin_amdgcn_raw_buffer_load_b128(rsb, a + 1024, 0, 0);
+      L.w[0] = __builtin_amdgcn_raw_buffer_load_b128(rsb, b, 0, 0);
+      L.w[1] = __builtin_amdgcn_raw_buffer_load_b128(rsb, b + 1024, 0, 0);
+      L.xu = __builtin_amdgcn_raw_buffer_load_b32(rsb, xoffU + po, 0, 0);
+      L.xw = __builtin_amdgcn_raw_buffer_load_b32(rsb, xoffW + po, 0, 0);
+      return;
+    }
     asm volatile("buffer_load_dwordx4 %0, %1, %2, 0 offen" : "=v"(L.u[0]) : "v"(a), "s"(rsv) : "memory");
     asm volatile("buffer_load_dwordx4 %0, %1, %2, 0 offen offset:1024" : "=v"(L.u[1]) : "v"(a), "s"(rsv) : "memory");
     asm volatile("buffer_load_dwordx4 %0, %1, %2, 0 offen" : "=v"(L.w[0]) : "v"(b), "s"(rsv) : "memory");
@@ -617,6 +651,7 @@ void count4_kernel(ExtractParams P) {
   // all but the newest six vector memory operations done (they retire in
   // issue order); ties L's registers
   auto wait_plane6 = [&](Plane4& L) {
+    if constexpr (ELEM == MCX_ELEM_F32) return;
     asm volatile("s_waitcnt vmcnt(6)" : "+v"(L.u[0]), "+v"(L.u[1]), "+v"(L.w[0]), "+v"(L.w[1]), "+v"(L.xu), "+v"(L.xw) :: "memory");
   };
   // Four plane buffers whose roles rotate over an unrolled loop of four steps
@@ -626,8 +661,9 @@ void count4_kernel(ExtractParams P) {
   load_plane(z0, A);
   load_plane(z0 + 1, B);
   load_plane(z0 + 2, C);
-  asm volatile("s_waitcnt vmcnt(12)" : "+v"(A.u[0]), "+v"(A.u[1]), "+v"(A.w[0]), "+v"(A.w[1]), "+v"(A.xu), "+v"(A.xw) :: "memory");
-  plane_signs(A);
+  if constexpr (ELEM == MCX_ELEM_SHORT2)
+    asm volatile("s_waitcnt vmcnt(12)" : "+v"(A.u[0]), "+v"(A.u[1]), "+v"(A.w[0]), "+v"(A.w[1]), "+v"(A.xu), "+v"(A.xw) :: "memory");
+  plane_signs<ELEM>(A);
 
   uint64_t nzmask = 0;  // planes zb + i of this column whose tile has vertices
   int zb = z0;
@@ -636,6 +672,7 @@ void count4_kernel(ExtractParams P) {
   // The plane two steps ahead is loaded at the end of a step, after the
   // step's record stores: the data a step waits for is then always older
   // than the newest loads (a fixed count), however many stores were issued.
+  auto neg_byte = [](uint32_t v) { return is_neg<ELEM>(v) ? 0xffu : 0u; };
   auto step = [&](Plane4& A, Plane4& B, Plane4& L, int z) __attribute__((always_inline)) {
 
     // ---- pass 1: active masks m[c][k] (bit L: cube 256c + 4L + k).  Signs
@@ -649,13 +686,21 @@ void count4_kernel(ExtractParams P) {
     // the minimum word over the eight corners below 0x10000 means some
     // weight is zero.
     wait_plane6(B);
-    plane_signs(B);
+    plane_signs<ELEM>(B);
     uint64_t m[2][4];
+    uint32_t nib[2];  // MASKS: the lane's four cubes of a chunk as bits
     uint32_t nxo, nxn, nxm;  // position 0 of the next chunk's lane 0 (wave-uniform)
     {
-      const uint32_t xo = A.xu | A.xw | B.xu | B.xw, xa = A.xu & A.xw & B.xu & B.xw;
-      nxo = (xo & 0x8000u) ? 0xffu : 0u;
-      nxn = (xa & 0x8000u) ? 0xffu : 0u;
+      if constexpr (ELEM == MCX_ELEM_SHORT2) {
+        const uint32_t xo = A.xu | A.xw | B.xu | B.xw, xa = A.xu & A.xw & B.xu & B.xw;
+        nxo = (xo & 0x8000u) ? 0xffu : 0u;
+        nxn = (xa & 0x8000u) ? 0xffu : 0u;
+      } else {
+        const uint32_t n0 = neg_byte(A.xu), n1 = neg_byte(A.xw), n2 = neg_byte(B.xu),
+                       n3 = neg_byte(B.xw);
+        nxo = n0 | n1 | n2 | n3;
+        nxn = n0 & n1 & n2 & n3;
+      }
       nxm = min(min(A.xu, A.xw), min(B.xu, B.xw));
     }
 #pragma unroll
@@ -672,8 +717,12 @@ void count4_kernel(ExtractParams P) {
       sg[1] = __ballot((int16_t)M < 0);
       sg[2] = __ballot((int8_t)(M >> 16) < 0);
       sg[3] = __ballot((int32_t)M < 0);
+      if (MASKS) nib[c] = ((M & 0x08040201u) * 0x01010101u) >> 24;
       uint32_t mn0 = 0;
-      if (sg[0] | sg[1] | sg[2] | sg[3]) {
+      if (ELEM == MCX_ELEM_F32) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) m[c][k] = sg[k];
+      } else if (sg[0] | sg[1] | sg[2] | sg[3]) {
         uint32_t mn[5];
 #pragma unroll
         for (int pos = 0; pos < 4; ++pos)
@@ -699,6 +748,7 @@ void count4_kernel(ExtractParams P) {
     if ((any_c0 | any_c1) == 0) {
       // no active cube: only the tile's vertex count (0) is read later
       if (lane == 0) P.tileT[t] = 0;
+      if (MASKS && lane < 16) reinterpret_cast<uint32_t*>(P.masks + (uint64_t)t * kCPW)[lane] = 0;
       load_plane(z + 3, L);
       t += tR;
       if (z - zb == 63 || z + 1 == z1) {
@@ -717,6 +767,13 @@ void count4_kernel(ExtractParams P) {
         zb = z + 1;
       }
       return;
+    }
+    if (MASKS) {
+      const int sh = 4 * (lane & 7);
+      const uint32_t w0 = or8(nib[0] << sh), w1 = or8(nib[1] << sh);
+      if ((lane & 7) < 2)
+        reinterpret_cast<uint32_t*>(P.masks + (uint64_t)t * kCPW)[(lane & 1) * 8 + (lane >> 3)] =
+            lane & 1 ? w1 : w0;
     }
     int nrec32 = 0;  // at most 512
 #pragma unroll
@@ -783,10 +840,10 @@ void count4_kernel(ExtractParams P) {
           x2 = __builtin_amdgcn_readlane(B.su[1], 0);
           x3 = __builtin_amdgcn_readlane(B.sw[1], 0);
         } else {
-          x0 = (A.xu & 0x8000u) ? 0xffu : 0u;
-          x1 = (A.xw & 0x8000u) ? 0xffu : 0u;
-          x2 = (B.xu & 0x8000u) ? 0xffu : 0u;
-          x3 = (B.xw & 0x8000u) ? 0xffu : 0u;
+          x0 = neg_byte(A.xu);
+          x1 = neg_byte(A.xw);
+          x2 = neg_byte(B.xu);
+          x3 = neg_byte(B.xw);
         }
         auto next = [&](uint32_t v, uint32_t x) {
           return __builtin_amdgcn_alignbyte(
@@ -1926,13 +1983,13 @@ int run_extract(ExtractParams& P, int elem, bool batch, int maxX, hipStream_t s,
   (void)maxX;
   // record scratch: per-column quotas; the wide count kernel keeps a quarter
   // of the scratch as a shared overflow pool
-  const bool wide = P.wide && elem == MCX_ELEM_SHORT2 && !P.write_masks;
+  const bool wide = P.wide;
   P.list_scan = emit;
-  const int64_t pool = wide ? P.rec_cap / 4 : 0;
+  const int64_t pool = wide && !P.write_masks ? P.rec_cap / 4 : 0;
   P.quota = P.ncols > 0 ? (P.rec_cap - pool) / P.ncols : 0;
   if (P.quota > (int64_t)kTile * P.slab_max) P.quota = (int64_t)kTile * P.slab_max;
   P.ovf_begin = P.quota * P.ncols;
-  P.ovf_cap = wide ? P.rec_cap - P.ovf_begin : 0;
+  P.ovf_cap = pool ? P.rec_cap - P.ovf_begin : 0;
   const unsigned k1_blocks = (unsigned)((P.ncols + 3) / 4);
   const unsigned k2_blocks = (unsigned)((P.n_tiles + kScanItems - 1) / kScanItems);
   const int64_t items = (P.n_tiles + 3) / 4;  // a workgroup is 4 waves, a wave takes tiles
@@ -1940,7 +1997,11 @@ int run_extract(ExtractParams& P, int elem, bool batch, int maxX, hipStream_t s,
   const unsigned k3_blocks = (unsigned)(items < k3_max ? items : k3_max);
 #define MCX_LAUNCH_SET(E, B)                                                                     \
   do {                                                                                           \
-    if (wide) hipLaunchKernelGGL(count4_kernel<B>, dim3(k1_blocks), dim3(256), 0, s, P);        \
+    if (wide && E == MCX_ELEM_F32 && P.write_masks)                                              \
+      hipLaunchKernelGGL((count4_kernel<E, B, E == MCX_ELEM_F32>), dim3(k1_blocks), dim3(256),   \
+                         0, s, P);                                                               \
+    else if (wide)                                                                               \
+      hipLaunchKernelGGL((count4_kernel<E, B, false>), dim3(k1_blocks), dim3(256), 0, s, P);     \
     else hipLaunchKernelGGL((count_kernel<E, B>), dim3(k1_blocks), dim3(256), 0, s, P);         \
     MCX_HIP(hipGetLastError());                                                                  \
     hipLaunchKernelGGL(scan_kernel, dim3(k2_blocks), dim3(256), 0, s, P);                        \

@@ -9,19 +9,28 @@
 // canonical order (the cubes interpolate the edge in different directions, so
 // their fp32 positions can differ in the last bit).
 //
-// W1 insert  hash table (open addressing, power of two >= 2V slots): the
-//            first lane of a wave holding a key (the smallest index of the
-//            key in the wave; vertices come in cube order, so a key often
-//            repeats within 64 vertices) claims the key's slot (atomicCAS)
-//            and records its index with atomicMin, so the slot ends with the
-//            first occurrence whatever the order of the atomics.
-// W2 flag    each vertex looks its key up: rep = first occurrence; unique
-//            vertices (rep == v) get flag 1; per-block flag sums.
-// W3 scan    exclusive scan of the block sums (one workgroup).
-// W4 place   unique index of every unique vertex; its position is copied;
-//            then every vertex's triangle index = unique index of its rep.
+// W1 insert  a workgroup takes 1024 vertices.  Its repeated keys are found in
+//            LDS (vertices come in cube order: about every third key of a
+//            block is new to it); the first of each claims the key's slot of a
+//            table of vertex indices in memory (open addressing, power of two
+//            >= 2V slots) with one atomicCAS, or lowers it with atomicMin, so
+//            a slot ends with the first occurrence whatever the order of the
+//            atomics.  Every vertex keeps its slot.
+// W2 rank    rep = table[slot] = the key's first occurrence; unique vertices
+//            (rep == v) get their rank in the block; per-block counts.
+// W3 scan    exclusive scan of the block counts (one workgroup).
+// W4 finish  triangle index = count before rep's block + rep's rank; unique
+//            vertices copy their position.
 // Deterministic: the table layout may vary between runs, what is read from
 // it (the minimum index per key) does not.
+//
+// Bound by the scattered atomics: of the insert's 41 us at 2.45 M vertices (a
+// 400^3 room) they are 25, the rest of the five launches 40.  A table of keys
+// and another of values, two atomics a key and per-wave repeats only, with a
+// second probe for the first occurrences, took 200 us for the whole weld where
+// this takes 82.  Tried: workgroups of 256 and 1024 threads for the insert (43
+// us), a table hashed key by key (47 us), a read of the slot before the CAS
+// (the same).
 #include <hip/hip_runtime.h>
 
 #include "mcx_internal.h"
@@ -29,11 +38,11 @@
 namespace mcx {
 namespace {
 
-// An empty slot holds kEmptyKey.  A vertex whose key equals it (-1 as int64:
-// never a grid-edge key, but the entry point accepts any int64) is kept in
-// the extra value slot T past the table, so that every key works.
-constexpr uint64_t kEmptyKey = ~0ull;
-constexpr int kWeldBlock = 1024;  // vertices per flag block (256 threads x 4)
+constexpr uint32_t kEmpty = 0xffffffffu;  // empty slot (V < 2^31)
+constexpr int kWeldBlock = 1024;          // vertices per workgroup (256 threads x 4)
+constexpr uint32_t kInsert = 512;  // threads of an insert workgroup
+constexpr uint32_t kPer = kWeldBlock / kInsert;
+constexpr uint32_t kLocal = 2 * kWeldBlock;  // slots of a workgroup's LDS table
 
 __device__ __forceinline__ uint64_t mix64(uint64_t k) {
   k ^= k >> 33;
@@ -44,148 +53,187 @@ __device__ __forceinline__ uint64_t mix64(uint64_t k) {
   return k;
 }
 
-__device__ __forceinline__ uint64_t find_slot(const uint64_t* keys, uint64_t mask, uint64_t key) {
-  if (key == kEmptyKey) return mask + 1;  // its own slot past the table
-  uint64_t h = mix64(key) & mask;
-  while (keys[h] != key) h = (h + 1) & mask;  // the key is present (inserted by W1)
-  return h;
+// First slot of a key.  Groups of 32 consecutive keys (the edges of 10 voxels
+// along x) stay in one 128-byte line, whose place and inner order are hashed:
+// the keys of a surface patch share lines, and keys a multiple of 32 apart
+// still start anywhere in the table.
+__device__ __forceinline__ uint32_t first_slot(uint64_t key, uint32_t mask) {
+  const uint64_t m = mix64(key >> 5);
+  return (((uint32_t)m << 5) | (((uint32_t)key ^ (uint32_t)(m >> 59)) & 31u)) & mask;
 }
 
-__global__ __launch_bounds__(256) void weld_insert_kernel(const int64_t* __restrict__ ekey,
-                                                          int64_t V, uint64_t* keys,
-                                                          uint32_t* vals, uint64_t mask) {
-  const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t key = v < V ? (uint64_t)ekey[v] : kEmptyKey;
-  // a lower lane of the wave with the same key inserts for this one (lanes
-  // past V are the highest of the last wave, so no live lane compares with
-  // them)
-  const int lane = (int)(threadIdx.x & 63);
-  const uint32_t klo = (uint32_t)key, khi = (uint32_t)(key >> 32);
-  bool dup = false;
-  for (int i = 0; i < 63; ++i) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)klo, i);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)khi, i);
-    dup |= i < lane && lo == klo && hi == khi;
-  }
-  if (v >= V || dup) return;
-  if (key == kEmptyKey) {
-    atomicMin(vals + mask + 1, (uint32_t)v);
-    return;
-  }
-  uint64_t h = mix64(key) & mask;
-  // at most V distinct keys in >= 2V slots: the probe ends
-  for (;;) {
-    const unsigned long long old =
-        atomicCAS(reinterpret_cast<unsigned long long*>(keys + h), kEmptyKey, key);
-    if (old == kEmptyKey || old == key) {
-      atomicMin(vals + h, (uint32_t)v);
-      return;
-    }
-    h = (h + 1) & mask;
-  }
-}
-
-__global__ __launch_bounds__(256) void weld_flag_kernel(const int64_t* __restrict__ ekey,
-                                                        int64_t V, const uint64_t* keys,
-                                                        const uint32_t* vals, uint64_t mask,
-                                                        uint32_t* rep, uint32_t* bsum) {
-  __shared__ uint32_t s_w[4];
-  const int64_t base = (int64_t)blockIdx.x * kWeldBlock;
-  uint32_t cnt = 0;
+__global__ __launch_bounds__(kInsert) void weld_insert_kernel(const int64_t* __restrict__ ekey,
+                                                          uint32_t V, uint32_t* table,
+                                                          uint32_t mask, uint32_t* slot) {
+  __shared__ uint64_t s_key[kWeldBlock];
+  __shared__ uint32_t s_tab[kLocal];  // index in the block of a key's first vertex
+  __shared__ uint32_t s_first[kWeldBlock];
+  __shared__ uint32_t s_n;
+  uint32_t* const s_slot = s_tab;  // once the first vertices are listed
+  const uint32_t tid = threadIdx.x;
+  const uint32_t base = blockIdx.x * (uint32_t)kWeldBlock;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int64_t v = base + k * 256 + threadIdx.x;
-    if (v < V) {
-      const uint32_t r = vals[find_slot(keys, mask, (uint64_t)ekey[v])];
-      rep[v] = r;
-      cnt += r == (uint32_t)v;
-    }
-  }
-  uint32_t t = cnt;
+  for (uint32_t i = tid; i < kLocal; i += kInsert) s_tab[i] = kEmpty;
+  uint64_t key[kPer];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) t += (uint32_t)__shfl_xor((int)t, o);
-  if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = t;
+  for (uint32_t k = 0; k < kPer; ++k) {
+    const uint32_t v = base + k * kInsert + tid;
+    key[k] = v < V ? (uint64_t)ekey[v] : 0;
+    s_key[k * kInsert + tid] = key[k];
+  }
+  if (tid == 0) s_n = 0;
   __syncthreads();
-  if (threadIdx.x == 0) bsum[blockIdx.x] = s_w[0] + s_w[1] + s_w[2] + s_w[3];
-}
-
-// Exclusive scan of nb block sums in place (one workgroup of 256 threads);
-// bsum[nb] = total.
-__global__ __launch_bounds__(256) void weld_scan_kernel(uint32_t* bsum, int64_t nb,
-                                                        int64_t* d_nunique) {
-  __shared__ uint32_t s_w[4];
-  __shared__ uint32_t s_carry;
-  if (threadIdx.x == 0) s_carry = 0;
-  __syncthreads();
-  for (int64_t b0 = 0; b0 < nb; b0 += 256) {
-    const int64_t i = b0 + threadIdx.x;
-    const uint32_t x = i < nb ? bsum[i] : 0u;
-    const uint32_t inc = wave_incl_scan32(x);
-    if ((threadIdx.x & 63) == 63) s_w[threadIdx.x >> 6] = inc;
-    __syncthreads();
-    uint32_t pre = s_carry;
-    const int w = threadIdx.x >> 6;
-    for (int k = 0; k < w; ++k) pre += s_w[k];
-    if (i < nb) bsum[i] = pre + inc - x;
-    __syncthreads();
-    if (threadIdx.x == 255) s_carry = pre + inc;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    bsum[nb] = s_carry;
-    if (d_nunique) *d_nunique = s_carry;
-  }
-}
-
-// Unique index of each unique vertex (block offset + rank inside the block),
-// its position copied to upos.  uidx doubles as the per-vertex unique index.
-__global__ __launch_bounds__(256) void weld_place_kernel(int64_t V, const uint32_t* rep,
-                                                         const uint32_t* bsum, const float* pos,
-                                                         int64_t stride, uint32_t* uidx,
-                                                         float* upos) {
-  __shared__ uint32_t s_w[4];
-  const int64_t base = (int64_t)blockIdx.x * kWeldBlock;
-  const int tid = threadIdx.x;
-  // thread owns vertices base + 4 tid .. +3 (consecutive: ranks in order)
-  uint32_t f[4];
-  uint32_t cnt = 0;
+  uint32_t at[kPer];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int64_t v = base + 4 * tid + k;
-    f[k] = v < V && rep[v] == (uint32_t)v;
-    cnt += f[k];
-  }
-  const uint32_t inc = wave_incl_scan32(cnt);
-  if ((tid & 63) == 63) s_w[tid >> 6] = inc;
-  __syncthreads();
-  uint32_t pre = bsum[blockIdx.x];
-  for (int k = 0; k < (tid >> 6); ++k) pre += s_w[k];
-  uint32_t r = pre + inc - cnt;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int64_t v = base + 4 * tid + k;
-    if (f[k]) {
-      uidx[v] = r;
-      upos[3 * (int64_t)r + 0] = pos[v * stride + 0];
-      upos[3 * (int64_t)r + 1] = pos[v * stride + 1];
-      upos[3 * (int64_t)r + 2] = pos[v * stride + 2];
-      ++r;
+  for (uint32_t k = 0; k < kPer; ++k) {
+    const uint32_t l = k * kInsert + tid;
+    at[k] = 0;
+    if (base + l >= V) continue;
+    uint32_t h = (uint32_t)mix64(key[k]) & (kLocal - 1);
+    for (;;) {  // at most 1024 keys in 2048 slots: the probe ends
+      const uint32_t old = atomicCAS(s_tab + h, kEmpty, l);
+      if (old == kEmpty) break;
+      if (s_key[old] == key[k]) {
+        if (l < old) atomicMin(s_tab + h, l);
+        break;
+      }
+      h = (h + 1) & (kLocal - 1);
     }
+    at[k] = h;
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < kPer; ++k) {
+    const uint32_t l = k * kInsert + tid;
+    if (base + l >= V) continue;
+    at[k] = s_tab[at[k]];
+    if (at[k] == l) s_first[atomicAdd(&s_n, 1u)] = l;
+  }
+  __syncthreads();
+  const uint32_t n = s_n;
+  for (uint32_t i = tid; i < n; i += kInsert) {
+    const uint32_t l = s_first[i], v = base + l;
+    const uint64_t mine = s_key[l];
+    uint32_t h = first_slot(mine, mask);
+    for (;;) {  // at most V distinct keys in >= 2V slots: the probe ends
+      const uint32_t old = atomicCAS(table + h, kEmpty, v);
+      if (old == kEmpty) break;
+      // a slot's index only changes to a lower one of the same key
+      if ((uint64_t)ekey[old] == mine) {
+        if (v < old) atomicMin(table + h, v);
+        break;
+      }
+      h = (h + 1) & mask;
+    }
+    s_slot[l] = h;
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < kPer; ++k) {
+    const uint32_t v = base + k * kInsert + tid;
+    if (v < V) slot[v] = s_slot[at[k]];
   }
 }
 
-__global__ __launch_bounds__(256) void weld_index_kernel(int64_t V, const uint32_t* rep,
-                                                         const uint32_t* uidx, int32_t* idx) {
-  const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (v < V) {
-    const uint32_t r = rep[v];  // the key's first occurrence: r <= v
-    idx[v] = r < (uint64_t)V ? (int32_t)uidx[r] : -1;
+// rep_of: a vertex's slot in, its key's first occurrence out.
+__global__ __launch_bounds__(256) void weld_rank_kernel(uint32_t V,
+                                                        const uint32_t* __restrict__ table,
+                                                        uint32_t* rep_of, uint32_t* rank,
+                                                        uint32_t* bsum) {
+  __shared__ uint32_t s_n[16];
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint32_t base = blockIdx.x * (uint32_t)kWeldBlock;
+  uint32_t s[4], r[4];
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    const uint32_t v = base + k * 256 + tid;
+    s[k] = v < V ? rep_of[v] : 0;
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) r[k] = base + k * 256 + tid < V ? table[s[k]] : kEmpty;
+  uint64_t first[4];
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    const uint32_t v = base + k * 256 + tid;
+    if (v < V) rep_of[v] = r[k];
+    first[k] = __ballot(r[k] == v);  // v >= V: r is kEmpty, never v
+    if (lane == 0) s_n[k * 4 + (tid >> 6)] = (uint32_t)__popcll(first[k]);
+  }
+  __syncthreads();
+  // 16 runs of 64 consecutive vertices
+  uint32_t before[4] = {0, 0, 0, 0}, all = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < 16; ++j) {
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+      if (j < k * 4 + (tid >> 6)) before[k] += s_n[j];
+    all += s_n[j];
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    const uint32_t v = base + k * 256 + tid;
+    if (r[k] == v)
+      rank[v] = before[k] + (uint32_t)__popcll(first[k] & ((1ull << lane) - 1));
+  }
+  if (tid == 0) bsum[blockIdx.x] = all;
+}
+
+// Exclusive scan of nb block sums in place (one workgroup of 1024 threads,
+// four sums a thread: one pass up to 4 million vertices); bsum[nb] = total.
+__global__ __launch_bounds__(1024) void weld_scan_kernel(uint32_t* bsum, uint32_t nb,
+                                                         int64_t* d_nunique) {
+  __shared__ uint32_t s_w[16];
+  const uint32_t tid = threadIdx.x;
+  uint32_t carry = 0;
+  for (uint32_t b0 = 0; b0 < nb; b0 += 4096) {
+    const uint32_t i = b0 + 4 * tid;
+    uint32_t x[4], sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+      x[k] = i + k < nb ? bsum[i + k] : 0u;
+      sum += x[k];
+    }
+    const uint32_t inc = wave_incl_scan32(sum);
+    if ((tid & 63) == 63) s_w[tid >> 6] = inc;
+    __syncthreads();
+    uint32_t pre = carry + inc - sum;
+#pragma unroll
+    for (uint32_t k = 0; k < 16; ++k) {
+      if (k < (tid >> 6)) pre += s_w[k];
+      carry += s_w[k];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+      if (i + k < nb) bsum[i + k] = pre;
+      pre += x[k];
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    bsum[nb] = carry;
+    if (d_nunique) *d_nunique = carry;
   }
 }
 
-__global__ __launch_bounds__(256) void fill_u64_kernel(uint64_t* p, int64_t n, uint64_t val) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = val;
+__global__ __launch_bounds__(256) void weld_finish_kernel(uint32_t V,
+                                                          const uint32_t* __restrict__ rep,
+                                                          const uint32_t* __restrict__ rank,
+                                                          const uint32_t* __restrict__ bsum,
+                                                          const float* __restrict__ pos,
+                                                          int64_t stride, int32_t* idx,
+                                                          float* upos) {
+  const uint32_t v = blockIdx.x * 256u + threadIdx.x;
+  if (v >= V) return;
+  const uint32_t r = rep[v];
+  const uint32_t u = bsum[r / kWeldBlock] + rank[r];
+  idx[v] = (int32_t)u;
+  if (r == v) {
+    const float* p = pos + (int64_t)v * stride;
+    float* q = upos + 3 * (int64_t)u;
+    q[0] = p[0];
+    q[1] = p[1];
+    q[2] = p[2];
+  }
 }
 
 uint64_t table_slots(int64_t V) {
@@ -229,37 +277,26 @@ extern "C" int mcx_weld(const int64_t* d_edge_key, const float* d_pos, int64_t s
   const uint64_t T = table_slots(V);
   const int64_t nb = (V + kWeldBlock - 1) / kWeldBlock;
   char* b = static_cast<char*>(d_ws);
-  uint64_t* keys = reinterpret_cast<uint64_t*>(b);
-  b += al256(T * 8);
-  uint32_t* vals = reinterpret_cast<uint32_t*>(b);
-  b += al256((T + 1) * 4);
-  uint32_t* rep = reinterpret_cast<uint32_t*>(b);
-  b += al256((size_t)V * 4 + 4);
-  uint32_t* uidx = reinterpret_cast<uint32_t*>(b);
-  b += al256((size_t)V * 4 + 4);
-  b += al256((size_t)V * 4 + 4);  // reserved
+  uint32_t* table = reinterpret_cast<uint32_t*>(b);
+  b += al256(T * 4);
+  uint32_t* rep = reinterpret_cast<uint32_t*>(b);  // slots, then first occurrences
+  b += al256((size_t)V * 4);
+  uint32_t* rank = reinterpret_cast<uint32_t*>(b);
+  b += al256((size_t)V * 4);
   uint32_t* bsum = reinterpret_cast<uint32_t*>(b);
-  int64_t fb = (int64_t)(T + 255) / 256;
-  if (fb > 65536) fb = 65536;
-  hipLaunchKernelGGL(fill_u64_kernel, dim3((unsigned)fb), dim3(256), 0, s, keys, (int64_t)T,
-                     kEmptyKey);
-  MCX_HIP(hipGetLastError());
-  int rc = fill_u32(vals, 0xffffffffu, (size_t)T + 1, s);
+  int rc = fill_u32(table, kEmpty, (size_t)T, s);
   if (rc) return rc;
-  const uint64_t mask = T - 1;
-  hipLaunchKernelGGL(weld_insert_kernel, dim3(grid_for(V, 256)), dim3(256), 0, s, d_edge_key, V,
-                     keys, vals, mask);
+  const uint32_t n = (uint32_t)V, mask = (uint32_t)(T - 1);
+  hipLaunchKernelGGL(weld_insert_kernel, dim3((unsigned)nb), dim3(kInsert), 0, s, d_edge_key, n, table,
+                     mask, rep);
   MCX_HIP(hipGetLastError());
-  hipLaunchKernelGGL(weld_flag_kernel, dim3((unsigned)nb), dim3(256), 0, s, d_edge_key, V, keys,
-                     vals, mask, rep, bsum);
+  hipLaunchKernelGGL(weld_rank_kernel, dim3((unsigned)nb), dim3(256), 0, s, n, table, rep, rank,
+                     bsum);
   MCX_HIP(hipGetLastError());
-  hipLaunchKernelGGL(weld_scan_kernel, dim3(1), dim3(256), 0, s, bsum, nb, d_nunique);
+  hipLaunchKernelGGL(weld_scan_kernel, dim3(1), dim3(1024), 0, s, bsum, (uint32_t)nb, d_nunique);
   MCX_HIP(hipGetLastError());
-  hipLaunchKernelGGL(weld_place_kernel, dim3((unsigned)nb), dim3(256), 0, s, V, rep, bsum, d_pos,
-                     stride_floats, uidx, d_upos);
-  MCX_HIP(hipGetLastError());
-  hipLaunchKernelGGL(weld_index_kernel, dim3(grid_for(V, 256)), dim3(256), 0, s, V, rep, uidx,
-                     d_indices);
+  hipLaunchKernelGGL(weld_finish_kernel, dim3(grid_for(V, 256)), dim3(256), 0, s, n, rep, rank,
+                     bsum, d_pos, stride_floats, d_indices, d_upos);
   MCX_HIP(hipGetLastError());
   if (h_nunique) {
     uint32_t total = 0;

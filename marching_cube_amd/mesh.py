@@ -133,6 +133,12 @@ def extract_into(vol, h, *, vv=None, pos=None, v2vox=None, ver_voxel=None, cap=N
     return int(hc.value) if sync else None
 
 
+def default_cap(X, Y, Z):
+    """Vertices that a mesh is first allocated for; a larger one is extracted
+    a second time."""
+    return max(4096, min(27_000_000, (X * Y * Z) // 16))
+
+
 def extract(vol, h, *, want=("vv",), cap=None, workspace=None):
     """Extract the mesh of `vol`; returns ExtractResult with tensors sized to
     the vertex count.  `want` selects among vv, pos, v2vox, ver_voxel.  The
@@ -141,7 +147,7 @@ def extract(vol, h, *, want=("vv",), cap=None, workspace=None):
     elem, X, Y, Z = volume_kind(vol)
     dev = vol.device
     if cap is None:
-        cap = max(4096, min(27_000_000, (X * Y * Z) // 16))
+        cap = default_cap(X, Y, Z)
     for _ in range(2):
         bufs = {
             "vv": torch.empty((cap, VV_WORDS), dtype=torch.int32, device=dev) if "vv" in want else None,
@@ -170,14 +176,20 @@ def indexed_mesh(vol, h, workspace=None):
     lib = _capi.load()
     ws = workspace or default_workspace(vol.device)
     ws.ensure(lib.mcx_extract_workspace_size(X, Y, Z))
-    n = extract_into(vol, h, cap=0, workspace=ws)
     dev = vol.device
-    pos = torch.empty((max(n, 1), 3), dtype=torch.float32, device=dev)
-    key = torch.empty(max(n, 1), dtype=torch.int64, device=dev)
+    cap = default_cap(X, Y, Z)
     hc = ctypes.c_int64(0)
-    _capi.check(lib.mcx_extract_ex(_ptr(vol), elem, X, Y, Z, float(h), None, _ptr(pos), None,
-                                   None, _ptr(key), n, None, ctypes.byref(hc), ws.ptr,
-                                   ws.nbytes, _stream_handle(dev)), "mcx_extract_ex")
+    for _ in range(2):
+        pos = torch.empty((cap, 3), dtype=torch.float32, device=dev)
+        key = torch.empty(cap, dtype=torch.int64, device=dev)
+        st = lib.mcx_extract_ex(_ptr(vol), elem, X, Y, Z, float(h), None, _ptr(pos), None, None,
+                                _ptr(key), cap, None, ctypes.byref(hc), ws.ptr, ws.nbytes,
+                                _stream_handle(dev))
+        if st != _capi.ERR_CAPACITY:
+            break
+        cap = hc.value
+    _capi.check(st, "mcx_extract_ex")
+    n = hc.value
     upos = torch.empty((max(n, 1), 3), dtype=torch.float32, device=dev)
     idx = torch.empty(max(n, 1), dtype=torch.int32, device=dev)
     wws = torch.empty(max(4096, lib.mcx_weld_workspace_size(n)), dtype=torch.uint8, device=dev)

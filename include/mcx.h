@@ -367,8 +367,8 @@ int mcx_raycast(const void* d_vol, int X, int Y, int Z, float h, float origin,
  *   d_dump (2-byte aligned, dump_cap bytes; mcx_rle_encode_bound(X, Y, nz)
  *   always suffices); the size goes to *d_dump_bytes and *h_dump_bytes (each
  *   may be NULL).  MCX_ERR_CAPACITY (nothing written) if it exceeds dump_cap.
- *   Workspace: mcx_rle_encode_workspace_size(X, Y, nz) bytes (16 per voxel:
- *   encode large volumes in slabs).  Synchronises the stream.
+ *   Workspace: mcx_rle_encode_workspace_size(X, Y, nz) bytes (40 per started
+ *   4096 voxels of a slice, and a little).  Synchronises the stream.
  * mcx_rle_decode: nz slices into d_vol[nz][Y][X]; slice j's uint32 byte
  *   count sits at byte h_slice_offsets[j] (host array) of d_dump (2-byte
  *   aligned, dump_bytes).  MCX_ERR_FORMAT for a malformed slice (offset

@@ -8,27 +8,41 @@
 // follows.  A run is a maximal stretch of equal tsdf (weights are not
 // compared; the record keeps the run's first voxel), cut every 0x3fff voxels.
 //
-// Encode (flat over the slab's voxels, no sequential pass):
-//   E1 count   tsdf change points per 1024 voxels (slice starts always);
-//   scan       exclusive prefix of the counts;
-//   E2 compact change-point positions in order;
-//   E3 size    bytes of each change point's records (+4 for a slice start);
-//   scan       byte offsets;
-//   E4 write   records (and slice byte counts) at their offsets.
+// Encode (flat over the slab's voxels, no sequential pass).  A run's bytes are
+// known where the next one starts, so a block of 4096 voxels accounts for the
+// runs that end in it, and blocks compose: (first and last run start, bytes of
+// the runs between) of two neighbours give those of both, with the run that
+// crosses from one to the other.
+//   E1 runs    the state of every block;
+//   scan       exclusive composition of the states (groups of 1024);
+//   E2 write   the volume's second and last reading: every block writes the
+//              records of the runs that end in it (a crossing run's by all
+//              its threads) and, for a slice start, the slice's byte count.
+// Bound by the two readings.  512^3 (a fused room, 28 MB of dump) in one call:
+// E1 104 us (the copy rate), E2 190; in calls of 2^24 voxels 670 us, most of it
+// eight ramps and read-backs.  With lists of run starts and of their bytes (16
+// bytes of workspace a voxel, two more passes, the number of runs read back)
+// it took 397 and 824.  1024 voxels a block: 720 instead of 670.
 // Decode (records are 1 or 3 words, so a record boundary cannot be told
 // from a word alone):
 //   D0 index   each slice's payload range from the caller's offsets;
-//   D1 resolve one workgroup per slice; every thread parses a 64-word
-//              chunk from each of the three possible entry offsets (the
-//              first record at or after the chunk start begins 0, 1 or 2
-//              words in), giving a map entry offset -> (exit offset, voxels,
-//              records); a block scan composes the maps, so each chunk
-//              learns its true entry offset, voxel and record positions; it
-//              re-parses and writes (first voxel, value) per record and, for
-//              every 4096-voxel tile, the record covering the tile's start;
-//   D2 fill    one workgroup per tile stages the tile's records in LDS and
-//              writes the voxels (coalesced, balanced whatever the run
-//              lengths).
+//   D1 resolve one workgroup per slice, 16 K words at a time through LDS;
+//              every thread parses a 32-word chunk from each of the three
+//              possible entry offsets (the first record at or after the chunk
+//              start begins 0, 1 or 2 words in), giving a map entry offset ->
+//              (exit offset, voxels, records); a block scan composes the maps,
+//              so each chunk learns its true entry offset, voxel and record
+//              positions; it re-parses and writes (first voxel, value) per
+//              record and, for every 4096-voxel tile, the record covering the
+//              tile's start;
+//   D2 fill    one workgroup per tile stages the tile's runs in LDS, marks the
+//              voxels where they start and writes every voxel by rank
+//              (coalesced, balanced whatever the run lengths).
+// The same dump: D1 84 us, bound by the chains of dependent record headers, D2
+// 114 us, the rate that memory takes writes at; 64-word chunks parsed from
+// memory one entry after the other took 196, a search for each voxel's run
+// 200.  D1 with 1024 threads or 16-word chunks 99-134 us (more maps to compose
+// for shorter chains), 256 threads 117-150.
 // Malformed input (a run of length 0, runs past the slice, a truncated
 // record, bytes left over, offsets outside the dump) is detected on the
 // device and reported as MCX_ERR_FORMAT; every access stays in bounds.
@@ -43,11 +57,14 @@ namespace {
 
 constexpr uint32_t kRunMax = 0x3fff;
 constexpr int kMaxT = 32766;
-constexpr int kBlk = 1024;        // scan block / encode count block (256 threads x 4)
-constexpr int kChunkWords = 64;   // decode: words per speculative-parse chunk
+constexpr int kSub = 1024;        // encode: voxels a workgroup reads at once (4 a thread)
+constexpr int kSubs = 4;          // ... and how many times
+constexpr int kEncBlk = kSub * kSubs;  // voxels of an encode block
+constexpr int kBlk = 1024;        // states of a scan group
+constexpr int64_t kMaxRuns = (int64_t)1 << 31;  // more are refused
+constexpr int kChunkWords = 32;   // decode: words per speculative-parse chunk
+constexpr int kResolve = 512;     // decode: threads (chunks) per slice and round
 constexpr int kFillTile = 4096;   // decode: voxels per fill workgroup
-constexpr int kFillStage = kFillTile + 256;
-constexpr uint64_t kSliceStart = 1ull << 63;
 constexpr uint32_t kNoRecord = 0xffffffffu;
 
 __device__ __forceinline__ int tsdf_of(uint32_t v) { return (int)(int16_t)(v & 0xffffu); }
@@ -55,198 +72,325 @@ __device__ __forceinline__ bool saturated(int t) { return t == kMaxT || t == -kM
 
 size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// ------------------------------------------------------------ int64 scan
-// Exclusive scan in place of a[0..n), a[n] = total (a holds n + 1).
-__global__ __launch_bounds__(256) void scan_block_kernel(int64_t* a, int64_t n, int64_t* bsum) {
-  __shared__ int64_t s_w[4];
-  const int tid = threadIdx.x;
-  const int64_t base = (int64_t)blockIdx.x * kBlk + 4 * tid;
-  int64_t v[4];
-  int64_t t = 0;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    v[k] = base + k < n ? a[base + k] : 0;
-    t += v[k];
-  }
-  const int64_t inc = (int64_t)wave_incl_scan((uint64_t)t);
-  if ((tid & 63) == 63) s_w[tid >> 6] = inc;
-  __syncthreads();
-  int64_t pre = 0;
-  for (int w = 0; w < (tid >> 6); ++w) pre += s_w[w];
-  int64_t run = pre + inc - t;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (base + k < n) a[base + k] = run;
-    run += v[k];
-  }
-  if (tid == 255) {
-    if (bsum)
-      bsum[blockIdx.x] = run;
-    else
-      a[n] = run;  // single block: the total
-  }
-}
-
-__global__ __launch_bounds__(256) void scan_add_kernel(int64_t* a, int64_t n, const int64_t* boff,
-                                                       int64_t nb) {
-  const int64_t base = (int64_t)blockIdx.x * kBlk + 4 * threadIdx.x;
-  const int64_t add = boff[blockIdx.x];
-#pragma unroll
-  for (int k = 0; k < 4; ++k)
-    if (base + k < n) a[base + k] += add;
-  if (blockIdx.x == 0 && threadIdx.x == 0) a[n] = boff[nb];
-}
-
-int64_t scan_tmp_elems(int64_t n) {
-  if (n <= kBlk) return 0;
-  const int64_t nb = (n + kBlk - 1) / kBlk;
-  return nb + 1 + scan_tmp_elems(nb);
-}
-
-int scan_excl(int64_t* a, int64_t n, int64_t* tmp, hipStream_t s) {
-  if (n <= 0) return fill_bytes_zero(a, sizeof(int64_t), s);
-  const int64_t nb = (n + kBlk - 1) / kBlk;
-  if (nb == 1) {
-    hipLaunchKernelGGL(scan_block_kernel, dim3(1), dim3(256), 0, s, a, n, (int64_t*)nullptr);
-    MCX_HIP(hipGetLastError());
-    return MCX_OK;
-  }
-  hipLaunchKernelGGL(scan_block_kernel, dim3((unsigned)nb), dim3(256), 0, s, a, n, tmp);
-  MCX_HIP(hipGetLastError());
-  int rc = scan_excl(tmp, nb, tmp + nb + 1, s);
-  if (rc) return rc;
-  hipLaunchKernelGGL(scan_add_kernel, dim3((unsigned)nb), dim3(256), 0, s, a, n, tmp, nb);
-  MCX_HIP(hipGetLastError());
-  return MCX_OK;
-}
-
 // ---------------------------------------------------------------- encode
 typedef uint32_t u32x4a4 __attribute__((ext_vector_type(4), aligned(4)));  // 4-byte aligned
 
-// grid (blocks per slice, nz): change points among 1024 voxels of slice z.
-// Bit k: voxel i0 + k starts a run (the first of the slice, or a tsdf that
-// differs from the voxel before it).
-__device__ __forceinline__ uint32_t change_flags(const uint32_t* __restrict__ sl, int64_t XY,
-                                                 int64_t i0) {
-  uint32_t f = 0;
-  if (i0 + 4 <= XY) {
-    // the four voxels in one 128-bit load (the slice is 4-byte aligned,
-    // which the vector memory path accepts), the one before in another
-    const u32x4a4 v = *reinterpret_cast<const u32x4a4*>(sl + i0);
-    int prev = i0 > 0 ? tsdf_of(sl[i0 - 1]) : 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int t = tsdf_of(v[k]);
-      if (i0 + k == 0 || t != prev) f |= 1u << k;
-      prev = t;
-    }
-    return f;
-  }
-  int prev = i0 > 0 && i0 - 1 < XY ? tsdf_of(sl[i0 - 1]) : 0;
+// The runs of a stretch of voxels: where the first and the last start (flat
+// indices; first < 0: none starts here), bytes of those that end before the
+// last start, how many start, and the last one's bytes a record and lead (a
+// slice's byte count before its first run).
+struct Runs {
+  int64_t first, last, bytes, count;
+  uint32_t rec, lead;
+};
+
+__device__ __forceinline__ uint32_t records(int64_t s, int64_t e) {  // of a run [s, e)
+  return ((uint32_t)(e - s) + kRunMax - 1) / kRunMax;
+}
+
+// Bytes of a's last run, which ends at e.
+__device__ __forceinline__ int64_t last_bytes(const Runs& a, int64_t e) {
+  return a.first < 0 ? 0 : (int64_t)records(a.last, e) * a.rec + a.lead;
+}
+
+// a, then b
+__device__ __forceinline__ Runs then(const Runs& a, const Runs& b) {
+  Runs o = b.first < 0 ? a : b;
+  o.first = a.first < 0 ? b.first : a.first;
+  o.bytes = a.bytes + b.bytes + (b.first < 0 ? 0 : last_bytes(a, b.first));
+  o.count = a.count + b.count;
+  return o;
+}
+
+__device__ __forceinline__ Runs no_runs() { return Runs{-1, -1, 0, 0, 0, 0}; }
+
+__device__ __forceinline__ Runs shfl_up_runs(const Runs& a, int d) {
+  Runs o;
+  o.first = __shfl_up((long long)a.first, d, kWave);
+  o.last = __shfl_up((long long)a.last, d, kWave);
+  o.bytes = __shfl_up((long long)a.bytes, d, kWave);
+  o.count = __shfl_up((long long)a.count, d, kWave);
+  o.rec = __shfl_up(a.rec, d, kWave);
+  o.lead = __shfl_up(a.lead, d, kWave);
+  return o;
+}
+
+// Exclusive composition of 1024 states in place (kBlk a workgroup, four a
+// thread); group[block] = all of them.
+__global__ __launch_bounds__(256) void enc_scan_kernel(Runs* a, int64_t n, Runs* group) {
+  __shared__ Runs s_w[4];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int64_t base = (int64_t)blockIdx.x * kBlk + 4 * tid;
+  Runs v[4], all = no_runs();
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const int64_t i = i0 + k;
-    if (i < XY) {
-      const int t = tsdf_of(sl[i]);
-      if (i == 0 || t != prev) f |= 1u << k;
-      prev = t;
-    }
+    v[k] = base + k < n ? a[base + k] : no_runs();
+    all = then(all, v[k]);
   }
-  return f;
-}
-
-__global__ __launch_bounds__(256) void enc_count_kernel(const uint32_t* __restrict__ vol,
-                                                        int64_t XY, int64_t* cnt) {
-  __shared__ uint32_t s_w[4];
-  const int tid = threadIdx.x;
-  const int64_t z = blockIdx.y;
-  const uint32_t f = change_flags(vol + z * XY, XY, (int64_t)blockIdx.x * kBlk + 4 * tid);
-  uint32_t c = __popc(f);
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) c += (uint32_t)__shfl_xor((int)c, o);
-  if ((tid & 63) == 0) s_w[tid >> 6] = c;
-  __syncthreads();
-  if (tid == 0) cnt[z * gridDim.x + blockIdx.x] = s_w[0] + s_w[1] + s_w[2] + s_w[3];
-}
-
-__global__ __launch_bounds__(256) void enc_compact_kernel(const uint32_t* __restrict__ vol,
-                                                          int64_t XY, const int64_t* ofs,
-                                                          uint64_t* cp, int64_t* slice_first) {
-  __shared__ uint32_t s_w[4];
-  const int tid = threadIdx.x;
-  const int64_t z = blockIdx.y;
-  const int64_t i0 = (int64_t)blockIdx.x * kBlk + 4 * tid;
-  const uint32_t f = change_flags(vol + z * XY, XY, i0);
-  const uint32_t c = __popc(f);
-  const uint32_t inc = wave_incl_scan32(c);
-  if ((tid & 63) == 63) s_w[tid >> 6] = inc;
-  __syncthreads();
-  uint32_t pre = 0;
-  for (int w = 0; w < (tid >> 6); ++w) pre += s_w[w];
-  int64_t k = ofs[z * gridDim.x + blockIdx.x] + pre + inc - c;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    if (f & (1u << e)) {
-      const int64_t i = i0 + e;
-      cp[k] = (uint64_t)(z * XY + i) | (i == 0 ? kSliceStart : 0);
-      if (i == 0) slice_first[z] = k;
-      ++k;
-    }
+  for (int d = 1; d < kWave; d <<= 1) {
+    const Runs g = shfl_up_runs(all, d);
+    if (lane >= d) all = then(g, all);
   }
+  if (lane == 63) s_w[wv] = all;
+  __syncthreads();
+  Runs pre = no_runs();
+  for (int k = 0; k < wv; ++k) pre = then(pre, s_w[k]);
+  const Runs up = shfl_up_runs(all, 1);
+  if (lane > 0) pre = then(pre, up);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (base + k < n) a[base + k] = pre;
+    pre = then(pre, v[k]);
+  }
+  if (tid == 255) group[blockIdx.x] = pre;
 }
 
-__global__ __launch_bounds__(256) void enc_size_kernel(const uint32_t* __restrict__ vol,
-                                                       const uint64_t* cp, int64_t M, int64_t N,
-                                                       int64_t* bytes) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= M) return;
-  const uint64_t c = cp[k];
-  const int64_t s = (int64_t)(c & ~kSliceStart);
-  const int64_t e = k + 1 < M ? (int64_t)(cp[k + 1] & ~kSliceStart) : N;
-  const int64_t nrec = (e - s + kRunMax - 1) / kRunMax;
-  const int64_t rs = saturated(tsdf_of(vol[s])) ? 2 : 6;
-  bytes[k] = nrec * rs + ((c & kSliceStart) ? 4 : 0);
+// Levels above the first: a[i] becomes what is before it, all the way down.
+__global__ __launch_bounds__(256) void enc_lift_kernel(Runs* a, int64_t n, const Runs* group) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) a[i] = then(group[i / kBlk], a[i]);
+}
+
+// The four voxels of a thread and the run starts among them (bit k: the first
+// voxel of the slice, or a tsdf that differs from the voxel before it).
+struct Four {
+  uint32_t v[4];
+  uint32_t starts;
+};
+
+// sl: a slice, i0: the thread's first voxel; all lanes of a wave take part.
+__device__ __forceinline__ Four four_voxels(const uint32_t* __restrict__ sl, int64_t XY,
+                                            int64_t i0) {
+  Four q;
+  if (i0 + 4 <= XY) {
+    // one 128-bit load (the slice is 4-byte aligned, which the vector memory
+    // path accepts)
+    const u32x4a4 v = *reinterpret_cast<const u32x4a4*>(sl + i0);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) q.v[k] = v[k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) q.v[k] = i0 + k < XY ? sl[i0 + k] : 0u;
+  }
+  uint32_t before = __shfl_up(q.v[3], 1, kWave);
+  if ((threadIdx.x & 63) == 0 && i0 > 0 && i0 < XY) before = sl[i0 - 1];
+  q.starts = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const bool change = i0 + k == 0 || tsdf_of(q.v[k]) != tsdf_of(k ? q.v[k - 1] : before);
+    if (change && i0 + k < XY) q.starts |= 1u << k;
+  }
+  return q;
+}
+
+// Bytes of a record of a run that starts with voxel v.
+__device__ __forceinline__ uint32_t record_bytes(uint32_t v) {
+  return saturated(tsdf_of(v)) ? 2u : 6u;
+}
+
+// Bytes of one record for each of a thread's run starts (no run inside a
+// block is longer than a record: kBlk <= kRunMax), and the slice's lead.
+__device__ __forceinline__ uint32_t four_bytes(const Four& q, int64_t i0) {
+  uint32_t b = i0 == 0 ? 4u : 0u;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (q.starts >> k & 1u) b += record_bytes(q.v[k]);
+  return b;
+}
+static_assert(kEncBlk <= (int)kRunMax, "a run inside a block is one record");
+
+// grid (blocks per slice, nz)
+__global__ __launch_bounds__(256) void enc_runs_kernel(const uint32_t* __restrict__ vol,
+                                                       int64_t XY, Runs* a) {
+  // of each wave: bytes of a record for every start (and the lead) << 16 |
+  // starts; first start (kEncBlk: none) and last start (-1) in the block;
+  // bytes of the last one's records, and its lead in bit 8
+  __shared__ uint32_t s_sum[4], s_rec[4];
+  __shared__ int s_first[4], s_last[4];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int64_t z = blockIdx.y;
+  const int64_t base = (int64_t)blockIdx.x * kEncBlk;
+  Four q[kSubs];
+#pragma unroll
+  for (int j = 0; j < kSubs; ++j) q[j] = four_voxels(vol + z * XY, XY, base + j * kSub + 4 * tid);
+  uint32_t sum = 0, rec = 0;
+  int first = kEncBlk, last = -1;
+#pragma unroll
+  for (int j = 0; j < kSubs; ++j) {
+    const uint64_t any = __ballot(q[j].starts != 0);
+    if (any == 0) continue;
+    const int i = j * kSub + 4 * tid;
+    sum += four_bytes(q[j], base + i) << 16 | (uint32_t)__popc(q[j].starts);
+    const int k = 31 - __clz(q[j].starts | 1u);
+    const uint32_t v = k == 0 ? q[j].v[0] : k == 1 ? q[j].v[1] : k == 2 ? q[j].v[2] : q[j].v[3];
+    const int lo = __ffsll((unsigned long long)any) - 1, hi = 63 - __clzll((long long)any);
+    const uint32_t r = record_bytes(v) | (base + i + k == 0 ? 4u << 8 : 0u);
+    first = min(first, __builtin_amdgcn_readlane(i + __ffs(q[j].starts) - 1, lo));
+    last = __builtin_amdgcn_readlane(i + k, hi);
+    rec = __builtin_amdgcn_readlane(r, hi);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);  // a wave's bytes < 2^13
+  if (lane == 0) {
+    s_sum[wv] = sum;
+    s_rec[wv] = rec;
+    s_first[wv] = first;
+    s_last[wv] = last;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    sum = s_sum[0];
+    for (int w = 1; w < 4; ++w) {
+      sum += s_sum[w];
+      first = min(first, s_first[w]);
+      if (s_last[w] > last) {
+        last = s_last[w];
+        rec = s_rec[w];
+      }
+    }
+    Runs r = no_runs();
+    if (last >= 0) {
+      r.first = z * XY + base + first;
+      r.last = z * XY + base + last;
+      r.rec = rec & 0xffu;
+      r.lead = rec >> 8;
+      r.bytes = (int64_t)(sum >> 16) - r.rec - r.lead;
+      r.count = sum & 0xffffu;
+    }
+    a[z * gridDim.x + blockIdx.x] = r;
+  }
 }
 
 __device__ __forceinline__ void put16(uint16_t* out16, int64_t byte_pos, uint32_t v) {
   out16[byte_pos >> 1] = (uint16_t)v;
 }
 
-__global__ __launch_bounds__(256) void enc_write_kernel(const uint32_t* __restrict__ vol,
-                                                        int64_t XY, const uint64_t* cp, int64_t M,
-                                                        int64_t N, const int64_t* ofs,
-                                                        const int64_t* slice_first, int nz,
-                                                        uint16_t* out16, int64_t cap,
-                                                        int64_t* d_total) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t total = ofs[M];
-  if (k == 0 && d_total) *d_total = total;
-  if (k >= M || total > cap) return;
-  const uint64_t c = cp[k];
-  const int64_t s = (int64_t)(c & ~kSliceStart);
-  const int64_t e = k + 1 < M ? (int64_t)(cp[k + 1] & ~kSliceStart) : N;
-  int64_t pos = ofs[k];
-  if (c & kSliceStart) {
-    const int64_t z = s / XY;
-    const int64_t next = z + 1 < nz ? ofs[slice_first[z + 1]] : total;
-    const uint32_t sz = (uint32_t)(next - pos - 4);
-    put16(out16, pos, sz & 0xffffu);
-    put16(out16, pos + 2, sz >> 16);
-    pos += 4;
+// One record of n voxels, the first of them v.
+__device__ __forceinline__ void put_record(uint16_t* out16, int64_t pos, uint32_t n, uint32_t v) {
+  const int t = tsdf_of(v);
+  const uint32_t kind = t == kMaxT ? 1u : t == -kMaxT ? 2u : 3u;
+  put16(out16, pos, n | (kind << 14));
+  if (kind == 3u) {
+    put16(out16, pos + 2, v & 0xffffu);
+    put16(out16, pos + 4, v >> 16);
   }
-  const int t = tsdf_of(vol[s]);
-  const uint32_t v = t == kMaxT ? 1u : t == -kMaxT ? 2u : 3u;
-  for (int64_t r = s; r < e; r += kRunMax) {
-    const uint32_t n = (uint32_t)min((int64_t)kRunMax, e - r);
-    put16(out16, pos, n | (v << 14));
-    pos += 2;
-    if (v == 3u) {
-      const uint32_t val = vol[r];
-      put16(out16, pos, val & 0xffffu);
-      put16(out16, pos + 2, val >> 16);
-      pos += 4;
+}
+
+// What is before block b of the slab (group: null if there is one group).
+__device__ __forceinline__ Runs before(const Runs* a, const Runs* group, int64_t b) {
+  return group ? then(group[b / kBlk], a[b]) : a[b];
+}
+
+// All records of the last run of `a`, which ends at e, the last of them ending
+// at byte `end`; the workgroup's threads take them in turn.
+__device__ __forceinline__ void put_run(uint16_t* out16, const uint32_t* __restrict__ vol,
+                                        const Runs& a, int64_t e, int64_t end) {
+  const uint32_t n = records(a.last, e);
+  for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) {
+    const int64_t r = a.last + (int64_t)k * kRunMax;
+    put_record(out16, end - (int64_t)(n - k) * a.rec, (uint32_t)min((int64_t)kRunMax, e - r),
+               vol[r]);
+  }
+}
+
+// all: the slab's state; totals: [bytes, runs]
+__global__ __launch_bounds__(256) void enc_write_kernel(const uint32_t* __restrict__ vol,
+                                                        int64_t XY, int64_t N, const Runs* a,
+                                                        const Runs* group, const Runs* all,
+                                                        uint16_t* out16, int64_t cap,
+                                                        int64_t* totals, int64_t* d_total) {
+  // of each run of 256 voxels: bytes, and the first start in the block
+  // (kEncBlk: none)
+  __shared__ uint32_t s_bytes[4 * kSubs];
+  __shared__ uint32_t s_first[4 * kSubs];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int64_t z = blockIdx.y, nblk = (int64_t)gridDim.x * gridDim.y;
+  const int64_t b = z * gridDim.x + blockIdx.x;
+  const int64_t base = (int64_t)blockIdx.x * kEncBlk;
+  // all loads at once: a block's life is short
+  Four q[kSubs];
+#pragma unroll
+  for (int j = 0; j < kSubs; ++j) q[j] = four_voxels(vol + z * XY, XY, base + j * kSub + 4 * tid);
+  const Runs pre = before(a, group, b);
+  const Runs end = *all;
+  const int64_t total = end.bytes + last_bytes(end, N);
+  if (b == 0 && tid == 0) {
+    totals[0] = total;
+    totals[1] = end.count;
+    if (d_total && end.count < kMaxRuns) *d_total = total;
+  }
+  if (total > cap || end.count >= kMaxRuns) return;
+  uint64_t any[kSubs];
+  uint32_t off[kSubs];  // bytes of the run's earlier starts
+#pragma unroll
+  for (int j = 0; j < kSubs; ++j) {
+    any[j] = __ballot(q[j].starts != 0);
+    uint32_t bytes = 0, first = kEncBlk;
+    off[j] = 0;
+    if (any[j]) {
+      const int i = j * kSub + 4 * tid;
+      const uint32_t mine = four_bytes(q[j], base + i);
+      const uint32_t inc = wave_incl_scan32(mine);
+      off[j] = inc - mine;
+      bytes = __builtin_amdgcn_readlane(inc, 63);
+      first = __builtin_amdgcn_readlane(i + __ffs(q[j].starts) - 1,
+                                        __ffsll((unsigned long long)any[j]) - 1);
+    }
+    if (lane == 0) {
+      s_bytes[4 * j + wv] = bytes;
+      s_first[4 * j + wv] = first;
     }
   }
+  __syncthreads();
+  uint32_t first = kEncBlk;
+#pragma unroll
+  for (int k = 4 * kSubs - 1; k >= 0; --k) first = min(first, s_first[k]);
+  if (first < (uint32_t)kEncBlk) {  // uniform over the block
+    // the run before the block's first, which ends here
+    const int64_t begin = pre.bytes + last_bytes(pre, z * XY + base + first);
+    if (pre.first >= 0) put_run(out16, vol, pre, z * XY + base + first, begin);
+#pragma unroll
+    for (int j = 0; j < kSubs; ++j) {
+      if (any[j] == 0) continue;
+      const int i = j * kSub + 4 * tid;
+      // what the earlier runs of 256 take, and the next start after this one
+      uint32_t skip = 0, next = kEncBlk;
+#pragma unroll
+      for (int k = 0; k < 4 * kSubs; ++k) {
+        if (k < 4 * j + wv) skip += s_bytes[k];
+        if (k > 4 * j + wv) next = min(next, s_first[k]);
+      }
+      // the next start after this thread's own
+      const uint64_t later = lane < 63 ? any[j] >> (lane + 1) << (lane + 1) : 0;
+      const uint32_t in_wave = __shfl((uint32_t)(i + __ffs(q[j].starts) - 1),
+                                      later ? __ffsll((unsigned long long)later) - 1 : 0, kWave);
+      if (later) next = in_wave;
+      int64_t pos = begin + skip + off[j];
+      if (base + i == 0) {
+        int64_t stop = total;
+        if (z + 1 < (int64_t)gridDim.y) {
+          const Runs p = before(a, group, b + gridDim.x);
+          stop = p.bytes + last_bytes(p, (z + 1) * XY);
+        }
+        const uint32_t size = (uint32_t)(stop - pos - 4);
+        put16(out16, pos, size & 0xffffu);
+        put16(out16, pos + 2, size >> 16);
+        pos += 4;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (!(q[j].starts >> k & 1u)) continue;
+        const uint32_t above = q[j].starts >> (k + 1);
+        const uint32_t at = i + k;
+        const uint32_t stop = above ? at + __ffs(above) : next;
+        // the block's last run ends in a later block, which writes it
+        if (stop < (uint32_t)kEncBlk) put_record(out16, pos, stop - at, q[j].v[k]);
+        pos += record_bytes(q[j].v[k]);
+      }
+    }
+  }
+  if (b + 1 == nblk) put_run(out16, vol, end, N, total);
 }
 
 // ---------------------------------------------------------------- decode
@@ -328,44 +472,63 @@ __global__ __launch_bounds__(256) void dec_index_kernel(const uint16_t* __restri
   info[j] = si;
 }
 
-__global__ __launch_bounds__(256) void dec_resolve_kernel(const uint16_t* __restrict__ d16,
-                                                          int64_t XY, int tps, SliceInfo* info,
-                                                          uint32_t* rec_start, uint32_t* rec_val,
-                                                          uint32_t* tile_first, uint32_t* err) {
-  __shared__ Fn s_fn[4];
+// Place of word i of a round in LDS: a dword of padding per chunk, so that the
+// lanes' chunks (17 dwords apart) start in different banks.
+__device__ __forceinline__ int staged(int i) { return i + 2 * (i / kChunkWords); }
+
+__global__ __launch_bounds__(kResolve) void dec_resolve_kernel(const uint16_t* __restrict__ d16,
+                                                               int64_t XY, int tps,
+                                                               SliceInfo* info, uint2* rec,
+                                                               uint32_t* tile_first,
+                                                               uint32_t* err) {
+  constexpr int kRound = kResolve * kChunkWords;  // words a workgroup resolves at once
+  __shared__ Fn s_fn[kResolve / kWave];
+  __shared__ uint16_t s_w[kRound + 2 * kResolve + 4];  // and the two after them
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int j = blockIdx.x;
   const SliceInfo si = info[j];
   if (si.words == 0) return;  // flagged by the index kernel
   const uint16_t* __restrict__ w = d16 + si.word_base;
   const int64_t L = si.words;
-  const int64_t nch = (L + kChunkWords - 1) / kChunkWords;
-  uint32_t* rs = rec_start + si.word_base;
-  uint32_t* rv = rec_val + si.word_base;
+  uint2* rs = rec + si.word_base;
   uint32_t* tf = tile_first + (int64_t)j * tps;
   uint32_t cp = 0, cv = 0, cr = 0;  // carry: entry offset, voxels, records
   bool bad = false;
-  for (int64_t c0 = 0; c0 < nch; c0 += 256) {
-    const int64_t c = c0 + tid;
-    const int64_t beg = c * kChunkWords;
-    const int64_t end = min(beg + kChunkWords, L);
+  for (int64_t w0 = 0; w0 < L; w0 += kRound) {
+    const int n_words = (int)min((int64_t)kRound, L - w0);
+    uint16_t in[kChunkWords];
+#pragma unroll
+    for (int k = 0; k < kChunkWords; ++k) {
+      const int i = k * kResolve + tid;
+      in[k] = i < n_words ? w[w0 + i] : (uint16_t)0;
+    }
+#pragma unroll
+    for (int k = 0; k < kChunkWords; ++k) s_w[staged(k * kResolve + tid)] = in[k];
+    if (tid < 2) s_w[staged(kRound + tid)] = w0 + kRound + tid < L ? w[w0 + kRound + tid] : 0;
+    __syncthreads();
+    const int beg = tid * kChunkWords;
+    const int end = min(beg + kChunkWords, n_words);
     Fn f = fn_identity();
-    if (c < nch) {
-      f.ex = 0;
-#pragma unroll 1
-      for (uint32_t p = 0; p < 3; ++p) {
-        int64_t pos = beg + p;
-        uint32_t vox = 0, rec = 0;
-        while (pos < end) {
-          const uint32_t h = w[pos];
-          vox = sat_add(vox, h & kRunMax);
-          ++rec;
-          pos += record_words(h);
+    if (beg < n_words) {
+      // the three entry offsets side by side: three loads in flight
+      int pos[3] = {beg, beg + 1, beg + 2};
+      bool more = true;
+      while (more) {
+        more = false;
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          if (pos[p] < end) {
+            const uint32_t h = s_w[staged(pos[p])];
+            f.v[p] = sat_add(f.v[p], h & kRunMax);
+            ++f.r[p];
+            pos[p] += record_words(h);
+            more = true;
+          }
         }
-        f.ex |= (uint32_t)(pos - end) << (2 * p);
-        f.v[p] = vox;
-        f.r[p] = rec;
       }
+      f.ex = 0;
+#pragma unroll
+      for (int p = 0; p < 3; ++p) f.ex |= (uint32_t)(pos[p] - end) << (2 * p);
     }
     // inclusive scan of the maps over the block
     Fn incl = f;
@@ -376,23 +539,23 @@ __global__ __launch_bounds__(256) void dec_resolve_kernel(const uint16_t* __rest
     }
     if (lane == 63) s_fn[wv] = incl;
     __syncthreads();
-    Fn pre = fn_identity();
-    for (int k = 0; k < wv; ++k) pre = compose(pre, s_fn[k]);
+    Fn pre = fn_identity(), total = fn_identity();
+    for (int k = 0; k < kResolve / kWave; ++k) {
+      if (k == wv) pre = total;
+      total = compose(total, s_fn[k]);
+    }
     const Fn up = shfl_up_fn(incl, 1);
     const Fn excl = lane == 0 ? pre : compose(pre, up);
-    Fn total = s_fn[0];
-    for (int k = 1; k < 4; ++k) total = compose(total, s_fn[k]);
-    __syncthreads();  // s_fn is rewritten by the next batch
-    if (c < nch) {
+    if (beg < n_words) {
       // true entry state of this chunk, then its records
-      int64_t pos = beg + ex_at(excl.ex, cp);
+      int pos = beg + ex_at(excl.ex, cp);
       uint64_t v0 = (uint64_t)sat_add(cv, sel3(excl.v, cp));
       uint32_t r = cr + sel3(excl.r, cp);
       while (pos < end) {
-        const uint32_t h = w[pos];
+        const uint32_t h = s_w[staged(pos)];
         const uint32_t n = h & kRunMax, v = h >> 14;
         const uint32_t len = record_words(h);
-        if (n == 0 || pos + len > L || v0 + n > (uint64_t)XY) {
+        if (n == 0 || w0 + pos + len > L || v0 + n > (uint64_t)XY) {
           bad = true;
           break;
         }
@@ -402,9 +565,8 @@ __global__ __launch_bounds__(256) void dec_resolve_kernel(const uint16_t* __rest
         else if (v == 2u)
           val = (uint32_t)(uint16_t)(int16_t)-kMaxT;
         else
-          val = (uint32_t)w[pos + 1] | ((uint32_t)w[pos + 2] << 16);
-        rs[r] = (uint32_t)v0;
-        rv[r] = val;
+          val = (uint32_t)s_w[staged(pos + 1)] | ((uint32_t)s_w[staged(pos + 2)] << 16);
+        rs[r] = make_uint2((uint32_t)v0, val);
         for (uint64_t t = (v0 + kFillTile - 1) / kFillTile; t * kFillTile < v0 + n; ++t)
           tf[t] = r;
         v0 += n;
@@ -416,6 +578,7 @@ __global__ __launch_bounds__(256) void dec_resolve_kernel(const uint16_t* __rest
     cv = sat_add(cv, sel3(total.v, cp));
     cr += sel3(total.r, cp);
     cp = np;
+    __syncthreads();  // s_w and s_fn are rewritten by the next round
   }
   if (bad) atomicOr(err, 2u);
   if (tid == 0) {
@@ -425,64 +588,59 @@ __global__ __launch_bounds__(256) void dec_resolve_kernel(const uint16_t* __rest
 }
 
 __global__ __launch_bounds__(256) void dec_fill_kernel(const SliceInfo* info, int64_t XY, int tps,
-                                                       const uint32_t* rec_start,
-                                                       const uint32_t* rec_val,
+                                                       const uint2* __restrict__ rec,
                                                        const uint32_t* tile_first,
-                                                       const uint32_t* err, uint32_t* out,
-                                                       int vec) {
-  // staged runs: start - vb clamped to [0, kFillTile] (16 bits, so six
-  // workgroups fit a CU's LDS; for every voxel q >= vb of the tile,
-  // start <= q exactly when the clamped value <= q - vb), and voxel value
-  __shared__ uint16_t s_start[kFillStage];
-  __shared__ uint32_t s_val[kFillStage];
-  static_assert(kFillTile <= 0xffff, "tile offsets in 16 bits");
+                                                       const uint32_t* err, uint32_t* out) {
+  // the tile's run values in order, a bit per voxel where a run starts, and
+  // the starts before each 32 voxels: a voxel's run is a rank, not a search
+  __shared__ uint32_t s_val[kFillTile + 1];
+  __shared__ uint32_t s_bit[kFillTile / 32];
+  __shared__ uint32_t s_pre[kFillTile / 32];
   if (*err) return;  // malformed input: the call reports it, outputs are undefined
   const int tid = threadIdx.x;
   const int j = blockIdx.y, t = blockIdx.x;
   const SliceInfo si = info[j];
-  const uint32_t r0 = tile_first[(int64_t)j * tps + t];
+  const uint32_t* tf = tile_first + (int64_t)j * tps + t;
+  const uint32_t r0 = tf[0];
   if (r0 == kNoRecord || r0 >= si.nrec) return;
-  const uint32_t* rs = rec_start + si.word_base;
-  const uint32_t* rv = rec_val + si.word_base;
+  // up to the run that covers the next tile's first voxel (it may start there)
+  const uint32_t r1 = t + 1 < tps ? min(tf[1], si.nrec - 1) : si.nrec - 1;
+  const int m = (int)min(r1 - r0, (uint32_t)kFillTile) + 1;
+  const uint2* rs = rec + si.word_base + r0;
   const int64_t vb = (int64_t)t * kFillTile;
   const int64_t ve = min(vb + kFillTile, XY);
-  int m = 0;
-  for (int round = 0; round * 256 < kFillTile + 1; ++round) {
-    const int64_t ri = (int64_t)r0 + round * 256 + tid;
-    bool in = false;
-    if (ri < si.nrec) {
-      const uint32_t s = rs[ri];
-      in = ri == r0 || (int64_t)s < ve;
-      if (in) {
-        s_start[round * 256 + tid] = (uint16_t)min(max((int64_t)s - vb, (int64_t)0), (int64_t)kFillTile);
-        s_val[round * 256 + tid] = rv[ri];
-      }
-    }
-    const int got = __syncthreads_count(in);
-    m += got;
-    if (got < 256) break;
+  if (tid < kFillTile / 32) s_bit[tid] = tid == 0 ? 1u : 0u;  // the first run
+  __syncthreads();
+  for (int i = tid; i < m; i += 256) {
+    const uint2 r = rs[i];
+    s_val[i] = r.y;
+    const uint32_t q = r.x - (uint32_t)vb;
+    if (i > 0 && q < (uint32_t)kFillTile) atomicOr(&s_bit[q >> 5], 1u << (q & 31));
   }
   __syncthreads();
+  if (tid < kWave) {
+    const uint32_t a = __popc(s_bit[2 * tid]), b = __popc(s_bit[2 * tid + 1]);
+    const uint32_t inc = wave_incl_scan32(a + b);
+    s_pre[2 * tid] = inc - a - b;
+    s_pre[2 * tid + 1] = inc - b;
+  }
+  static_assert(kFillTile / 32 == 2 * kWave, "two words of starts a lane");
+  __syncthreads();
   uint32_t* o = out + (int64_t)j * XY;
-  for (int64_t q = vb + 4 * tid; q < ve; q += 4 * 256) {
-    const int qr = (int)(q - vb);
-    int lo = 0, hi = m - 1;  // last staged record with start <= q
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if ((int)s_start[mid] <= qr)
-        lo = mid;
-      else
-        hi = mid - 1;
-    }
-    uint32_t v4[4];
-    int idx = lo;
+#pragma unroll
+  for (int k = 0; k < kFillTile / 1024; ++k) {
+    const int qr = k * 1024 + 4 * tid;
+    const int64_t q = vb + qr;
+    if (q >= ve) break;
+    const uint32_t bits = s_bit[qr >> 5], pre = s_pre[qr >> 5];
+    u32x4a4 v4;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      while (idx + 1 < m && (int)s_start[idx + 1] <= qr + e) ++idx;
-      v4[e] = s_val[idx];
+      const uint32_t upto = 0xffffffffu >> (31 - ((qr & 31) + e));
+      v4[e] = s_val[pre + __popc(bits & upto) - 1];
     }
-    if (vec && q + 3 < ve) {
-      *reinterpret_cast<uint4*>(o + q) = make_uint4(v4[0], v4[1], v4[2], v4[3]);
+    if (q + 3 < ve) {
+      *reinterpret_cast<u32x4a4*>(o + q) = v4;
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -499,13 +657,40 @@ unsigned grid_for(int64_t n, int64_t per) { return (unsigned)((n + per - 1) / pe
 using namespace mcx;
 
 // ------------------------------------------------------------------ C ABI
+namespace {
+// States of all levels of the scan over n blocks, the last level's single one
+// included.
+int64_t run_states(int64_t n) {
+  const int64_t ng = (n + kBlk - 1) / kBlk;
+  return n + (ng > 1 ? run_states(ng) : 1);
+}
+
+// a[i] becomes what is before it in its group of kBlk, the groups' prefixes
+// (from the slab's start) follow a; *all = the state of everything.
+int scan_runs(Runs* a, int64_t n, Runs** all, hipStream_t s) {
+  const int64_t ng = (n + kBlk - 1) / kBlk;
+  Runs* group = a + n;
+  hipLaunchKernelGGL(enc_scan_kernel, dim3((unsigned)ng), dim3(256), 0, s, a, n, group);
+  MCX_HIP(hipGetLastError());
+  if (ng == 1) {
+    *all = group;
+    return MCX_OK;
+  }
+  const int rc = scan_runs(group, ng, all, s);
+  if (rc) return rc;
+  if (ng > kBlk) {
+    hipLaunchKernelGGL(enc_lift_kernel, dim3((unsigned)((ng + 255) / 256)), dim3(256), 0, s,
+                       group, ng, group + ng);
+    MCX_HIP(hipGetLastError());
+  }
+  return MCX_OK;
+}
+}  // namespace
+
 extern "C" size_t mcx_rle_encode_workspace_size(int X, int Y, int nz) {
   if (X < 1 || Y < 1 || nz < 1) return 0;
-  const int64_t XY = (int64_t)X * Y, N = XY * nz;
-  const int64_t nblk = ((XY + kBlk - 1) / kBlk) * nz;
-  const int64_t tmp = std::max(scan_tmp_elems(nblk), scan_tmp_elems(N));
-  return al256((size_t)(nblk + 1) * 8) + al256((size_t)N * 8) + al256((size_t)(N + 1) * 8) +
-         al256((size_t)nz * 8) + al256((size_t)(tmp + 1) * 8) + 256;
+  const int64_t nblk = ((int64_t)X * Y + kEncBlk - 1) / kEncBlk * nz;
+  return al256((size_t)run_states(nblk) * sizeof(Runs)) + 256;
 }
 
 extern "C" size_t mcx_rle_encode_bound(int X, int Y, int nz) {
@@ -523,44 +708,28 @@ extern "C" int mcx_rle_encode(const void* d_vol, int X, int Y, int Z, int z0, in
   if (!d_ws || ws_bytes < mcx_rle_encode_workspace_size(X, Y, nz)) return MCX_ERR_WORKSPACE;
   hipStream_t s = as_stream(stream);
   const int64_t XY = (int64_t)X * Y, N = XY * nz;
-  const int64_t bps = (XY + kBlk - 1) / kBlk, nblk = bps * nz;
+  const int64_t bps = (XY + kEncBlk - 1) / kEncBlk, nblk = bps * nz;
   if (bps > 0x7fffffff || nz > 65535) return MCX_ERR_ARG;
   const uint32_t* vol = static_cast<const uint32_t*>(d_vol) + (int64_t)z0 * XY;
-  char* b = static_cast<char*>(d_ws);
-  int64_t* cnt = reinterpret_cast<int64_t*>(b);
-  b += al256((size_t)(nblk + 1) * 8);
-  uint64_t* cp = reinterpret_cast<uint64_t*>(b);
-  b += al256((size_t)N * 8);
-  int64_t* bytes = reinterpret_cast<int64_t*>(b);
-  b += al256((size_t)(N + 1) * 8);
-  int64_t* slice_first = reinterpret_cast<int64_t*>(b);
-  b += al256((size_t)nz * 8);
-  int64_t* tmp = reinterpret_cast<int64_t*>(b);
+  int64_t* totals = static_cast<int64_t*>(d_ws);
+  Runs* a = reinterpret_cast<Runs*>(static_cast<char*>(d_ws) + 256);
   const dim3 g2((unsigned)bps, (unsigned)nz);
-  hipLaunchKernelGGL(enc_count_kernel, g2, dim3(256), 0, s, vol, XY, cnt);
+  hipLaunchKernelGGL(enc_runs_kernel, g2, dim3(256), 0, s, vol, XY, a);
   MCX_HIP(hipGetLastError());
-  int rc = scan_excl(cnt, nblk, tmp, s);
+  Runs* all = nullptr;
+  const int rc = scan_runs(a, nblk, &all, s);
   if (rc) return rc;
-  int64_t M = 0;
-  MCX_HIP(hipMemcpyAsync(&M, cnt + nblk, sizeof(M), hipMemcpyDeviceToHost, s));
+  const Runs* group = nblk > kBlk ? a + nblk : nullptr;  // nothing is before a single one
+  hipLaunchKernelGGL(enc_write_kernel, g2, dim3(256), 0, s, vol, XY, N, a,
+                     group, all, static_cast<uint16_t*>(d_dump),
+                     (int64_t)dump_cap, totals, d_dump_bytes);
+  MCX_HIP(hipGetLastError());
+  int64_t h[2] = {0, 0};
+  MCX_HIP(hipMemcpyAsync(h, totals, sizeof(h), hipMemcpyDeviceToHost, s));
   MCX_HIP(hipStreamSynchronize(s));
-  if (M < nz || M > N) return MCX_ERR_INTERNAL;
-  // one thread per run below: the grid (in work-items) must fit 32 bits
-  if (M >= ((int64_t)1 << 31)) return MCX_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(enc_compact_kernel, g2, dim3(256), 0, s, vol, XY, cnt, cp, slice_first);
-  MCX_HIP(hipGetLastError());
-  hipLaunchKernelGGL(enc_size_kernel, dim3(grid_for(M, 256)), dim3(256), 0, s, vol, cp, M, N,
-                     bytes);
-  MCX_HIP(hipGetLastError());
-  rc = scan_excl(bytes, M, tmp, s);
-  if (rc) return rc;
-  hipLaunchKernelGGL(enc_write_kernel, dim3(grid_for(M, 256)), dim3(256), 0, s, vol, XY, cp, M, N,
-                     bytes, slice_first, nz, static_cast<uint16_t*>(d_dump), (int64_t)dump_cap,
-                     d_dump_bytes);
-  MCX_HIP(hipGetLastError());
-  int64_t total = 0;
-  MCX_HIP(hipMemcpyAsync(&total, bytes + M, sizeof(total), hipMemcpyDeviceToHost, s));
-  MCX_HIP(hipStreamSynchronize(s));
+  const int64_t total = h[0];
+  if (h[1] < nz || h[1] > N) return MCX_ERR_INTERNAL;
+  if (h[1] >= kMaxRuns) return MCX_ERR_UNSUPPORTED;
   if (h_dump_bytes) *h_dump_bytes = total;
   return total > (int64_t)dump_cap ? MCX_ERR_CAPACITY : MCX_OK;
 }
@@ -586,7 +755,6 @@ extern "C" int mcx_rle_decode(const void* d_dump, int64_t dump_bytes,
     return MCX_ERR_WORKSPACE;
   hipStream_t s = as_stream(stream);
   const int64_t tps = (XY + kFillTile - 1) / kFillTile;
-  const size_t words = (size_t)(dump_bytes / 2) + 1;
   char* b = static_cast<char*>(d_ws);
   uint32_t* err = reinterpret_cast<uint32_t*>(b);
   b += 256;
@@ -596,9 +764,7 @@ extern "C" int mcx_rle_decode(const void* d_dump, int64_t dump_bytes,
   b += al256((size_t)nz * 8);
   uint32_t* tile_first = reinterpret_cast<uint32_t*>(b);
   b += al256((size_t)nz * tps * 4);
-  uint32_t* rec_start = reinterpret_cast<uint32_t*>(b);
-  b += al256(words * 4);
-  uint32_t* rec_val = reinterpret_cast<uint32_t*>(b);
+  uint2* rec = reinterpret_cast<uint2*>(b);  // first voxel and value of each record
   MCX_HIP(hipMemcpyAsync(offs, h_slice_offsets, (size_t)nz * 8, hipMemcpyHostToDevice, s));
   int rc = fill_u32(err, 0u, 1, s);
   if (!rc) rc = fill_u32(tile_first, kNoRecord, (size_t)nz * tps, s);
@@ -607,13 +773,11 @@ extern "C" int mcx_rle_decode(const void* d_dump, int64_t dump_bytes,
   hipLaunchKernelGGL(dec_index_kernel, dim3(grid_for(nz, 256)), dim3(256), 0, s, d16, dump_bytes,
                      offs, nz, info, err);
   MCX_HIP(hipGetLastError());
-  hipLaunchKernelGGL(dec_resolve_kernel, dim3((unsigned)nz), dim3(256), 0, s, d16, XY, (int)tps,
-                     info, rec_start, rec_val, tile_first, err);
+  hipLaunchKernelGGL(dec_resolve_kernel, dim3((unsigned)nz), dim3(kResolve), 0, s, d16, XY,
+                     (int)tps, info, rec, tile_first, err);
   MCX_HIP(hipGetLastError());
-  const int vec = (XY % 4 == 0) && ((reinterpret_cast<uintptr_t>(d_vol) & 15) == 0);
   hipLaunchKernelGGL(dec_fill_kernel, dim3((unsigned)tps, (unsigned)nz), dim3(256), 0, s, info, XY,
-                     (int)tps, rec_start, rec_val, tile_first, err, static_cast<uint32_t*>(d_vol),
-                     vec);
+                     (int)tps, rec, tile_first, err, static_cast<uint32_t*>(d_vol));
   MCX_HIP(hipGetLastError());
   uint32_t herr = 0;
   MCX_HIP(hipMemcpyAsync(&herr, err, sizeof(herr), hipMemcpyDeviceToHost, s));

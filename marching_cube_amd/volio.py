@@ -30,7 +30,7 @@ from .mesh import CuVoxel, _ptr, _stream_handle
 
 VOLUME_FORMAT = b"VOLUME_TSDF_RGB\x00"
 HEADER = struct.Struct("<16s3i3f")
-ENCODE_SLAB_VOXELS = 1 << 24  # voxels per encode call (16 bytes of workspace each)
+ENCODE_SLAB_VOXELS = 1 << 24  # voxels per encode call (up to 6 bytes of dump each)
 
 
 def _lib():

@@ -60,3 +60,21 @@ def test_many_blocks(dev, X, nz):
                                    mesh._stream_handle(dev)), "mcx_rle_encode")
     assert total.value == out.numel()
     assert out.cpu().numpy().tobytes() == one.tobytes() * nz
+
+
+@pytest.mark.parametrize("n", [volio.STAGE_BYTES + d for d in (-1, 0, 1)] +
+                         [3 * volio.STAGE_BYTES - 1, 3 * volio.STAGE_BYTES + 5])
+def test_staged_copies(dev, n):
+    print(f"[case] staged copies of {n} bytes", flush=True)
+    data = np.random.default_rng(n).integers(0, 256, n, dtype=np.uint8).tobytes()
+    d = volio._to_device(data, dev)
+    assert d.cpu().numpy().tobytes() == data
+    assert volio._to_bytes(d) == data
+
+
+def test_slabs_when_the_dump_is_large(dev):
+    """All slices at once would need more than the slab's buffer."""
+    print("[case] rle slabs", flush=True)
+    v = np.arange(9 * 70 * 80, dtype=np.uint32).reshape(9, 70, 80) % 1000 | np.uint32(7 << 16)
+    for slices in (1, 2, 4, 9):
+        assert volio.encode(dev_vol(v, dev), slab_voxels=slices * 5600) == O.rle_encode_dump(v)

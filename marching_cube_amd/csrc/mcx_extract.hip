@@ -1653,21 +1653,34 @@ __global__ __launch_bounds__(kEmitThreads) void contrib_kernel(ExtractParams P, 
 
 // Backward BW2: dL/dv of every voxel = the sum, over the up to 8 cubes it
 // is corner k of (k = 0..7 in corner order), of the cube's contribution k.
-// A workgroup takes kGatherSpan consecutive voxels of one plane z.  The
-// cubes they are corners of lie in planes z - 1 and z and, per plane, in two
-// in-plane windows (rows y and y - 1: cube ids [q0 - 1, q0 + span) and the
-// same minus X), each within 4 consecutive tiles: the workgroup stages those
-// tiles' active-cube mask words, the popcount prefix of each word and the
-// tiles' first records in LDS, so a voxel's lookups read LDS and only active
-// cubes read their contribution (record index = tile's first record + rank
-// of the cube's bit).  A wave takes 64 consecutive voxels at a time: each
-// lane finds which of its (at most 8) cubes are active (the cube (x - dx,
-// y - dy) has in-plane index q - dx - dy X), the wave packs the active
-// (voxel, corner) pairs onto consecutive lanes (about 1.6 % of the cubes are
-// active, so one round of 64 lanes usually takes them all) to rank them and
-// read their contributions, and each voxel lane then adds its values in
+// A wave takes kGatherSpan consecutive voxels of one plane z.  The cubes they
+// are corners of lie in planes z - 1 and z and, per plane, in two in-plane
+// windows (rows y and y - 1: cube ids [q0 - 1, q0 + span) and the same minus
+// X), each within two consecutive tiles: 4 windows x 16 words of active-cube
+// masks, a word a lane, with its rank in its tile and the tile's first record.
+// No LDS and no barrier.  If no cube is active (most spans), the span is
+// zeroed.  Else the wave goes through it by 64 voxels: the cubes that have
+// them as corner k are 64 consecutive cube ids, so which of them are active is
+// one wave-uniform 64-bit mask, shifted out of two of the words (a voxel on
+// the volume's border meets ids of the row before, whose last cube is never
+// active).  A lane's record is the first one's index plus its rank in the mask
+// (a window meets at most one tile boundary, past which the records start
+// anew); only lanes with an active cube read, and each adds its values in
 // corner order, the order of the per-corner sum, so the bits are the same.
-constexpr int kGatherSpan = 1024;  // voxels per workgroup (4 per thread)
+// Bound by the scalar work for each read of few lanes (2.6 on average at 256^3)
+// and by the output (13 and 44 us of the times that follow): 256^3
+// (bumps) 62 us, a batch of 64 volumes of 64-192 a side 166 us; with a workgroup
+// for 1024 voxels, their masks in LDS behind barriers and the active (voxel,
+// corner) pairs of a wave packed through LDS, 67 and 232.
+constexpr int kGatherSpan = 512;  // voxels per wave, four waves a workgroup
+constexpr int kGatherAhead = 4;   // ... 64 at a time, whose reads are in flight together
+
+__device__ __forceinline__ uint64_t readlane64(uint64_t v, int lane) {
+  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)v, lane);
+  const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(v >> 32), lane);
+  return (uint64_t)hi << 32 | lo;
+}
+
 // Batched launches: workgroup blk belongs to the volume whose gather range
 // [gblk_begin, next) holds it, and writes that volume's part of the
 // concatenated gradient (from vox_begin).  With maxg, the largest |dL/dv| of
@@ -1675,154 +1688,135 @@ constexpr int kGatherSpan = 1024;  // voxels per workgroup (4 per thread)
 template <bool BATCH>
 __global__ __launch_bounds__(256) void gather_kernel(ExtractParams P, const float* contrib,
                                                      float* gvol, uint32_t* maxg) {
-  __shared__ uint64_t s_mask[2][2][4][kCPW];  // [dz][dy][tile slot][word]
-  __shared__ uint32_t s_pre[2][2][4][kCPW];   // set bits of the tile's earlier words
-  __shared__ int64_t s_rec[2][2][4];          // first record of the tile
-  __shared__ uint32_t s_max[4];
-  __shared__ uint16_t s_pair[4][64 * 8];  // per wave: lane << 3 | corner of each active pair
-  __shared__ float s_val[4][64 * 8];      // the pair's contribution
   int vi = 0;
   const int64_t gblk = P.first_block + blockIdx.x;
-  uint32_t blk = (uint32_t)gblk;  // single volumes: below 2^31
+  int64_t blk = gblk;
   if constexpr (BATCH) {
     vi = batch_volume_of<&BatchVol::gblk_begin>(P.bvol, P.nvol, gblk);
-    blk = (uint32_t)(gblk - P.bvol[vi].gblk_begin);
+    blk = gblk - P.bvol[vi].gblk_begin;
     gvol += P.bvol[vi].vox_begin;
   }
   const VolDesc& V = vol_at<BATCH>(P, vi);
   const int X = V.X, Y = V.Y, Z = V.Z;
   const uint32_t XY = (uint32_t)X * (uint32_t)Y;  // < 2^30 (plane_ok)
   const uint32_t per_plane = (XY + kGatherSpan - 1) / kGatherSpan;
-  const int z = (int)(blk / per_plane);
-  const uint32_t q0 = (blk - (uint32_t)z * per_plane) * kGatherSpan;
-  const int tid = threadIdx.x;
-  // first tile of each window (cube ids below 0 are never looked up)
-  int base[2];
-#pragma unroll
-  for (int dy = 0; dy < 2; ++dy) {
-    const int64_t lo = (int64_t)q0 - 1 - (dy ? X : 0);
-    base[dy] = (int)(max(lo, (int64_t)0) >> 9);
+  const int lane = threadIdx.x & 63;
+  // units: at most N / 512 + Z, below 2^31 for any volume that fits in memory
+  const uint32_t unit =
+      (uint32_t)blk * 4 + (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int z = (int)(unit / per_plane);
+  if (z >= Z) return;
+  const int q0 = (int)(unit - (uint32_t)z * per_plane) * kGatherSpan;
+  // lane 16 d + 8 slot + word, d = 2 dz + dy (cube ids below 0 are never
+  // looked up)
+  const int first[2] = {max(q0 - 1, 0) >> 9, max(q0 - 1 - X, 0) >> 9};  // tiles
+  uint64_t word = 0;
+  int64_t rec = 0;
+  {
+    const int d = lane >> 4, cz = z - (d >> 1);
+    const int r = ((d & 1) ? first[1] : first[0]) + ((lane >> 3) & 1);
+    if (cz >= 0 && cz <= Z - 2 && r < V.R) {
+      const int64_t t = V.tile_begin + (int64_t)cz * V.R + r;
+      word = P.masks[t * kCPW + (lane & 7)];
+      rec = P.tile_rec[t];
+    }
   }
-  uint64_t m = 0;  // the staged mask word of threads 0..127
-  if (tid < 128) {
-    const int dz = tid >> 6, dy = (tid >> 5) & 1, slot = (tid >> 3) & 3, word = tid & 7;
-    const int cz = z - dz, r = base[dy] + slot;
-    if (cz >= 0 && cz <= Z - 2 && r < V.R)
-      m = P.masks[(V.tile_begin + (int64_t)cz * V.R + r) * kCPW + word];
-    s_mask[dz][dy][slot][word] = m;
-  } else if (tid < 128 + 16) {
-    const int e = tid - 128, dz = e >> 3, dy = (e >> 2) & 1, slot = e & 3;
-    const int cz = z - dz, r = base[dy] + slot;
-    int64_t rs = 0;
-    if (cz >= 0 && cz <= Z - 2 && r < V.R) rs = P.tile_rec[V.tile_begin + (int64_t)cz * V.R + r];
-    s_rec[dz][dy][slot] = rs;
-  }
-  if (!__syncthreads_or(m != 0)) {
+  float* const gz = gvol + (int64_t)z * XY;
+  if (!__any(word != 0)) {
     // no active cube has a corner in the span: its gradient is zero (the
     // sums below would all be empty), and it raises no maximum
-    float* const gz0 = gvol + (int64_t)z * XY;
 #pragma unroll
-    for (int j = 0; j < kGatherSpan / 256; ++j) {
-      const uint32_t q = q0 + (uint32_t)(j * 256 + tid);
-      if (q < XY) gz0[q] = 0.0f;
+    for (int j = 0; j < kGatherSpan; j += 256) {
+      const uint32_t q = (uint32_t)(q0 + j + 4 * lane);
+      if (q + 4 <= XY) {
+        *reinterpret_cast<u32x4a4*>(gz + q) = u32x4a4{0, 0, 0, 0};
+      } else {
+        for (uint32_t e = q; e < XY; ++e) gz[e] = 0.0f;
+      }
     }
     return;
   }
-  if (tid < 16) {
-    const int dz = tid >> 3, dy = (tid >> 2) & 1, slot = tid & 3;
-    uint32_t pre = 0;
+  uint32_t pre = (uint32_t)__popcll(word);  // then the set bits of the tile's earlier words
+  {
+    const uint32_t own = pre;
 #pragma unroll
-    for (int w = 0; w < kCPW; ++w) {
-      s_pre[dz][dy][slot][w] = pre;
-      pre += (uint32_t)__popcll(s_mask[dz][dy][slot][w]);
+    for (int o = 1; o < 8; o <<= 1) {
+      const uint32_t up = __shfl_up(pre, o, 8);
+      if ((lane & 7) >= o) pre += up;
     }
+    pre -= own;
   }
-  __syncthreads();
-  float* const gz = gvol + (int64_t)z * XY;
   uint32_t gmax = 0;  // largest |g| bits of this thread
-  const int lane = tid & 63, wv = tid >> 6;
-  uint16_t* const pairs = s_pair[wv];
-  float* const vals = s_val[wv];
-#pragma unroll 1
-  for (int j = 0; j < kGatherSpan / 256; ++j) {
-    // which of the (at most 8) cubes having this voxel as a corner are active
-    const uint32_t qb = q0 + (uint32_t)(j * 256 + wv * 64);
-    const uint32_t q = qb + (uint32_t)lane;
-    const bool inq = q < XY;
-    uint32_t act = 0;
-    if (inq) {
-      const uint32_t y = V.divX.div(q);
-      const int x = (int)(q - y * (uint32_t)X);
-      // cube (x - dx, y - dy) has in-plane index q - dx - dy X
-      const bool okx[2] = {x <= X - 2, x >= 1}, oky[2] = {(int)y <= Y - 2, y >= 1};
-      const bool okz[2] = {z <= Z - 2, z >= 1};
+  // Window d of the first 64 voxels: its first cube id (dx = 1), the lane of
+  // that id's word, the shift into it; 64 voxels on, the next lane and the same
+  // shift.  words: the lanes that the 64 voxels' windows read (all, where a
+  // window begins before the plane).
+  const uint64_t active = __ballot(word != 0);
+  int s0[4], lane0[4];
+  uint64_t words = 0;
 #pragma unroll
-      for (int dy = 0; dy < 2; ++dy) {
+  for (int d = 0; d < 4; ++d) {
+    s0[d] = q0 - 1 - ((d & 1) ? X : 0);
+    lane0[d] = 16 * d + (s0[d] >> 6) - 8 * first[d & 1];
+    words |= s0[d] >= 0 ? 3ull << lane0[d] : ~0ull;
+  }
+#pragma unroll 1
+  for (int c0 = 0; c0 < kGatherSpan / 64; c0 += kGatherAhead) {
+    float val[kGatherAhead][8] = {};
+#pragma unroll
+    for (int u = 0; u < kGatherAhead; ++u) {
+      const int c = c0 + u;
+      if ((active & (s0[1] >= 0 ? words << c : words)) == 0) continue;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        // cube ids s + lane (dx = 1) and s + 1 + lane (dx = 0): two words
+        const int s = s0[d] + 64 * c, sh = s & 63;
+        const int l0 = lane0[d] + c, l1 = l0 + 1;
+        const uint64_t m0 = s >= 0 ? readlane64(word, l0) : 0;
+        const uint64_t m1 = s >= -64 ? readlane64(word, l1) : 0;
+        const uint64_t with = sh ? m0 >> sh | m1 << (64 - sh) : m0;
+        const uint64_t past = with >> 1 | (m1 >> sh & 1ull) << 63;
+        if ((with | past) == 0) continue;
+        // the record of the window's first cube, in the first word's tile and,
+        // where the second word begins a tile, in that
+        const bool two = (l1 & 7) == 0;
+        const int64_t i0 = s >= 0 ? (int64_t)readlane64((uint64_t)rec, l0) +
+                                        (uint32_t)__builtin_amdgcn_readlane(pre, l0) +
+                                        __popcll(m0 & ((1ull << sh) - 1))
+                                  : 0;
+        const int64_t i1 = (int64_t)readlane64((uint64_t)rec, l1) - __popcll(m0 >> sh);
 #pragma unroll
         for (int dx = 0; dx < 2; ++dx) {
-          if (!(okx[dx] && oky[dy])) continue;
-          const uint32_t p = q - (uint32_t)dx - (dy ? (uint32_t)X : 0u);
-          const int slot = (int)(p >> 9) - base[dy];
-          const uint32_t word = (p >> 6) & 7u, bit = p & 63u;
-          const int c = dy ? (dx ? 2 : 3) : dx;  // corner index in the plane
-#pragma unroll
-          for (int dz = 0; dz < 2; ++dz)
-            if (okz[dz]) act |= (uint32_t)((s_mask[dz][dy][slot][word] >> bit) & 1ull) << (4 * dz + c);
+          const uint64_t act = dx ? with : past;
+          const int k = 4 * (d >> 1) + ((d & 1) ? (dx ? 2 : 3) : dx);
+          const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+              (uint32_t)(act >> 32),
+              __builtin_amdgcn_mbcnt_lo((uint32_t)act, dx ? 0u : (uint32_t)(with & 1ull)));
+          const float* at = contrib + i0 * 8 + k;
+          if (two && lane >= 64 - sh - (1 - dx)) at = contrib + i1 * 8 + k;
+          if (__builtin_amdgcn_inverse_ballot_w64(act)) val[u][k] = at[rank * 8];
         }
       }
     }
-    // the wave's active (voxel, corner) pairs, packed in corner order per voxel
-    const uint32_t cnt = (uint32_t)__popc(act);
-    const uint32_t incl = wave_incl_scan32(cnt);
-    const uint32_t excl = incl - cnt;
-    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(incl, 63);
-    {
-      uint32_t a = act, e = excl;
-      while (a) {
-        const int k = __builtin_ctz(a);
-        a &= a - 1u;
-        pairs[e++] = (uint16_t)((lane << 3) | k);
+#pragma unroll
+    for (int u = 0; u < kGatherAhead; ++u) {
+      const uint32_t q = (uint32_t)(q0 + 64 * (c0 + u) + lane);
+      if (q < XY) {
+        float g = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) g += val[u][k];  // + 0 where inactive: g is never -0
+        gz[q] = g;
+        gmax = max(gmax, __float_as_uint(g) & 0x7fffffffu);
       }
     }
-    wave_sync();
-    for (uint32_t pr = (uint32_t)lane; pr < total; pr += 64) {
-      const uint32_t d = pairs[pr];
-      const int k = (int)(d & 7u);
-      const uint32_t ql = qb + (d >> 3);
-      const int dx = corner_dx(k), dy = corner_dy(k), dz = corner_dz(k);
-      const uint32_t p = ql - (uint32_t)dx - (dy ? (uint32_t)X : 0u);
-      const int slot = (int)(p >> 9) - base[dy];
-      const int word = (int)((p >> 6) & 7u), bit = (int)(p & 63u);
-      const uint64_t m = s_mask[dz][dy][slot][word];
-      const uint32_t rank = s_pre[dz][dy][slot][word] + (uint32_t)__popcll(m & ((1ull << bit) - 1ull));
-      vals[pr] = contrib[(s_rec[dz][dy][slot] + rank) * 8 + k];
-    }
-    wave_sync();
-    if (inq) {
-      // the voxel's sum in corner order, as the per-corner loop adds it
-      float g = 0.0f;
-      uint32_t a = act, e = excl;
-      while (a) {
-        a &= a - 1u;
-        g += vals[e++];
-      }
-      gz[q] = g;
-      gmax = max(gmax, __float_as_uint(g) & 0x7fffffffu);
-    }
-    wave_sync();
   }
   if (maxg) {
-    // one atomic per workgroup, only where it can raise the maximum (the
-    // plain read is a filter: a stale value only lets an atomic through)
+    // one atomic per wave, only where it can raise the maximum (the plain
+    // read is a filter: a stale value only lets an atomic through)
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) gmax = max(gmax, (uint32_t)__shfl_xor((int)gmax, o));
-    if ((tid & 63) == 0) s_max[tid >> 6] = gmax;
-    __syncthreads();
-    if (tid == 0) {
-      const uint32_t m = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
-      if (m > __hip_atomic_load(maxg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMax(maxg, m);
-    }
+    if (lane == 0 && gmax > __hip_atomic_load(maxg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(maxg, gmax);
   }
 }
 
@@ -1866,6 +1860,10 @@ int launch_contrib(ExtractParams P, int64_t nb, const float* gpos, float* contri
     MCX_HIP(hipGetLastError());
   }
   return MCX_OK;
+}
+
+int64_t gather_blocks(int X, int Y, int Z) {
+  return (((int64_t)X * Y + kGatherSpan - 1) / kGatherSpan * Z + 3) / 4;
 }
 
 template <bool BATCH>
@@ -2318,7 +2316,7 @@ int backward_impl(const float* d_vol, int X, int Y, int Z, float h, const float*
   const int64_t g1 = (n_tiles + kTilesPerContribGroup - 1) / kTilesPerContribGroup;
   rc = launch_contrib<false>(P, g1, d_grad_pos, contrib, s);
   if (rc) return rc;
-  const int64_t g2 = ((int64_t)X * Y + kGatherSpan - 1) / kGatherSpan * Z;
+  const int64_t g2 = gather_blocks(X, Y, Z);
   if (g2 >= ((int64_t)1 << 31)) return MCX_ERR_UNSUPPORTED;
   return launch_gather<false>(P, g2, contrib, d_grad_vol, nullptr, s);
 }
@@ -2373,7 +2371,7 @@ extern "C" int mcx_batch_create(mcx_batch** out, int nvol, const int* dims_xyz, 
     blk_begin[b] = blocks;
     voxels += nv;
     blocks += (int64_t)rx * ry * rz;
-    gblocks += ((int64_t)X * Y + kGatherSpan - 1) / kGatherSpan * Z;
+    gblocks += gather_blocks(X, Y, Z);
     const int64_t nt = tiles_of(X, Y, Z);
     if (nt > 0) {
       // one column per in-plane range, slabs of the plan's planes per column

@@ -2,7 +2,8 @@
 planes that end at, just past and just before a tile of 512 voxels, widths that
 are no multiple of a lane's four voxels, rows longer than a tile, the smallest
 volumes; signed zeros, denormals, infinities and NaN (only f < 0 is inside);
-with the active-cube masks that the backward reads, and batched."""
+with the active-cube masks that the backward's gather reads in runs of 512 voxels,
+and batched."""
 import numpy as np
 import pytest
 import torch

@@ -177,8 +177,8 @@ extern "C" int mcx_chamfer_batched(const float* d_pos, const int64_t* d_vbase, i
   if (!d_ws || ws_bytes < mcx_chamfer_workspace_size(cap)) return MCX_ERR_WORKSPACE;
   hipStream_t s = as_stream(stream);
   float* vloss = static_cast<float*>(d_ws);
+  if (cap > kMaxLaunchBlocks * 256) return MCX_ERR_UNSUPPORTED;
   const int64_t blocks = (cap + 256 * kRows - 1) / (256 * kRows);
-  if (blocks > kMaxLaunchBlocks) return MCX_ERR_UNSUPPORTED;  // grid in work-items: 32 bits
   hipLaunchKernelGGL(chamfer_vertex_kernel, dim3((unsigned)blocks), dim3(256), 0, s, d_pos,
                      d_vbase, nvol, d_targets, M, cap, d_grad_pos, vloss);
   MCX_HIP(hipGetLastError());

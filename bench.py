@@ -63,10 +63,6 @@ def parse():
     return ap.parse_args()
 
 
-def nvox_int(dim):
-    return dim * dim * dim
-
-
 def host_threads(requested=0):
     """Threads for the all-cores CPU baseline: `requested`, or every core this
     process may run on (its affinity set), capped by OMP_NUM_THREADS."""
@@ -647,8 +643,13 @@ def main():
     torch.cuda.synchronize()
     per_frame_ms = e0.elapsed_time(e1) / args.frames
     assert torch.equal(vox1.data, vox.data)  # same updates in the same order
+    # a voxel moves only where the frame updates it: with a cap that no voxel
+    # reaches, the weights count the updates
+    vox1 = fusion.voxel_new((dim, dim, dim), cfg["trunc"], h, device=dev)
+    fusion.integrate(vox1, intr, poses, depth, trunc=cfg["trunc"], max_w=args.frames)
+    updates = int(((vox1.data >> 16) & 0xffff).sum(dtype=torch.int64))
     del vox1, depth
-    frame_bytes = 8 * nvox_int(dim) + 2 * cfg["W"] * cfg["H"]
+    frame_bytes = 8 * updates // args.frames + 2 * cfg["W"] * cfg["H"]
     per_frame = {"workload": f"kinfu{dim}_integrate_per_frame", "frames": args.frames,
                  "ms_per_frame": round(per_frame_ms, 4),
                  "algorithmic_bytes_per_frame": frame_bytes,
@@ -658,7 +659,7 @@ def main():
                               "frac": round(frame_bytes / (per_frame_ms * 1e-3) / 1e9
                                             / HBM_PEAK_GBS, 4)},
                  "note": "one mcx_integrate call per frame; a voxel is read and written only "
-                         "where the frame updates it"}
+                         "where the frame updates it (bytes: the updates, counted)"}
     print(f"[bench] integrate per frame {per_frame}", file=sys.stderr, flush=True)
     vols = [vox.data, vox.data.clone()]
     print(f"[bench] volume {dim}^3 fused from {args.frames} frames in {integrate_ms:.1f} ms "

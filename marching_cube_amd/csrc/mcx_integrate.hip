@@ -7,12 +7,12 @@
 //   _cu_voxel_volumetric_integration       :534-549
 // The reference gives each thread one (y, z) row and walks x inside the
 // thread, so a wave strides the volume by 4*X bytes (uncoalesced), and it
-// sweeps the whole volume once per frame.  Here a wave owns a brick of
-// 8 x 8 x 4 voxels (a lane one x, y and four z) and a workgroup four bricks in
-// a row of x (32 consecutive voxels: whole 128-byte lines), and K frames are
-// fused per sweep: the voxel is read once, updated for every frame in order
-// in registers, and written once, so a sweep costs 8 B/voxel plus the depth
-// reads instead of 8 B/voxel/frame.
+// sweeps the whole volume once per frame.  Here a wave, a workgroup of its
+// own, owns bricks of 8 x 8 x 4 voxels (a lane one x, y and four z), four
+// neighbouring waves a row of x (32 consecutive voxels: whole 128-byte
+// lines), and K frames are fused per sweep: the voxel is read once, updated
+// for every frame in order in registers, and written once, so a sweep costs
+// 8 B/voxel plus the depth reads instead of 8 B/voxel/frame.
 //
 // Per voxel and frame (bit-for-bit the oracle's update_voxel):
 //   p = ((i + 0.5) h) per axis; q = R^T (p - t)          (camera-to-world pose)
@@ -24,9 +24,9 @@
 //   and max_t of the volume; one truncation gives clamp(sdf / trunc, -1, 1));
 //   running average with integer weights capped at max_w; tsdf stored as
 //   trunc(t * 32767) clamped to +-32767.
-// A wave first tests eight frames at a time against its brick (test_box) and
-// passes over those that none of its voxels can observe: out of the frame's
-// view, or behind everything the frame measured there.  The per-voxel
+// A wave first tests 64 (brick, frame) pairs at a time, one a lane
+// (test_brick), and passes over those that no voxel can observe: out of the
+// frame's view, or behind everything the frame measured there.  The per-voxel
 // arithmetic and its results are those of every voxel taken by itself.
 #include <float.h>
 #include <hip/hip_runtime.h>

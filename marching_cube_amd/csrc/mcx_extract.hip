@@ -84,7 +84,6 @@ struct Tuning {
   int batch_slab = 64;
 };
 Tuning g_tuning;
-constexpr int kTilesPerContribGroup = 8;  // backward BW1: tiles per workgroup
 // third word of a gfx9 raw buffer resource (stride 0, 32-bit data format)
 constexpr int kBufferWord3 = 0x00020000;
 
@@ -1148,36 +1147,6 @@ __global__ __launch_bounds__(256) void vbase_kernel(ExtractParams P) {
 }
 
 // ============================================================ K3: emit
-// Exclusive scan of one int per thread over a 256-thread workgroup; returns
-// the thread's exclusive prefix and the total through *tot (s_tmp: 4 ints).
-__device__ __forceinline__ int block_excl_scan(int v, int* s_tmp, int* tot) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint32_t incl = wave_incl_scan32((uint32_t)v);
-  if (lane == 63) s_tmp[wave] = (int)incl;
-  __syncthreads();
-  int pre = 0, all = 0;
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    if (w < wave) pre += s_tmp[w];
-    all += s_tmp[w];
-  }
-  __syncthreads();
-  *tot = all;
-  return (int)incl - v + pre;
-}
-
-struct TileInfo {      // backward BW1 per-tile info in LDS (10 words)
-  int64_t delta;       // output index of the tile's first record vertex minus
-                       // the item-list vertex prefix at that record
-  int64_t rstart;      // first record in scratch
-  int64_t t;           // tile id
-  int32_t nrec;        // records (-1: staged path)
-  int32_t T;           // vertices
-  int32_t lbeg;        // first position in the item's record list
-  int32_t vi;          // volume
-};
-static_assert(sizeof(TileInfo) == 40, "tile info is 10 words");
-
 // Per-wave LDS area of the emit kernel (32-bit words): 64 records (cube
 // offset << 8 | case, 8 corners), the vertex -> record map (u8, at most 15
 // vertices a record), the first vertex of each record, and per record its
@@ -1425,6 +1394,85 @@ __device__ __forceinline__ void emit_staged_tile(const ExtractParams& P, const u
   }
 }
 
+// Unit k: the records 64 k .. 64 k + R - 1 of the list's tiles, in list order
+// (R, at most 64, is returned); lane l < R gets record l, its index in the
+// scratch, the output index of its first vertex, its cube's in-plane index and
+// plane and its volume.  mark: 64 bytes of the wave's, zero before and after.
+template <bool BATCH>
+__device__ __forceinline__ int load_unit(const ExtractParams& P, int64_t k, uint32_t nl,
+                                         int64_t total, uint8_t* mark, const uint8_t* s_nv,
+                                         uint32_t (&rec)[kRecWords], int64_t* ri, int64_t* out,
+                                         uint32_t* p, uint32_t* zk, uint32_t* vik) {
+  const int lane = threadIdx.x & 63;
+  const int64_t g0 = k << 6;
+  const int R = (int)min((int64_t)64, total - g0);
+  // lane l: clist entry units[k] + l, its records [pre, pre + nrec)
+  const uint32_t i = P.units[k] + (uint32_t)lane;
+  const uint32_t ic = min(i, nl);
+  const int64_t pre = P.lpre[ic];
+  const int64_t nrec = i < nl ? P.lpre[ic + 1] - pre : 0;
+  const uint32_t t = i < nl ? P.clist[i] : 0u;
+  const int64_t trec = i < nl ? P.lrs[i] : 0;  // the tile's first record
+  const uint32_t vi = BATCH && i < nl ? P.clist_vol[i] : 0u;
+  const bool inu = nrec > 0 && pre < g0 + R;  // the entry has records in the unit
+  const int first = (int)max(pre - g0, (int64_t)0);  // its first record in the unit
+  int64_t rs = 0, off = 0;
+  uint32_t p0 = 0, z = 0;
+  if (inu) {
+    rs = trec + (g0 + first - pre);  // the record of unit position `first`
+    off = P.voff[t];
+    const VolDesc& Vl = vol_at<BATCH>(P, (int)vi);
+    const uint32_t local = (uint32_t)(t - Vl.tile_begin);
+    z = Vl.divR.div(local);
+    p0 = (local - z * (uint32_t)Vl.R) * (uint32_t)kTile;
+    mark[first] = (uint8_t)(lane + 1);
+  }
+  // records of the first entry's tile before the unit: their vertices
+  const int64_t head = g0 - __shfl(pre, 0);
+  const int64_t rs0 = __shfl(rs, 0) - head;  // the tile's first record
+  wave_sync();
+  uint32_t mk = 0;
+  if (lane < R) {
+    mk = mark[lane];
+    mark[lane] = 0;
+  }
+  const int kk = lane < R ? (int)wave_incl_max32(mk) - 1 : 0;
+  const int fr = __shfl(first, kk);
+  const int64_t rsk = __shfl(rs, kk);
+  if (lane < R) {
+    const uint32_t* src = P.rec + (rsk + (lane - fr)) * kRecWords;
+#pragma unroll
+    for (int q = 0; q < kRecWords; ++q) rec[q] = src[q];
+  } else {
+#pragma unroll
+    for (int q = 0; q < kRecWords; ++q) rec[q] = 0;
+  }
+  // a tile has at most kTile records: head < 512, eight loads per lane
+  uint32_t hv = 0;
+  if (head > 0) {
+    uint32_t hw[kTile / 64];
+#pragma unroll
+    for (int q = 0; q < kTile / 64; ++q) {
+      const int64_t j = lane + 64 * q;
+      hw[q] = j < head ? P.rec[(rs0 + j) * kRecWords] : 0u;
+    }
+#pragma unroll
+    for (int q = 0; q < kTile / 64; ++q) hv += lane + 64 * q < head ? s_nv[hw[q] & 0xffu] : 0u;
+    hv = wave_sum32(hv);
+  }
+  const uint32_t nv = lane < R ? s_nv[rec[0] & 0xffu] : 0u;
+  const uint32_t vincl = wave_incl_scan32(nv);
+  const uint32_t vex = vincl - nv;
+  const uint32_t vfirst = (uint32_t)__shfl((int)vex, fr);
+  const int64_t offk = __shfl(off, kk) + (kk == 0 ? (int64_t)hv : 0);
+  *out = offk + (int64_t)(vex - vfirst);
+  *ri = rsk + (lane - fr);
+  *p = (uint32_t)__shfl((int)p0, kk) + (rec[0] >> 8);
+  *zk = (uint32_t)__shfl((int)z, kk);
+  *vik = BATCH ? (uint32_t)__shfl((int)vi, kk) : 0u;
+  return R;
+}
+
 // Single volumes, balanced by records: the records of the list's tiles, in
 // list order, are cut into units of 64 (the scan's clist / lpre / units
 // tables) and wave w takes units w, w + nwaves, ..., then the staged-path
@@ -1474,82 +1522,19 @@ void emit_units_kernel(ExtractParams P) {
       emit_staged_tile<ELEM, BATCH>(P, s_slot, s_nv, s_w, P.dense_list[k - n_units]);
       continue;
     }
-    const int64_t g0 = k << 6;
-    const int R = (int)min((int64_t)64, total - g0);
-    // lane l: clist entry units[k] + l, its records [pre, pre + nrec)
-    const uint32_t i = P.units[k] + (uint32_t)lane;
-    const uint32_t ic = min(i, nl);
-    const int64_t pre = P.lpre[ic];
-    const int64_t nrec = i < nl ? P.lpre[ic + 1] - pre : 0;
-    const uint32_t t = i < nl ? P.clist[i] : 0u;
-    const int64_t trec = i < nl ? P.lrs[i] : 0;  // the tile's first record
-    const uint32_t vi = BATCH && i < nl ? P.clist_vol[i] : 0u;
-    const bool inu = nrec > 0 && pre < g0 + R;  // the entry has records in the unit
-    const int first = (int)max(pre - g0, (int64_t)0);  // its first record in the unit
-    int64_t rs = 0, off = 0;
-    uint32_t p0 = 0, z = 0;
-    if (inu) {
-      rs = trec + (g0 + first - pre);  // the record of unit position `first`
-      off = P.voff[t];
-      const VolDesc& Vl = vol_at<BATCH>(P, (int)vi);
-      const uint32_t local = (uint32_t)(t - Vl.tile_begin);
-      z = Vl.divR.div(local);
-      p0 = (local - z * (uint32_t)Vl.R) * (uint32_t)kTile;
-      mark[first] = (uint8_t)(lane + 1);
-    }
-    // records of the first entry's tile before the unit: their vertices
-    const int64_t head = g0 - __shfl(pre, 0);
-    const int64_t rs0 = __shfl(rs, 0) - head;  // the tile's first record
-    wave_sync();
-    uint32_t mk = 0;
-    if (lane < R) {
-      mk = mark[lane];
-      mark[lane] = 0;
-    }
-    const int kk = lane < R ? (int)wave_incl_max32(mk) - 1 : 0;
-    const int fr = __shfl(first, kk);
-    const int64_t rsk = __shfl(rs, kk);
     uint32_t rec[kRecWords];
-    if (lane < R) {
-      const uint32_t* src = P.rec + (rsk + (lane - fr)) * kRecWords;
-#pragma unroll
-      for (int q = 0; q < kRecWords; ++q) rec[q] = src[q];
-    } else {
-#pragma unroll
-      for (int q = 0; q < kRecWords; ++q) rec[q] = 0;
-    }
-    // a tile has at most kTile records: head < 512, eight loads per lane
-    uint32_t hv = 0;
-    if (head > 0) {
-      uint32_t hw[kTile / 64];
-#pragma unroll
-      for (int q = 0; q < kTile / 64; ++q) {
-        const int64_t j = lane + 64 * q;
-        hw[q] = j < head ? P.rec[(rs0 + j) * kRecWords] : 0u;
-      }
-#pragma unroll
-      for (int q = 0; q < kTile / 64; ++q) hv += lane + 64 * q < head ? s_nv[hw[q] & 0xffu] : 0u;
-      hv = wave_sum32(hv);
-    }
-    const uint32_t nv = lane < R ? s_nv[rec[0] & 0xffu] : 0u;
-    const uint32_t vincl = wave_incl_scan32(nv);
-    const uint32_t vex = vincl - nv;
-    const uint32_t vfirst = (uint32_t)__shfl((int)vex, fr);
-    const int64_t offk = __shfl(off, kk) + (kk == 0 ? (int64_t)hv : 0);
-    const uint32_t p0k = (uint32_t)__shfl((int)p0, kk);
-    const uint32_t zk = (uint32_t)__shfl((int)z, kk);
-    const uint32_t vik = BATCH ? (uint32_t)__shfl((int)vi, kk) : 0u;
+    int64_t ri, o;
+    uint32_t p, zk, vik;
+    const int R = load_unit<BATCH>(P, k, nl, total, mark, s_nv, rec, &ri, &o, &p, &zk, &vik);
     GridDims dl{0, 0, 0, 0.0f, 0u};
     if (lane < R) {
 #pragma unroll
       for (int q = 0; q < kRecWords; ++q) s_w[lane * kRecWords + q] = rec[q];
-      const uint64_t o = (uint64_t)(offk + (int64_t)(vex - vfirst));
-      const uint32_t p = p0k + (rec[0] >> 8);
       const VolDesc& Vk = vol_at<BATCH>(P, (int)vik);
       const uint32_t y = Vk.divX.div(p);
       uint32_t* mt = s_meta + 4 * lane;
       mt[0] = (uint32_t)o;
-      mt[1] = meta_hi(o, zk);
+      mt[1] = meta_hi((uint64_t)o, zk);
       mt[2] = p - y * (uint32_t)Vk.X;
       mt[3] = y;
       if constexpr (BATCH) dl = GridDims{Vk.X, Vk.Y, Vk.Z, Vk.h, vik};
@@ -1567,106 +1552,71 @@ void emit_units_kernel(ExtractParams P) {
 // cube's vertices, in slot order, into 8 per-corner sums.  BW2: every voxel
 // sums the corner sums of the (at most 8) active cubes it is a corner of, in
 // corner order.  No atomics, so the result is bitwise reproducible.
+// Units of 64 records as in the emit kernel: a wave takes units w, w + nwaves,
+// ..., a lane a record, whose vertices are consecutive.  Bound by the chain of
+// dependent reads to a record and by its vertices' gradients: 256^3 (bumps)
+// 18 us, a batch of 64 volumes 18 us; with eight tiles a workgroup, their
+// records spread over 256 threads after six barriers (a fifth of the threads
+// had one), 25 and 61.
 template <bool BATCH>
 __global__ __launch_bounds__(kEmitThreads) void contrib_kernel(ExtractParams P, const float* gpos,
                                                                float* contrib) {
   __shared__ uint64_t s_case[256];
   __shared__ uint8_t s_nv[256];
-  __shared__ int s_tmp[8];
-  __shared__ TileInfo s_tile[kTilesPerContribGroup];
-  const int tid = threadIdx.x;
-  const int64_t t0 = (P.first_block + blockIdx.x) * kTilesPerContribGroup;
-  s_case[tid] = dCase[tid];
-  s_nv[tid] = dNumVerts[tid];
-  if (tid < kTilesPerContribGroup) {
-    const int64_t t = t0 + tid;
-    TileInfo ti{};
-    if (t < P.n_tiles) {
-      ti.T = P.tileT[t];
-      ti.nrec = P.tile_nrec[t];
-      ti.rstart = P.tile_rec[t];
-      ti.delta = P.voff[t];
-      ti.vi = BATCH ? volume_of_tile(P, t) : 0;
-    }
-    s_tile[tid] = ti;
-  }
+  __shared__ uint8_t s_mark[kEmitThreads / 64][64];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  s_case[threadIdx.x] = dCase[threadIdx.x];
+  s_nv[threadIdx.x] = dNumVerts[threadIdx.x];
+  s_mark[wv][lane] = 0;
   __syncthreads();
-  if (tid == 0) {
-    int lpos = 0;
-    int64_t vpre = 0;
-    for (int u = 0; u < kTilesPerContribGroup; ++u) {
-      TileInfo& ti = s_tile[u];
-      ti.lbeg = lpos;
-      ti.delta -= vpre;
-      if (ti.T > 0 && ti.nrec >= 0) {
-        lpos += ti.nrec;
-        vpre += ti.T;
-      }
-    }
-    s_tmp[7] = lpos;
-  }
-  __syncthreads();
-  const int nlist = s_tmp[7];
+  const uint32_t nl = P.hdr->nz_total ? P.hdr->list_n : 0u;  // clist entries
+  const int64_t total = nl ? P.lpre[nl] : 0;  // records of the list
+  const int64_t n_units = (total + 63) >> 6;
+  const int64_t nwaves = (int64_t)gridDim.x * (kEmitThreads / 64);
   // records were dropped (staged path) by the forward: no exact gradient;
   // make it loud (NaN) rather than silently wrong
   const float poison = P.hdr->dense_last ? __uint_as_float(0x7fc00000u) : 0.0f;
-  int64_t carry = 0;
-  for (int rb = 0; rb < nlist; rb += kEmitThreads) {
-    const int k = rb + tid;
-    int nv = 0, u = 0;
-    uint32_t rc[kRecWords] = {};
-    int64_t ri = 0;
-    if (k < nlist) {
-      while (u + 1 < kTilesPerContribGroup &&
-             !(s_tile[u].T > 0 && s_tile[u].nrec >= 0 && k < s_tile[u].lbeg + s_tile[u].nrec))
-        ++u;
-      ri = s_tile[u].rstart + (k - s_tile[u].lbeg);
-      const uint32_t* src = P.rec + ri * kRecWords;
+  for (int64_t k = (int64_t)blockIdx.x * (kEmitThreads / 64) + wv; k < n_units; k += nwaves) {
+    uint32_t rc[kRecWords];
+    int64_t ri, first;
+    uint32_t p, z, vi;
+    const int R = load_unit<BATCH>(P, k, nl, total, s_mark[wv], s_nv, rc, &ri, &first, &p, &z, &vi);
+    if (lane >= R) continue;
+    const float h = vol_at<BATCH>(P, (int)vi).h;
+    const uint32_t ci = rc[0] & 0xffu;
+    const int nv = s_nv[ci];
+    float c[8];
 #pragma unroll
-      for (int q = 0; q < kRecWords; ++q) rc[q] = src[q];
-      nv = s_nv[rc[0] & 0xffu];
-    }
-    int tot;
-    const int ex = block_excl_scan(nv, s_tmp, &tot);
-    if (k < nlist) {
-      const TileInfo& ti = s_tile[u];
-      const VolDesc& V = vol_at<BATCH>(P, ti.vi);
-      const float h = V.h;
-      const uint32_t ci = rc[0] & 0xffu;
-      const int64_t first = ti.delta + carry + ex;
-      float c[8];
+    for (int q = 0; q < 8; ++q) c[q] = 0.0f;
+    for (int q = 0; q < nv; ++q) {
+      const int m = 3 * (q / 3) + 2 - (q % 3);
+      const int e = (int)((s_case[ci] >> (4 * m)) & 0xfu);
+      const int ca = (int)((kEdgeA >> (3 * e)) & 7u);
+      const int cb = (int)((kEdgeB >> (3 * e)) & 7u);
+      float fa = 0.f, fb = 0.f;
 #pragma unroll
-      for (int q = 0; q < 8; ++q) c[q] = 0.0f;
-      for (int q = 0; q < nv; ++q) {
-        const int m = 3 * (q / 3) + 2 - (q % 3);
-        const int e = (int)((s_case[ci] >> (4 * m)) & 0xfu);
-        const int ca = (int)((kEdgeA >> (3 * e)) & 7u);
-        const int cb = (int)((kEdgeB >> (3 * e)) & 7u);
-        float fa = 0.f, fb = 0.f;
-#pragma unroll
-        for (int w = 0; w < 8; ++w) {
-          fa = ca == w ? __uint_as_float(rc[1 + w]) : fa;
-          fb = cb == w ? __uint_as_float(rc[1 + w]) : fb;
-        }
-        // p_b - p_a is one signed grid step along one axis (same fp32 values
-        // as the forward's node coordinates)
-        const float dpx = (float)(corner_dx(cb) - corner_dx(ca)) * h;
-        const float dpy = (float)(corner_dy(cb) - corner_dy(ca)) * h;
-        const float dpz = (float)(corner_dz(cb) - corner_dz(ca)) * h;
-        const float* g = gpos + 3 * (first + q);
-        const float sdot = g[0] * dpx + g[1] * dpy + g[2] * dpz;
-        const float d = fb - fa + 1e-15f;
-        const float inv = 1.0f / (d * d);
-        const float ga = sdot * (-(fb + 1e-15f) * inv);
-        const float gb = sdot * (fa * inv);
-#pragma unroll
-        for (int w = 0; w < 8; ++w) c[w] += (ca == w ? ga : 0.0f) + (cb == w ? gb : 0.0f);
+      for (int w = 0; w < 8; ++w) {
+        fa = ca == w ? __uint_as_float(rc[1 + w]) : fa;
+        fb = cb == w ? __uint_as_float(rc[1 + w]) : fb;
       }
-      float4* dst = reinterpret_cast<float4*>(contrib + ri * 8);
-      dst[0] = make_float4(c[0] + poison, c[1] + poison, c[2] + poison, c[3] + poison);
-      dst[1] = make_float4(c[4] + poison, c[5] + poison, c[6] + poison, c[7] + poison);
+      // p_b - p_a is one signed grid step along one axis (same fp32 values
+      // as the forward's node coordinates)
+      const float dpx = (float)(corner_dx(cb) - corner_dx(ca)) * h;
+      const float dpy = (float)(corner_dy(cb) - corner_dy(ca)) * h;
+      const float dpz = (float)(corner_dz(cb) - corner_dz(ca)) * h;
+      const float* g = gpos + 3 * (first + q);
+      const float sdot = g[0] * dpx + g[1] * dpy + g[2] * dpz;
+      const float d = fb - fa + 1e-15f;
+      const float inv = 1.0f / (d * d);
+      const float ga = sdot * (-(fb + 1e-15f) * inv);
+      const float gb = sdot * (fa * inv);
+#pragma unroll
+      for (int w = 0; w < 8; ++w) c[w] += (ca == w ? ga : 0.0f) + (cb == w ? gb : 0.0f);
     }
-    carry += tot;
+    float4* dst = reinterpret_cast<float4*>(contrib + ri * 8);
+    dst[0] = make_float4(c[0] + poison, c[1] + poison, c[2] + poison, c[3] + poison);
+    dst[1] = make_float4(c[4] + poison, c[5] + poison, c[6] + poison, c[7] + poison);
   }
 }
 
@@ -1867,20 +1817,32 @@ __global__ __launch_bounds__(256) void classify_kernel(const uint32_t* __restric
 // ================================================================ host side
 size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// The backward's two launches over nb workgroups, in launches of at most
-// kMaxLaunchBlocks workgroups (each given its first workgroup).
+// Compute units of the current device (cached per device).
+int cu_count() {
+  static int cache[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) dev = 0;
+  if (dev >= 0 && dev < 64 && cache[dev] > 0) return cache[dev];
+  int n = 0;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+    n = 256;
+  if (dev >= 0 && dev < 64) cache[dev] = n;
+  return n;
+}
+
+// The backward's first launch: persistent workgroups (the number of records is
+// on the device).
 template <bool BATCH>
-int launch_contrib(ExtractParams P, int64_t nb, const float* gpos, float* contrib,
-                   hipStream_t s) {
-  for (int64_t b0 = 0; b0 < nb; b0 += kMaxLaunchBlocks) {
-    P.first_block = b0;
-    hipLaunchKernelGGL(contrib_kernel<BATCH>, dim3((unsigned)std::min(kMaxLaunchBlocks, nb - b0)),
-                       dim3(kEmitThreads), 0, s, P, gpos, contrib);
-    MCX_HIP(hipGetLastError());
-  }
+int launch_contrib(const ExtractParams& P, const float* gpos, float* contrib, hipStream_t s) {
+  const int64_t items = (P.n_tiles + 3) / 4, most = (int64_t)cu_count() * 8;
+  hipLaunchKernelGGL(contrib_kernel<BATCH>, dim3((unsigned)std::min(items, most)),
+                     dim3(kEmitThreads), 0, s, P, gpos, contrib);
+  MCX_HIP(hipGetLastError());
   return MCX_OK;
 }
 
+// Its second, over nb workgroups, in launches of at most kMaxLaunchBlocks
+// (each given its first workgroup).
 int64_t gather_blocks(int X, int Y, int Z) {
   return (((int64_t)X * Y + kGatherSpan - 1) / kGatherSpan * Z + 3) / 4;
 }
@@ -1979,19 +1941,6 @@ int layout_ws(void* d_ws, size_t ws_bytes, int64_t n_tiles, ExtractParams& P) {
   return MCX_OK;
 }
 
-// Compute units of the current device (cached per device).
-int cu_count() {
-  static int cache[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-  if (dev >= 0 && dev < 64 && cache[dev] > 0) return cache[dev];
-  int n = 0;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-    n = 256;
-  if (dev >= 0 && dev < 64) cache[dev] = n;
-  return n;
-}
-
 // Launch K1, K2, (vbase), K3 for prepared parameters; emit = false stops
 // after the scan (records, masks and tile offsets only: the backward's
 // recompute of the forward's per-cube records).
@@ -2001,7 +1950,7 @@ int run_extract(ExtractParams& P, int elem, bool batch, int maxX, hipStream_t s,
   // record scratch: per-column quotas; the wide count kernel keeps a quarter
   // of the scratch as a shared overflow pool
   const bool wide = P.wide;
-  P.list_scan = emit;
+  P.list_scan = emit || P.write_masks;  // the backward takes the list's units too
   const int64_t pool = wide && !P.write_masks ? P.rec_cap / 4 : 0;
   P.quota = P.ncols > 0 ? (P.rec_cap - pool) / P.ncols : 0;
   if (P.quota > (int64_t)kTile * P.slab_max) P.quota = (int64_t)kTile * P.slab_max;
@@ -2345,8 +2294,7 @@ int backward_impl(const float* d_vol, int X, int Y, int Z, float h, const float*
   }
   if (!d_scratch || scratch_bytes < (size_t)P.rec_cap * 8 * sizeof(float)) return MCX_ERR_WORKSPACE;
   float* contrib = static_cast<float*>(d_scratch);
-  const int64_t g1 = (n_tiles + kTilesPerContribGroup - 1) / kTilesPerContribGroup;
-  rc = launch_contrib<false>(P, g1, d_grad_pos, contrib, s);
+  rc = launch_contrib<false>(P, d_grad_pos, contrib, s);
   if (rc) return rc;
   const int64_t g2 = gather_blocks(X, Y, Z);
   if (g2 >= ((int64_t)1 << 31)) return MCX_ERR_UNSUPPORTED;
@@ -2600,8 +2548,7 @@ extern "C" int mcx_extract_backward_batched(const mcx_batch* plan, const float* 
   if (!d_scratch || scratch_bytes < (size_t)P.rec_cap * 8 * sizeof(float)) return MCX_ERR_WORKSPACE;
   if (plan->gather_blocks >= ((int64_t)1 << 31)) return MCX_ERR_UNSUPPORTED;
   float* contrib = static_cast<float*>(d_scratch);
-  const int64_t g1 = (plan->n_tiles + kTilesPerContribGroup - 1) / kTilesPerContribGroup;
-  rc = launch_contrib<true>(P, g1, d_grad_pos, contrib, s);
+  rc = launch_contrib<true>(P, d_grad_pos, contrib, s);
   if (rc) return rc;
   return launch_gather<true>(P, plan->gather_blocks, contrib, d_grad_vol, d_maxabs, s);
 }

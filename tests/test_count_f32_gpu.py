@@ -71,3 +71,28 @@ def test_batched(dev):
     for k, f in enumerate(fs):
         ref = O.extract(f, 0.01, want=("pos",))["pos"]
         assert pos[vb[k]:vb[k + 1]].tobytes() == ref.tobytes(), SHAPES[k]
+
+
+@pytest.mark.parametrize("recompute", [False, True])
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 16, 65])
+def test_units_of_the_backward(dev, n, recompute):
+    """n voxels inside, apart from one another: 8 n records, units of 64."""
+    print(f"[case] backward units, {8 * n} records, recompute {recompute}", flush=True)
+    f = np.full((14, 41, 50), 0.5, np.float32)
+    rng = np.random.default_rng(n)
+    spots = np.stack(np.meshgrid(range(1, 13, 3), range(1, 40, 3), range(1, 49, 3),
+                                 indexing="ij"), -1).reshape(-1, 3)
+    for z, y, x in spots[np.sort(rng.choice(len(spots), n, replace=False))]:
+        f[z, y, x] = -rng.uniform(0.25, 1.0)
+    h = 0.02
+    ref = O.extract(f, h, want=("pos",))
+    v = torch.from_numpy(f).to(dev).requires_grad_(True)
+    ex = diff.DiffExtractor(f.shape, dev, recompute=recompute)
+    p = diff.extract_positions(v, h, extractor=ex)
+    assert p.detach().cpu().numpy().tobytes() == ref["pos"].tobytes()
+    g = np.random.default_rng(1).standard_normal(ref["pos"].shape).astype(np.float32)
+    p.backward(torch.from_numpy(g).to(dev))
+    want = O.extract_backward_f64(f, h, g.astype(np.float64))
+    got = v.grad.cpu().numpy().astype(np.float64)
+    assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+    assert (got[want == 0] == 0).all()

@@ -76,6 +76,12 @@ int mcx_workspace_init(void* d_ws, size_t ws_bytes, void* stream);
  * made with h_count report (and clear) the mark themselves.  Meant for
  * callers that pass no h_count: asynchronous loops and captured graphs. */
 int mcx_workspace_status(void* d_ws, size_t ws_bytes, void* stream);
+/* Tiles of the last extraction on a workspace whose records did not fit its
+ * record scratch (their vertices are right; after mcx_extract_diff* the
+ * gradient is NaN unless this is 0).  Synchronises the stream.  For callers
+ * that pass no h_count. */
+int mcx_workspace_staged_tiles(const void* d_ws, size_t ws_bytes, int64_t* h_tiles,
+                               void* stream);
 
 /* ---- extraction (replaces MarchingCubes::run, cu_marching_cubes_v1.cu:417-467:
  *      getOccupiedVoxels :185-206, computeOffsetsAndTotalVertexes :208-225,
@@ -247,7 +253,9 @@ int mcx_normals(const void* d_vol, int X, int Y, int Z, float h, const float* d_
  * mcx_extract_backward: d_grad_vol[i] = sum over the vertices on edges at
  * voxel i of dL/dp . dp/df_i, from d_grad_pos (float3 per vertex), using the
  * workspace of the preceding mcx_extract_diff call on the same volume
- * (unchanged) and d_scratch of mcx_backward_scratch_size() bytes.
+ * (unchanged) and d_scratch of mcx_backward_scratch_size() bytes.  NaN
+ * throughout if the record scratch of that call (made without h_count) was
+ * too small: the same for the batched form.
  * Deterministic: fixed-order sums, no atomics. */
 int mcx_extract_diff(const float* d_vol, int X, int Y, int Z, float h, float* d_pos,
                      int64_t cap, int64_t* d_count, int64_t* h_count, void* d_ws,

@@ -123,3 +123,16 @@ extern "C" int mcx_workspace_status(void* d_ws, size_t ws_bytes, void* stream) {
   MCX_HIP(hipStreamSynchronize(s));
   return err ? take_error(d_ws, s) : MCX_OK;
 }
+
+extern "C" int mcx_workspace_staged_tiles(const void* d_ws, size_t ws_bytes, int64_t* h_tiles,
+                                          void* stream) {
+  if (!h_tiles) return MCX_ERR_ARG;
+  if (!d_ws || ws_bytes < kWsHeader) return MCX_ERR_WORKSPACE;
+  hipStream_t s = as_stream(stream);
+  uint32_t n = 0;
+  MCX_HIP(hipMemcpyAsync(&n, static_cast<const char*>(d_ws) + offsetof(WsHeader, dense_last),
+                         sizeof(n), hipMemcpyDeviceToHost, s));
+  MCX_HIP(hipStreamSynchronize(s));
+  *h_tiles = n;
+  return MCX_OK;
+}

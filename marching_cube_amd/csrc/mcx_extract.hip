@@ -156,7 +156,7 @@ struct ExtractParams {
   int64_t cap_desc;
   int32_t* tileT;        // vertex count per tile
   int32_t* tile_nrec;    // records per tile, -1 = staged path
-  int64_t* tile_rec;     // first record of the tile
+  int64_t* tile_rec;     // first record of the tile (0 on the staged path)
   int64_t* voff;         // exclusive vertex offset per tile
   uint64_t* masks;       // active-cube bits, kCPW words per tile
   uint32_t* nz_list;     // ids of the tiles with vertices (in append order)
@@ -407,7 +407,7 @@ __global__ __launch_bounds__(256) void count_kernel(ExtractParams P) {
     if (lane == 0) {
       P.tileT[t] = (int32_t)vsum;
       P.tile_nrec[t] = dense ? -1 : (int32_t)nrec;
-      P.tile_rec[t] = rec_base + used;
+      P.tile_rec[t] = dense ? 0 : rec_base + used;
       if (dense) atomicAdd(&P.hdr->dense_acc, 1u);
     }
     if (!dense) used += nrec;
@@ -899,7 +899,7 @@ void count4_kernel(ExtractParams P) {
     if (lane == 0) {
       P.tileT[t] = (int32_t)vsum;
       P.tile_nrec[t] = dense ? -1 : (int32_t)nrec;
-      P.tile_rec[t] = rbase;
+      P.tile_rec[t] = dense ? 0 : rbase;
       if (dense) atomicAdd(&P.hdr->dense_acc, 1u);
     }
     load_plane(z + 3, L);
@@ -1558,12 +1558,20 @@ void emit_units_kernel(ExtractParams P) {
 // 18 us, a batch of 64 volumes 18 us; with eight tiles a workgroup, their
 // records spread over 256 threads after six barriers (a fifth of the threads
 // had one), 25 and 61.
+//   Records that did not fit the scratch (staged-path tiles) have no
+// contribution: the forward then has no exact gradient, and the whole of it is
+// NaN, with no record or contribution read.
+__device__ __forceinline__ bool no_gradient(const ExtractParams& P) {
+  return P.hdr->dense_last != 0;
+}
+
 template <bool BATCH>
 __global__ __launch_bounds__(kEmitThreads) void contrib_kernel(ExtractParams P, const float* gpos,
                                                                float* contrib) {
   __shared__ uint64_t s_case[256];
   __shared__ uint8_t s_nv[256];
   __shared__ uint8_t s_mark[kEmitThreads / 64][64];
+  if (no_gradient(P)) return;
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   s_case[threadIdx.x] = dCase[threadIdx.x];
@@ -1574,9 +1582,6 @@ __global__ __launch_bounds__(kEmitThreads) void contrib_kernel(ExtractParams P, 
   const int64_t total = nl ? P.lpre[nl] : 0;  // records of the list
   const int64_t n_units = (total + 63) >> 6;
   const int64_t nwaves = (int64_t)gridDim.x * (kEmitThreads / 64);
-  // records were dropped (staged path) by the forward: no exact gradient;
-  // make it loud (NaN) rather than silently wrong
-  const float poison = P.hdr->dense_last ? __uint_as_float(0x7fc00000u) : 0.0f;
   for (int64_t k = (int64_t)blockIdx.x * (kEmitThreads / 64) + wv; k < n_units; k += nwaves) {
     uint32_t rc[kRecWords];
     int64_t ri, first;
@@ -1615,8 +1620,8 @@ __global__ __launch_bounds__(kEmitThreads) void contrib_kernel(ExtractParams P, 
       for (int w = 0; w < 8; ++w) c[w] += (ca == w ? ga : 0.0f) + (cb == w ? gb : 0.0f);
     }
     float4* dst = reinterpret_cast<float4*>(contrib + ri * 8);
-    dst[0] = make_float4(c[0] + poison, c[1] + poison, c[2] + poison, c[3] + poison);
-    dst[1] = make_float4(c[4] + poison, c[5] + poison, c[6] + poison, c[7] + poison);
+    dst[0] = make_float4(c[0], c[1], c[2], c[3]);
+    dst[1] = make_float4(c[4], c[5], c[6], c[7]);
   }
 }
 
@@ -1691,18 +1696,21 @@ __global__ __launch_bounds__(256) void gather_kernel(ExtractParams P, const floa
     }
   }
   float* const gz = gvol + (int64_t)z * XY;
-  if (!__any(word != 0)) {
+  const bool none = no_gradient(P);
+  if (none || !__any(word != 0)) {
     // no active cube has a corner in the span: its gradient is zero (the
     // sums below would all be empty), and it raises no maximum
+    const uint32_t g = none ? 0x7fc00000u : 0u;
 #pragma unroll
     for (int j = 0; j < kGatherSpan; j += 256) {
       const uint32_t q = (uint32_t)(q0 + j + 4 * lane);
       if (q + 4 <= XY) {
-        *reinterpret_cast<u32x4a4*>(gz + q) = u32x4a4{0, 0, 0, 0};
+        *reinterpret_cast<u32x4a4*>(gz + q) = u32x4a4{g, g, g, g};
       } else {
-        for (uint32_t e = q; e < XY; ++e) gz[e] = 0.0f;
+        for (uint32_t e = q; e < XY; ++e) gz[e] = __uint_as_float(g);
       }
     }
+    if (none && maxg && lane == 0 && blockIdx.x == 0) atomicMax(maxg, g);
     return;
   }
   uint32_t pre = (uint32_t)__popcll(word);  // then the set bits of the tile's earlier words

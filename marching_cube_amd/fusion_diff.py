@@ -280,11 +280,19 @@ class FusionGraph:
 
     def check(self):
         """Raise McxError if an extraction of the pass reported a device-side
-        error since the last check (synchronises the stream), or if the vertices
-        exceeded the capacity."""
-        _capi.check(_capi.load().mcx_workspace_status(_ptr(self.ws), self.ws.numel(),
-                                                      _stream_handle(self.dev)),
+        error since the last check (synchronises the stream), if its records did
+        not fit the workspace (the gradients are then not those of the loss), or
+        if the vertices exceeded the capacity."""
+        lib, s = _capi.load(), _stream_handle(self.dev)
+        _capi.check(lib.mcx_workspace_status(_ptr(self.ws), self.ws.numel(), s),
                     "fusion graph extraction workspace")
+        staged = ctypes.c_int64(0)
+        _capi.check(lib.mcx_workspace_staged_tiles(_ptr(self.ws), self.ws.numel(),
+                                                   ctypes.byref(staged), s),
+                    "fusion graph extraction workspace")
+        if staged.value:
+            raise _capi.McxError(_capi.ERR_WORKSPACE, f"FusionGraph: the records of "
+                                                      f"{staged.value} tiles did not fit")
         if int(self.total.item()) > self.cap:
             raise _capi.McxError(_capi.ERR_CAPACITY, f"FusionGraph: {int(self.total.item())} "
                                                      f"vertices exceed the capacity {self.cap}")

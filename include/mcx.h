@@ -183,6 +183,9 @@ int64_t mcx_batch_voxels(const mcx_batch* plan);
  *   mcx_extract_diff_batched of this plan and d_scratch of
  *   mcx_batch_backward_scratch_size bytes; d_maxabs (optional, device
  *   uint32) receives max |dL/dtsdf| as float bits.  Fixed-order sums.
+ *   _rows: d_grad_pos has `rows` rows; if the meshes have more vertices (a
+ *   forward without h_count whose cap they passed), dL/dtsdf is NaN
+ *   throughout and nothing past the rows is read.
  * mcx_integrate_tsdf_backward_batched: dL/d(depth value) [nvol][K][H][W]
  *   from dL/dtsdf, as mcx_integrate_tsdf_backward per volume; d_weight0: the
  *   weights before the fused frames (NULL: all 0); d_maxabs: max |dL/dtsdf|
@@ -201,6 +204,10 @@ int mcx_extract_backward_batched(const mcx_batch* plan, const float* d_grad_pos,
                                  float* d_grad_vol, uint32_t* d_maxabs, void* d_ws,
                                  size_t ws_bytes, void* d_scratch, size_t scratch_bytes,
                                  void* stream);
+int mcx_extract_backward_batched_rows(const mcx_batch* plan, const float* d_grad_pos,
+                                      int64_t rows, float* d_grad_vol, uint32_t* d_maxabs,
+                                      void* d_ws, size_t ws_bytes, void* d_scratch,
+                                      size_t scratch_bytes, void* stream);
 size_t mcx_integrate_tsdf_backward_batched_workspace_size(const mcx_batch* plan, int W, int H,
                                                           int K);
 int mcx_integrate_tsdf_backward_batched(const mcx_batch* plan, const float* d_grad_tsdf,

@@ -100,6 +100,8 @@ SIGNATURES = {
     "mcx_extract_diff_batched": (_i32, [_vp, _vp, _i64, _vp, _vp, _vp, _vp, _sz, _vp]),
     "mcx_batch_backward_scratch_size": (_sz, [_vp, _sz]),
     "mcx_extract_backward_batched": (_i32, [_vp, _vp, _vp, _vp, _vp, _sz, _vp, _sz, _vp]),
+    "mcx_extract_backward_batched_rows": (_i32, [_vp, _vp, _i64, _vp, _vp, _vp, _sz, _vp, _sz,
+                                                 _vp]),
     "mcx_integrate_tsdf_backward_batched_workspace_size": (_sz, [_vp, _i32, _i32, _i32]),
     "mcx_integrate_tsdf_backward_batched": (_i32, [_vp, _vp, _vp, _vp, _f32, _i32, _vp, _vp,
                                                    _vp, _f32, _i32, _i32, _i32, _vp, _vp, _sz,

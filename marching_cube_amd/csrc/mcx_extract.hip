@@ -177,6 +177,7 @@ struct ExtractParams {
   int64_t zero_bytes;
   uint32_t* rec;
   int64_t rec_cap;
+  int64_t grad_rows;     // backward: rows of the vertices' gradient
 };
 
 // The fp32 value of a voxel: tsdf / 32766 (tsdf_unit, correctly rounded) or
@@ -1559,10 +1560,11 @@ void emit_units_kernel(ExtractParams P) {
 // records spread over 256 threads after six barriers (a fifth of the threads
 // had one), 25 and 61.
 //   Records that did not fit the scratch (staged-path tiles) have no
-// contribution: the forward then has no exact gradient, and the whole of it is
-// NaN, with no record or contribution read.
+// contribution, vertices past the caller's rows no gradient: the forward then
+// has no exact gradient, and the whole of it is NaN, with no record, row or
+// contribution read.
 __device__ __forceinline__ bool no_gradient(const ExtractParams& P) {
-  return P.hdr->dense_last != 0;
+  return P.hdr->dense_last != 0 || P.hdr->count > P.grad_rows;
 }
 
 template <bool BATCH>
@@ -1571,14 +1573,14 @@ __global__ __launch_bounds__(kEmitThreads) void contrib_kernel(ExtractParams P, 
   __shared__ uint64_t s_case[256];
   __shared__ uint8_t s_nv[256];
   __shared__ uint8_t s_mark[kEmitThreads / 64][64];
-  if (no_gradient(P)) return;
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   s_case[threadIdx.x] = dCase[threadIdx.x];
   s_nv[threadIdx.x] = dNumVerts[threadIdx.x];
   s_mark[wv][lane] = 0;
   __syncthreads();
-  const uint32_t nl = P.hdr->nz_total ? P.hdr->list_n : 0u;  // clist entries
+  // clist entries
+  const uint32_t nl = P.hdr->nz_total && !no_gradient(P) ? P.hdr->list_n : 0u;
   const int64_t total = nl ? P.lpre[nl] : 0;  // records of the list
   const int64_t n_units = (total + 63) >> 6;
   const int64_t nwaves = (int64_t)gridDim.x * (kEmitThreads / 64);
@@ -2302,6 +2304,7 @@ int backward_impl(const float* d_vol, int X, int Y, int Z, float h, const float*
   }
   if (!d_scratch || scratch_bytes < (size_t)P.rec_cap * 8 * sizeof(float)) return MCX_ERR_WORKSPACE;
   float* contrib = static_cast<float*>(d_scratch);
+  P.grad_rows = INT64_MAX;  // the caller's rows are the forward's vertices
   rc = launch_contrib<false>(P, d_grad_pos, contrib, s);
   if (rc) return rc;
   const int64_t g2 = gather_blocks(X, Y, Z);
@@ -2539,7 +2542,16 @@ extern "C" int mcx_extract_backward_batched(const mcx_batch* plan, const float* 
                                             float* d_grad_vol, uint32_t* d_maxabs, void* d_ws,
                                             size_t ws_bytes, void* d_scratch,
                                             size_t scratch_bytes, void* stream) {
-  if (!plan || !d_grad_vol) return MCX_ERR_ARG;
+  return mcx_extract_backward_batched_rows(plan, d_grad_pos, INT64_MAX, d_grad_vol, d_maxabs, d_ws,
+                                           ws_bytes, d_scratch, scratch_bytes, stream);
+}
+
+extern "C" int mcx_extract_backward_batched_rows(const mcx_batch* plan, const float* d_grad_pos,
+                                                 int64_t rows, float* d_grad_vol,
+                                                 uint32_t* d_maxabs, void* d_ws, size_t ws_bytes,
+                                                 void* d_scratch, size_t scratch_bytes,
+                                                 void* stream) {
+  if (!plan || !d_grad_vol || rows < 0) return MCX_ERR_ARG;
   if (plan->elem != MCX_ELEM_F32) return MCX_ERR_ARG;
   hipStream_t s = as_stream(stream);
   int rc = MCX_OK;
@@ -2556,6 +2568,7 @@ extern "C" int mcx_extract_backward_batched(const mcx_batch* plan, const float* 
   if (!d_scratch || scratch_bytes < (size_t)P.rec_cap * 8 * sizeof(float)) return MCX_ERR_WORKSPACE;
   if (plan->gather_blocks >= ((int64_t)1 << 31)) return MCX_ERR_UNSUPPORTED;
   float* contrib = static_cast<float*>(d_scratch);
+  P.grad_rows = rows;
   rc = launch_contrib<true>(P, d_grad_pos, contrib, s);
   if (rc) return rc;
   return launch_gather<true>(P, plan->gather_blocks, contrib, d_grad_vol, d_maxabs, s);

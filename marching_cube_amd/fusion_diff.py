@@ -250,11 +250,10 @@ class FusionGraph:
                                             _ptr(self.targets_all), self.M, self.cap,
                                             _ptr(self.loss), _ptr(self.gpos), _ptr(self.ws_l),
                                             self.ws_l.numel(), s), "mcx_chamfer_batched")
-        _capi.check(lib.mcx_extract_backward_batched(h, _ptr(self.gpos), _ptr(self.gtsdf_all),
-                                                     _ptr(self.maxabs), _ptr(self.ws),
-                                                     self.ws.numel(), _ptr(self.scratch),
-                                                     self.scratch.numel(), s),
-                    "mcx_extract_backward_batched")
+        _capi.check(lib.mcx_extract_backward_batched_rows(
+            h, _ptr(self.gpos), self.cap, _ptr(self.gtsdf_all), _ptr(self.maxabs), _ptr(self.ws),
+            self.ws.numel(), _ptr(self.scratch), self.scratch.numel(), s),
+            "mcx_extract_backward_batched_rows")
         _capi.check(lib.mcx_integrate_tsdf_backward_batched(
             h, _ptr(self.gtsdf_all), None, _ptr(self.maxabs), self.trunc, self.max_w, self.intr,
             _ptr(self.poses_all), _ptr(self.depth_all), 1.0, self.W, self.H, self.K,

@@ -2,7 +2,8 @@
 small: the mesh is whole, and the gradient is NaN throughout (no contribution
 exists for the tiles that found no room, and none is read), for scratches that
 hold no tile, some tiles and all but the last of them, single, recomputed and
-batched; FusionGraph.check() reports it."""
+batched; the same for a batch whose vertices' gradient has too few rows;
+FusionGraph.check() reports both."""
 import ctypes
 
 import numpy as np
@@ -129,4 +130,55 @@ def test_fusion_graph_reports_it(dev):
     with pytest.raises(_capi.McxError) as e:
         g.check()
     assert e.value.status == _capi.ERR_WORKSPACE
+    assert torch.isnan(g.gtsdf_all).all()
+
+
+@pytest.mark.parametrize("missing", [-1, 0, 1, 10**6])
+def test_batched_rows(dev, missing):
+    """The gradient's rows as many as the vertices, one more, one fewer, none."""
+    print(f"[case] batched backward, {missing} rows short", flush=True)
+    lib, h = _capi.load(), 0.01
+    fs = [noisy(s, k) for k, s in enumerate([(9, 20, 21), (5, 16, 32)])]
+    flat = torch.from_numpy(np.concatenate([f.reshape(-1) for f in fs])).to(dev)
+    at = np.cumsum([0] + [f.size for f in fs])
+    plan = batch.BatchPlan([flat[at[k]:at[k + 1]].view(f.shape) for k, f in enumerate(fs)],
+                           [h] * len(fs))
+    n = sum(O.extract(f, h, want=("pos",))["n"] for f in fs)
+    rows = max(0, n - missing)
+    ws = workspace(lib.mcx_batch_workspace_size(plan.handle, 65536), dev)
+    scratch = torch.zeros(lib.mcx_batch_backward_scratch_size(plan.handle, ws.numel()),
+                          dtype=torch.uint8, device=dev)
+    vbase = torch.empty(len(fs) + 1, dtype=torch.int64, device=dev)
+    g = torch.from_numpy(np.random.default_rng(2).standard_normal((n + 1, 3)).astype(
+        np.float32)).to(dev)
+    gv, plain = torch.zeros_like(flat), torch.zeros_like(flat)
+    s = _stream_handle(dev)
+    _capi.check(lib.mcx_extract_diff_batched(plan.handle, None, 0, _ptr(vbase), None, None,
+                                             _ptr(ws), ws.numel(), s))
+    assert staged_tiles(ws, dev) == 0 and int(vbase[-1].item()) == n
+    _capi.check(lib.mcx_extract_backward_batched_rows(plan.handle, _ptr(g), rows, _ptr(gv), None,
+                                                      _ptr(ws), ws.numel(), _ptr(scratch),
+                                                      scratch.numel(), s))
+    _capi.check(lib.mcx_extract_backward_batched(plan.handle, _ptr(g), _ptr(plain), None, _ptr(ws),
+                                                 ws.numel(), _ptr(scratch), scratch.numel(), s))
+    assert plain.abs().max() > 0 and torch.isfinite(plain).all()
+    if rows < n:
+        assert torch.isnan(gv).all()
+    else:
+        assert torch.equal(gv, plain)
+
+
+def test_fusion_graph_past_its_capacity(dev):
+    print("[case] FusionGraph with more vertices than its cap", flush=True)
+    K, W, H = 2, 64, 48
+    depth = [torch.full((K, H, W), 1.0, device=dev)]
+    poses = [torch.tensor([[1, 0, 0, 0, 1, 0, 0, 0, 1, 0.5, 0.5, -0.5]] * K,
+                          dtype=torch.float32, device=dev)]
+    g = fusion_diff.FusionGraph([(24, 24, 24)], [1 / 24], depth, poses,
+                                [torch.full((4, 3), 0.5, device=dev)],
+                                [60.0, 60.0, 31.5, 23.5], trunc=0.1, cap=30)
+    g.step()
+    with pytest.raises(_capi.McxError) as e:
+        g.check()
+    assert e.value.status == _capi.ERR_CAPACITY
     assert torch.isnan(g.gtsdf_all).all()

@@ -65,6 +65,7 @@ struct IntegrateParams {
   int W, H, K;
   int TX, TY, TX1, TY1;    // tiles of kTile x kTile pixels; of 4 x 4 tiles
   int tiled;               // frames [0, tiled) have a tile table
+  int framed;              // sides of at most 2^22 pixels (test_brick)
   int plain;               // camera, scale and truncation within the fast forms' ranges
   FastDiv divX, divY;      // workgroups along x and y of the volume
   int64_t first_block;     // region of this launch's first workgroup
@@ -211,14 +212,17 @@ constexpr int kRegionX = 4 * kBrick;  // a workgroup's four bricks lie side by s
 // direction of its centre (|n| = 1, so |q(p)| >= q(p) . n, linear in p).
 //   kFree is the same argument from the other side: the least distance
 // measured against the centre's plus the half diagonal of e.
-// Margins: a voxel's fp32 q, and the box's, differ from the exact one by at
-// most d = 4e-7 * (|dx| + |dy| + |dz| + |p| + half sides) per component (the
-// coordinates, the subtraction and the fma chain, |R| <= 1), which widens e;
-// the rectangle is wider by one pixel, for the rounding to the nearest pixel
-// and the hardware reciprocals (|u|, |v| < 2^16: under 0.02 pixel).  Distances
-// differ by less than 1e-6 of the same sum, taken four times over.  So every
-// voxel of a skipped frame would have taken its q.z, window, dropout or
-// -trunc_neg skip.
+// Margins, in sum = (|dx| + |dy| + |dz| + |p| + half sides) * m, m the largest
+// |entry| of R (any matrix is a pose; at least 1): a voxel's fp32 q, and the
+// box's, differ from the exact one by at most 2.4e-7 sum per component (the
+// coordinates, the subtraction, the fma chain), the quotients by the hardware
+// reciprocals from the exact ones by 2.4e-7 of themselves, and |q| <= sum: d =
+// 8e-7 sum widens e for all of it.  The rectangle is wider by one pixel, half
+// of it for the rounding to the nearest pixel and half for that of u (2^-24 of
+// up to 2^22; wider frames are not tested).  Distances differ by less than
+// 1.6e-6 sum, taken as 4e-6.  So every voxel of a skipped frame would have
+// taken its q.z, window, dropout or -trunc_neg skip.  (d = 4e-7 and m = 1 left
+// out updates at sdf = -trunc_neg under matrices of scale 100 and more.)
 // Rectangles of up to 4 x 4 tiles are read from the table of 8-pixel tiles,
 // larger ones from the 32-pixel tiles; beyond that nothing is known of the
 // depth.
@@ -235,8 +239,12 @@ __device__ int test_brick(const IntegrateParams& P, int x0, int y0, int z0, int 
   const float r0 = R[0], r1 = R[1], r2 = R[2], r3 = R[3], r4 = R[4], r5 = R[5], r6 = R[6],
               r7 = R[7], r8 = R[8];
   const float dx = px - R[9], dy = py - R[10], dz = pz - R[11];
-  const float sum = fabsf(dx) + fabsf(dy) + fabsf(dz) + (px + hx) + (py + hy) + (pz + hz);
-  const float d = 4e-7f * sum;
+  const float m = fmaxf(fmaxf(fmaxf(fmaxf(1.0f, fabsf(r0)), fmaxf(fabsf(r1), fabsf(r2))),
+                              fmaxf(fmaxf(fabsf(r3), fabsf(r4)), fmaxf(fabsf(r5), fabsf(r6)))),
+                        fmaxf(fabsf(r7), fabsf(r8)));
+  const float sum =
+      (fabsf(dx) + fabsf(dy) + fabsf(dz) + (px + hx) + (py + hy) + (pz + hz)) * m;
+  const float d = 8e-7f * sum;
   const float qx = __fmaf_rn(r6, dz, __fmaf_rn(r3, dy, r0 * dx));
   const float qy = __fmaf_rn(r7, dz, __fmaf_rn(r4, dy, r1 * dx));
   const float qz = __fmaf_rn(r8, dz, __fmaf_rn(r5, dy, r2 * dx));
@@ -245,7 +253,7 @@ __device__ int test_brick(const IntegrateParams& P, int x0, int y0, int z0, int 
   const float ez = __fmaf_rn(fabsf(r8), hz, __fmaf_rn(fabsf(r5), hy, __fmaf_rn(fabsf(r2), hx, d)));
   if (qz + ez < -fmaxf(1e-4f, 4.0f * d)) return kSkip;
   const float zlo = qz - ez;
-  if (!(zlo > 0.01f)) return 0;
+  if (!(zlo > 0.01f) || !P.framed) return 0;
   const float rz = __builtin_amdgcn_rcpf(qz), rl = __builtin_amdgcn_rcpf(zlo);
   const float tx = qx * rz, ty = qy * rz;
   const float u = __fmaf_rn(P.fx, tx, P.cx), v = __fmaf_rn(P.fy, ty, P.cy);
@@ -1137,7 +1145,7 @@ extern "C" size_t mcx_integrate_workspace_size(int W, int H) {
   return rf ? al256(rf) + 256 + tile_tables_bytes(W, H) : 0;
 }
 
-// The smaller truncation, the reciprocals and whether everything lies where
+// The smaller truncation, the reciprocals, and whether everything lies where
 // the quick exact forms hold (kFast): pixel numbers below 2^22, finite ray
 // factors, truncations and scale within 2^-60 to 2^60.
 void set_trunc_neg(IntegrateParams& P, float trunc_neg) {
@@ -1147,7 +1155,8 @@ void set_trunc_neg(IntegrateParams& P, float trunc_neg) {
   const auto in = [](float v, float lo, float hi) {
     return std::fabs(v) >= lo && std::fabs(v) <= hi;
   };
-  P.plain = P.W <= (1 << 22) && P.H <= (1 << 22) && in(P.trunc, 0x1p-60f, 0x1p60f) &&
+  P.framed = P.W <= (1 << 22) && P.H <= (1 << 22);
+  P.plain = P.framed && in(P.trunc, 0x1p-60f, 0x1p60f) &&
             in(trunc_neg, 0x1p-60f, 0x1p60f) && P.depth_scale > 0.0f &&
             in(P.depth_scale, 0x1p-60f, 0x1p60f) && in(P.fx, 0x1p-20f, 0x1p20f) &&
             in(P.fy, 0x1p-20f, 0x1p20f) && in(P.cx, 0.0f, 0x1p22f) && in(P.cy, 0.0f, 0x1p22f);

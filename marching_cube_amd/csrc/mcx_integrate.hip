@@ -36,6 +36,7 @@
 #include <type_traits>
 
 #include "mcx_internal.h"
+#include "mcx_region_order.h"
 
 namespace mcx {
 namespace {
@@ -68,7 +69,7 @@ struct IntegrateParams {
   int framed;              // sides of at most 2^22 pixels (test_brick)
   int plain;               // camera, scale and truncation within the fast forms' ranges
   FastDiv divX, divY;      // workgroups along x and y of the volume
-  int64_t first_block;     // region of this launch's first workgroup
+  int64_t first_block, end_block;  // this launch's regions
   int log2_run;            // regions in a row of one XCD
 };
 
@@ -339,52 +340,31 @@ struct Brick {
 // A wave is a workgroup: the four waves of a region end at different times,
 // and a workgroup of four would hold the places of those that ended (3.1 waves
 // ran per SIMD where five fit; one frame into 512^3 111 -> 81 us, 300 frames
-// 12.6 -> 11.2 ms).  Workgroups go round the 8 XCDs, so a region's four waves
-// are those of every 8th workgroup: one L2 sees whole lines.  An XCD takes
-// 2^log2_run regions in a row.
-__device__ __forceinline__ int64_t region_of(int64_t first, int log2_run, int* wave) {
-  const uint32_t b = blockIdx.x, i = b >> 3, r = i >> 2;
-  *wave = (int)(i & 3);
-  return first + ((int64_t)(r >> log2_run) << (log2_run + 3)) + ((b & 7) << log2_run) +
-         (r & ((1u << log2_run) - 1));
+// 12.6 -> 11.2 ms).  This workgroup's region (-1: past the launch's last) and
+// which of the region's waves it is.
+__device__ __forceinline__ int64_t region_of(const IntegrateParams& P, int* wave) {
+  *wave = wave_of_block(blockIdx.x);
+  return region_of_block(blockIdx.x, P.first_block, P.end_block, P.log2_run);
 }
 
-// A wave's first brick of region `blk` of a volume; false past the volume's
-// edge.  Regions are numbered x first, or (BLOCKS) in blocks of 2 x 8 x 4
-// regions, smaller at the far sides: waves that run together then see the same
-// part of each frame, and an XCD's L2 holds it (300 frames into 512^3: 10.9 ms
-// x first, where the waves of an XCD lie all over a slab, 8.8 ms in blocks).
-constexpr int kBlockX = 2, kBlockY = 8, kBlockZ = 4;
+// A wave's first brick of region `blk` >= 0 of a volume; false past the
+// volume's edge.  Regions are numbered x first, or (BLOCKS) in blocks.
 template <bool BLOCKS>
 __device__ __forceinline__ bool brick_origin(const IntegrateParams& P, uint32_t blk, int wave,
                                              int zstep, int* x0, int* y0, int* z0) {
-  uint32_t x, y, z;
+  RegionAt at;
   if (BLOCKS) {
-    const uint32_t nx = P.divX.d, ny = P.divY.d, nz = (uint32_t)((P.Z + zstep - 1) / zstep);
-    const uint32_t bz = blk / (nx * ny * kBlockZ);
-    if (bz * kBlockZ >= nz) return false;
-    uint32_t r = blk - bz * (nx * ny * kBlockZ);
-    const uint32_t hz = min((uint32_t)kBlockZ, nz - bz * kBlockZ);
-    const uint32_t by = r / (nx * kBlockY * hz);
-    r -= by * (nx * kBlockY * hz);
-    const uint32_t hy = min((uint32_t)kBlockY, ny - by * kBlockY);
-    const uint32_t bx = r / (kBlockX * hy * hz);
-    r -= bx * (kBlockX * hy * hz);
-    const uint32_t hx = min((uint32_t)kBlockX, nx - bx * kBlockX);
-    const uint32_t iy = r / hx, iz = iy / hy;
-    x = bx * kBlockX + r - iy * hx;
-    y = by * kBlockY + iy - iz * hy;
-    z = bz * kBlockZ + iz;
+    at = blocked_region(blk, P.divX.d, P.divY.d, (uint32_t)((P.Z + zstep - 1) / zstep));
   } else {
     const uint32_t row = P.divX.div(blk);
-    z = P.divY.div(row);
-    x = blk - row * P.divX.d;
-    y = row - z * P.divY.d;
+    at.z = P.divY.div(row);
+    at.x = blk - row * P.divX.d;
+    at.y = row - at.z * P.divY.d;
   }
-  *x0 = __builtin_amdgcn_readfirstlane((int)x) * kRegionX + wave * kBrick;
-  *y0 = __builtin_amdgcn_readfirstlane((int)y) * kBrick;
-  *z0 = __builtin_amdgcn_readfirstlane((int)z) * zstep;
-  return *x0 < P.X && *z0 < P.Z;
+  *x0 = __builtin_amdgcn_readfirstlane((int)at.x) * kRegionX + wave * kBrick;
+  *y0 = __builtin_amdgcn_readfirstlane((int)at.y) * kBrick;
+  *z0 = __builtin_amdgcn_readfirstlane((int)at.z) * zstep;
+  return *x0 < P.X;
 }
 
 // The frames that bricks may observe.  A wave's 64 lanes test `lanes` frames
@@ -622,8 +602,9 @@ __device__ __forceinline__ float truncated(const IntegrateParams& P, float sdf) 
 template <typename DT>
 __global__ __launch_bounds__(64) void integrate_kernel(IntegrateParams P, int bricks) {
   int wave, x0, y0, z0;
-  const uint32_t blk = (uint32_t)region_of(P.first_block, P.log2_run, &wave);
-  if (!brick_origin<true>(P, blk, wave, kBrickZ * bricks, &x0, &y0, &z0)) return;
+  const int64_t blk = region_of(P, &wave);
+  if (blk < 0 || !brick_origin<true>(P, (uint32_t)blk, wave, kBrickZ * bricks, &x0, &y0, &z0))
+    return;
   const int64_t XY = (int64_t)P.X * P.Y;
   for_bricks<kBrickZ>(P, x0, y0, z0, bricks, [&](const Brick<kBrickZ>& B, Frames<kBrickZ>& F) {
     uint32_t* const v = P.vol + B.first(P);
@@ -660,8 +641,9 @@ __global__ __launch_bounds__(64) void integrate_kernel(IntegrateParams P, int br
 template <typename DT>
 __global__ __launch_bounds__(64) void integrate1_kernel(IntegrateParams P, int bricks) {
   int wave, x0, y0, z0;
-  const uint32_t blk = (uint32_t)region_of(P.first_block, P.log2_run, &wave);
-  if (!brick_origin<false>(P, blk, wave, kBrickZ * bricks, &x0, &y0, &z0)) return;
+  const int64_t blk = region_of(P, &wave);
+  if (blk < 0 || !brick_origin<false>(P, (uint32_t)blk, wave, kBrickZ * bricks, &x0, &y0, &z0))
+    return;
   const int64_t XY = (int64_t)P.X * P.Y;
   const int lane = threadIdx.x & 63, zt = z0 + lane * kBrickZ;
   const int cls =
@@ -777,8 +759,9 @@ __device__ __forceinline__ void integrate_tsdf_stored(const IntegrateParams& P,
 __global__ __launch_bounds__(64) void integrate_tsdf_kernel(IntegrateParams P, int bricks,
                                                              float* tsdf, int32_t* wvol) {
   int wave, x0, y0, z0;
-  const uint32_t blk = (uint32_t)region_of(P.first_block, P.log2_run, &wave);
-  if (!brick_origin<true>(P, blk, wave, kBrickZ * bricks, &x0, &y0, &z0)) return;
+  const int64_t blk = region_of(P, &wave);
+  if (blk < 0 || !brick_origin<true>(P, (uint32_t)blk, wave, kBrickZ * bricks, &x0, &y0, &z0))
+    return;
   for_bricks<kBrickZ>(P, x0, y0, z0, bricks, [&](const Brick<kBrickZ>& B, Frames<kBrickZ>& F) {
     integrate_tsdf_stored(P, B, F, tsdf, wvol);
   });
@@ -902,8 +885,8 @@ __global__ __launch_bounds__(64) void integrate_tsdf_backward_kernel(
     IntegrateParams P, const float* __restrict__ g, const int32_t* __restrict__ w0vol,
     const uint32_t* maxg, float max_dtdd, unsigned long long* acc) {
   int wave, x0, y0, z0;
-  const uint32_t blk = (uint32_t)region_of(P.first_block, P.log2_run, &wave);
-  if (!brick_origin<true>(P, blk, wave, NZ, &x0, &y0, &z0)) return;
+  const int64_t blk = region_of(P, &wave);
+  if (blk < 0 || !brick_origin<true>(P, (uint32_t)blk, wave, NZ, &x0, &y0, &z0)) return;
   backward_brick(P, Brick<NZ>(P, x0, y0, z0), g, w0vol, maxg, max_dtdd, acc);
 }
 
@@ -917,9 +900,7 @@ struct BatchIntegrateParams {
   int from_init;         // start every voxel from (init_value, 0) without reading it
   float init_value;
   int bricks;            // bricks above one another in a workgroup
-  int64_t end_block;     // regions [first_block, end_block) are this launch's
   int tiled_vol;         // volumes [tiled_vol, tiled_vol + base.tiled / K) have tile tables
-  int64_t first_block;   // workgroup index of this launch's blockIdx.x 0
 };
 
 // This workgroup's volume (binary search over the block ranges), its launch
@@ -928,8 +909,8 @@ __device__ __forceinline__ bool batch_setup(const BatchIntegrateParams& B, Integ
                                             int64_t* vox_begin, int* vol, int* x0, int* y0,
                                             int* z0) {
   int wave;
-  const int64_t blk = region_of(B.first_block, B.base.log2_run, &wave);
-  if (blk >= B.end_block) return false;
+  const int64_t blk = region_of(B.base, &wave);
+  if (blk < 0) return false;
   const int vi = __builtin_amdgcn_readfirstlane(
       batch_volume_of<&BatchVol::blk_begin>(B.bvol, B.nvol, blk));
   const BatchVol& V = B.bvol[vi];
@@ -1198,7 +1179,7 @@ int prepare_integrate(IntegrateParams& P, int X, int Y, int Z, float h, float tr
   P.K = 0;
   P.poses = nullptr;
   P.depth = nullptr;
-  P.first_block = 0;
+  P.first_block = P.end_block = 0;
   P.log2_run = 0;
   return MCX_OK;
 }
@@ -1236,12 +1217,12 @@ int frame_tiles(IntegrateParams& P, const DT* depth, int64_t frames, char* table
   return MCX_OK;
 }
 
-// Workgroups of a launch over `n` regions (whole rounds of the 8 XCDs), and
-// the most regions of a launch.
+// The launch over regions [b0, end), at most kMaxRegions of them.
 constexpr int64_t kMaxRegions = kMaxLaunchBlocks;
-unsigned region_groups(int64_t n, int log2_run) {
-  const int64_t round = (int64_t)8 << log2_run;
-  return (unsigned)((n + round - 1) / round * round * 4);
+dim3 region_grid(IntegrateParams& P, int64_t b0, int64_t end) {
+  P.first_block = b0;
+  P.end_block = std::min(end, b0 + kMaxRegions);
+  return dim3((unsigned)region_workgroups(P.end_block - b0, P.log2_run));
 }
 // Eight regions of a block in a row for one XCD, where several frames are
 // swept over regions enough for that (runs of 16 and 32 8.9 ms, of 64 10.7: the
@@ -1285,8 +1266,7 @@ int integrate_impl(void* d_vol, int X, int Y, int Z, float h, float trunc_neg, f
     const int64_t nb = regions(X, Y, Z, kBrickZ * bricks);
     P.log2_run = region_runs(nb, P.K);
     for (int64_t b0 = 0; b0 < nb; b0 += kMaxRegions) {
-      P.first_block = b0;
-      const dim3 grid(region_groups(std::min(kMaxRegions, nb - b0), P.log2_run));
+      const dim3 grid = region_grid(P, b0, nb);
       if (P.K == 1)
         hipLaunchKernelGGL(integrate1_kernel<DT>, grid, dim3(64), 0, s, P, bricks);
       else
@@ -1397,8 +1377,7 @@ extern "C" int mcx_integrate_tsdf(float* d_tsdf, int32_t* d_weight, int X, int Y
     const int64_t nb = regions(X, Y, Z, kBrickZ * bricks);
     P.log2_run = region_runs(nb, P.K);
     for (int64_t b0 = 0; b0 < nb; b0 += kMaxRegions) {
-      P.first_block = b0;
-      const dim3 grid(region_groups(std::min(kMaxRegions, nb - b0), P.log2_run));
+      const dim3 grid = region_grid(P, b0, nb);
       hipLaunchKernelGGL(integrate_tsdf_kernel, grid, dim3(64), 0, s, P, bricks, d_tsdf, d_weight);
       MCX_HIP(hipGetLastError());
     }
@@ -1457,8 +1436,7 @@ extern "C" int mcx_integrate_tsdf_backward(const float* d_grad_tsdf, const int32
   const int64_t nb = regions(X, Y, Z, small ? 1 : kBrickZ);
   P.log2_run = region_runs(nb, K);
   for (int64_t b0 = 0; b0 < nb; b0 += kMaxRegions) {
-    P.first_block = b0;
-    const dim3 grid(region_groups(std::min(kMaxRegions, nb - b0), P.log2_run));
+    const dim3 grid = region_grid(P, b0, nb);
     if (small)
       hipLaunchKernelGGL(integrate_tsdf_backward_kernel<1>, grid, dim3(64), 0, s, P, d_grad_tsdf,
                          d_weight0, maxg, mdt, acc);
@@ -1528,9 +1506,7 @@ extern "C" int mcx_integrate_tsdf_batched(const mcx_batch* plan, float* d_tsdf, 
     B.tiled_vol = v0;
     const int64_t end = plan->blk_begin[v1];
     for (int64_t b0 = plan->blk_begin[v0]; b0 < end; b0 += kMaxRegions) {
-      B.first_block = b0;
-      B.end_block = std::min(end, b0 + kMaxRegions);
-      const dim3 grid(region_groups(B.end_block - b0, B.base.log2_run));
+      const dim3 grid = region_grid(B.base, b0, end);
       hipLaunchKernelGGL(integrate_tsdf_batched_kernel, grid, dim3(64), 0, s, B, d_tsdf, d_weight);
       MCX_HIP(hipGetLastError());
     }
@@ -1602,9 +1578,7 @@ extern "C" int mcx_integrate_tsdf_backward_batched(const mcx_batch* plan,
   B.from_init = 0;
   B.init_value = 0.0f;
   for (int64_t b0 = 0; b0 < plan->blocks; b0 += kMaxRegions) {
-    B.first_block = b0;
-    B.end_block = std::min(plan->blocks, b0 + kMaxRegions);
-    const dim3 grid(region_groups(B.end_block - b0, B.base.log2_run));
+    const dim3 grid = region_grid(B.base, b0, plan->blocks);
     hipLaunchKernelGGL(integrate_tsdf_backward_batched_kernel, grid, dim3(64), 0, s, B,
                        d_grad_tsdf, d_weight0, mg, mdt, acc);
     MCX_HIP(hipGetLastError());

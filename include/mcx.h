@@ -174,7 +174,7 @@ int64_t mcx_batch_voxels(const mcx_batch* plan);
  * all volumes and only launches kernels (capturable in a hipGraph).
  * mcx_integrate_tsdf_batched: from_init != 0 starts every voxel from
  *   (init_value, 0) without reading the arrays (else from their contents).
- *   K <= 512.  Workspace: mcx_integrate_workspace_size(W, H).
+ *   K <= 512.  Workspace: mcx_integrate_workspace_size_frames(W, H, nvol * K).
  * mcx_extract_diff_batched: mcx_extract_diff of every volume (float3
  *   positions, vertex ranges in d_vbase as mcx_extract_batched), keeping in
  *   the workspace what the backward needs.
@@ -294,11 +294,15 @@ int mcx_volume_init(void* d_vol, int X, int Y, int Z, void* stream);
  * intr (host): {fx, fy, cx, cy}.  d_poses: K x 12 floats, camera-to-world
  * {R row-major, t}.  d_depth: K x H x W uint16, metres = value * depth_scale,
  * 0 = no measurement.  Frames are fused in order, all K in one sweep of the
- * volume.  Workspace: mcx_integrate_workspace_size(W, H) bytes (per-pixel ray
- * factors and the frames' tile tables, recomputed by every call; W * H * 4
- * bytes are enough, and slower: no frame is passed over for what it hides).
- * Frames of W * H * 4 >= 2^31 bytes: MCX_ERR_UNSUPPORTED. */
+ * volume.  Workspace: per-pixel ray factors and the frames' tile tables,
+ * recomputed by every call.  mcx_integrate_workspace_size_frames(W, H, frames)
+ * bytes serve calls of up to `frames` frames (of all volumes together in the
+ * batched form; more than 512 of one volume are fused 512 at a time and need
+ * no more than that); mcx_integrate_workspace_size(W, H) bytes, about 32 MiB,
+ * any number.  W * H * 4 bytes are enough, and slower: no frame is passed over
+ * for what it hides.  Frames of W * H * 4 >= 2^31 bytes: MCX_ERR_UNSUPPORTED. */
 size_t mcx_integrate_workspace_size(int W, int H);
+size_t mcx_integrate_workspace_size_frames(int W, int H, int64_t frames);
 int mcx_integrate(void* d_vol, int X, int Y, int Z, float h, float trunc, int max_w,
                   const float* intr, const float* d_poses, const uint16_t* d_depth,
                   float depth_scale, int W, int H, int K, void* d_ws, size_t ws_bytes,
@@ -329,7 +333,7 @@ int mcx_integrate_ex(void* d_vol, int X, int Y, int Z, float h, float trunc_neg,
  *        t = clamp(sdf / trunc, -1, 1),
  *      with float depth frames (metres = value * depth_scale).
  * mcx_tsdf_init: every voxel = (tsdf_value, 0).
- * mcx_integrate_tsdf: fuse K frames (workspace: mcx_integrate_workspace_size).
+ * mcx_integrate_tsdf: fuse K frames (workspace: as mcx_integrate).
  * mcx_integrate_tsdf_backward: d_grad_depth (K x H x W) = dL/d(depth value)
  *   from d_grad_tsdf = dL/df after the call that fused these K frames into a
  *   volume whose weights before that call were d_weight0 (NULL: all 0).  Per

@@ -80,6 +80,7 @@ SIGNATURES = {
                                            _vp, _vp, _f32, _i32, _i32, _i32, _vp, _vp, _sz,
                                            _vp]),
     "mcx_integrate_workspace_size": (_sz, [_i32, _i32]),
+    "mcx_integrate_workspace_size_frames": (_sz, [_i32, _i32, _i64]),
     "mcx_integrate": (_i32, [_vp, _i32, _i32, _i32, _f32, _f32, _i32, _vp, _vp, _vp, _f32, _i32,
                              _i32, _i32, _vp, _sz, _vp]),
     "mcx_integrate_f32": (_i32, [_vp, _i32, _i32, _i32, _f32, _f32, _i32, _vp, _vp, _vp, _f32,

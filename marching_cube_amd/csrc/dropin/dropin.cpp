@@ -215,7 +215,7 @@ void _cu_voxel_volumetric_integration(cu_voxel v, float_camera_intrinsic ci,
                           c[0].z, c[1].z, c[2].z, ce.t.x, ce.t.y, ce.t.z};
   cu_array<float> dpose;
   dpose.upload(pose, 12);
-  cu_array<unsigned char> ws(mcx_integrate_workspace_size(size.x, size.y));
+  cu_array<unsigned char> ws(mcx_integrate_workspace_size_frames(size.x, size.y, 1));
   // the volume's two truncation distances: min_t behind the surface, max_t
   // in front of it (cu_kinect_fusion_v1.cu:455-463)
   check_mcx(mcx_integrate_ex(v.data, v.size.x, v.size.y, v.size.z, v.grid_s, v.min_t, v.max_t,

@@ -1102,18 +1102,19 @@ extern "C" int mcx_volume_init(void* d_vol, int X, int Y, int Z, void* stream) {
 
 size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Tile tables: bytes per frame, and of as many frames as 32 MiB hold, at least
-// one (a 640x480 frame takes 38 KB, so a sweep's 512 frames fit; a 320x240
-// frame 9.6 KB: 3,495, the frames of 218 volumes of a batch with 16 each).
+// Tile tables: bytes per frame, and of `frames` frames, but of no more than 32
+// MiB hold, at least one (a 640x480 frame takes 40.8 KB, so a sweep's 512 frames
+// fit; a 320x240 frame 10.2 KB: 3,276, the frames of 204 volumes of a batch with
+// 16 each).
 size_t tile_bytes(int W, int H) {
   const auto tiles = [&](int side) {
     return (size_t)((W + side - 1) / side) * ((H + side - 1) / side);
   };
   return (tiles(kTile) + tiles(kTile * kTiles1)) * sizeof(float2);
 }
-size_t tile_tables_bytes(int W, int H) {
+size_t tile_tables_bytes(int W, int H, int64_t frames) {
   const size_t per = tile_bytes(W, H), most = (size_t)32 << 20;
-  return per * std::max((size_t)1, most / std::max(per, (size_t)1));
+  return per * std::min((size_t)frames, std::max((size_t)1, most / std::max(per, (size_t)1)));
 }
 
 // The ray factors alone would do (they are what a call cannot run without);
@@ -1121,9 +1122,13 @@ size_t tile_tables_bytes(int W, int H) {
 size_t rayfac_bytes(int W, int H) {
   return (size_t)(W > 0 ? W : 0) * (size_t)(H > 0 ? H : 0) * sizeof(float);
 }
-extern "C" size_t mcx_integrate_workspace_size(int W, int H) {
+extern "C" size_t mcx_integrate_workspace_size_frames(int W, int H, int64_t frames) {
   const size_t rf = rayfac_bytes(W, H);
-  return rf ? al256(rf) + 256 + tile_tables_bytes(W, H) : 0;
+  return rf && frames >= 0 ? al256(rf) + 256 + tile_tables_bytes(W, H, frames) : 0;
+}
+
+extern "C" size_t mcx_integrate_workspace_size(int W, int H) {
+  return mcx_integrate_workspace_size_frames(W, H, INT64_MAX);
 }
 
 // The smaller truncation, the reciprocals, and whether everything lies where

@@ -74,8 +74,8 @@ def integrate(volume, intr, poses, depth, *, trunc=None, min_t=None, max_t=None,
     K, H, W = depth.shape
     poses = torch.as_tensor(poses, dtype=torch.float32).reshape(K, 12).to(vol.device).contiguous()
     lib = _lib()
-    ws = torch.empty(max(1, lib.mcx_integrate_workspace_size(W, H)), dtype=torch.uint8,
-                     device=vol.device)
+    ws = torch.empty(max(1, lib.mcx_integrate_workspace_size_frames(W, H, min(K, 512))),
+                     dtype=torch.uint8, device=vol.device)
     hi, hp = _host_f32(intr)
     _capi.check(lib.mcx_integrate_ex(_ptr(vol), X, Y, Z, float(h), float(min_t), float(max_t),
                                      int(max_w), hp, _ptr(poses), _ptr(depth.contiguous()), kind,

@@ -39,24 +39,26 @@ def tsdf_init(shape, device, value=1.0):
 
 
 class _Integrator:
-    """Launch helper with its own workspaces (ray factors, accumulators)."""
+    """Launch helper with the backward's workspace (the forward's is its call's)."""
 
     def __init__(self, shape, W, H, K, h, trunc, max_w, intr, device):
         self.Z, self.Y, self.X = (int(a) for a in shape)
         self.W, self.H, self.K = int(W), int(H), int(K)
         self.h, self.trunc, self.max_w = float(h), float(trunc), int(max_w)
         self.intr = _intr_arr(intr)
-        lib = _capi.load()
-        self.ws_f = torch.empty(max(4096, lib.mcx_integrate_workspace_size(W, H)),
-                                dtype=torch.uint8, device=device)
-        self.ws_b = torch.empty(max(4096, lib.mcx_integrate_tsdf_backward_workspace_size(W, H, K)),
-                                dtype=torch.uint8, device=device)
+        self.ws_b = torch.empty(
+            max(4096, _capi.load().mcx_integrate_tsdf_backward_workspace_size(W, H, K)),
+            dtype=torch.uint8, device=device)
 
     def forward(self, tsdf, w, poses, depth, depth_scale=1.0):
-        _capi.check(_capi.load().mcx_integrate_tsdf(
+        lib = _capi.load()
+        ws = torch.empty(max(4096, lib.mcx_integrate_workspace_size_frames(self.W, self.H,
+                                                                           min(self.K, 512))),
+                         dtype=torch.uint8, device=tsdf.device)
+        _capi.check(lib.mcx_integrate_tsdf(
             _ptr(tsdf), _ptr(w), self.X, self.Y, self.Z, self.h, self.trunc, self.max_w,
             self.intr, _ptr(poses), _ptr(depth), float(depth_scale), self.W, self.H, self.K,
-            _ptr(self.ws_f), self.ws_f.numel(), _stream_handle(tsdf.device)), "mcx_integrate_tsdf")
+            _ptr(ws), ws.numel(), _stream_handle(tsdf.device)), "mcx_integrate_tsdf")
 
     def backward(self, grad_tsdf, w0, poses, depth, grad_depth, depth_scale=1.0):
         _capi.check(_capi.load().mcx_integrate_tsdf_backward(
@@ -190,8 +192,8 @@ class FusionGraph:
         self.total = torch.zeros(1, dtype=torch.int64, device=self.dev)
         self.loss = torch.zeros(self.B, dtype=torch.float32, device=self.dev)
         self.maxabs = torch.zeros(1, dtype=torch.int32, device=self.dev)
-        self.ws_f = torch.empty(max(4096, lib.mcx_integrate_workspace_size(self.W, self.H)),
-                                dtype=torch.uint8, device=self.dev)
+        self.ws_f = torch.empty(max(4096, lib.mcx_integrate_workspace_size_frames(
+            self.W, self.H, self.B * self.K)), dtype=torch.uint8, device=self.dev)
         self.ws_b = torch.empty(max(4096, lib.mcx_integrate_tsdf_backward_batched_workspace_size(
             self.plan.handle, self.W, self.H, self.K)), dtype=torch.uint8, device=self.dev)
         # extraction workspace (every record kept: the backward needs them) and

@@ -246,17 +246,24 @@ size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 unsigned grid_for(int64_t n, int64_t per) { return (unsigned)((n + per - 1) / per); }
 
+// Byte offsets of the workspace's arrays, the table first.
+struct Layout {
+  uint64_t slots;
+  int64_t blocks;
+  size_t rep, rank, bsum, bytes;
+  explicit Layout(int64_t V)
+      : slots(table_slots(V)), blocks((V + kWeldBlock - 1) / kWeldBlock), rep(al256(slots * 4)),
+        rank(rep + al256((size_t)V * 4)), bsum(rank + al256((size_t)V * 4)),
+        bytes(bsum + al256((size_t)(blocks + 1) * 4)) {}
+};
+
 }  // namespace
 }  // namespace mcx
 
 using namespace mcx;
 
 extern "C" size_t mcx_weld_workspace_size(int64_t V) {
-  if (V < 0) return 0;
-  const uint64_t T = table_slots(V);
-  const int64_t nb = (V + kWeldBlock - 1) / kWeldBlock;
-  return al256(T * 8) + al256((T + 1) * 4) + 3 * al256((size_t)V * 4 + 4) +
-         al256((size_t)(nb + 1) * 4);
+  return V < 0 ? 0 : Layout(V).bytes;
 }
 
 extern "C" int mcx_weld(const int64_t* d_edge_key, const float* d_pos, int64_t stride_floats,
@@ -273,20 +280,17 @@ extern "C" int mcx_weld(const int64_t* d_edge_key, const float* d_pos, int64_t s
     return MCX_OK;
   }
   if (!d_edge_key || !d_pos || !d_upos || !d_indices) return MCX_ERR_ARG;
-  if (!d_ws || ws_bytes < mcx_weld_workspace_size(V)) return MCX_ERR_WORKSPACE;
-  const uint64_t T = table_slots(V);
-  const int64_t nb = (V + kWeldBlock - 1) / kWeldBlock;
+  const Layout L(V);
+  if (!d_ws || ws_bytes < L.bytes) return MCX_ERR_WORKSPACE;
+  const int64_t nb = L.blocks;
   char* b = static_cast<char*>(d_ws);
   uint32_t* table = reinterpret_cast<uint32_t*>(b);
-  b += al256(T * 4);
-  uint32_t* rep = reinterpret_cast<uint32_t*>(b);  // slots, then first occurrences
-  b += al256((size_t)V * 4);
-  uint32_t* rank = reinterpret_cast<uint32_t*>(b);
-  b += al256((size_t)V * 4);
-  uint32_t* bsum = reinterpret_cast<uint32_t*>(b);
-  int rc = fill_u32(table, kEmpty, (size_t)T, s);
+  uint32_t* rep = reinterpret_cast<uint32_t*>(b + L.rep);  // slots, then first occurrences
+  uint32_t* rank = reinterpret_cast<uint32_t*>(b + L.rank);
+  uint32_t* bsum = reinterpret_cast<uint32_t*>(b + L.bsum);
+  int rc = fill_u32(table, kEmpty, (size_t)L.slots, s);
   if (rc) return rc;
-  const uint32_t n = (uint32_t)V, mask = (uint32_t)(T - 1);
+  const uint32_t n = (uint32_t)V, mask = (uint32_t)(L.slots - 1);
   hipLaunchKernelGGL(weld_insert_kernel, dim3((unsigned)nb), dim3(kInsert), 0, s, d_edge_key, n, table,
                      mask, rep);
   MCX_HIP(hipGetLastError());

@@ -53,7 +53,8 @@ __device__ __forceinline__ void nearest(const float (&p)[N][3], int M, At at,
 }
 
 // Two vertex rows a thread, 256 apart (rows past the total or past cap:
-// gradient 0).  The targets of the volume of the workgroup's first vertex are
+// gradient 0; a wave of only such rows looks at no target: 2 M rows without a
+// vertex, 1024 targets, 9 us, and 348 where it did).  The targets of the volume of the workgroup's first vertex are
 // staged in LDS, one 16-byte read of all lanes for both rows; a wave with a
 // vertex of another volume (a workgroup spanning a boundary) reads targets from
 // memory.  Bound by the arithmetic (9 instructions a row and target) and by what
@@ -94,9 +95,11 @@ __global__ __launch_bounds__(256) void chamfer_vertex_kernel(const float* pos,
       p[r][2] = pos[3 * u + 2];
     }
   }
-  float best[kRows];
-  int j[kRows], b[kRows];
-  if (__all(same)) {
+  float best[kRows] = {};
+  int j[kRows] = {}, b[kRows] = {};
+  if (!__any(v[0] < live)) {
+    // no vertex: v[0] is the lower of a thread's rows
+  } else if (__all(same)) {
 #pragma unroll
     for (int r = 0; r < kRows; ++r) b[r] = b0;
     nearest(p, M, [&](int m) { return s_t[m]; }, best, j);

@@ -1629,11 +1629,12 @@ __global__ __launch_bounds__(kEmitThreads) void contrib_kernel(ExtractParams P, 
 
 // Backward BW2: dL/dv of every voxel = the sum, over the up to 8 cubes it
 // is corner k of (k = 0..7 in corner order), of the cube's contribution k.
-// A wave takes kGatherSpan consecutive voxels of one plane z.  The cubes they
-// are corners of lie in planes z - 1 and z and, per plane, in two in-plane
-// windows (rows y and y - 1: cube ids [q0 - 1, q0 + span) and the same minus
-// X), each within two consecutive tiles: 4 windows x 16 words of active-cube
-// masks, a word a lane, with its rank in its tile and the tile's first record.
+// A wave takes a window of kGatherSpan consecutive voxels of one plane z, or one
+// SPLIT-th of it.  The cubes they are corners of lie in planes z - 1 and z and,
+// per plane, in two runs of cube ids (rows y and y - 1: [q0 - 1, q0 + 512) and
+// the same minus X), each within two consecutive tiles: 4 runs x 16 words of
+// active-cube masks, a word a lane, with its rank in its tile and the tile's
+// first record.
 // No LDS and no barrier.  If no cube is active (most spans), the span is
 // zeroed.  Else the wave goes through it by 64 voxels: the cubes that have
 // them as corner k are 64 consecutive cube ids, so which of them are active is
@@ -1648,8 +1649,8 @@ __global__ __launch_bounds__(kEmitThreads) void contrib_kernel(ExtractParams P, 
 // (bumps) 62 us, a batch of 64 volumes of 64-192 a side 166 us; with a workgroup
 // for 1024 voxels, their masks in LDS behind barriers and the active (voxel,
 // corner) pairs of a wave packed through LDS, 67 and 232.
-constexpr int kGatherSpan = 512;  // voxels per wave, four waves a workgroup
-constexpr int kGatherAhead = 4;   // ... 64 at a time, whose reads are in flight together
+constexpr int kGatherSpan = 512;  // voxels of a window, four waves a workgroup
+constexpr int kGatherAhead = 4;   // at most so many of its 64s have reads in flight together
 
 __device__ __forceinline__ uint64_t readlane64(uint64_t v, int lane) {
   const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)v, lane);
@@ -1661,9 +1662,11 @@ __device__ __forceinline__ uint64_t readlane64(uint64_t v, int lane) {
 // [gblk_begin, next) holds it, and writes that volume's part of the
 // concatenated gradient (from vox_begin).  With maxg, the largest |dL/dv| of
 // the launch goes there as float bits (atomicMax; order-independent).
-template <bool BATCH>
+template <bool BATCH, int SPLIT>
 __global__ __launch_bounds__(256) void gather_kernel(ExtractParams P, const float* contrib,
                                                      float* gvol, uint32_t* maxg) {
+  constexpr int kGroups = kGatherSpan / 64 / SPLIT;  // 64s of a wave
+  constexpr int kAhead = kGroups < kGatherAhead ? kGroups : kGatherAhead;
   int vi = 0;
   const int64_t gblk = P.first_block + blockIdx.x;
   int64_t blk = gblk;
@@ -1677,12 +1680,14 @@ __global__ __launch_bounds__(256) void gather_kernel(ExtractParams P, const floa
   const uint32_t XY = (uint32_t)X * (uint32_t)Y;  // < 2^30 (plane_ok)
   const uint32_t per_plane = (XY + kGatherSpan - 1) / kGatherSpan;
   const int lane = threadIdx.x & 63;
-  // units: at most N / 512 + Z, below 2^31 for any volume that fits in memory
+  // windows: at most N / 512 + Z, below 2^31 for any volume that fits in memory
   const uint32_t unit =
       (uint32_t)blk * 4 + (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int z = (int)(unit / per_plane);
+  const uint32_t window = unit / SPLIT;
+  const int z = (int)(window / per_plane);
   if (z >= Z) return;
-  const int q0 = (int)(unit - (uint32_t)z * per_plane) * kGatherSpan;
+  const int q0 = (int)(window - (uint32_t)z * per_plane) * kGatherSpan;
+  const int cb = (int)(unit % SPLIT) * kGroups;  // the wave's first 64
   // lane 16 d + 8 slot + word, d = 2 dz + dy (cube ids below 0 are never
   // looked up)
   const int first[2] = {max(q0 - 1, 0) >> 9, max(q0 - 1 - X, 0) >> 9};  // tiles
@@ -1704,8 +1709,9 @@ __global__ __launch_bounds__(256) void gather_kernel(ExtractParams P, const floa
     // sums below would all be empty), and it raises no maximum
     const uint32_t g = none ? 0x7fc00000u : 0u;
 #pragma unroll
-    for (int j = 0; j < kGatherSpan; j += 256) {
-      const uint32_t q = (uint32_t)(q0 + j + 4 * lane);
+    for (int j = 0; j < 64 * kGroups; j += 256) {
+      const uint32_t q = (uint32_t)(q0 + 64 * cb + j + 4 * lane);
+      if (kGroups < 4 && lane >= 16 * kGroups) break;
       if (q + 4 <= XY) {
         *reinterpret_cast<u32x4a4*>(gz + q) = u32x4a4{g, g, g, g};
       } else {
@@ -1740,10 +1746,10 @@ __global__ __launch_bounds__(256) void gather_kernel(ExtractParams P, const floa
     words |= s0[d] >= 0 ? 3ull << lane0[d] : ~0ull;
   }
 #pragma unroll 1
-  for (int c0 = 0; c0 < kGatherSpan / 64; c0 += kGatherAhead) {
-    float val[kGatherAhead][8] = {};
+  for (int c0 = cb; c0 < cb + kGroups; c0 += kAhead) {
+    float val[kAhead][8] = {};
 #pragma unroll
-    for (int u = 0; u < kGatherAhead; ++u) {
+    for (int u = 0; u < kAhead; ++u) {
       const int c = c0 + u;
       if ((active & (s0[1] >= 0 ? words << c : words)) == 0) continue;
 #pragma unroll
@@ -1778,7 +1784,7 @@ __global__ __launch_bounds__(256) void gather_kernel(ExtractParams P, const floa
       }
     }
 #pragma unroll
-    for (int u = 0; u < kGatherAhead; ++u) {
+    for (int u = 0; u < kAhead; ++u) {
       const uint32_t q = (uint32_t)(q0 + 64 * (c0 + u) + lane);
       if (q < XY) {
         float g = 0.0f;
@@ -1851,19 +1857,35 @@ int launch_contrib(const ExtractParams& P, const float* gpos, float* contrib, hi
   return MCX_OK;
 }
 
-// Its second, over nb workgroups, in launches of at most kMaxLaunchBlocks
-// (each given its first workgroup).
-int64_t gather_blocks(int X, int Y, int Z) {
-  return (((int64_t)X * Y + kGatherSpan - 1) / kGatherSpan * Z + 3) / 4;
+// Its second: how many waves share a window, the workgroups of a volume, and the
+// launches over nb workgroups, at most kMaxLaunchBlocks each (given its first
+// workgroup).
+//   Below 2^23 voxels a wave per window leaves SIMDs with few waves or none, each
+// going through eight 64s: two waves share a window there and four below 2^21
+// (the reading of its masks is repeated), 64 waves per CU either way.  The
+// backward with 1, 2 and 4: 64^3 23.5, 17.2 and 14.2 us; 128^3 24.7, 19.5, 19.2;
+// 200^3 32.1, 27.8, 29.5; batches of 16 64^3 44.9, 38.6, 45.2 and of 8 128^3 65.5,
+// 70.2, 93.7.
+int gather_split(double voxels) {
+  return voxels <= (double)(1 << 21) ? 4 : voxels <= (double)(1 << 23) ? 2 : 1;
+}
+
+int64_t gather_blocks(int X, int Y, int Z, int split) {
+  return (((int64_t)X * Y + kGatherSpan - 1) / kGatherSpan * Z * split + 3) / 4;
 }
 
 template <bool BATCH>
-int launch_gather(ExtractParams P, int64_t nb, const float* contrib, float* gvol,
+int launch_gather(ExtractParams P, int64_t nb, int split, const float* contrib, float* gvol,
                   uint32_t* maxg, hipStream_t s) {
   for (int64_t b0 = 0; b0 < nb; b0 += kMaxLaunchBlocks) {
     P.first_block = b0;
-    hipLaunchKernelGGL(gather_kernel<BATCH>, dim3((unsigned)std::min(kMaxLaunchBlocks, nb - b0)),
-                       dim3(256), 0, s, P, contrib, gvol, maxg);
+    const dim3 grid((unsigned)std::min(kMaxLaunchBlocks, nb - b0));
+    if (split == 1)
+      hipLaunchKernelGGL((gather_kernel<BATCH, 1>), grid, dim3(256), 0, s, P, contrib, gvol, maxg);
+    else if (split == 2)
+      hipLaunchKernelGGL((gather_kernel<BATCH, 2>), grid, dim3(256), 0, s, P, contrib, gvol, maxg);
+    else
+      hipLaunchKernelGGL((gather_kernel<BATCH, 4>), grid, dim3(256), 0, s, P, contrib, gvol, maxg);
     MCX_HIP(hipGetLastError());
   }
   return MCX_OK;
@@ -2307,9 +2329,10 @@ int backward_impl(const float* d_vol, int X, int Y, int Z, float h, const float*
   P.grad_rows = INT64_MAX;  // the caller's rows are the forward's vertices
   rc = launch_contrib<false>(P, d_grad_pos, contrib, s);
   if (rc) return rc;
-  const int64_t g2 = gather_blocks(X, Y, Z);
+  const int split = gather_split((double)N);
+  const int64_t g2 = gather_blocks(X, Y, Z, split);
   if (g2 >= ((int64_t)1 << 31)) return MCX_ERR_UNSUPPORTED;
-  return launch_gather<false>(P, g2, contrib, d_grad_vol, nullptr, s);
+  return launch_gather<false>(P, g2, split, contrib, d_grad_vol, nullptr, s);
 }
 }  // namespace
 
@@ -2350,6 +2373,7 @@ extern "C" int mcx_batch_create(mcx_batch** out, int nvol, const int* dims_xyz, 
   for (int b = 0; b < nvol; ++b)
     all += (double)dims_xyz[3 * b] * dims_xyz[3 * b + 1] * dims_xyz[3 * b + 2];
   const int bricks = all >= (double)(1 << 24) ? 4 : 1;
+  const int split = gather_split(all);
   for (int b = 0; b < nvol; ++b) {
     const int X = dims_xyz[3 * b], Y = dims_xyz[3 * b + 1], Z = dims_xyz[3 * b + 2];
     if (X < 1 || Y < 1 || Z < 1 || !d_vols[b]) return MCX_ERR_ARG;
@@ -2362,7 +2386,7 @@ extern "C" int mcx_batch_create(mcx_batch** out, int nvol, const int* dims_xyz, 
     blk_begin[b] = blocks;
     voxels += nv;
     blocks += (int64_t)rx * ry * rz;
-    gblocks += gather_blocks(X, Y, Z);
+    gblocks += gather_blocks(X, Y, Z, split);
     const int64_t nt = tiles_of(X, Y, Z);
     if (nt > 0) {
       // one column per in-plane range, slabs of the plan's planes per column
@@ -2394,6 +2418,7 @@ extern "C" int mcx_batch_create(mcx_batch** out, int nvol, const int* dims_xyz, 
   p->blk_begin = std::move(blk_begin);
   p->bricks = bricks;
   p->gather_blocks = gblocks;
+  p->gather_split = split;
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&p->d_vols), sizeof(VolDesc) * nvol);
   if (e == hipSuccess)
     e = hipMalloc(reinterpret_cast<void**>(&p->d_bvol), sizeof(BatchVol) * nvol);
@@ -2571,7 +2596,7 @@ extern "C" int mcx_extract_backward_batched_rows(const mcx_batch* plan, const fl
   P.grad_rows = rows;
   rc = launch_contrib<true>(P, d_grad_pos, contrib, s);
   if (rc) return rc;
-  return launch_gather<true>(P, plan->gather_blocks, contrib, d_grad_vol, d_maxabs, s);
+  return launch_gather<true>(P, plan->gather_blocks, plan->gather_split, contrib, d_grad_vol, d_maxabs, s);
 }
 
 // ---- launch-shape tunables (no counterpart in the reference) ------------

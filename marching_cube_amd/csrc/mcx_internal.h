@@ -352,6 +352,7 @@ struct mcx_batch {
   std::vector<int64_t> blk_begin;  // each volume's first one, then their number
   int bricks = 1;           // bricks above one another that an integration wave takes
   int64_t gather_blocks = 0;
+  int gather_split = 1;     // waves that share a window of the batched gather
   mcx::VolDesc* d_vols = nullptr;
   mcx::Column* d_cols = nullptr;
   mcx::BatchVol* d_bvol = nullptr;

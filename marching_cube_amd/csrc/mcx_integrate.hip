@@ -228,13 +228,6 @@ constexpr int kRegionX = 4 * kBrick;  // a workgroup's four bricks lie side by s
 // larger ones from the 32-pixel tiles; beyond that nothing is known of the
 // depth.
 constexpr int kSkip = 1, kFast = 2, kInside = 4, kFree = 8;
-// The largest of |a|, |b| and |c| (fmaxf makes every operand a quiet NaN first,
-// an instruction each).
-__device__ __forceinline__ float max3_abs(float a, float b, float c) {
-  float m;
-  asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(m) : "v"(a), "v"(b), "v"(c));
-  return m;
-}
 template <int NZ>
 __device__ int test_brick(const IntegrateParams& P, int x0, int y0, int z0, int k) {
   const float* R = P.poses + 12 * k;
@@ -247,8 +240,9 @@ __device__ int test_brick(const IntegrateParams& P, int x0, int y0, int z0, int 
   const float r0 = R[0], r1 = R[1], r2 = R[2], r3 = R[3], r4 = R[4], r5 = R[5], r6 = R[6],
               r7 = R[7], r8 = R[8];
   const float dx = px - R[9], dy = py - R[10], dz = pz - R[11];
-  const float m = fmaxf(
-      max3_abs(max3_abs(max3_abs(max3_abs(1.0f, r0, r1), r2, r3), r4, r5), r6, r7), fabsf(r8));
+  const float m = fmaxf(fmaxf(fmaxf(fmaxf(1.0f, fabsf(r0)), fmaxf(fabsf(r1), fabsf(r2))),
+                              fmaxf(fmaxf(fabsf(r3), fabsf(r4)), fmaxf(fabsf(r5), fabsf(r6)))),
+                        fmaxf(fabsf(r7), fabsf(r8)));
   const float sum =
       (fabsf(dx) + fabsf(dy) + fabsf(dz) + (px + hx) + (py + hy) + (pz + hz)) * m;
   const float d = 8e-7f * sum;

@@ -44,3 +44,38 @@ def test_live_fusions_hold_no_forward_workspace(dev):
     assert torch.cuda.memory_allocated(dev) - before <= 8 * (128 << 10)
     sum(t.sum() for t in live).backward()
     assert torch.isfinite(depth.grad).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("offset", [0, 4, 8, 16])
+@pytest.mark.parametrize("W", [64, 72, 70])
+def test_unaligned_workspace(dev, W, offset):
+    """Ray factors are written 16 bytes at a time only where rows and workspace
+    allow it."""
+    import ctypes
+
+    import numpy as np
+    import torch
+
+    from marching_cube_amd.mesh import _ptr, _stream_handle
+    from oracle import oracle as O
+    from test_integrate_bricks_gpu import H0, random_depth, random_poses
+    print(f"[case] workspace at {offset} bytes, frames {W} wide", flush=True)
+    rng = np.random.default_rng(W + offset)
+    dims, K, H = (70, 67, 61), 9, 40
+    X, Y, Z = dims
+    poses, depth = random_poses(rng, K, dims), random_depth(rng, K, H, W, True)
+    intr = np.array([0.9 * W, 0.8 * W, 0.5 * W - 0.5, 0.45 * H], np.float32)
+    ref = np.zeros((Z, Y, X), np.uint32)
+    O.integrate_ex(ref, H0, 0.07, 0.05, 8, intr, poses, depth)
+    lib = _capi.load()
+    n = lib.mcx_integrate_workspace_size_frames(W, H, K)
+    ws = torch.full((n + 4096,), 0x5a, dtype=torch.uint8, device=dev)
+    vol = torch.zeros((Z, Y, X), dtype=torch.int32, device=dev)
+    d_depth, d_poses = torch.from_numpy(depth).to(dev), torch.from_numpy(poses).to(dev)
+    _capi.check(lib.mcx_integrate_ex(
+        _ptr(vol), X, Y, Z, H0, 0.07, 0.05, 8, (ctypes.c_float * 4)(*intr), _ptr(d_poses),
+        _ptr(d_depth), _capi.DEPTH_F32, 0.001, W, H, K, ctypes.c_void_p(ws.data_ptr() + offset), n,
+        _stream_handle(dev)), "mcx_integrate_ex")
+    assert vol.cpu().numpy().view(np.uint32).tobytes() == ref.tobytes()
+    assert (ws[:offset] == 0x5a).all() and (ws[offset + n:] == 0x5a).all()

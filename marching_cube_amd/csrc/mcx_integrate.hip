@@ -826,7 +826,10 @@ __device__ __forceinline__ double grad_scale(uint32_t maxg_bits, float max_dtdd)
 // contribution g * df/dt_i * dt_i/dd goes to the observed pixel of acc (K
 // frames of W x H) as an int64 fixed-point atomic add (integer sums do not
 // depend on the order).  Bricks without a gradient (most: only the corners of
-// active cubes carry one) are left after reading it.
+// active cubes carry one) are left after reading it, and lanes without one look
+// at no pixel: with a gradient on one voxel in 37, 16 frames of 320x240 of eight
+// 40^3 volumes each 151 -> 104 us (110 with a wave for 64 voxels of a row whose
+// lanes left by themselves), of 64 128^3 volumes 3275 -> 2438.
 template <int NZ>
 __device__ __forceinline__ void backward_brick(const IntegrateParams& P, const Brick<NZ>& B,
                                                const float* __restrict__ g,
@@ -841,6 +844,9 @@ __device__ __forceinline__ void backward_brick(const IntegrateParams& P, const B
 #pragma unroll
   for (int j = 0; j < NZ; ++j) any |= gi[j] != 0.0f;
   if (!__any(any)) return;
+  Brick<NZ> A = B;  // with the lanes that carry a gradient
+  A.inside = any;
+  const int drop = __all(any) ? 0 : kInside;
   const double scale = grad_scale(*maxg, max_dtdd);
   const int M = P.max_w;
   int nobs[NZ] = {}, o[NZ] = {}, w0[NZ] = {};
@@ -852,7 +858,7 @@ __device__ __forceinline__ void backward_brick(const IntegrateParams& P, const B
   Frames<NZ> F(P, B.x0, B.y0, B.z0);
   F.each([&](int k, int cls) {
     observe_brick<float>(
-        P, B, k, cls, [&](auto, int j, float, float, uint32_t) { ++nobs[j]; },
+        P, A, k, cls & ~drop, [&](auto, int j, float, float, uint32_t) { ++nobs[j]; },
         [&](int j) { ++nobs[j]; });
   });
   const double cap_a = (double)M / (double)(M + 1);
@@ -887,7 +893,7 @@ __device__ __forceinline__ void backward_brick(const IntegrateParams& P, const B
       }
     };
     // where t is known to be +1 the slope is 0: the observation only counts
-    observe_brick<float>(P, B, k, cls, add, [&](int j) { ++o[j]; });
+    observe_brick<float>(P, A, k, cls & ~drop, add, [&](int j) { ++o[j]; });
   });
 }
 

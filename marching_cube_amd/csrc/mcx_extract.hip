@@ -2373,6 +2373,8 @@ extern "C" int mcx_batch_create(mcx_batch** out, int nvol, const int* dims_xyz, 
   for (int b = 0; b < nvol; ++b)
     all += (double)dims_xyz[3 * b] * dims_xyz[3 * b + 1] * dims_xyz[3 * b + 2];
   const int bricks = all >= (double)(1 << 24) ? 4 : 1;
+  // ... one plane high up to 2^17 voxels (brick_planes)
+  const int nz = all <= (double)(1 << 17) ? 1 : 4;
   const int split = gather_split(all);
   for (int b = 0; b < nvol; ++b) {
     const int X = dims_xyz[3 * b], Y = dims_xyz[3 * b + 1], Z = dims_xyz[3 * b + 2];
@@ -2380,7 +2382,7 @@ extern "C" int mcx_batch_create(mcx_batch** out, int nvol, const int* dims_xyz, 
     if (!size_ok(X, Y, Z)) return MCX_ERR_UNSUPPORTED;
     vols[b] = make_vol(d_vols[b], X, Y, Z, h[b], nullptr, tb);
     const int64_t nv = (int64_t)X * Y * Z;
-    const int rx = (X + 31) / 32, ry = (Y + 7) / 8, rz = (Z + 4 * bricks - 1) / (4 * bricks);
+    const int rx = (X + 31) / 32, ry = (Y + 7) / 8, rz = (Z + nz * bricks - 1) / (nz * bricks);
     bvol[b] = BatchVol{X, Y, Z, h[b], voxels, blocks, gblocks, FastDiv((uint32_t)rx),
                        FastDiv((uint32_t)ry)};
     blk_begin[b] = blocks;
@@ -2417,6 +2419,7 @@ extern "C" int mcx_batch_create(mcx_batch** out, int nvol, const int* dims_xyz, 
   p->blocks = blk_begin[nvol] = blocks;
   p->blk_begin = std::move(blk_begin);
   p->bricks = bricks;
+  p->brick_planes = nz;
   p->gather_blocks = gblocks;
   p->gather_split = split;
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&p->d_vols), sizeof(VolDesc) * nvol);

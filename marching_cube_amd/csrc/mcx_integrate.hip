@@ -192,7 +192,7 @@ __device__ __forceinline__ float frame_rayfac(const IntegrateParams& P, uint32_t
 }
 
 // ---- bricks ---------------------------------------------------------------
-// A wave's 8 x 8 x NZ voxels (NZ = 4, or 1 in the backward of small volumes):
+// A wave's 8 x 8 x NZ voxels (NZ = 4, or 1 in small volumes):
 // compact, so that its image is a few tiles (256 voxels in a row of x, the
 // former split, cover a line of some 300 pixels) and one test serves 256
 // voxels; a lane's NZ voxels share x, y and so two of the three products of
@@ -610,23 +610,23 @@ __device__ __forceinline__ float truncated(const IntegrateParams& P, float sdf) 
 // update_voxel).  A brick is read when its first frame comes up and a voxel is
 // written only if some frame updated it: outside every frustum and behind
 // every surface it costs no memory traffic.
-template <typename DT>
+template <typename DT, int NZ>
 __global__ __launch_bounds__(64) void integrate_kernel(IntegrateParams P, int bricks) {
   int wave, x0, y0, z0;
   const int64_t blk = region_of(P, &wave);
-  if (blk < 0 || !brick_origin<true>(P, (uint32_t)blk, wave, kBrickZ * bricks, &x0, &y0, &z0))
+  if (blk < 0 || !brick_origin<true>(P, (uint32_t)blk, wave, NZ * bricks, &x0, &y0, &z0))
     return;
   const int64_t XY = (int64_t)P.X * P.Y;
-  for_bricks<kBrickZ>(P, x0, y0, z0, bricks, [&](const Brick<kBrickZ>& B, Frames<kBrickZ>& F) {
+  for_bricks<NZ>(P, x0, y0, z0, bricks, [&](const Brick<NZ>& B, Frames<NZ>& F) {
     uint32_t* const v = P.vol + B.first(P);
-    uint32_t cur[kBrickZ] = {};
+    uint32_t cur[NZ] = {};
     uint32_t changed = 0;
     bool have = false;
     F.each([&](int k, int cls) {
       if (!have) {
         have = true;
 #pragma unroll
-        for (int j = 0; j < kBrickZ; ++j)
+        for (int j = 0; j < NZ; ++j)
           if (B.inside && j < B.nz) cur[j] = v[j * XY];
       }
       observe_brick<DT>(
@@ -641,7 +641,7 @@ __global__ __launch_bounds__(64) void integrate_kernel(IntegrateParams P, int br
           });
     });
 #pragma unroll
-    for (int j = 0; j < kBrickZ; ++j)
+    for (int j = 0; j < NZ; ++j)
       if (changed & (1u << j)) v[j * XY] = cur[j];
   });
 }
@@ -716,11 +716,11 @@ __device__ __forceinline__ float observation_slope(const IntegrateParams& P, flo
 
 // fp32 update of a brick by frames [0, K), from (f, w) as given.  Returns the
 // voxels (bits j) that some frame updated.
-template <typename LOAD>
+template <int NZ, typename LOAD>
 __device__ __forceinline__ uint32_t integrate_tsdf_brick(const IntegrateParams& P,
-                                                         const Brick<kBrickZ>& B,
-                                                         Frames<kBrickZ>& F, float (&f)[kBrickZ],
-                                                         int (&w)[kBrickZ], LOAD&& load) {
+                                                         const Brick<NZ>& B, Frames<NZ>& F,
+                                                         float (&f)[NZ], int (&w)[NZ],
+                                                         LOAD&& load) {
   uint32_t changed = 0;
   bool have = false;
   F.each([&](int k, int cls) {
@@ -744,36 +744,37 @@ __device__ __forceinline__ uint32_t integrate_tsdf_brick(const IntegrateParams& 
 
 // The brick's voxels are read when the first frame that may observe it comes
 // up; only updated voxels are written.
+template <int NZ>
 __device__ __forceinline__ void integrate_tsdf_stored(const IntegrateParams& P,
-                                                      const Brick<kBrickZ>& B,
-                                                      Frames<kBrickZ>& F, float* tsdf,
-                                                      int32_t* wvol) {
+                                                      const Brick<NZ>& B, Frames<NZ>& F,
+                                                      float* tsdf, int32_t* wvol) {
   const int64_t i = B.first(P), XY = (int64_t)P.X * P.Y;
-  float f[kBrickZ] = {};
-  int w[kBrickZ] = {};
+  float f[NZ] = {};
+  int w[NZ] = {};
   const uint32_t changed = integrate_tsdf_brick(P, B, F, f, w, [&]() {
 #pragma unroll
-    for (int j = 0; j < kBrickZ; ++j)
+    for (int j = 0; j < NZ; ++j)
       if (B.inside && j < B.nz) {
         f[j] = tsdf[i + j * XY];
         w[j] = wvol[i + j * XY];
       }
   });
 #pragma unroll
-  for (int j = 0; j < kBrickZ; ++j)
+  for (int j = 0; j < NZ; ++j)
     if (changed & (1u << j)) {
       tsdf[i + j * XY] = f[j];
       wvol[i + j * XY] = w[j];
     }
 }
 
+template <int NZ>
 __global__ __launch_bounds__(64) void integrate_tsdf_kernel(IntegrateParams P, int bricks,
                                                              float* tsdf, int32_t* wvol) {
   int wave, x0, y0, z0;
   const int64_t blk = region_of(P, &wave);
-  if (blk < 0 || !brick_origin<true>(P, (uint32_t)blk, wave, kBrickZ * bricks, &x0, &y0, &z0))
+  if (blk < 0 || !brick_origin<true>(P, (uint32_t)blk, wave, NZ * bricks, &x0, &y0, &z0))
     return;
-  for_bricks<kBrickZ>(P, x0, y0, z0, bricks, [&](const Brick<kBrickZ>& B, Frames<kBrickZ>& F) {
+  for_bricks<NZ>(P, x0, y0, z0, bricks, [&](const Brick<NZ>& B, Frames<NZ>& F) {
     integrate_tsdf_stored(P, B, F, tsdf, wvol);
   });
 }
@@ -922,6 +923,7 @@ struct BatchIntegrateParams {
 
 // This workgroup's volume (binary search over the block ranges), its launch
 // parameters and this wave's brick; false past the volume's edge.
+template <int NZ>
 __device__ __forceinline__ bool batch_setup(const BatchIntegrateParams& B, IntegrateParams& P,
                                             int64_t* vox_begin, int* vol, int* x0, int* y0,
                                             int* z0) {
@@ -944,29 +946,30 @@ __device__ __forceinline__ bool batch_setup(const BatchIntegrateParams& B, Integ
   P.tiles = B.base.tiles + (int64_t)(vi - B.tiled_vol) * P.K * (P.TX * P.TY + P.TX1 * P.TY1);
   *vox_begin = V.vox_begin;
   *vol = vi;
-  return brick_origin<true>(P, (uint32_t)(blk - V.blk_begin), wave, kBrickZ * B.bricks, x0, y0, z0);
+  return brick_origin<true>(P, (uint32_t)(blk - V.blk_begin), wave, NZ * B.bricks, x0, y0, z0);
 }
 
+template <int NZ>
 __global__ __launch_bounds__(64) void integrate_tsdf_batched_kernel(BatchIntegrateParams B,
                                                                      float* tsdf, int32_t* wvol) {
   IntegrateParams P;
   int64_t vb;
   int vi, x0, y0, z0;
-  if (!batch_setup(B, P, &vb, &vi, &x0, &y0, &z0)) return;
-  for_bricks<kBrickZ>(P, x0, y0, z0, B.bricks, [&](const Brick<kBrickZ>& K, Frames<kBrickZ>& F) {
+  if (!batch_setup<NZ>(B, P, &vb, &vi, &x0, &y0, &z0)) return;
+  for_bricks<NZ>(P, x0, y0, z0, B.bricks, [&](const Brick<NZ>& K, Frames<NZ>& F) {
     if (!B.from_init) {
       integrate_tsdf_stored(P, K, F, tsdf + vb, wvol + vb);
       return;
     }
     // every voxel is written: the start value where no frame observes it
-    float f[kBrickZ];
-    int w[kBrickZ] = {};
+    float f[NZ];
+    int w[NZ] = {};
 #pragma unroll
-    for (int j = 0; j < kBrickZ; ++j) f[j] = B.init_value;
+    for (int j = 0; j < NZ; ++j) f[j] = B.init_value;
     integrate_tsdf_brick(P, K, F, f, w, []() {});
     const int64_t i = vb + K.first(P), XY = (int64_t)P.X * P.Y;
 #pragma unroll
-    for (int j = 0; j < kBrickZ; ++j)
+    for (int j = 0; j < NZ; ++j)
       if (K.inside && j < K.nz) {
         tsdf[i + j * XY] = f[j];
         wvol[i + j * XY] = w[j];
@@ -974,15 +977,16 @@ __global__ __launch_bounds__(64) void integrate_tsdf_batched_kernel(BatchIntegra
   });
 }
 
+template <int NZ>
 __global__ __launch_bounds__(64) void integrate_tsdf_backward_batched_kernel(
     BatchIntegrateParams B, const float* __restrict__ g, const int32_t* __restrict__ w0vol,
     const uint32_t* maxg, float max_dtdd, unsigned long long* acc) {
   IntegrateParams P;
   int64_t vb;
   int vi, x0, y0, z0;
-  if (!batch_setup(B, P, &vb, &vi, &x0, &y0, &z0)) return;
-  for (int b = 0; b < B.bricks && z0 < P.Z; ++b, z0 += kBrickZ)
-    backward_brick(P, Brick<kBrickZ>(P, x0, y0, z0), g + vb, w0vol ? w0vol + vb : nullptr, maxg,
+  if (!batch_setup<NZ>(B, P, &vb, &vi, &x0, &y0, &z0)) return;
+  for (int b = 0; b < B.bricks && z0 < P.Z; ++b, z0 += NZ)
+    backward_brick(P, Brick<NZ>(P, x0, y0, z0), g + vb, w0vol ? w0vol + vb : nullptr, maxg,
                    max_dtdd, acc + (int64_t)vi * P.K * P.W * P.H);
 }
 
@@ -1212,16 +1216,16 @@ int64_t regions(int X, int Y, int Z, int zstep) {
          ((Z + zstep - 1) / zstep);
 }
 
-// The ray factors, and the tile tables of as many of `frames` frames (from
-// `depth`) as [tables, end) holds; P.tiled says how many.
+// The ray factors, and if wanted the tile tables of as many of `frames` frames
+// (from `depth`) as [tables, end) holds; P.tiled says how many.
 template <typename DT>
-int frame_tiles(IntegrateParams& P, const DT* depth, int64_t frames, char* tables, char* end,
-                hipStream_t s) {
+int frame_tiles(IntegrateParams& P, bool tables_wanted, const DT* depth, int64_t frames,
+                char* tables, char* end, hipStream_t s) {
   tables = reinterpret_cast<char*>(al256(reinterpret_cast<uintptr_t>(tables)));
   const size_t per = tile_bytes(P.W, P.H);
   const int64_t room = tables < end ? (int64_t)((size_t)(end - tables) / per) : 0;
   P.tiles = reinterpret_cast<const float2*>(tables);
-  P.tiled = (int)std::min(frames, room);
+  P.tiled = tables_wanted ? (int)std::min(frames, room) : 0;
   const int gx = (P.TX + 7) / 8;
   // about 16 waves per SIMD in all; each takes every gz-th frame
   const int64_t plane = (int64_t)gx * P.TY1;
@@ -1264,6 +1268,29 @@ int bricks_per_wave(int64_t voxels, int K) {
   return n;
 }
 
+// Planes of a brick.  Up to 2^18 voxels four leave one wave a SIMD or fewer, each
+// going through the frames alone; one plane gives four times the waves and each a
+// quarter of the work a frame.  Above 2^17 that pays while the frames are few or
+// stay in a CU's vector cache (2^15 pixels of 2 bytes): more waves read each
+// frame.  Four planes against one, without tile tables: 32^3, 16 VGA frames 28 and
+// 17 us, 300 429 and 208; 48^3 31 and 23, 452 and 308; 64^3, 16 of 320x240 25 and
+// 20, 300 VGA 432 and 503, 600 of 160x120 710 and 423; 80^3, 16 VGA 46 and 55.
+int brick_planes(int64_t voxels, int K, int64_t pixels) {
+  if (voxels > (1 << 18)) return kBrickZ;
+  return voxels <= (1 << 17) || K <= 32 || pixels <= (1 << 15) ? 1 : kBrickZ;
+}
+
+// Whether the frames' tile tables give back the reading of every frame: a frame's
+// table costs its pixels, and saves part of the observations, as many as there are
+// voxels (`each`: of one volume of a batch); nothing where the sweep is as short
+// as the table's kernel.  With and without, us: 64^3, 4 VGA frames 16.4 and 13.3,
+// 300 471 and 432; 80^3, 4 17.0 and 15.7, 16 42.7 and 46.2; 96^3, 4 of 1920x1080
+// 41.9 and 35.7; 128^3, 4 VGA 23.5 and 25.8, 4 of 1920x1080 45.9 and 53.4, one of
+// 3840x2160 41.6 and 39.5; 160^3, one VGA 15.0 and 16.5.
+bool tables_pay(int64_t voxels, int64_t each, int K, int64_t pixels) {
+  return voxels > (1 << 18) && each >= pixels && (K >= 8 || voxels >= (1 << 20));
+}
+
 template <typename DT>
 int integrate_impl(void* d_vol, int X, int Y, int Z, float h, float trunc_neg, float trunc,
                    int max_w, const float* intr, const float* d_poses, const DT* d_depth,
@@ -1281,22 +1308,27 @@ int integrate_impl(void* d_vol, int X, int Y, int Z, float h, float trunc_neg, f
   if (rc) return rc;
   P.vol = static_cast<uint32_t*>(d_vol);
   set_trunc_neg(P, trunc_neg);
+  const int64_t voxels = (int64_t)X * Y * Z, pixels = (int64_t)W * H;
   for (int k0 = 0; k0 < K; k0 += kFramesPerPass) {
     P.K = K - k0 < kFramesPerPass ? K - k0 : kFramesPerPass;
     P.poses = d_poses + (int64_t)12 * k0;
-    P.depth = d_depth + (int64_t)k0 * W * H;
-    rc = frame_tiles(P, d_depth + (int64_t)k0 * W * H, P.K, ws + rayfac_bytes(W, H), ws + ws_bytes,
-                     s);
+    P.depth = d_depth + k0 * pixels;
+    rc = frame_tiles(P, tables_pay(voxels, voxels, P.K, pixels), d_depth + k0 * pixels, P.K,
+                     ws + rayfac_bytes(W, H), ws + ws_bytes, s);
     if (rc) return rc;
-    const int bricks = bricks_per_wave((int64_t)X * Y * Z, P.K);
-    const int64_t nb = regions(X, Y, Z, kBrickZ * bricks);
+    // (integrate1_kernel has bricks of four)
+    const int nz = P.K == 1 ? kBrickZ : brick_planes(voxels, P.K, pixels);
+    const int bricks = bricks_per_wave(voxels, P.K);
+    const int64_t nb = regions(X, Y, Z, nz * bricks);
     P.log2_run = region_runs(nb, P.K);
     for (int64_t b0 = 0; b0 < nb; b0 += kMaxRegions) {
       const dim3 grid = region_grid(P, b0, nb);
       if (P.K == 1)
         hipLaunchKernelGGL(integrate1_kernel<DT>, grid, dim3(64), 0, s, P, bricks);
+      else if (nz == 1)
+        hipLaunchKernelGGL((integrate_kernel<DT, 1>), grid, dim3(64), 0, s, P, bricks);
       else
-        hipLaunchKernelGGL(integrate_kernel<DT>, grid, dim3(64), 0, s, P, bricks);
+        hipLaunchKernelGGL((integrate_kernel<DT, kBrickZ>), grid, dim3(64), 0, s, P, bricks);
       MCX_HIP(hipGetLastError());
     }
   }
@@ -1392,19 +1424,26 @@ extern "C" int mcx_integrate_tsdf(float* d_tsdf, int32_t* d_weight, int X, int Y
   int rc = prepare_integrate(P, X, Y, Z, h, trunc, max_w, intr, depth_scale, W, H, K,
                              reinterpret_cast<float*>(ws));
   if (rc) return rc;
+  const int64_t voxels = (int64_t)X * Y * Z, pixels = (int64_t)W * H;
   for (int k0 = 0; k0 < K; k0 += kFramesPerPass) {
     P.K = K - k0 < kFramesPerPass ? K - k0 : kFramesPerPass;
     P.poses = d_poses + (int64_t)12 * k0;
-    P.depth = d_depth + (int64_t)k0 * W * H;
-    rc = frame_tiles(P, d_depth + (int64_t)k0 * W * H, P.K, ws + rayfac_bytes(W, H), ws + ws_bytes,
-                     s);
+    P.depth = d_depth + k0 * pixels;
+    rc = frame_tiles(P, tables_pay(voxels, voxels, P.K, pixels), d_depth + k0 * pixels, P.K,
+                     ws + rayfac_bytes(W, H), ws + ws_bytes, s);
     if (rc) return rc;
-    const int bricks = bricks_per_wave((int64_t)X * Y * Z, P.K);
-    const int64_t nb = regions(X, Y, Z, kBrickZ * bricks);
+    const int nz = brick_planes(voxels, P.K, pixels);
+    const int bricks = bricks_per_wave(voxels, P.K);
+    const int64_t nb = regions(X, Y, Z, nz * bricks);
     P.log2_run = region_runs(nb, P.K);
     for (int64_t b0 = 0; b0 < nb; b0 += kMaxRegions) {
       const dim3 grid = region_grid(P, b0, nb);
-      hipLaunchKernelGGL(integrate_tsdf_kernel, grid, dim3(64), 0, s, P, bricks, d_tsdf, d_weight);
+      if (nz == 1)
+        hipLaunchKernelGGL(integrate_tsdf_kernel<1>, grid, dim3(64), 0, s, P, bricks, d_tsdf,
+                           d_weight);
+      else
+        hipLaunchKernelGGL(integrate_tsdf_kernel<kBrickZ>, grid, dim3(64), 0, s, P, bricks, d_tsdf,
+                           d_weight);
       MCX_HIP(hipGetLastError());
     }
   }
@@ -1443,9 +1482,10 @@ extern "C" int mcx_integrate_tsdf_backward(const float* d_grad_tsdf, const int32
   IntegrateParams P;
   int rc = prepare_integrate(P, X, Y, Z, h, trunc, max_w, intr, depth_scale, W, H, K, rayfac);
   if (rc) return rc;
-  rc = frame_tiles(P, d_depth, K, b + backward_bytes(W, H, K), b + ws_bytes, s);
-  if (rc) return rc;
   const int64_t n = (int64_t)X * Y * Z;
+  rc = frame_tiles(P, tables_pay(n, n, K, (int64_t)W * H), d_depth, K, b + backward_bytes(W, H, K),
+                   b + ws_bytes, s);
+  if (rc) return rc;
   const int64_t npix = (int64_t)K * W * H;
   rc = fill_bytes_zero(maxg, 256 + (size_t)npix * 8, s);  // max and accumulators
   if (rc) return rc;
@@ -1523,17 +1563,25 @@ extern "C" int mcx_integrate_tsdf_batched(const mcx_batch* plan, float* d_tsdf, 
   // volumes in turn of as many as the workspace holds tile tables for
   char* const ws = static_cast<char*>(d_ws);
   const int64_t pixels = (int64_t)W * H * K;
-  const int turn = volumes_per_turn(ws + rayfac_bytes(W, H), ws + ws_bytes, W, H, K, plan->nvol);
+  const bool tables = tables_pay(plan->voxels, plan->voxels / plan->nvol, K, (int64_t)W * H);
+  const int turn = tables ? volumes_per_turn(ws + rayfac_bytes(W, H), ws + ws_bytes, W, H, K,
+                                             plan->nvol)
+                          : plan->nvol;
   for (int v0 = 0; v0 < plan->nvol; v0 += turn) {
     const int v1 = std::min(plan->nvol, v0 + turn);
-    rc = frame_tiles(B.base, d_depth + v0 * pixels, (int64_t)(v1 - v0) * K,
+    rc = frame_tiles(B.base, tables, d_depth + v0 * pixels, (int64_t)(v1 - v0) * K,
                      ws + rayfac_bytes(W, H), ws + ws_bytes, s);
     if (rc) return rc;
     B.tiled_vol = v0;
     const int64_t end = plan->blk_begin[v1];
     for (int64_t b0 = plan->blk_begin[v0]; b0 < end; b0 += kMaxRegions) {
       const dim3 grid = region_grid(B.base, b0, end);
-      hipLaunchKernelGGL(integrate_tsdf_batched_kernel, grid, dim3(64), 0, s, B, d_tsdf, d_weight);
+      if (plan->brick_planes == 1)
+        hipLaunchKernelGGL(integrate_tsdf_batched_kernel<1>, grid, dim3(64), 0, s, B, d_tsdf,
+                           d_weight);
+      else
+        hipLaunchKernelGGL(integrate_tsdf_batched_kernel<kBrickZ>, grid, dim3(64), 0, s, B, d_tsdf,
+                           d_weight);
       MCX_HIP(hipGetLastError());
     }
   }
@@ -1575,8 +1623,10 @@ extern "C" int mcx_integrate_tsdf_backward_batched(const mcx_batch* plan,
   int rc = prepare_integrate(B.base, 1, 1, 1, 1.0f, trunc, max_w, intr, depth_scale, W, H, K,
                              rayfac);
   if (rc) return rc;
-  rc = frame_tiles(B.base, d_depth, (int64_t)plan->nvol * K,
-                   b + backward_bytes(W, H, (int64_t)plan->nvol * K), b + ws_bytes, s);
+  rc = frame_tiles(B.base,
+                   tables_pay(plan->voxels, plan->voxels / plan->nvol, K, (int64_t)W * H), d_depth,
+                   (int64_t)plan->nvol * K, b + backward_bytes(W, H, (int64_t)plan->nvol * K),
+                   b + ws_bytes, s);
   if (rc) return rc;
   B.tiled_vol = 0;
   const int64_t npix = (int64_t)plan->nvol * K * W * H;
@@ -1605,8 +1655,12 @@ extern "C" int mcx_integrate_tsdf_backward_batched(const mcx_batch* plan,
   B.init_value = 0.0f;
   for (int64_t b0 = 0; b0 < plan->blocks; b0 += kMaxRegions) {
     const dim3 grid = region_grid(B.base, b0, plan->blocks);
-    hipLaunchKernelGGL(integrate_tsdf_backward_batched_kernel, grid, dim3(64), 0, s, B,
-                       d_grad_tsdf, d_weight0, mg, mdt, acc);
+    if (plan->brick_planes == 1)
+      hipLaunchKernelGGL(integrate_tsdf_backward_batched_kernel<1>, grid, dim3(64), 0, s, B,
+                         d_grad_tsdf, d_weight0, mg, mdt, acc);
+    else
+      hipLaunchKernelGGL(integrate_tsdf_backward_batched_kernel<kBrickZ>, grid, dim3(64), 0, s, B,
+                         d_grad_tsdf, d_weight0, mg, mdt, acc);
     MCX_HIP(hipGetLastError());
   }
   hipLaunchKernelGGL(fixed_to_float_kernel, dim3(blocks_for((npix + 1) / 2)), dim3(256), 0, s, acc, npix,

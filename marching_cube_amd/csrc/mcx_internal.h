@@ -301,10 +301,11 @@ __device__ __forceinline__ int64_t lookback(const uint64_t* desc, int64_t t, uin
 // Per-volume table of a batch plan (device memory), shared by the batched
 // extraction, MC backward and integration kernels.  Per-voxel arrays of a
 // batch (fp32 TSDF, weights, gradients) are concatenated in volume order:
-// volume b's voxels start at vox_begin.  Workgroups of the integration kernels
-// take 32 x 8 x (4 * the plan's bricks) voxels of one volume (blk_begin: the
-// volume's first such workgroup; divX, divY: workgroups along x and y); the
-// batched gather takes 1024 voxels of one plane (gblk_begin).
+// volume b's voxels start at vox_begin.  The integration kernels take regions of
+// 32 x 8 x (the plan's brick_planes * bricks) voxels of one volume (blk_begin:
+// the volume's first; divX, divY: regions along x and y); a workgroup of the
+// batched gather takes four windows of 512 voxels of one plane, or parts of
+// windows (gblk_begin).
 struct BatchVol {
   int X, Y, Z;
   float h;
@@ -317,13 +318,13 @@ struct BatchVol {
 struct VolDesc;  // extraction descriptors (mcx_extract.hip)
 struct Column;
 
-// Volume of workgroup `blk` (the last b with begin[b] <= blk), by binary
 // A dispatch carries its grid size in work-items as a 32-bit number, so a
 // grid of one workgroup per 256 or more items (volumes of 2^32 voxels and
 // more) is issued as several launches of at most this many workgroups, each
 // told the index of its first workgroup.
 constexpr int64_t kMaxLaunchBlocks = (int64_t)1 << 23;
 
+// Volume of workgroup `blk` (the last b with begin[b] <= blk), by binary
 // search over a BatchVol table; the member selects which begin.
 template <int64_t BatchVol::*BEGIN>
 __device__ __forceinline__ int batch_volume_of(const BatchVol* bv, int nvol, int64_t blk) {
@@ -348,8 +349,9 @@ struct mcx_batch {
   int64_t ncols = 0;
   int64_t cubes = 0;
   int64_t voxels = 0;       // all volumes' voxels
-  int64_t blocks = 0;       // workgroups of the integration kernels
+  int64_t blocks = 0;       // regions of the integration kernels
   std::vector<int64_t> blk_begin;  // each volume's first one, then their number
+  int brick_planes = 4;     // planes of an integration brick
   int bricks = 1;           // bricks above one another that an integration wave takes
   int64_t gather_blocks = 0;
   int gather_split = 1;     // waves that share a window of the batched gather

@@ -63,7 +63,7 @@ def frames_at_the_edge(rng, voxel, scale, mirror, trunc):
 
 @pytest.mark.parametrize("mirror", [False, True])
 @pytest.mark.parametrize("scale", [0.001, 1.0, 1000.0])
-@pytest.mark.parametrize("dims", [(1, 1, 1), (9, 9, 5)])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (9, 9, 5), (65, 65, 65)])
 def test_updates_at_minus_trunc(dev, dims, scale, mirror):
     print(f"[case] {dims}, matrices of scale {scale}, mirrored {mirror}", flush=True)
     X, Y, Z = dims

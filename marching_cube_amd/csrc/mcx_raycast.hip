@@ -19,18 +19,19 @@
 // which the ray can lie in the volume grown by one voxel (all later samples
 // would be skipped), and 2^20 steps.
 //
-// Layout: eight lanes take a ray and its next eight samples at once; a wave
-// holds 2 x 4 pixels, an XCD the waves of 16 x 16 pixels in a row.  Each sample
-// reads its eight corner words as four x-neighbour pairs (one 64-bit load
-// each).  With a ray to a lane the march was as slow as its slowest waves: a
-// ray along a surface takes hundreds of fine steps, some 1500 cycles each, one
-// after the other (640x480 rays through 512^3: 1.28 ms, of which most waves
-// ran 0.3).  Eight samples a step cut that chain, also where the samples are
-// only free space (four lanes 0.49 ms, sixteen 0.50), and patches per XCD cut
-// the L2 misses to an eighth (0.475 -> 0.458 ms).  What bounds it now is the
-// vector cache: 34 accesses a load, 0.98 M a CU in 1.05 M cycles.  A map of the
-// bricks without a surface, built in every call by a pass over the volume,
-// needs memory that the entry point is not given and left 0.42 ms.
+// Layout: LANES lanes take a ray and its next LANES samples at once; a wave
+// holds 64 / LANES pixels, an XCD the waves of 16 x 16 pixels in a row.  Each
+// sample reads its eight corner words as four x-neighbour pairs (one 64-bit load
+// each).  With a ray to a lane the march is as slow as its slowest waves: a ray
+// along a surface takes hundreds of fine steps, some 1500 cycles each, one after
+// the other (640x480 rays through 512^3: 1.28 ms, of which most waves ran 0.3).
+// Eight samples a step cut that chain, also where the samples are only free
+// space (four lanes 0.49 ms, sixteen 0.50), and patches per XCD cut the L2 misses
+// to an eighth (0.475 -> 0.458 ms).  What bounds it then is the vector cache: 34
+// accesses a load, 0.98 M a CU in 1.05 M cycles.  Where the rays fill the chip by
+// themselves, samples past a ray's end are only waste: ray_lanes.  A map of the
+// bricks without a surface, built in every call by a pass over the volume, needs
+// memory that the entry point is not given and left 0.42 ms.
 // Bit-exact with the CPU oracle: every fused multiply-add is explicit and the
 // build disables contraction.
 #include <hip/hip_runtime.h>
@@ -46,13 +47,16 @@ namespace {
 
 constexpr int kMaxTsdf = 32766;
 constexpr int kRayMaxSteps = 1 << 20;
-// kLanes lanes take a ray; a wave's rays are a tile of kTileW x kTileH pixels.
-constexpr int kLanes = 8;
-constexpr int kTileW = 2, kTileH = 64 / kLanes / kTileW;
 // Workgroups go round the 8 XCDs; an XCD's are the tiles of patches of kPatch x
 // kPatch pixels, one after the other, so that its L2 holds what they share.
 constexpr int kPatch = 16;
-constexpr int kPatchTilesX = kPatch / kTileW, kPatchTiles = kPatchTilesX * (kPatch / kTileH);
+// LANES lanes take a ray; a wave's rays are a tile of W x H pixels.
+template <int LANES>
+struct Tile {
+  static constexpr int kW = LANES == 8 ? 2 : 8, kH = 64 / LANES / kW;
+  static constexpr int kPatchX = kPatch / kW;               // tiles in a patch's row
+  static constexpr int kInPatch = kPatchX * (kPatch / kH);  // tiles of a patch
+};
 
 struct RaycastArgs {
   const int16_t* vol16;  // tsdf halves: word i's tsdf at vol16[2 i]
@@ -164,23 +168,27 @@ __device__ void surface_normal(const RaycastArgs& A, int64_t XY, float px, float
   n[2] = gz;
 }
 
-// The value of lane `from` (0 to kLanes - 1) of this lane's group.
+// The value of lane `from` (0 to LANES - 1) of this lane's group.
+template <int LANES>
 __device__ __forceinline__ float group_get(float v, int from) {
-  return __shfl(v, from, kLanes);
+  return __shfl(v, from, LANES);
 }
 // This group's bits of a condition over the wave.
+template <int LANES>
 __device__ __forceinline__ uint32_t group_bits(bool c) {
-  const int first = threadIdx.x & (64 - kLanes);
-  return (uint32_t)(__ballot(c) >> first) & ((1u << kLanes) - 1u);
+  const int first = threadIdx.x & (64 - LANES);
+  return (uint32_t)(__ballot(c) >> first) & ((1u << LANES) - 1u);
 }
 
+template <int LANES>
 __global__ __launch_bounds__(64) void raycast_kernel(RaycastArgs A) {
-  const int j = threadIdx.x & (kLanes - 1), ray = threadIdx.x / kLanes;
-  const int b = blockIdx.x >> 3, tile = b % kPatchTiles;
-  const int patch = A.first_patch + b / kPatchTiles * 8 + (blockIdx.x & 7);
+  using T = Tile<LANES>;
+  const int j = threadIdx.x & (LANES - 1), ray = threadIdx.x / LANES;
+  const int b = blockIdx.x >> 3, tile = b % T::kInPatch;
+  const int patch = A.first_patch + b / T::kInPatch * 8 + (blockIdx.x & 7);
   const int py = patch / A.patches_x, px = patch - py * A.patches_x;
-  const int x = px * kPatch + tile % kPatchTilesX * kTileW + ray % kTileW;
-  const int y = py * kPatch + tile / kPatchTilesX * kTileH + ray / kTileW;
+  const int x = px * kPatch + tile % T::kPatchX * T::kW + ray % T::kW;
+  const int y = py * kPatch + tile / T::kPatchX * T::kH + ray / T::kW;
   const bool live = x < A.W && y < A.H;
   const float xf = (float)x, yf = (float)y;
   float r[3];
@@ -225,7 +233,7 @@ __global__ __launch_bounds__(64) void raycast_kernel(RaycastArgs A) {
   t_far = t_far + fabsf(t_far) * 0x1p-20f + 1.0f;
   const int64_t XY = (int64_t)A.X * A.Y;
 
-  // The march, kLanes samples at a time: lane j takes the j-th next one.  The
+  // The march, LANES samples at a time: lane j takes the j-th next one.  The
   // samples are those of a step-by-step march up to the first event (the end,
   // a hit, a back face, a change between coarse and fine steps); what was
   // sampled past an event is dropped.  State, the same in a group's lanes:
@@ -237,7 +245,7 @@ __global__ __launch_bounds__(64) void raycast_kernel(RaycastArgs A) {
   while (__any(marching)) {
     float ts = t, last = t;          // this lane's sample, the group's last one
 #pragma unroll
-    for (int i = 1; i < kLanes; ++i) {
+    for (int i = 1; i < LANES; ++i) {
       last = last + dt;
       ts = j >= i ? last : ts;
     }
@@ -257,28 +265,28 @@ __global__ __launch_bounds__(64) void raycast_kernel(RaycastArgs A) {
     }
     // all lanes in free or unseen space, taking coarse steps: on
     if (__all(!marching || (in && side != 0 && !fine))) {
-      steps += kLanes;
-      sdf1 = group_get(sdf, kLanes - 1);
+      steps += LANES;
+      sdf1 = group_get<LANES>(sdf, LANES - 1);
       t = last + dt;
       continue;
     }
     // the sample before this lane's (samples outside the volume do not count,
     // and lie before all or after all of the others)
-    const float before = __shfl_up(sdf, 1, kLanes), t_before = __shfl_up(ts, 1, kLanes);
-    const uint32_t ins = group_bits(in);
+    const float before = __shfl_up(sdf, 1, LANES), t_before = __shfl_up(ts, 1, LANES);
+    const uint32_t ins = group_bits<LANES>(in);
     const bool carried = j == 0 || !(ins >> (j - 1) & 1u);
     const float prev = carried ? sdf1 : before, t_prev = carried ? t1 : t_before;
     const bool band = sdf > -1.0f && sdf < 1.0f;
     const bool crossed = sdf < 0.0f && sdf > -1.0f && prev >= 0.0f && prev < 1.0f;
     const bool back = prev <= 0.0f && prev > -1.0f && sdf >= 0.0f && sdf < 1.0f;
-    const uint32_t events = group_bits(stop || (in && (crossed || back || band != fine)));
+    const uint32_t events = group_bits<LANES>(stop || (in && (crossed || back || band != fine)));
     if (!marching) continue;
     if (!events) {
-      steps += kLanes;
+      steps += LANES;
       if (ins) {
         const int l = 31 - __builtin_clz(ins);
-        sdf1 = group_get(sdf, l);
-        t1 = group_get(ts, l);
+        sdf1 = group_get<LANES>(sdf, l);
+        t1 = group_get<LANES>(ts, l);
       }
       t = last + dt;
       continue;
@@ -290,9 +298,9 @@ __global__ __launch_bounds__(64) void raycast_kernel(RaycastArgs A) {
       hit = true;
       hit_t = t_prev - dt * prev / (sdf - prev);
     }
-    const bool ended = __shfl((int)ends, e, kLanes);
-    const float te = group_get(ts, e), sdfe = group_get(sdf, e), preve = group_get(prev, e),
-                t_preve = group_get(t_prev, e);
+    const bool ended = __shfl((int)ends, e, LANES);
+    const float te = group_get<LANES>(ts, e), sdfe = group_get<LANES>(sdf, e), preve = group_get<LANES>(prev, e),
+                t_preve = group_get<LANES>(t_prev, e);
     if (ended) {
       marching = false;
       continue;
@@ -311,7 +319,7 @@ __global__ __launch_bounds__(64) void raycast_kernel(RaycastArgs A) {
     }
     t += dt;
   }
-  const uint32_t hits = group_bits(hit);
+  const uint32_t hits = group_bits<LANES>(hit);
   if (!live || !(hits ? hit : j == 0)) return;
   float out_d = 0.0f, out_n[3] = {0.0f, 0.0f, 0.0f};
   if (hit) {
@@ -361,6 +369,35 @@ bool camera_inverse(const float* intr, const float* R, float* im) {
   return true;
 }
 
+// Lanes of a ray.  One fills every SIMD with a wave for each 2^16 rays; with 14
+// waves the next ones hide the slowest, whatever the volume; from 4 on two lanes
+// do, the longer the volume's marches the later; else the chip would idle behind
+// the slow rays.  Eight, two and one lanes, us, through a fused scene and through
+// one without a surface: 640x480, 64^3 147, 123, 171 and 88, 65, 59; 160^3 211, 210,
+// 260 and 199, 169, 167; 256^3 290, 313, 409 and 315, 283, 311; 512^3 573, 738,
+// 1022 and 738, 914, 1360.  1024x768, 512^3 1273, 1196, 1658 and 1585, 1498, 2053.
+// 1280x720, 64^3 388, 251, 258 and 244, 170, 136; 512^3 1481, 1288, 1484 and 1871,
+// 1655, 1864.  1920x1080, 512^3 3236, 2498, 2459 and 4161, 3301, 3227.  480x360,
+// 96^3 109, 127, 180 and 75, 61, 68.
+int ray_lanes(int64_t rays, int side) {
+  if (rays >= (int64_t)14 << 16) return 1;
+  return rays >= (int64_t)4 << 16 && (int64_t)side << 16 <= 40 * rays ? 2 : 8;
+}
+
+// All patches, in launches of at most 2^25 waves.
+template <int LANES>
+int launch_rays(RaycastArgs A, int64_t patches, hipStream_t s) {
+  constexpr int kTiles = Tile<LANES>::kInPatch;
+  constexpr int64_t kMost = ((int64_t)1 << 25) / kTiles;
+  for (int64_t p = 0; p < patches; p += kMost) {
+    A.first_patch = (int)p;
+    const int64_t n = (std::min(kMost, patches - p) + 7) / 8 * 8 * kTiles;
+    hipLaunchKernelGGL(raycast_kernel<LANES>, dim3((unsigned)n), dim3(64), 0, s, A);
+    MCX_HIP(hipGetLastError());
+  }
+  return MCX_OK;
+}
+
 }  // namespace
 }  // namespace mcx
 
@@ -390,16 +427,11 @@ extern "C" int mcx_raycast(const void* d_vol, int X, int Y, int Z, float h, floa
   A.cx = intr[2];
   A.cy = intr[3];
   if ((H + 15) / 16 > 65535) return MCX_ERR_ARG;
-  // patches in launches of at most 2^25 waves
   A.patches_x = (W + kPatch - 1) / kPatch;
   const int64_t patches = (int64_t)A.patches_x * ((H + kPatch - 1) / kPatch);
-  constexpr int64_t kMost = ((int64_t)1 << 25) / kPatchTiles;
   if (patches >= ((int64_t)1 << 31)) return MCX_ERR_ARG;
-  for (int64_t p = 0; p < patches; p += kMost) {
-    A.first_patch = (int)p;
-    const int64_t n = (std::min(kMost, patches - p) + 7) / 8 * 8 * kPatchTiles;
-    hipLaunchKernelGGL(raycast_kernel, dim3((unsigned)n), dim3(64), 0, as_stream(stream), A);
-    MCX_HIP(hipGetLastError());
-  }
-  return MCX_OK;
+  const int lanes = ray_lanes((int64_t)W * H, std::max(X, std::max(Y, Z)));
+  if (lanes == 1) return launch_rays<1>(A, patches, as_stream(stream));
+  if (lanes == 2) return launch_rays<2>(A, patches, as_stream(stream));
+  return launch_rays<8>(A, patches, as_stream(stream));
 }

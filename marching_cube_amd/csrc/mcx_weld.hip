@@ -24,13 +24,15 @@
 // Deterministic: the table layout may vary between runs, what is read from
 // it (the minimum index per key) does not.
 //
-// Bound by the scattered atomics: of the insert's 41 us at 2.45 M vertices (a
-// 400^3 room) they are 25, the rest of the five launches 40.  A table of keys
-// and another of values, two atomics a key and per-wave repeats only, with a
-// second probe for the first occurrences, took 200 us for the whole weld where
-// this takes 82.  Tried: workgroups of 256 and 1024 threads for the insert (43
-// us), a table hashed key by key (47 us), a read of the slot before the CAS
-// (the same).
+// Bound by the scattered atomics of the insert: 31 us at 2.45 M vertices (a 400^3
+// room), the rest of the five launches 38.  A table of keys and another of
+// values, two atomics a key and per-wave repeats only, with a second probe for
+// the first occurrences, took 200 us for the whole weld where this takes 69.
+// Steps of one slot where groups of keys meet took 43 us for the insert there,
+// and 433 for the weld of 1 M consecutive keys (now 40; shuffled 1230 and 103).
+// Tried, with those steps: workgroups of 256 and 1024 threads for the insert (43
+// us), a table hashed key by key (47 us), a read of the slot before the CAS (the
+// same).
 #include <hip/hip_runtime.h>
 
 #include "mcx_internal.h"
@@ -53,13 +55,25 @@ __device__ __forceinline__ uint64_t mix64(uint64_t k) {
   return k;
 }
 
-// First slot of a key.  Groups of 32 consecutive keys (the edges of 10 voxels
-// along x) stay in one 128-byte line, whose place and inner order are hashed:
-// the keys of a surface patch share lines, and keys a multiple of 32 apart
-// still start anywhere in the table.
-__device__ __forceinline__ uint32_t first_slot(uint64_t key, uint32_t mask) {
+// The slots of a key.  Groups of 32 consecutive keys (the edges of 10 voxels
+// along x) stay in one 128-byte line, whose place and inner order are hashed: the
+// keys of a surface patch share lines, and keys a multiple of 32 apart still
+// start anywhere in the table.  A key whose slot is taken goes on to the same
+// place of other lines, the group's (a group that meets another moves as a whole:
+// by steps of one slot, 32 dense keys walk over 32 taken ones each), and from the
+// kLines-th line on to the next slots, all of the table if need be.
+constexpr uint32_t kLines = 16;
+struct Probe {
+  uint32_t h, step, n;
+};
+__device__ __forceinline__ Probe first_slot(uint64_t key, uint32_t mask) {
   const uint64_t m = mix64(key >> 5);
-  return (((uint32_t)m << 5) | (((uint32_t)key ^ (uint32_t)(m >> 59)) & 31u)) & mask;
+  return Probe{(((uint32_t)m << 5) | (((uint32_t)key ^ (uint32_t)(m >> 59)) & 31u)) & mask,
+               (uint32_t)(m >> 32) << 6 | 32u, 1};
+}
+__device__ __forceinline__ void next_slot(Probe& p, uint32_t mask) {
+  p.h = (p.h + (p.n < kLines ? p.step : 1u)) & mask;
+  ++p.n;
 }
 
 __global__ __launch_bounds__(kInsert) void weld_insert_kernel(const int64_t* __restrict__ ekey,
@@ -114,18 +128,18 @@ __global__ __launch_bounds__(kInsert) void weld_insert_kernel(const int64_t* __r
   for (uint32_t i = tid; i < n; i += kInsert) {
     const uint32_t l = s_first[i], v = base + l;
     const uint64_t mine = s_key[l];
-    uint32_t h = first_slot(mine, mask);
+    Probe p = first_slot(mine, mask);
     for (;;) {  // at most V distinct keys in >= 2V slots: the probe ends
-      const uint32_t old = atomicCAS(table + h, kEmpty, v);
+      const uint32_t old = atomicCAS(table + p.h, kEmpty, v);
       if (old == kEmpty) break;
       // a slot's index only changes to a lower one of the same key
       if ((uint64_t)ekey[old] == mine) {
-        if (v < old) atomicMin(table + h, v);
+        if (v < old) atomicMin(table + p.h, v);
         break;
       }
-      h = (h + 1) & mask;
+      next_slot(p, mask);
     }
-    s_slot[l] = h;
+    s_slot[l] = p.h;
   }
   __syncthreads();
 #pragma unroll

@@ -668,6 +668,13 @@ void count4_kernel(ExtractParams P) {
     asm volatile("s_waitcnt vmcnt(12)" : "+v"(A.u[0]), "+v"(A.u[1]), "+v"(A.w[0]), "+v"(A.w[1]), "+v"(A.xu), "+v"(A.xw) :: "memory");
   plane_signs<ELEM>(A);
 
+  // The pool's counter only grows, and a take that failed leaves it past the end:
+  // a wave asks no more, and counts its staged tiles once, instead of two atomics
+  // a tile on one line (128^3, 98 % of the cubes active: 110 us, now 40).  In short2
+  // volumes (111 us there) it costs 0.25 % of a batch whose records fit: left out.
+  constexpr bool kAskOnce = ELEM == MCX_ELEM_F32;
+  bool pool_full = kAskOnce && P.ovf_cap == 0;
+  uint32_t n_dense = 0;
   uint64_t nzmask = 0;  // planes zb + i of this column whose tile has vertices
   int zb = z0;
   uint32_t t = (uint32_t)(V.tile_begin + (int64_t)z0 * V.R + r);  // this step's tile
@@ -793,12 +800,18 @@ void count4_kernel(ExtractParams P) {
     int64_t rbase = wg_base + got;
     bool dense = false;
     if (got + (uint32_t)nrec32 > wg_size) {
-      unsigned long long ob = 0;
-      if (lane == 0) ob = atomicAdd(reinterpret_cast<unsigned long long*>(&P.hdr->ovf_next),
-                                    (unsigned long long)nrec);
-      ob = __shfl(ob, 0);
-      if ((int64_t)ob + nrec <= P.ovf_cap) rbase = P.ovf_begin + (int64_t)ob;
-      else dense = true;
+      if (pool_full) {
+        dense = true;
+      } else {
+        unsigned long long ob = 0;
+        if (lane == 0) ob = atomicAdd(reinterpret_cast<unsigned long long*>(&P.hdr->ovf_next),
+                                      (unsigned long long)nrec);
+        ob = __shfl(ob, 0);
+        if ((int64_t)ob + nrec <= P.ovf_cap) rbase = P.ovf_begin + (int64_t)ob;
+        else dense = true;
+        if (kAskOnce) pool_full = dense;
+      }
+      if (kAskOnce) n_dense += dense;
     }
 
     // ---- pass 2: the active cubes of a chunk are staged in the wave's LDS
@@ -901,7 +914,7 @@ void count4_kernel(ExtractParams P) {
       P.tileT[t] = (int32_t)vsum;
       P.tile_nrec[t] = dense ? -1 : (int32_t)nrec;
       P.tile_rec[t] = dense ? 0 : rbase;
-      if (dense) atomicAdd(&P.hdr->dense_acc, 1u);
+      if (!kAskOnce && dense) atomicAdd(&P.hdr->dense_acc, 1u);
     }
     load_plane(z + 3, L);
     t += tR;
@@ -929,6 +942,7 @@ void count4_kernel(ExtractParams P) {
     if (z + 2 < z1) step(C, D, B, z + 2);
     if (z + 3 < z1) step(D, A, C, z + 3);
   }
+  if (kAskOnce && n_dense && lane == 0) atomicAdd(&P.hdr->dense_acc, n_dense);
 }
 
 // ============================================================ K2: scan

@@ -182,3 +182,42 @@ def test_fusion_graph_past_its_capacity(dev):
         g.check()
     assert e.value.status == _capi.ERR_CAPACITY
     assert torch.isnan(g.gtsdf_all).all()
+
+
+@pytest.mark.parametrize("share", [0.0, 0.25, 0.5, 0.9, 1.3, 8.0])
+@pytest.mark.parametrize("kind", ["short2", "f32"])
+def test_plain_extraction(dev, kind, share):
+    """No room, a pool that runs out on the way, room for all: the same mesh."""
+    print(f"[case] plain extraction {kind}, records for {share} of the cubes", flush=True)
+    from marching_cube_amd import synth
+    lib, h, (Z, Y, X) = _capi.load(), 0.01, (40, 61, 67)
+    if kind == "short2":
+        f = synth.noise_volume((Z, Y, X), seed=3, p_zero_w=0.02)
+        ref = O.extract(f, h, want=("vv",))
+        want = ref["vv"].view(np.int32).reshape(-1, 7)
+        v, elem = torch.from_numpy(f.view(np.int32)).to(dev), _capi.ELEM_SHORT2
+    else:
+        f = noisy((Z, Y, X), 3)
+        ref = O.extract(f, h, want=("pos",))
+        want = ref["pos"]
+        v, elem = torch.from_numpy(f).to(dev), _capi.ELEM_F32
+    tiles = (Z - 1) * ((X * Y + 511) // 512)
+    records = int(share * (Z - 1) * (Y - 1) * (X - 1))
+    ws = workspace(lib.mcx_extract_workspace_size_ex(X, Y, Z, records), dev)
+    n = ctypes.c_int64(0)
+    out = torch.empty(want.shape, dtype=torch.int32 if kind == "short2" else torch.float32,
+                      device=dev)
+    for _ in range(2):
+        out.zero_()
+        _capi.check(lib.mcx_extract(_ptr(v), elem, X, Y, Z, h,
+                                    _ptr(out) if kind == "short2" else None,
+                                    None if kind == "short2" else _ptr(out), None, None, len(want),
+                                    None, ctypes.byref(n), _ptr(ws), ws.numel(),
+                                    _stream_handle(dev)), "mcx_extract")
+        assert n.value == len(want) and out.cpu().numpy().tobytes() == want.tobytes()
+        staged = staged_tiles(ws, dev)
+        assert staged <= tiles
+        if share in (0.0, 0.25, 0.5):  # (at 0.9 the active cubes may all fit)
+            assert staged > 0
+        if share == 8.0:
+            assert staged == 0

@@ -16,7 +16,6 @@ namespace mcx {
 namespace {
 
 constexpr int kMaxTargets = 1024;  // targets staged in LDS per workgroup
-constexpr int kRows = 2;           // vertex rows a thread
 
 // Volume of vertex v: the last b with vbase[b] <= v (vbase ascending).
 __device__ __forceinline__ int volume_of_vertex(const int64_t* vbase, int nvol, int64_t v) {
@@ -28,39 +27,34 @@ __device__ __forceinline__ int volume_of_vertex(const int64_t* vbase, int nvol, 
   return lo;
 }
 
-// The first nearest of M targets (at(m): target m) to each of a thread's rows.
-template <int N, class At>
-__device__ __forceinline__ void nearest(const float (&p)[N][3], int M, At at,
-                                        float (&best)[N], int (&j)[N]) {
-#pragma unroll
-  for (int r = 0; r < N; ++r) {
-    best[r] = __builtin_inff();
-    j[r] = 0;
-  }
+// The first nearest of M targets (at(m): target m) to p, and its distance squared.
+template <class At>
+__device__ __forceinline__ float nearest(const float (&p)[3], int M, At at, int* j) {
+  float best = __builtin_inff();
+  *j = 0;
 #pragma unroll 4
   for (int m = 0; m < M; ++m) {
     const float4 t = at(m);
-#pragma unroll
-    for (int r = 0; r < N; ++r) {
-      const float dx = p[r][0] - t.x, dy = p[r][1] - t.y, dz = p[r][2] - t.z;
-      const float d2 = __fmaf_rn(dz, dz, __fmaf_rn(dy, dy, dx * dx));
-      if (d2 < best[r]) {
-        best[r] = d2;
-        j[r] = m;
-      }
+    const float dx = p[0] - t.x, dy = p[1] - t.y, dz = p[2] - t.z;
+    const float d2 = __fmaf_rn(dz, dz, __fmaf_rn(dy, dy, dx * dx));
+    if (d2 < best) {
+      best = d2;
+      *j = m;
     }
   }
+  return best;
 }
 
-// Two vertex rows a thread, 256 apart (rows past the total or past cap:
-// gradient 0; a wave of only such rows looks at no target: 2 M rows without a
-// vertex, 1024 targets, 9 us, and 348 where it did).  The targets of the volume of the workgroup's first vertex are
-// staged in LDS, one 16-byte read of all lanes for both rows; a wave with a
+// One thread per vertex row (rows past the total or past cap: gradient 0; a wave
+// of only such rows looks at no target: 2 M rows without a vertex, 1024 targets,
+// 9 us, and 348 where it did).  The targets of the volume of the workgroup's first
+// vertex are staged in LDS, one 16-byte read of all lanes for each; a wave with a
 // vertex of another volume (a workgroup spanning a boundary) reads targets from
 // memory.  Bound by the arithmetic (9 instructions a row and target) and by what
-// a row reads and writes: a batch of 64 fused volumes of 64-192 a side, 64
-// targets each, takes 31 us (131 with a row a thread and three reads a target
-// through a pointer that could be either).
+// a row reads and writes.  Loss and sum: 64 volumes, 0.9 M rows, 64 targets 24 us
+// (98 with three reads a target through a pointer that could be either, as with
+// two rows a thread); 4 volumes, 30,000 rows 9.2 us, 300, 0.1 M rows, 1024 targets
+// 49 (12.1 and 89 with two rows, on half the waves).
 __global__ __launch_bounds__(256) void chamfer_vertex_kernel(const float* pos,
                                                              const int64_t* vbase, int nvol,
                                                              const float* targets, int M,
@@ -68,7 +62,7 @@ __global__ __launch_bounds__(256) void chamfer_vertex_kernel(const float* pos,
                                                              float* vloss) {
   __shared__ float4 s_t[kMaxTargets];
   __shared__ int s_b0;
-  const int64_t v0 = (int64_t)blockIdx.x * (256 * kRows);
+  const int64_t v0 = (int64_t)blockIdx.x * 256;
   const int64_t total = vbase[nvol];
   if (threadIdx.x == 0) s_b0 = v0 < total ? volume_of_vertex(vbase, nvol, v0) : 0;
   __syncthreads();
@@ -79,57 +73,35 @@ __global__ __launch_bounds__(256) void chamfer_vertex_kernel(const float* pos,
       s_t[i] = make_float4(t[3 * i], t[3 * i + 1], t[3 * i + 2], 0.0f);
   }
   __syncthreads();
-  const int64_t live = min(total, cap);
-  int64_t v[kRows];
-  float p[kRows][3];
-  bool same = true;
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    v[r] = v0 + r * 256 + threadIdx.x;
-    const int64_t u = min(v[r], live - 1);  // idle lanes: any row
-    p[r][0] = p[r][1] = p[r][2] = 0.0f;
-    if (v[r] < live) {
-      same = same && u < vbase[b0 + 1];
-      p[r][0] = pos[3 * u];
-      p[r][1] = pos[3 * u + 1];
-      p[r][2] = pos[3 * u + 2];
+  const int64_t live = min(total, cap), v = v0 + threadIdx.x;
+  const bool row = v < live;
+  float p[3] = {0.0f, 0.0f, 0.0f}, best = 0.0f;
+  int j = 0, b = b0;
+  if (__any(row)) {
+    if (row) {
+      p[0] = pos[3 * v];
+      p[1] = pos[3 * v + 1];
+      p[2] = pos[3 * v + 2];
+    }
+    if (__all(!row || v < vbase[b0 + 1])) {
+      best = nearest(p, M, [&](int m) { return s_t[m]; }, &j);
+    } else {
+      if (row) b = volume_of_vertex(vbase, nvol, v);
+      const float* t = targets + (int64_t)b * M * 3;
+      best = nearest(
+          p, M, [&](int m) { return make_float4(t[3 * m], t[3 * m + 1], t[3 * m + 2], 0.0f); }, &j);
     }
   }
-  float best[kRows] = {};
-  int j[kRows] = {}, b[kRows] = {};
-  if (!__any(v[0] < live)) {
-    // no vertex: v[0] is the lower of a thread's rows
-  } else if (__all(same)) {
+  if (v >= cap) return;
+  float g[3] = {0.0f, 0.0f, 0.0f};
+  if (row) {
+    const float* t = targets + ((int64_t)b * M + j) * 3;
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) b[r] = b0;
-    nearest(p, M, [&](int m) { return s_t[m]; }, best, j);
-  } else {
-#pragma unroll
-    for (int r = 0; r < kRows; ++r) {
-      b[r] = v[r] < live ? volume_of_vertex(vbase, nvol, v[r]) : b0;
-      const float* t = targets + (int64_t)b[r] * M * 3;
-      const float q[1][3] = {{p[r][0], p[r][1], p[r][2]}};
-      float d[1];
-      int k[1];
-      nearest(q, M, [&](int m) { return make_float4(t[3 * m], t[3 * m + 1], t[3 * m + 2], 0.0f); },
-              d, k);
-      best[r] = d[0];
-      j[r] = k[0];
-    }
+    for (int c = 0; c < 3; ++c) g[c] = 2.0f * (p[c] - t[c]);
+    vloss[v] = best;
   }
 #pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    if (v[r] >= cap) continue;
-    float g[3] = {0.0f, 0.0f, 0.0f};
-    if (v[r] < live) {
-      const float* t = targets + ((int64_t)b[r] * M + j[r]) * 3;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) g[c] = 2.0f * (p[r][c] - t[c]);
-      vloss[v[r]] = best[r];
-    }
-#pragma unroll
-    for (int c = 0; c < 3; ++c) gpos[3 * v[r] + c] = g[c];
-  }
+  for (int c = 0; c < 3; ++c) gpos[3 * v + c] = g[c];
 }
 
 // One workgroup per volume: the sum of its vertex losses (vertices below cap).
@@ -181,7 +153,7 @@ extern "C" int mcx_chamfer_batched(const float* d_pos, const int64_t* d_vbase, i
   hipStream_t s = as_stream(stream);
   float* vloss = static_cast<float*>(d_ws);
   if (cap > kMaxLaunchBlocks * 256) return MCX_ERR_UNSUPPORTED;
-  const int64_t blocks = (cap + 256 * kRows - 1) / (256 * kRows);
+  const int64_t blocks = (cap + 255) / 256;
   hipLaunchKernelGGL(chamfer_vertex_kernel, dim3((unsigned)blocks), dim3(256), 0, s, d_pos,
                      d_vbase, nvol, d_targets, M, cap, d_grad_pos, vloss);
   MCX_HIP(hipGetLastError());

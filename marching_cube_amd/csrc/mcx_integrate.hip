@@ -1496,9 +1496,11 @@ extern "C" int mcx_integrate_tsdf_backward(const float* d_grad_tsdf, const int32
   P.K = K;
   P.poses = d_poses;
   P.depth = d_depth;
-  // One plane a wave below 2^23 voxels: few bricks hold a surface there, and
-  // each one's frames run in series.
-  const bool small = n < ((int64_t)1 << 23);
+  // One plane a wave up to 2^22 voxels: few bricks hold a surface there, and each
+  // one's frames run in series.  One and four, gradients at the surface, us: 96^3,
+  // 16 frames 69 and 87; 128^3, 1 30 and 27, 4 38 and 41, 16 71 and 90; 160^3, 1 41
+  // and 33, 16 88 and 94; 192^3, 1 54 and 38, 16 111 and 101; 256^3, 16 154 and 129.
+  const bool small = n <= ((int64_t)1 << 22);
   const int64_t nb = regions(X, Y, Z, small ? 1 : kBrickZ);
   P.log2_run = region_runs(nb, K);
   for (int64_t b0 = 0; b0 < nb; b0 += kMaxRegions) {

@@ -160,8 +160,8 @@ struct ExtractParams {
   int64_t* voff;         // exclusive vertex offset per tile
   uint64_t* masks;       // active-cube bits, kCPW words per tile
   uint32_t* nz_list;     // ids of the tiles with vertices (in append order)
-  // emission in units of 64 records (single volumes): the scan also scans
-  // the records of the list's tiles in list order
+  // emission and the backward's contributions go in units of 64 records: the
+  // scan also scans the records of the list's tiles in list order
   bool list_scan;
   uint32_t* clist;       // the list's tiles with records, in list order
   int64_t* lpre;         // [n + 1] first record of clist entry j (lpre[n]: all records)
@@ -1978,7 +1978,7 @@ int layout_ws(void* d_ws, size_t ws_bytes, int64_t n_tiles, ExtractParams& P) {
   o += al256(8 * (size_t)(n_tiles + 1));
   P.lrs = reinterpret_cast<int64_t*>(b + o);
   o += al256(8 * (size_t)n_tiles);
-  P.list_scan = false;  // set by run_extract for single-volume emission
+  P.list_scan = false;  // set by run_extract: emission and masks take the list's units
   const int64_t rc = rec_cap_of(ws_bytes - o);
   P.units = reinterpret_cast<uint32_t*>(b + o);
   o += al256(4 * (size_t)(rc / 64 + 2));
@@ -2382,7 +2382,10 @@ extern "C" int mcx_batch_create(mcx_batch** out, int nvol, const int* dims_xyz, 
   int maxX = 1;
   bool wide = true;
   // integration workgroups take one brick of 8 x 8 x 4 voxels a wave, or four
-  // above one another where that leaves 16 waves per SIMD (2^24 voxels)
+  // above one another where that leaves 16 waves per SIMD (2^24 voxels).  One and
+  // four, 320x240 frames, forward and backward, us: 16 volumes of 64^3, 4 frames 52
+  // and 74 (forward), 16 165 and 273; 8 of 128^3, 4 101 and 81, 16 211 and 239, 226
+  // and 313; 64 of 128^3, 4 804 and 593, 822 and 726, 16 1696 and 1759, 1703 and 1914.
   double all = 0;
   for (int b = 0; b < nvol; ++b)
     all += (double)dims_xyz[3 * b] * dims_xyz[3 * b + 1] * dims_xyz[3 * b + 2];

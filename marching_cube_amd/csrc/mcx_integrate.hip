@@ -41,7 +41,7 @@
 namespace mcx {
 namespace {
 
-constexpr int kFramesPerPass = 512;  // poses staged in LDS per launch
+constexpr int kFramesPerPass = 512;  // frames of one sweep; calls of more are several
 
 __global__ __launch_bounds__(256) void init_kernel(uint32_t* vol, int64_t n) {
   const uint32_t v = (uint32_t)(uint16_t)(int16_t)-32766;  // (-CU_VOXEL_MAX_TSDF, 0)
@@ -1255,8 +1255,11 @@ dim3 region_grid(IntegrateParams& P, int64_t b0, int64_t end) {
   return dim3((unsigned)region_workgroups(P.end_block - b0, P.log2_run));
 }
 // Eight regions of a block in a row for one XCD, where several frames are
-// swept over regions enough for that (runs of 16 and 32 8.9 ms, of 64 10.7: the
-// XCDs' shares of the surfaces become uneven).
+// swept over regions enough for that (300 frames, 512^3: runs of 16 and 32 8.9 ms,
+// of 64 10.7: the XCDs' shares of the surfaces become uneven).  One region and
+// eight, 100 640x480 frames, us: 96^3 (864 regions) 311 and 323, 160^3 (4,000) 468
+// and 454, 200^3 (8,750) 612 and 585, 256^3 766 and 790, 512^3 2635 and 2636; 16
+// frames, 96^3 52 and 57, 200^3 105 and 100.
 int region_runs(int64_t n, int K) { return K > 1 && n >= 4096 ? 3 : 0; }
 
 // Bricks above one another that a wave takes (their frames are tested

@@ -426,7 +426,7 @@ extern "C" int mcx_raycast(const void* d_vol, int X, int Y, int Z, float h, floa
   A.fy = intr[1];
   A.cx = intr[2];
   A.cy = intr[3];
-  if ((H + 15) / 16 > 65535) return MCX_ERR_ARG;
+  if ((H + 15) / 16 > 65535) return MCX_ERR_ARG;  // the entry point's limit of rows
   A.patches_x = (W + kPatch - 1) / kPatch;
   const int64_t patches = (int64_t)A.patches_x * ((H + kPatch - 1) / kPatch);
   if (patches >= ((int64_t)1 << 31)) return MCX_ERR_ARG;

@@ -190,7 +190,7 @@ __device__ __forceinline__ uint32_t record_bytes(uint32_t v) {
 }
 
 // Bytes of one record for each of a thread's run starts (no run inside a
-// block is longer than a record: kBlk <= kRunMax), and the slice's lead.
+// block is longer than a record: kEncBlk <= kRunMax), and the slice's lead.
 __device__ __forceinline__ uint32_t four_bytes(const Four& q, int64_t i0) {
   uint32_t b = i0 == 0 ? 4u : 0u;
 #pragma unroll
